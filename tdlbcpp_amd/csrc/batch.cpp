@@ -395,15 +395,16 @@ int build_plan(tdlb_batch* b, int64_t K, bool* structure_changed) {
         const int t = std::atoi(v);
         if (t >= 64 && t <= kForcePlaneBlock && t % 64 == 0) p.force_bs = t;
     }
-    // The force values of a solo plane stay in LDS through its levels when they
-    // fit a share of the CU's LDS that keeps the workgroups resident together
-    // that the registers allow (at most 128 VGPRs: 1024 lanes per CU); larger
-    // planes keep them in HBM.  All batch formats compute in 4-byte floats.
-    // The launch-sized LDS stays within 64 KB, which needs no kernel attribute.
+    // The force values (and moments) of a solo plane stay in LDS through its
+    // levels when they fit a share of the CU's LDS that keeps the workgroups
+    // resident together that the registers allow (at most 128 VGPRs: 1024 lanes
+    // per CU); larger planes keep them in HBM.  All batch formats compute in
+    // 4-byte floats.  The launch-sized LDS stays within 64 KB, which needs no
+    // kernel attribute.
     {
         const int64_t per_cu = std::max<int64_t>(1, kForcePlaneBlock / p.force_bs);
         const int64_t bytes = (int64_t)std::min<size_t>({kPlaneLdsBytes, kCuLdsBytes / (size_t)per_cu, 64 * 1024});
-        p.force_lds_cells = std::min<int64_t>(solo_cells, bytes / (3 * (int64_t)sizeof(float)));
+        p.force_lds_bytes = std::min<int64_t>(solo_cells * 7 * (int64_t)sizeof(float), bytes) / 16 * 16;
     }
     p.tot_coll = tot_coll;
     p.tot_rot = tot_rot;
@@ -415,7 +416,7 @@ int build_plan(tdlb_batch* b, int64_t K, bool* structure_changed) {
     // A captured step bakes in every launch size and kernel argument: recapture
     // whenever any of them differs (member identity alone is not enough, a freed
     // handle's address can come back for a tank of another size).
-    std::vector<int64_t> sig = {M, tot_coll, tot_rot, tot_words, p.n_tasks, p.bs, p.force_bs, p.force_lds_cells,
+    std::vector<int64_t> sig = {M, tot_coll, tot_rot, tot_words, p.n_tasks, p.bs, p.force_bs, p.force_lds_bytes,
                                 (int64_t)(uintptr_t)b->d_mem.p, (int64_t)(uintptr_t)b->d_tab.p,
                                 (int64_t)(uintptr_t)b->d_tasks.p, (int64_t)(uintptr_t)b->d_bm.p};
     *structure_changed = moved || sig != b->launch_sig || key != b->key || b->buffers_moved;

@@ -539,6 +539,29 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
     return TDLB_OK;
 }
 
+// Stencil rows of the static points (uploaded in plane order before) and room
+// for the blades'; the positions sidx are not needed after that.
+int build_rows(tdlb_cu* cu) {
+    IndexedSet& set = cu->static_set;
+    const size_t row = cu->tsize == 4 ? sizeof(ForceRow<float>) : sizeof(ForceRow<double>);
+    const size_t n = (size_t)(cu->n_static + cu->n_rot);
+    if (n == 0) return TDLB_OK;
+    std::vector<int32_t> plane_of_j((size_t)cu->yg, 0);
+    for (size_t t = 0; t < set.plane_list.size(); t++) plane_of_j[set.plane_list[t].j] = (int32_t)t;
+    int32_t* dj = nullptr;
+    if (hipMalloc(&set.rows, 3 * n * row) != hipSuccess) return fail(TDLB_ERR_NOMEM, "IB stencil rows");
+    if (hipMalloc((void**)&dj, plane_of_j.size() * 4) != hipSuccess) return fail(TDLB_ERR_NOMEM, "IB stencil rows");
+    hipError_t e = hipMemcpyAsync(dj, plane_of_j.data(), plane_of_j.size() * 4, hipMemcpyHostToDevice, cu->stream);
+    if (e == hipSuccess)
+        e = launch_static_rows(cu->eprec(), cu->pts.d, cu->n_static, set.sidx, set.planes, dj, set.rows, cu->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
+    (void)hipFree(dj);
+    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("IB stencil rows: ") + hipGetErrorString(e));
+    if (set.sidx) (void)hipFree(set.sidx);
+    set.sidx = nullptr;
+    return TDLB_OK;
+}
+
 // Whether this process's GPU can run the one-launch step: workgroups of a
 // launch must see every XCC id (each XCD's work queue needs workers); checked
 // once per device.  The step is opt-in (TDLB_PIPE=1): at 512^3 its rows run
@@ -694,7 +717,8 @@ int gen_blades(tdlb_cu* cu, double angle, double omega) {
     Rushton R(cu->rp);
     R.blade_trig(angle, st.cosb, st.sinb);
     st.omega = omega;
-    HIPCHK(launch_gen_blades(cu->prec(), cu->blade, st, cu->pts.d, cu->n_static, cu->stream));
+    HIPCHK(launch_gen_blades(cu->prec(), cu->blade, st, cu->pts.d, cu->static_set.rows, cu->g, cu->n_static,
+                             cu->stream));
     return TDLB_OK;
 }
 
@@ -1255,6 +1279,7 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     // blade colour classes never overlap (blade_colours: a colour per blade in small tanks)
     // blades are generated on the device at any angle: their whole swept disk and
     // the planes they occupy must lie inside the interior
+    bool wraps = false;  // a blade stencil may wrap to the other side of the tank
     {
         const double ro = p->blade_outer_radius;
         const double lo_i = std::floor(p->center_x - ro + 0.5), hi_i = std::floor(p->center_x + ro + 0.5);
@@ -1263,6 +1288,7 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
             p->blade_plane_lo < 0 || p->blade_plane_lo + p->blade_planes > cu->prm.y || p->blade_planes < 1 ||
             p->blade_inner_radius < 0)
             return fail(TDLB_ERR_INVALID, "impeller does not fit inside the ComputeUnit interior");
+        wraps = lo_i < 1 || hi_i > (double)(cu->prm.x - 2) || lo_k < 1 || hi_k > (double)(cu->prm.z - 2);
     }
 
     // main.cpp:277-303: increment for the current step, fixed, non-updating, rotating
@@ -1283,6 +1309,7 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     to_host_points(cu, stat.data(), order, hs);
     CHK(cu->pts.reserve(cu->n_static + cu->n_rot, cu->tsize));
     CHK(upload_points(cu, cu->pts, 0, hs));
+    CHK(build_rows(cu));
     if (cu->rot_cache) (void)hipFree(cu->rot_cache);
     cu->rot_cache = nullptr;
     if (cu->n_rot > 0 && hipMalloc(&cu->rot_cache, (size_t)cu->n_rot * 9 * 4 * cu->tsize) != hipSuccess)
@@ -1297,6 +1324,7 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     cu->blade.cx = p->center_x;
     cu->blade.cz = p->center_z;
     cu->blade.ghost = (int32_t)cu->prm.ghost;
+    cu->blade.merged = !wraps && blades_apart(p->n_blades, p->blade_inner_radius) ? 1 : 0;
     cu->rp = *p;
 
     // static occupancy bits: run the prepare kernel on an empty mask

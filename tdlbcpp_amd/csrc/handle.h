@@ -95,6 +95,7 @@ inline void set_q_geometry(Grid& g, int dlay, size_t ssize) {
 struct IndexedSet {
     uint32_t* cells = nullptr;
     int32_t* sidx = nullptr;
+    void* rows = nullptr;  // bound tank: ForceRow x 3 per static and blade point
     void* cache = nullptr;
     PlaneDesc* planes = nullptr;
     int64_t* lev_off = nullptr;
@@ -106,11 +107,12 @@ struct IndexedSet {
     std::vector<PlaneBlock> block_list;  // host copy of blocks
     std::vector<PlaneDesc> plane_list;   // host copy of planes
     void release() {
-        void* ptrs[] = {cells, sidx, cache, planes, lev_off, blocks, bar};
+        void* ptrs[] = {cells, sidx, rows, cache, planes, lev_off, blocks, bar};
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
         cells = nullptr;
         sidx = nullptr;
+        rows = nullptr;
         cache = nullptr;
         planes = nullptr;
         lev_off = nullptr;
@@ -183,7 +185,7 @@ struct tdlb_cu {
     IndexedSet static_set;               // stencil cells of the static points
     void* rot_cache = nullptr;           // 9 moment entries per blade point
     int64_t n_static = 0, n_rot = 0;
-    int32_t n_blade_classes = 0;         // blade colour classes (one forcing level each)
+    int32_t n_blade_classes = 0;         // blade colour classes of the generated list
     BladeLayout blade{};
     double alfa = 0.97, beta = 1.9;
 
@@ -235,7 +237,7 @@ struct tdlb_cu {
         f.n_static = n_static;
         f.n_rot = n_rot;
         f.cells = static_set.cells;
-        f.sidx = static_set.sidx;
+        f.rows = static_set.rows;
         f.scache = static_set.cache;
         f.rcache = rot_cache;
         f.planes = static_set.planes;

@@ -53,6 +53,7 @@ struct BladeLayout {
     double r_inner;          // radius of the first point; spacing 1
     double cx, cz;           // axis position (pre-ghost grid coordinates)
     int32_t ghost;
+    int32_t merged;          // 1: no two blades ever share a stencil cell (blades_apart)
 };
 struct BladeStep {
     double cosb[16], sinb[16];  // per-blade orientation this step
@@ -137,11 +138,21 @@ struct PlaneDesc {
 struct PlaneBlock {
     int32_t plane, rank;
 };
+// One row (k1 = c - 1) of a point's 3 x 3 stencil: what the forcing of a point
+// needs besides the flow, 32 bytes in FP32.  lane c of the point's quad loads
+// rows[3 q + c].
+template <typename T>
+struct alignas(16) ForceRow {
+    T w[3];        // weights of the cells i1 = -1, 0, 1
+    T vel;         // component c of the wall velocity
+    int32_t e[3];  // static point: the cells' entries in its plane's list; blade: their cell_index
+    int32_t pad;
+};
 struct ForceGeom {
     PointsDev pts;           // static points [0, n_static) plane by plane, level by level; blades after
     int64_t n_static, n_rot;
     const uint32_t* cells;   // unique static stencil cells, grouped by plane
-    const int32_t* sidx;     // per static point: the 9 positions of its stencil cells in cells
+    void* rows;              // ForceRow x 3 per point, static points first, blades after
     void* scache;            // {rho, jx, jy, jz} in T per entry of cells
     void* rcache;            // {rho, jx, jy, jz} in T x 9 per blade point
     const PlaneDesc* planes;
@@ -155,21 +166,14 @@ struct ForceGeom {
                              // (launches deal workgroups to the XCDs in turn)
 };
 constexpr int kBarWords = 4;
-// points one pass of a plane task handles: 16 wavefronts of 21 groups of 3 lanes
-constexpr int kForcePlanePoints = 336;
+// points one pass of a plane task handles: a quad of lanes per point
+constexpr int kForcePlanePoints = 256;
 constexpr int kForcePlaneBlock = 1024;  // threads of a plane task's workgroup, at most
 // LDS of a single tank's plane-task workgroup for the force values of a solo
 // plane's static cells: 8192 cells in FP32 (6570 per plane at 512^3).  The
 // workgroup's registers already hold a CU to one workgroup.
 constexpr size_t kPlaneLdsBytes = 96 * 1024;
 constexpr size_t kCuLdsBytes = 160 * 1024;  // LDS of a gfx950 CU
-// A single tank's plane keeps its force values in LDS only from this many
-// static cells on: with few planes per CU (tanks to about 256^3) the pass is
-// not bandwidth-bound and the copy in and out costs more than the levels save
-// (64 tanks of 48..160^3 one at a time: 3.5 % slower with every plane in LDS;
-// 512^3, 6570 cells per plane: 4.5 % faster).  Batches, whose thousands of
-// tasks keep every CU gathering, use LDS for every plane that fits.
-constexpr int64_t kPlaneLdsMinCells = 4096;
 // Workgroup of a batch's forcing planes for a mean of `cells` static stencil
 // cells per task: a lane per ~4 cells, a power of two from 128 to
 // kForcePlaneBlock lanes (batches of 48^3 tanks: 128 lanes 1.7x faster than
@@ -272,8 +276,13 @@ hipError_t launch_plane_xz(int prec, int layout, const void* Q, const void* F, c
 hipError_t launch_vorticity(int prec, int layout, int streaming, int momsrc, int even, const void* Q, const Grid& g,
                             int axis, int cut, const uint8_t* exclude, void* out, float rho0, hipStream_t s);
 
-hipError_t launch_gen_blades(int prec, const BladeLayout& bl, const BladeStep& st, const PointsDev& out,
-                             int64_t offset, hipStream_t s);
+// blade points of a step into out[offset ..], their stencil rows into rows[3 offset ..]
+hipError_t launch_gen_blades(int prec, const BladeLayout& bl, const BladeStep& st, const PointsDev& out, void* rows,
+                             const Grid& g, int64_t offset, hipStream_t s);
+// stencil rows of the n static points p, from the positions sidx (9 per point) of
+// their cells in the plane-grouped list; plane_of_j: index into planes of plane j
+hipError_t launch_static_rows(int prec, const PointsDev& p, int64_t n, const int32_t* sidx, const PlaneDesc* planes,
+                              const int32_t* plane_of_j, void* rows, hipStream_t s);
 hipError_t launch_solid_mask(double cx, double cz, double radius, uint8_t* out, const Grid& g, int ghost,
                              hipStream_t s);
 
@@ -330,7 +339,7 @@ struct BatchPlan {
     int64_t tot_coll, tot_rot, tot_words, n_tasks;
     int32_t bs;  // threads per block of the fused kernel (256 or 512)
     int32_t force_bs;  // threads per workgroup of the forcing pass (64 .. kForcePlaneBlock, a multiple of 64)
-    int64_t force_lds_cells;  // force values of a solo plane task kept in LDS, at most (0: none)
+    int64_t force_lds_bytes;  // LDS of a plane task's workgroup for force values and moments (0: none)
 };
 
 // Enqueue `steps` main-loop steps of every active member: per step blade

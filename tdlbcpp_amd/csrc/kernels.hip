@@ -1238,38 +1238,11 @@ __global__ __launch_bounds__(kBlock) void k_ib_moments_points(PointsDev p, int64
 constexpr int kGroup = 3;                    // lanes per point
 constexpr int kGroupsPerWave = 64 / kGroup;  // 21 points per wavefront, lane 63 idle
 
-// The inputs of stencil row c of point q, as loaded (force_point9 in two
-// parts, so that a pass can load the next pass's points while it computes).
-template <typename T>
-struct PointRaw {
-    int pi, pj, pk;
-    T ifr, kfr, u, v, w;
-    int64_t e[3];  // cache entries of the row's cells
-};
-template <typename T, bool INDEXED>
-__device__ __forceinline__ PointRaw<T> point_raw(const PointsDev& p, int64_t q, bool valid, int c,
-                                                 const int32_t* __restrict__ sidx, int64_t cache_base) {
-    PointRaw<T> r{};
-    if (valid) {
-        r.pi = p.i[q];
-        r.pj = p.j[q];
-        r.pk = p.k[q];
-        r.ifr = static_cast<const T*>(p.ifrac)[q];
-        r.kfr = static_cast<const T*>(p.kfrac)[q];
-        r.u = static_cast<const T*>(p.u)[q];
-        r.v = static_cast<const T*>(p.v)[q];
-        r.w = static_cast<const T*>(p.w)[q];
-#pragma unroll
-        for (int m = 0; m < 3; m++)
-            r.e[m] = INDEXED ? (int64_t)sidx[9 * q + 3 * c + m] : 9 * (q - cache_base) + 3 * c + m;
-    }
-    return r;
-}
-
-template <typename T, typename D>
-__device__ __forceinline__ void force_point9_raw(const PointRaw<T>& r, bool valid, int c, int base,
-                                                 const Mom4<T>* __restrict__ cache, T* __restrict__ F, const Grid& g,
-                                                 T alfa, T beta) {
+template <typename T, typename D, bool INDEXED>
+__device__ __forceinline__ void force_point9(const PointsDev& p, int64_t q, bool valid, int c, int base,
+                                             const int32_t* __restrict__ sidx, int64_t cache_base,
+                                             const Mom4<T>* __restrict__ cache, T* __restrict__ F, const Grid& g,
+                                             T alfa, T beta) {
     T w[3], tr[3], tx[3], ty[3], tz[3], fo[3][3];
     uint64_t cell[3];
 #pragma unroll
@@ -1278,21 +1251,22 @@ __device__ __forceinline__ void force_point9_raw(const PointRaw<T>& r, bool vali
         cell[m] = 0;
     }
     if (valid) {
-        const T wk = ib_weight<T>(-r.kfr + T(c - 1));
-        const int k2 = wrap_ik(r.pk + c - 1, g.zg1);
+        const T ifr = static_cast<const T*>(p.ifrac)[q], kfr = static_cast<const T*>(p.kfrac)[q];
+        const T wk = ib_weight<T>(-kfr + T(c - 1));
+        const int pi = p.i[q], pj = p.j[q], k2 = wrap_ik(p.k[q] + c - 1, g.zg1);
         Mom4<T> mo[3];
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            const int i2 = wrap_ik(r.pi + m - 1, g.xg1);
-            cell[m] = cell_index(g, i2, r.pj, k2);
-            mo[m] = cache[r.e[m]];
+            const int i2 = wrap_ik(pi + m - 1, g.xg1);
+            cell[m] = cell_index(g, i2, pj, k2);
+            mo[m] = cache[INDEXED ? (int64_t)sidx[9 * q + 3 * c + m] : 9 * (q - cache_base) + 3 * c + m];
             fo[m][0] = F[3 * cell[m] + 0];
             fo[m][1] = F[3 * cell[m] + 1];
             fo[m][2] = F[3 * cell[m] + 2];
         }
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            w[m] = ib_weight<T>(-r.ifr + T(m - 1)) * wk;
+            w[m] = ib_weight<T>(-ifr + T(m - 1)) * wk;
             const T xx = (T)((D)mo[m].x + D(0.5) * (D)fo[m][0]);
             const T yy = (T)((D)mo[m].y + D(0.5) * (D)fo[m][1]);
             const T zz = (T)((D)mo[m].z + D(0.5) * (D)fo[m][2]);
@@ -1314,9 +1288,9 @@ __device__ __forceinline__ void force_point9_raw(const PointRaw<T>& r, bool vali
             zSum += __shfl(tz[m], base + c2, 64);
         }
     if (!valid) return;
-    xSum -= rhoSum * r.u;
-    ySum -= rhoSum * r.v;
-    zSum -= rhoSum * r.w;
+    xSum -= rhoSum * static_cast<const T*>(p.u)[q];
+    ySum -= rhoSum * static_cast<const T*>(p.v)[q];
+    zSum -= rhoSum * static_cast<const T*>(p.w)[q];
 #pragma unroll
     for (int m = 0; m < 3; m++) {
         const T bp = beta * w[m];
@@ -1324,74 +1298,6 @@ __device__ __forceinline__ void force_point9_raw(const PointRaw<T>& r, bool vali
         F[3 * cell[m] + 1] = alfa * fo[m][1] - bp * ySum;
         F[3 * cell[m] + 2] = alfa * fo[m][2] - bp * zSum;
     }
-}
-
-// force_point9_raw with the row's force values in LDS: entry e of the
-// plane's static cells at lds[3 (e - cb)], the same arithmetic in the same order.
-template <typename T, typename D>
-__device__ __forceinline__ void force_point9_lds(const PointRaw<T>& r, bool valid, int c, int base,
-                                                 const Mom4<T>* __restrict__ cache, T* lds, int64_t cb, T alfa,
-                                                 T beta) {
-    T w[3], tr[3], tx[3], ty[3], tz[3], fo[3][3];
-    int li[3];
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-        w[m] = tr[m] = tx[m] = ty[m] = tz[m] = fo[m][0] = fo[m][1] = fo[m][2] = T(0);
-        li[m] = 0;
-    }
-    if (valid) {
-        const T wk = ib_weight<T>(-r.kfr + T(c - 1));
-        Mom4<T> mo[3];
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            li[m] = 3 * (int)(r.e[m] - cb);
-            mo[m] = cache[r.e[m]];
-            fo[m][0] = lds[li[m] + 0];
-            fo[m][1] = lds[li[m] + 1];
-            fo[m][2] = lds[li[m] + 2];
-        }
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            w[m] = ib_weight<T>(-r.ifr + T(m - 1)) * wk;
-            const T xx = (T)((D)mo[m].x + D(0.5) * (D)fo[m][0]);
-            const T yy = (T)((D)mo[m].y + D(0.5) * (D)fo[m][1]);
-            const T zz = (T)((D)mo[m].z + D(0.5) * (D)fo[m][2]);
-            tr[m] = w[m] * mo[m].r;
-            tx[m] = w[m] * xx;
-            ty[m] = w[m] * yy;
-            tz[m] = w[m] * zz;
-        }
-    }
-    T rhoSum = T(0.0), xSum = T(0.0), ySum = T(0.0), zSum = T(0.0);
-#pragma unroll
-    for (int c2 = 0; c2 < kGroup; c2++)
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            rhoSum += __shfl(tr[m], base + c2, 64);
-            xSum += __shfl(tx[m], base + c2, 64);
-            ySum += __shfl(ty[m], base + c2, 64);
-            zSum += __shfl(tz[m], base + c2, 64);
-        }
-    if (!valid) return;
-    xSum -= rhoSum * r.u;
-    ySum -= rhoSum * r.v;
-    zSum -= rhoSum * r.w;
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-        const T bp = beta * w[m];
-        lds[li[m] + 0] = alfa * fo[m][0] - bp * xSum;
-        lds[li[m] + 1] = alfa * fo[m][1] - bp * ySum;
-        lds[li[m] + 2] = alfa * fo[m][2] - bp * zSum;
-    }
-}
-
-template <typename T, typename D, bool INDEXED>
-__device__ __forceinline__ void force_point9(const PointsDev& p, int64_t q, bool valid, int c, int base,
-                                             const int32_t* __restrict__ sidx, int64_t cache_base,
-                                             const Mom4<T>* __restrict__ cache, T* __restrict__ F, const Grid& g,
-                                             T alfa, T beta) {
-    const PointRaw<T> r = point_raw<T, INDEXED>(p, q, valid, c, sidx, cache_base);
-    force_point9_raw<T, D>(r, valid, c, base, cache, F, g, alfa, beta);
 }
 
 // lane -> (point index within the launch, stencil row, group base lane)
@@ -1426,15 +1332,15 @@ __global__ __launch_bounds__(kBlock) void k_force_level_cached(PointsDev p, int6
 // kernels.h).  A task first clears F and sets the occupancy bit of the blade
 // stencil cells missing from the previous mask (prepare_point) and computes the
 // density and momentum of its static and blade stencil cells; then it runs its
-// static levels and its blade colour classes in order, passes of up to
-// kPlanePoints points per workgroup, 3 lanes per point (force_point9), with a
-// barrier after every level: the sequential list order of Forcing.hpp:73-135
-// within the plane, without a kernel launch per level.  A plane with many
+// static levels and its blade levels in order, passes of up to kPlanePoints
+// points per workgroup, a quad of lanes per point (force_row), with a barrier
+// after every level: the sequential list order of Forcing.hpp:73-135 within the
+// plane, without a kernel launch per level.  A plane with many
 // points runs on a team of workgroups that meet at a barrier in global memory
 // (team_barrier); teams are the first workgroups of the launch, so they are
 // dispatched, and resident, before any other workgroup of it.
 constexpr int kPlaneBlock = kForcePlaneBlock;
-constexpr int kPlanePoints = (kPlaneBlock / 64) * kGroupsPerWave;
+constexpr int kPlanePoints = kPlaneBlock / 4;
 static_assert(kPlanePoints == kForcePlanePoints, "points per pass of a plane task");
 // polls of a team barrier before it gives up and flags a time-out (about a
 // second; every member of a team is resident, so a healthy barrier takes
@@ -1495,20 +1401,113 @@ __device__ __forceinline__ void team_barrier(uint32_t* bar, int team, bool local
     if (local) asm volatile("buffer_inv sc1" ::: "memory");
 }
 
-// lane -> point slot of a pass (wave-major, 21 groups of 3 lanes per wave), -1 for lane 63
-__device__ __forceinline__ int plane_slot(int& c, int& base) {
-    const int lane = (int)(threadIdx.x & 63), grp = lane / kGroup;
-    c = lane - grp * kGroup;
-    base = grp * kGroup;
-    return grp < kGroupsPerWave ? (int)(threadIdx.x >> 6) * kGroupsPerWave + grp : -1;
+// ---- A point of a plane task on a quad of lanes: lane c = 0..2 of the quad
+// takes stencil row k1 = c - 1 (cells s = 3c + m for i1 = m - 1), lane 3 repeats
+// row 2 and writes nothing.  Everything of the row that does not depend on the
+// flow is in its ForceRow (weights, wall velocity, stencil entries), laid out
+// once for the static points and once a step for the blades, so a pass is two
+// 16-byte loads, the gather, the sums and the spread.  The nine terms are added
+// in the reference's order (s = 0..8) by every lane, each term taken from its
+// lane of the quad as a DPP operand of the add: no LDS traffic and no latency
+// beyond the add's own.  A level is a chain (gather, sums, spread, barrier) of a
+// few hundred lanes, bound by latency: three lanes per point with LDS shuffles
+// and the weights' FP64 square roots in every pass took about 9 us a level,
+// this form 1 us with the plane in LDS.  Whole forcing pass of a tank, FP32:
+// 36^3 68 -> 37 us, 60^3 80 -> 41, 96^3 91 -> 47, 256^3 290 -> 226, 512^3 633 -> 597.
+template <int C>
+__device__ __forceinline__ float quad_lane(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), C * 0x55, 0xf, 0xf, true));
+}
+template <int C>
+__device__ __forceinline__ double quad_lane(double x) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(x), C * 0x55, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(x), C * 0x55, 0xf, 0xf, true));
+}
+template <int C, typename T>
+__device__ __forceinline__ void quad_add(T& sum, const T (&t)[3]) {
+#pragma unroll
+    for (int m = 0; m < 3; m++) sum += quad_lane<C>(t[m]);
+}
+template <typename T>
+__device__ __forceinline__ T quad_sum(const T (&t)[3]) {
+    T sum = T(0.0);
+    quad_add<0>(sum, t);
+    quad_add<1>(sum, t);
+    quad_add<2>(sum, t);
+    return sum;
+}
+// j + 0.5 F rounded once, which is what the reference's double sum rounded to T
+// gives: exact for T = double, and for T = float a sum of two floats rounded
+// first to 53 and then to 24 bits is the correctly rounded sum (53 >= 2 * 24 + 2)
+__device__ __forceinline__ float add_half(float j, float f) { return fmaf(0.5f, f, j); }
+__device__ __forceinline__ double add_half(double j, double f) { return j + 0.5 * f; }
+
+// the row's nine terms, the point's sums and the row's new force values (f in place)
+template <typename T>
+__device__ __forceinline__ void force_row(const ForceRow<T>& r, const Mom4<T> (&mo)[3], T (&f)[3][3], T alfa, T beta) {
+    T tr[3], tx[3], ty[3], tz[3];
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        tr[m] = r.w[m] * mo[m].r;
+        tx[m] = r.w[m] * add_half(mo[m].x, f[m][0]);
+        ty[m] = r.w[m] * add_half(mo[m].y, f[m][1]);
+        tz[m] = r.w[m] * add_half(mo[m].z, f[m][2]);
+    }
+    const T rho = quad_sum(tr);
+    T x = quad_sum(tx), y = quad_sum(ty), z = quad_sum(tz);
+    x -= rho * quad_lane<0>(r.vel);
+    y -= rho * quad_lane<1>(r.vel);
+    z -= rho * quad_lane<2>(r.vel);
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        const T bp = beta * r.w[m];
+        f[m][0] = alfa * f[m][0] - bp * x;
+        f[m][1] = alfa * f[m][1] - bp * y;
+        f[m][2] = alfa * f[m][2] - bp * z;
+    }
 }
 
-// Blade colour class c of the generator's colour-major list (rushton.h
-// blade_decode): its first list index, blades and radial points; point
-// (blade bi, plane bp, radial ri) of the class is at base + (bi * planes + bp) * nr + ri.
-struct BladeClass {
-    int64_t base;
-    int nb, nr;
+// stencil row c of a point: weights as ib_weight gives them in the point's own
+// precision, component c of its wall velocity
+template <typename T>
+__device__ __forceinline__ ForceRow<T> make_row(T ifr, T kfr, int c, T vel) {
+    ForceRow<T> r;
+    const T wk = ib_weight<T>(-kfr + T(c - 1));
+#pragma unroll
+    for (int m = 0; m < 3; m++) r.w[m] = ib_weight<T>(-ifr + T(m - 1)) * wk;
+    r.vel = vel;
+    r.pad = 0;
+    return r;
+}
+
+// ForceRow of every static point: e[m] = the cell's entry in its plane's list
+// (cell_of maps the point to its plane's first entry)
+template <typename T>
+__global__ void k_static_rows(PointsDev p, int64_t n, const int32_t* __restrict__ sidx,
+                              const PlaneDesc* __restrict__ planes, const int32_t* __restrict__ plane_of_j,
+                              ForceRow<T>* __restrict__ rows) {
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t >= 3 * n) return;
+    const int64_t q = t / 3;
+    const int c = (int)(t - 3 * q);
+    const T* vel = static_cast<const T*>(c == 0 ? p.u : c == 1 ? p.v : p.w);
+    ForceRow<T> r = make_row<T>(static_cast<const T*>(p.ifrac)[q], static_cast<const T*>(p.kfrac)[q], c, vel[q]);
+    const int64_t first = planes[plane_of_j[p.j[q]]].cell_begin;
+#pragma unroll
+    for (int m = 0; m < 3; m++) r.e[m] = (int32_t)(sidx[9 * q + 3 * c + m] - first);
+    rows[t] = r;
+}
+
+// Blade levels of a plane.  The generator's list is colour-major (rushton.h
+// blade_decode): classes (blade colour, radial index mod 5) of points that never
+// share a stencil cell.  Blades at least 3 sqrt(2) cells apart at the inner
+// radius never share one either, so one level then takes all blades' points of a
+// radial class (5 levels, merged); in smaller tanks a level is one class.
+struct BladeLevel {
+    BladeEnum e;
+    int rmod, nr;        // radial class and its points per blade
+    int first, stride;   // blades first, first + stride, ...
+    int count;           // points of the level on one plane
 };
 __device__ __forceinline__ BladeEnum blade_enum_of(const BladeLayout& bl) {
     BladeEnum e;
@@ -1518,19 +1517,37 @@ __device__ __forceinline__ BladeEnum blade_enum_of(const BladeLayout& bl) {
     e.n_bcol = bl.n_bcol;
     return e;
 }
-__device__ __forceinline__ BladeClass blade_class(const BladeEnum& e, int c, int64_t base) {
-    const int bcol = c / 5, rmod = c % 5;
-    BladeClass bc;
-    bc.base = base;
-    bc.nb = e.n_blades > bcol ? (e.n_blades - bcol + e.n_bcol - 1) / e.n_bcol : 0;
-    bc.nr = e.n_radial > rmod ? (e.n_radial - rmod + 4) / 5 : 0;
-    return bc;
+__device__ __forceinline__ BladeLevel blade_level(const BladeLayout& bl, int l) {
+    BladeLevel v;
+    v.e = blade_enum_of(bl);
+    v.rmod = l % 5;
+    v.nr = v.e.n_radial > v.rmod ? (v.e.n_radial - v.rmod + 4) / 5 : 0;
+    v.first = bl.merged ? 0 : l / 5;
+    v.stride = bl.merged ? 1 : v.e.n_bcol;
+    const int nb = v.e.n_blades > v.first ? (v.e.n_blades - v.first + v.stride - 1) / v.stride : 0;
+    v.count = nb * v.nr;
+    return v;
 }
-// blade plane index of plane j (ghost included) and its colour classes (0: no blades)
-__device__ __forceinline__ int blade_plane(const ForceGeom& fg, int j, int& ncls) {
+// list index of radial point r of blade b on blade plane bp
+__device__ __forceinline__ int blade_index(const BladeEnum& e, int b, int r, int bp) {
+    const int bcol = b % e.n_bcol, bi = b / e.n_bcol, rmod = r % 5;
+    const int nb = (e.n_blades - bcol + e.n_bcol - 1) / e.n_bcol;
+    int before = 0;  // points per plane of the colours before bcol, then of this colour's radial classes before rmod
+    for (int a = 0; a < bcol; a++) before += (e.n_blades - a + e.n_bcol - 1) / e.n_bcol;
+    before *= e.n_radial;
+    for (int a = 0; a < rmod; a++) before += nb * (e.n_radial > a ? (e.n_radial - a + 4) / 5 : 0);
+    return before * e.n_planes + (bi * e.n_planes + bp) * ((e.n_radial - rmod + 4) / 5) + r / 5;
+}
+// list index of point t of the level on blade plane bp
+__device__ __forceinline__ int level_index(const BladeLevel& v, int t, int bp) {
+    const int s = t / v.nr, ri = t - s * v.nr;
+    return blade_index(v.e, v.first + s * v.stride, v.rmod + 5 * ri, bp);
+}
+// blade plane index of plane j and its blade levels (0: no blades)
+__device__ __forceinline__ int blade_plane(const ForceGeom& fg, int j, int& nlev) {
     const BladeLayout& bl = fg.blade;
     const int bp = j - bl.ghost - bl.j_lo;
-    ncls = (bl.n_blades > 0 && fg.n_rot > 0 && bp >= 0 && bp < bl.n_planes) ? 5 * blade_enum_of(bl).n_bcol : 0;
+    nlev = (bl.n_blades > 0 && fg.n_rot > 0 && bp >= 0 && bp < bl.n_planes) ? (bl.merged ? 5 : 5 * bl.n_bcol) : 0;
     return bp;
 }
 
@@ -1554,162 +1571,236 @@ __device__ __forceinline__ void gather_cells(const ForceGeom& fg, int64_t c0, in
 // previous mask lacks the cell (prepare_point), density and momentum into the
 // blade cache.
 template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
-__device__ void gather_blades(const ForceGeom& fg, int j, int64_t t0, int64_t threads,
+__device__ void gather_blades(const ForceGeom& fg, int j, int t0, int threads,
                               const typename PR::S* __restrict__ Q, typename PR::T* __restrict__ F,
                               const uint64_t* __restrict__ prev, uint64_t* __restrict__ next, const Grid& g,
                               float rho0) {
     using T = typename PR::T;
     auto* rcache = static_cast<Mom4<T>*>(fg.rcache);
-    int ncls;
-    const int bp = blade_plane(fg, j, ncls);
+    int nlev;
+    const int bp = blade_plane(fg, j, nlev);
+    if (nlev == 0) return;
     const BladeEnum be = blade_enum_of(fg.blade);
-    int64_t base = 0;
-    for (int c = 0; c < ncls; c++) {
-        const BladeClass bc = blade_class(be, c, base);
-        const int64_t n9 = 9 * (int64_t)bc.nb * bc.nr;
-        for (int64_t t = t0; t < n9; t += threads) {
-            const int64_t pt = t / 9;
-            const int s = (int)(t - 9 * pt);
-            const int bi = (int)(pt / bc.nr), ri = (int)(pt - (int64_t)bi * bc.nr);
-            const int64_t e = bc.base + ((int64_t)bi * fg.blade.n_planes + bp) * bc.nr + ri;
-            const int64_t q = fg.n_static + e;
-            const int pj = fg.pts.j[q];
-            const int i2 = wrap_ik(fg.pts.i[q] + (s % 3) - 1, g.xg1), k2 = wrap_ik(fg.pts.k[q] + (s / 3) - 1, g.zg1);
-            if (!mask_test(prev, g, i2, pj, k2)) {
-                const uint64_t cc = cell_index(g, i2, pj, k2);
-                F[3 * cc + 0] = T(0);
-                F[3 * cc + 1] = T(0);
-                F[3 * cc + 2] = T(0);
-            }
-            atomicOr((unsigned long long*)&next[mask_word_index(g, i2, pj, k2)], 1ull << (k2 & 63));
-            Mom4<T> m;
-            cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i2, pj, k2, m.r, m.x, m.y, m.z, rho0);
-            rcache[9 * e + s] = m;
+    const int n9 = 9 * be.n_blades * be.n_radial;
+    for (int t = t0; t < n9; t += threads) {
+        const int pt = t / 9, s = t - 9 * pt;
+        const int b = pt / be.n_radial, e = blade_index(be, b, pt - b * be.n_radial, bp);
+        const int64_t q = fg.n_static + e;
+        const int i2 = wrap_ik(fg.pts.i[q] + (s % 3) - 1, g.xg1), k2 = wrap_ik(fg.pts.k[q] + (s / 3) - 1, g.zg1);
+        if (!mask_test(prev, g, i2, j, k2)) {
+            const uint64_t cc = cell_index(g, i2, j, k2);
+            F[3 * cc + 0] = T(0);
+            F[3 * cc + 1] = T(0);
+            F[3 * cc + 2] = T(0);
         }
-        base += blade_class_size(be, c);
+        atomicOr((unsigned long long*)&next[mask_word_index(g, i2, j, k2)], 1ull << (k2 & 63));
+        Mom4<T> m;
+        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i2, j, k2, m.r, m.x, m.y, m.z, rho0);
+        rcache[9 * (int64_t)e + s] = m;
     }
 }
 
-// The plane's static levels, then its blade colour classes, by workgroup
-// `rank` of a team of `team` (passes of (blockDim.x / 64) * 7 points), with
-// sync() after every level.
-template <typename T, typename D, typename Sync>
-__device__ void plane_levels(const ForceGeom& fg, const PlaneDesc& pd, int rank, int team, T* __restrict__ F,
-                             const Grid& g, T alfa, T beta, Sync&& sync, T* lds = nullptr) {
-    if constexpr (sizeof(T) > 4) lds = nullptr;  // FP64: the registers of the LDS form spill
-    const auto* scache = static_cast<const Mom4<T>*>(fg.scache);
-    const auto* rcache = static_cast<const Mom4<T>*>(fg.rcache);
-    int row, gbase;
-    const int slot = plane_slot(row, gbase);
-    const int64_t per = (int64_t)(blockDim.x >> 6) * kGroupsPerWave;
-    const int64_t p0 = (int64_t)rank * per, pstride = (int64_t)team * per;
-    // Each pass loads the next pass's points (positions, fractions, velocities,
-    // cache entries) before it computes: the point lists do not change during
-    // the pass.  Every static level ends with one sync(), also a level this
-    // workgroup has no pass in.
+// The plane's static levels by workgroup `rank` of a team of `team`, passes of a
+// point per quad of lanes, with sync() after every level.  Each pass loads the
+// next pass's rows before it computes (the rows do not change during the pass).
+// lm: the moments, by entry of the plane, in LDS or the cache in HBM; lf: the
+// force values by entry in LDS, or null: in F.
+template <typename T, typename Sync>
+__device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDesc& pd, int rank, int team,
+                                              const Mom4<T>* lm, T* lf, T* __restrict__ F, T alfa, T beta,
+                                              Sync&& sync) {
+    const ForceRow<T>* __restrict__ rows = static_cast<const ForceRow<T>*>(fg.rows);
+    const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), c = min(lane, 2);
+    const int per = (int)(blockDim.x >> 2), p0 = rank * per, pstride = team * per;
     const int nlev = pd.n_levels;
-    auto lev_end = [&](int lv) { return fg.lev_off[pd.lev + lv + 1]; };
-    auto first = [&](int lv) { return fg.lev_off[pd.lev + lv] + p0; };
-    auto raw_at = [&](int lv, int64_t qq) {
-        const bool ok = lv < nlev && slot >= 0 && qq + slot < lev_end(lv);
-        return point_raw<T, true>(fg.pts, ok ? qq + slot : 0, ok, row, fg.sidx, 0);
+    const int64_t* __restrict__ off = fg.lev_off + pd.lev;
+    struct Pass {
+        ForceRow<T> r;
+        uint32_t cell[3];  // cell_index of the entries (force values in F only)
+        bool ok;
     };
-    int l = 0;
-    while (l < nlev && first(l) >= lev_end(l)) {
-        sync();
-        l++;
-    }
-    int64_t q = l < nlev ? first(l) : 0;
-    PointRaw<T> cur = raw_at(l, q);
+    auto load = [&](int l, int64_t q) {
+        Pass a{};
+        a.ok = l < nlev && q + slot < off[l + 1];
+        if (a.ok) {
+            a.r = rows[3 * (q + slot) + c];
+            if (!lf)
+#pragma unroll
+                for (int m = 0; m < 3; m++) a.cell[m] = fg.cells[pd.cell_begin + a.r.e[m]];
+        }
+        return a;
+    };
+    // the first pass of this workgroup at or after level l: empty levels still end with a sync
+    auto skip = [&](int l) {
+        while (l < nlev && off[l] + p0 >= off[l + 1]) l++;
+        return l;
+    };
+    int l = skip(0);
+    for (int k = 0; k < l; k++) sync();
+    int64_t q = l < nlev ? off[l] + p0 : 0;
+    Pass cur = load(l, q);
     while (l < nlev) {
-        // the next pass of this workgroup: later in level l, else the first of the next level that has one
         int nl = l;
         int64_t nq = q + pstride;
-        if (nq >= lev_end(l)) {
-            nl = l + 1;
-            while (nl < nlev && first(nl) >= lev_end(nl)) nl++;
-            nq = nl < nlev ? first(nl) : 0;
+        if (nq >= off[l + 1]) {
+            nl = skip(l + 1);
+            nq = nl < nlev ? off[nl] + p0 : 0;
         }
-        const PointRaw<T> nxt = raw_at(nl, nq);
-        if (lds)
-            force_point9_lds<T, D>(cur, slot >= 0 && q + slot < lev_end(l), row, gbase, scache, lds, pd.cell_begin,
-                                   alfa, beta);
-        else
-            force_point9_raw<T, D>(cur, slot >= 0 && q + slot < lev_end(l), row, gbase, scache, F, g, alfa, beta);
+        const Pass nxt = load(nl, nq);
+        if (cur.ok) {
+            Mom4<T> mo[3];
+            T f[3][3];
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                const T* fp = lf ? lf + 3 * cur.r.e[m] : F + 3 * (uint64_t)cur.cell[m];
+                mo[m] = lm[cur.r.e[m]];
+                f[m][0] = fp[0];
+                f[m][1] = fp[1];
+                f[m][2] = fp[2];
+            }
+            force_row(cur.r, mo, f, alfa, beta);
+            if (lane < 3)
+#pragma unroll
+                for (int m = 0; m < 3; m++) {
+                    T* fp = lf ? lf + 3 * cur.r.e[m] : F + 3 * (uint64_t)cur.cell[m];
+                    fp[0] = f[m][0];
+                    fp[1] = f[m][1];
+                    fp[2] = f[m][2];
+                }
+        }
         for (int k = l; k < nl; k++) sync();  // levels l .. nl - 1 are done
         l = nl;
         q = nq;
         cur = nxt;
     }
-    if (lds) {
-        // the static levels are done (each ended with a barrier): their force
-        // values back to F before the blade classes read it
-        for (int64_t e = threadIdx.x; e < pd.cell_end - pd.cell_begin; e += blockDim.x) {
-            const uint64_t cc = fg.cells[pd.cell_begin + e];  // cell_index of the entry
-            F[3 * cc + 0] = lds[3 * e + 0];
-            F[3 * cc + 1] = lds[3 * e + 1];
-            F[3 * cc + 2] = lds[3 * e + 2];
+}
+
+// The plane's blade levels, as static_levels: force values in F, moments in the
+// blade cache, the next level's rows and moments loaded a level ahead.
+template <typename T, typename Sync>
+__device__ __forceinline__ void blade_levels(const ForceGeom& fg, int j, int rank, int team, T* __restrict__ F,
+                                             T alfa, T beta, Sync&& sync) {
+    int nlev;
+    const int bp = blade_plane(fg, j, nlev);
+    if (nlev == 0) return;
+    const ForceRow<T>* __restrict__ rows = static_cast<const ForceRow<T>*>(fg.rows) + 3 * fg.n_static;
+    const Mom4<T>* __restrict__ cache = static_cast<const Mom4<T>*>(fg.rcache);
+    const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), c = min(lane, 2);
+    const int per = (int)(blockDim.x >> 2), p0 = rank * per, pstride = team * per;
+    struct Pass {
+        ForceRow<T> r;
+        Mom4<T> mo[3];
+        bool ok;
+    };
+    auto load = [&](int l, int t) {
+        Pass a{};
+        if (l >= nlev) return a;
+        const BladeLevel v = blade_level(fg.blade, l);
+        a.ok = t < v.count;
+        if (a.ok) {
+            const int64_t e = level_index(v, t, bp);
+            a.r = rows[3 * e + c];
+#pragma unroll
+            for (int m = 0; m < 3; m++) a.mo[m] = cache[9 * e + 3 * c + m];
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-    }
-    int ncls;
-    const int bp = blade_plane(fg, pd.j, ncls);
-    const BladeEnum be = blade_enum_of(fg.blade);
-    int64_t base = 0;
-    for (int c = 0; c < ncls; c++) {
-        const BladeClass bc = blade_class(be, c, base);
-        const int64_t n = (int64_t)bc.nb * bc.nr;
-        for (int64_t u0 = p0; u0 < n; u0 += pstride) {
-            const int64_t t = u0 + slot;
-            const bool valid = slot >= 0 && t < n;
-            int64_t qb = fg.n_static;
-            if (valid) {
-                const int bi = (int)(t / bc.nr), ri = (int)(t - (int64_t)bi * bc.nr);
-                qb += bc.base + ((int64_t)bi * fg.blade.n_planes + bp) * bc.nr + ri;
+        return a;
+    };
+    auto count = [&](int l) { return blade_level(fg.blade, l).count; };
+    int l = 0, u = p0;
+    Pass cur = load(0, u + slot);
+    while (l < nlev) {
+        int nl = l, nu = u + pstride;
+        if (nu >= count(l)) {
+            nl = l + 1;
+            nu = p0;
+        }
+        const Pass nxt = load(nl, nu + slot);
+        if (cur.ok) {
+            T f[3][3];
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                const T* fp = F + 3 * (uint64_t)(uint32_t)cur.r.e[m];
+                f[m][0] = fp[0];
+                f[m][1] = fp[1];
+                f[m][2] = fp[2];
             }
-            force_point9<T, D, false>(fg.pts, qb, valid, row, gbase, nullptr, fg.n_static, rcache, F, g, alfa, beta);
+            force_row(cur.r, cur.mo, f, alfa, beta);
+            if (lane < 3)
+#pragma unroll
+                for (int m = 0; m < 3; m++) {
+                    T* fp = F + 3 * (uint64_t)(uint32_t)cur.r.e[m];
+                    fp[0] = f[m][0];
+                    fp[1] = f[m][1];
+                    fp[2] = f[m][2];
+                }
         }
-        sync();
-        base += blade_class_size(be, c);
+        if (nl != l) sync();
+        l = nl;
+        u = nu;
+        cur = nxt;
     }
 }
 
-// workgroup `rank` of the plane's team
+// Workgroup `rank` of the plane's team.  A solo plane whose static cells fit
+// keeps their force values in LDS through the static levels, and their moments
+// too when both fit (every stencil cell of a plane task lies in its own plane,
+// which no other task touches): a level then waits on LDS alone.  The blade
+// cells' zeroing does not reach a static cell that holds a force value: the
+// static cells are in the previous mask, or were cleared before the pass.
 template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
 __device__ void force_plane(const ForceGeom& fg, const PlaneDesc& pd, int rank,
                             const typename PR::S* __restrict__ Q, typename PR::T* __restrict__ F,
                             const uint64_t* __restrict__ prev, uint64_t* __restrict__ next, const Grid& g,
-                            typename PR::T alfa, typename PR::T beta, float rho0,
-                            typename PR::T* lds_buf = nullptr, int64_t lds_cells = 0, int64_t lds_min = 0) {
+                            typename PR::T alfa, typename PR::T beta, float rho0, void* lds_buf, int64_t lds_bytes) {
+    using T = typename PR::T;
     const int team = pd.team;
     uint32_t* bar = team > 1 ? fg.bar + kBarWords * pd.bar : nullptr;
-    const int64_t t0 = (int64_t)rank * blockDim.x + threadIdx.x, threads = (int64_t)team * blockDim.x;
+    const int t0 = rank * (int)blockDim.x + (int)threadIdx.x, threads = team * (int)blockDim.x;
     const bool local = fg.local_teams != 0;
     auto sync = [&]() {
         if (team > 1) team_barrier(bar, team, local);
         else __syncthreads();
     };
-    gather_cells<PR, L, STREAM, MOMSRC, EVEN>(fg, pd.cell_begin, pd.cell_end, t0, threads, Q, g, rho0);
+    const int nc = (int)(pd.cell_end - pd.cell_begin);
+    const int64_t mom_bytes = (int64_t)nc * sizeof(Mom4<T>), f_bytes = (int64_t)nc * 3 * sizeof(T);
+    const bool in_lds = lds_buf && team == 1 && f_bytes <= lds_bytes;
+    const bool mom_lds = in_lds && mom_bytes + f_bytes <= lds_bytes;
+    auto* gm = static_cast<Mom4<T>*>(fg.scache) + pd.cell_begin;
+    auto* lm = static_cast<Mom4<T>*>(lds_buf);
+    T* lf = mom_lds ? reinterpret_cast<T*>(lm + nc) : static_cast<T*>(lds_buf);
+    const uint32_t* __restrict__ cells = fg.cells + pd.cell_begin;
+    for (int e = t0; e < nc; e += threads) {
+        const uint32_t n = cells[e];
+        const int i = (int)(n / g.yz), k = (int)(n - (uint32_t)i * g.yz - (uint32_t)pd.j * (uint32_t)g.zg);
+        T f[3];
+        if (in_lds)
+#pragma unroll
+            for (int a = 0; a < 3; a++) f[a] = F[3 * (uint64_t)n + a];
+        Mom4<T> m;
+        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i, pd.j, k, m.r, m.x, m.y, m.z, rho0);
+        if (mom_lds) lm[e] = m;
+        else gm[e] = m;
+        if (in_lds)
+#pragma unroll
+            for (int a = 0; a < 3; a++) lf[3 * e + a] = f[a];
+    }
     gather_blades<PR, L, STREAM, MOMSRC, EVEN>(fg, pd.j, t0, threads, Q, F, prev, next, g, rho0);
     sync();
-    // A solo plane whose static cells fit keeps their force values in LDS
-    // through the static levels (every stencil cell of a plane task lies in
-    // its own plane, which no other task touches): each level then waits on
-    // LDS instead of on F in HBM.  Loaded after the blade cells' zeroing.
-    using T = typename PR::T;
-    const int64_t nc = pd.cell_end - pd.cell_begin;
-    T* lds = (sizeof(T) <= 4 && lds_buf && team == 1 && nc <= lds_cells && nc >= lds_min) ? lds_buf : nullptr;
-    if (lds) {
-        for (int64_t e = threadIdx.x; e < nc; e += blockDim.x) {
-            const uint64_t cc = fg.cells[pd.cell_begin + e];  // cell_index of the entry
-            lds[3 * e + 0] = F[3 * cc + 0];
-            lds[3 * e + 1] = F[3 * cc + 1];
-            lds[3 * e + 2] = F[3 * cc + 2];
+    // the three homes of moments and force values are loops of their own, each with one address space
+    if (mom_lds) static_levels<T>(fg, pd, 0, 1, lm, lf, F, alfa, beta, sync);
+    else if (in_lds) static_levels<T>(fg, pd, 0, 1, gm, lf, F, alfa, beta, sync);
+    else static_levels<T>(fg, pd, rank, team, gm, (T*)nullptr, F, alfa, beta, sync);
+    if (in_lds) {
+        // every static level ended with a barrier: the force values back to F before the blade levels read it
+        for (int e = (int)threadIdx.x; e < nc; e += (int)blockDim.x) {
+            const uint64_t n = cells[e];
+#pragma unroll
+            for (int a = 0; a < 3; a++) F[3 * n + a] = lf[3 * e + a];
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
-    plane_levels<T, typename PR::D>(fg, pd, rank, team, F, g, alfa, beta, sync, lds);
+    blade_levels<T>(fg, pd.j, rank, team, F, alfa, beta, sync);
 }
 
 template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
@@ -1718,13 +1809,11 @@ __global__ __launch_bounds__(kPlaneBlock) void k_force_planes(ForceGeom fg, cons
                                                               const uint64_t* __restrict__ prev,
                                                               uint64_t* __restrict__ next, Grid g,
                                                               typename PR::T alfa, typename PR::T beta, float rho0) {
-    __shared__ float4 lds_f[kPlaneLdsBytes / sizeof(float4)];
+    __shared__ float4 lds[kPlaneLdsBytes / sizeof(float4)];
     const PlaneBlock pb = fg.blocks[blockIdx.x];
     if (pb.plane < 0) return;
-    using T = typename PR::T;
     force_plane<PR, L, STREAM, MOMSRC, EVEN>(fg, fg.planes[pb.plane], pb.rank, Q, F, prev, next, g, alfa, beta,
-                                             rho0, reinterpret_cast<T*>(lds_f),
-                                             (int64_t)(kPlaneLdsBytes / (3 * sizeof(T))), kPlaneLdsMinCells);
+                                             rho0, lds, (int64_t)kPlaneLdsBytes);
 }
 
 // The levels of every plane after the gathers of the one-launch step: a
@@ -1747,9 +1836,11 @@ __global__ __launch_bounds__(kLevelBlock) void k_force_levels(ForceGeom fg, cons
         else __syncthreads();
     };
     gather_blades<PR, LayoutLIJK, StreamEsotwist, MOMSRC_ESO_POPS, EVEN>(
-        fg, pd.j, (int64_t)pb.rank * blockDim.x + threadIdx.x, (int64_t)team * blockDim.x, Q, F, prev, next, g, rho0);
+        fg, pd.j, pb.rank * (int)blockDim.x + (int)threadIdx.x, team * (int)blockDim.x, Q, F, prev, next, g, rho0);
     sync();
-    plane_levels<float, typename PR::D>(fg, pd, pb.rank, team, F, g, alfa, beta, sync);
+    static_levels<float>(fg, pd, pb.rank, team, static_cast<const Mom4<float>*>(fg.scache) + pd.cell_begin,
+                         (float*)nullptr, F, alfa, beta, sync);
+    blade_levels<float>(fg, pd.j, pb.rank, team, F, alfa, beta, sync);
 }
 
 // ------------------------------------------------------------------ pipelined Esotwist step
@@ -2188,7 +2279,8 @@ __global__ void k_vorticity(const typename PR::S* __restrict__ Q, Grid g, int ax
 // ------------------------------------------------------------------ geometry on the device
 template <typename T>
 __device__ __forceinline__ void blade_gen_point(const BladeLayout& bl, const BladeStep& st, const PointsDev& out,
-                                                int64_t offset, int64_t t) {
+                                                ForceRow<T>* __restrict__ rows, const Grid& g, int64_t offset,
+                                                int64_t t) {
     BladeEnum e;
     e.n_blades = bl.n_blades;
     e.n_planes = bl.n_planes;
@@ -2207,13 +2299,25 @@ __device__ __forceinline__ void blade_gen_point(const BladeLayout& bl, const Bla
     static_cast<T*>(out.u)[q] = (T)pt.u_delta;
     static_cast<T*>(out.v)[q] = (T)pt.v_delta;
     static_cast<T*>(out.w)[q] = (T)pt.w_delta;
+    // its three stencil rows for the blade levels (e: cell_index of the cells)
+    const T vel[3] = {(T)pt.u_delta, (T)pt.v_delta, (T)pt.w_delta};
+    const int i = (int)pt.i + bl.ghost, j = (int)pt.j + bl.ghost, k = (int)pt.k + bl.ghost;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        ForceRow<T> row = make_row<T>((T)pt.i_frac, (T)pt.k_frac, c, vel[c]);
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+            row.e[m] = (int32_t)cell_index(g, wrap_ik(i + m - 1, g.xg1), j, wrap_ik(k + c - 1, g.zg1));
+        rows[3 * q + c] = row;
+    }
 }
 
 template <typename T>
-__global__ void k_gen_blades(BladeLayout bl, BladeStep st, PointsDev out, int64_t offset, int64_t count) {
+__global__ void k_gen_blades(BladeLayout bl, BladeStep st, PointsDev out, ForceRow<T>* __restrict__ rows, Grid g,
+                             int64_t offset, int64_t count) {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (t >= count) return;
-    blade_gen_point<T>(bl, st, out, offset, t);
+    blade_gen_point<T>(bl, st, out, rows, g, offset, t);
 }
 
 // getExternalPoints as a mask: a cell is outside when its centre lies beyond the
@@ -2959,13 +3063,22 @@ hipError_t launch_vorticity(int prec, int layout, int streaming, int momsrc, int
     return e;
 }
 
-hipError_t launch_gen_blades(int prec, const BladeLayout& bl, const BladeStep& st, const PointsDev& out,
-                             int64_t offset, hipStream_t s) {
+hipError_t launch_gen_blades(int prec, const BladeLayout& bl, const BladeStep& st, const PointsDev& out, void* rows,
+                             const Grid& g, int64_t offset, hipStream_t s) {
     const int64_t count = (int64_t)bl.n_blades * bl.n_planes * bl.n_radial;
     if (count <= 0) return hipSuccess;
     const uint32_t nb = (uint32_t)((count + kBlock - 1) / kBlock);
-    if (prec != 1) hipLaunchKernelGGL(k_gen_blades<float>, dim3(nb), dim3(kBlock), 0, s, bl, st, out, offset, count);
-    else hipLaunchKernelGGL(k_gen_blades<double>, dim3(nb), dim3(kBlock), 0, s, bl, st, out, offset, count);
+    if (prec != 1) hipLaunchKernelGGL(k_gen_blades<float>, dim3(nb), dim3(kBlock), 0, s, bl, st, out, (ForceRow<float>*)rows, g, offset, count);
+    else hipLaunchKernelGGL(k_gen_blades<double>, dim3(nb), dim3(kBlock), 0, s, bl, st, out, (ForceRow<double>*)rows, g, offset, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_static_rows(int prec, const PointsDev& p, int64_t n, const int32_t* sidx, const PlaneDesc* planes,
+                              const int32_t* plane_of_j, void* rows, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    const uint32_t nb = (uint32_t)((3 * n + kBlock - 1) / kBlock);
+    if (prec != 1) hipLaunchKernelGGL(k_static_rows<float>, dim3(nb), dim3(kBlock), 0, s, p, n, sidx, planes, plane_of_j, (ForceRow<float>*)rows);
+    else hipLaunchKernelGGL(k_static_rows<double>, dim3(nb), dim3(kBlock), 0, s, p, n, sidx, planes, plane_of_j, (ForceRow<double>*)rows);
     return hipGetLastError();
 }
 
@@ -3059,7 +3172,8 @@ __global__ void k_batch_blades(const MemberDev* __restrict__ mem, const int64_t*
     const int m = find_slot(off, n, t);
     const MemberDev& md = mem[m];
     if (!md.active) return;
-    blade_gen_point<float>(md.fg.blade, md.steps[md.done], md.fg.pts, md.fg.n_static, t - off[m]);
+    blade_gen_point<float>(md.fg.blade, md.steps[md.done], md.fg.pts, static_cast<ForceRow<float>*>(md.fg.rows), md.g,
+                           md.fg.n_static, t - off[m]);
 }
 
 // the new occupancy mask starts from the static stencil bits
@@ -3078,14 +3192,13 @@ __global__ void k_batch_mask_init(const MemberDev* __restrict__ mem, const int64
 template <typename PR, int L, int STREAM>
 __global__ __launch_bounds__(kPlaneBlock) void k_batch_force_planes(const MemberDev* __restrict__ mem,
                                                                     const PlaneTask* __restrict__ tasks,
-                                                                    int64_t lds_cells) {
-    extern __shared__ float4 batch_lds[];  // lds_cells force values (3 T each), launch-sized
+                                                                    int64_t lds_bytes) {
+    extern __shared__ float4 batch_lds[];  // lds_bytes for force values and moments, launch-sized
     const PlaneTask tk = tasks[blockIdx.x];
     const MemberDev& md = mem[tk.member];
     if (!md.active) return;
     using S = typename PR::S;
-    using T = typename PR::T;
-    T* lds = lds_cells > 0 ? reinterpret_cast<T*>(batch_lds) : nullptr;
+    void* lds = lds_bytes > 0 ? batch_lds : nullptr;
     const PlaneBlock pb = md.fg.blocks[tk.block];
     if (pb.plane < 0) return;
     const PlaneDesc& pd = md.fg.planes[pb.plane];
@@ -3095,14 +3208,14 @@ __global__ __launch_bounds__(kPlaneBlock) void k_batch_force_planes(const Member
         const S* Q = static_cast<const S*>(md.Q[0]);
         if (md.even)
             force_plane<PR, L, STREAM, MOMSRC_ESO_POPS, 0>(md.fg, pd, pb.rank, Q, md.F, prev, next, md.g, md.alfa, md.beta,
-                                                            md.rho0, lds, lds_cells);
+                                                            md.rho0, lds, lds_bytes);
         else
             force_plane<PR, L, STREAM, MOMSRC_ESO_POPS, 1>(md.fg, pd, pb.rank, Q, md.F, prev, next, md.g, md.alfa, md.beta,
-                                                            md.rho0, lds, lds_cells);
+                                                            md.rho0, lds, lds_bytes);
     } else {
         const S* Q = static_cast<const S*>(md.Q[1 - md.cur]);
         force_plane<PR, L, STREAM, MOMSRC_PULL_POPS, 1>(md.fg, pd, pb.rank, Q, md.F, prev, next, md.g, md.alfa, md.beta,
-                                                         md.rho0, lds, lds_cells);
+                                                         md.rho0, lds, lds_bytes);
     }
 }
 
@@ -3144,8 +3257,7 @@ hipError_t batch_step_t(const BatchPlan& p, hipStream_t s) {
     if (p.n_tasks > 0)
         hipLaunchKernelGGL((k_batch_force_planes<PR, L, STREAM>), dim3((uint32_t)p.n_tasks),
                            dim3(p.force_bs > 0 ? p.force_bs : kPlaneBlock),
-                           (uint32_t)(p.force_lds_cells * 3 * sizeof(typename PR::T)), s, p.mem, p.tasks,
-                           p.force_lds_cells);
+                           (uint32_t)p.force_lds_bytes, s, p.mem, p.tasks, p.force_lds_bytes);
     hipLaunchKernelGGL(k_batch_advance<STREAM>, dim3(nblk(n, 64)), dim3(64), 0, s, p.mem_rw, n);
     return hipGetLastError();
 }

@@ -60,6 +60,13 @@ TDLB_HD inline int32_t blade_colours(int32_t n_blades, double r_inner) {
     return sep < 3.0 * 1.4142135623730951 + 1e-9 ? n_blades : c;
 }
 
+// No two blades ever share a stencil cell: neighbouring blades are more than
+// 3 sqrt(2) cells apart at the inner radius.
+TDLB_HD inline bool blades_apart(int32_t n_blades, double r_inner) {
+    if (n_blades < 2) return true;
+    return 2.0 * r_inner * sin(3.14159265358979323846 / n_blades) >= 3.0 * 1.4142135623730951 + 1e-9;
+}
+
 // Number of blade points of colour class c (c = bcol*5 + rmod).
 TDLB_HD inline int64_t blade_class_size(const BladeEnum& e, int c) {
     int bcol = c / 5, rmod = c % 5;
