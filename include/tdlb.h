@@ -310,7 +310,7 @@ int tdlb_batch_member(tdlb_batch_t b, tdlb_cu_t cu, uint64_t* step, double* angl
 /* members, kernel launches per step of the last run, and each member's tile (0 row, 1 plane, 2 flat) */
 int tdlb_batch_info(tdlb_batch_t b, int64_t* n_members, int64_t* launches_per_step, int32_t* tiles, int64_t cap);
 /* the fused kernel's block size of the last run, the steps one graph replay
- * advances and the forcing pass's workgroup size (chosen from the members'
+ * advances and the workgroup size of the forcing levels (chosen from the members'
  * mean stencil cells per plane task; TDLB_BATCH_FORCE_BLOCK overrides it) */
 int tdlb_batch_shape(tdlb_batch_t b, int32_t* block_size, int32_t* graph_steps, int32_t* forcing_block);
 

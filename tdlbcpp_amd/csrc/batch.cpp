@@ -90,7 +90,7 @@ struct tdlb_batch {
     DevBuf<int64_t> d_tab;
     DevBuf<PlaneTask> d_tasks;
     DevBuf<BladeStep> d_steps;
-    DevBuf<int32_t> d_bm;  // member of each fused-kernel block
+    DevBuf<int32_t> d_bm;  // member of each fused-kernel block, then of each gather block
 
     // plan of the last run and its graph
     BatchPlan plan{};
@@ -145,7 +145,7 @@ MemberDev describe(const tdlb_batch* b, const Member& m) {
     md.fmask[1] = cu->fmask[1];
     md.static_base = cu->static_base;
     md.fg = cu->fgeom();
-    md.fg.local_teams = 0;  // the batch orders workgroups by member, not by XCD
+    md.gb = gather_blocks(cu->n_rot, md.fg.n_cells, (int64_t)cu->mask_words);
     md.even = cu->even ? 1 : 0;
     md.cur = cu->cur;
     md.fm = cu->fm;
@@ -290,35 +290,25 @@ int build_plan(tdlb_batch* b, int64_t K, bool* structure_changed) {
     for (int a : idx) key.push_back({b->members[a].cu, b->members[a].tile});
 
     std::vector<MemberDev> mem(M);
-    std::vector<int64_t> tab(3 * (size_t)(M + 1), 0);
+    std::vector<int64_t> tab(2 * (size_t)(M + 1), 0);
     int64_t* off_coll = tab.data();
-    int64_t* off_rot = off_coll + (M + 1);
-    int64_t* off_words = off_rot + (M + 1);
+    int64_t* off_gather = off_coll + (M + 1);
     std::vector<BladeStep> steps;
     std::vector<size_t> step_base(M);
-    // forcing workgroups: the teams of every member first (a team's workgroups
-    // must be resident together), then every solo plane, longest first
-    std::vector<PlaneTask> team_tasks;
+    // levels workgroups: every plane of every member, longest first
     std::vector<std::pair<float, PlaneTask>> tk;
-    int64_t solo_cells = 0;  // static cells of the largest solo plane
+    int64_t most_lds = 0;  // bytes that would hold everything of every plane
     for (int r = 0; r < M; r++) {
         Member& m = b->members[idx[r]];
         tdlb_cu* cu = m.cu;
         m.n_steps = std::min<int64_t>(m.call, K);
         off_coll[r + 1] = off_coll[r] + batch_coll_blocks(cu->g, m.tile, b->bs);
-        off_rot[r + 1] = off_rot[r] + cu->n_rot;
-        off_words[r + 1] = off_words[r] + (int64_t)cu->mask_words;
-        const auto& bl = cu->static_set.block_list;
         const auto& pl = cu->static_set.plane_list;
-        for (int32_t b = 0; b < (int32_t)bl.size(); b++) {
-            if (bl[b].plane < 0) continue;  // an empty slot of the single-tank launch
-            const PlaneDesc& pd = pl[bl[b].plane];
-            if (pd.team > 1) {
-                team_tasks.push_back(PlaneTask{r, b});
-            } else {
-                tk.push_back({cu->static_set.plane_cost[bl[b].plane], PlaneTask{r, b}});
-                solo_cells = std::max<int64_t>(solo_cells, pd.cell_end - pd.cell_begin);
-            }
+        for (int32_t t = 0; t < (int32_t)pl.size(); t++) {
+            tk.push_back({cu->static_set.plane_cost[t], PlaneTask{r, t}});
+            const int64_t rows = (int64_t)cu->blade.n_blades * cu->blade.n_radial * blade_row_bytes(sizeof(float));
+            most_lds = std::max<int64_t>({most_lds, (pl[t].cell_end - pl[t].cell_begin) * 7 * (int64_t)sizeof(float),
+                                          rows + plane_force_bytes(cu->g, sizeof(float))});
         }
         // blade orientation of each step (the single-handle loop computes the same)
         Rushton R(cu->rp);
@@ -337,17 +327,51 @@ int build_plan(tdlb_batch* b, int64_t K, bool* structure_changed) {
             st.omega = delta;
         }
         mem[r] = describe(b, m);
+        const GatherBlocks& gb = mem[r].gb;
+        off_gather[r + 1] = off_gather[r] + gb.blades + gb.cells + gb.words;
         mem[r].n_steps = m.n_steps;
         mem[r].active = m.n_steps > 0 ? 1 : 0;
         mem[r].done = 0;
     }
     std::stable_sort(tk.begin(), tk.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
-    std::vector<PlaneTask> tasks(team_tasks);
+    std::vector<PlaneTask> tasks;
     for (const auto& t : tk) tasks.push_back(t.second);
-    const int64_t tot_coll = off_coll[M], tot_rot = off_rot[M], tot_words = off_words[M];
-    std::vector<int32_t> blk_member((size_t)tot_coll);
-    for (int r = 0; r < M; r++)
+    const int64_t tot_coll = off_coll[M], tot_gather = off_gather[M];
+    std::vector<int32_t> blk_member((size_t)(tot_coll + tot_gather));
+    for (int r = 0; r < M; r++) {
         std::fill(blk_member.begin() + off_coll[r], blk_member.begin() + off_coll[r + 1], (int32_t)r);
+        std::fill(blk_member.begin() + tot_coll + off_gather[r], blk_member.begin() + tot_coll + off_gather[r + 1],
+                  (int32_t)r);
+    }
+
+    BatchPlan& p = b->plan;
+    // small levels workgroups only with enough tasks to keep every CU busy
+    // several times over (a batch of one tank runs faster with 1024 lanes)
+    p.force_bs = kForcePlaneBlock;
+    if ((int64_t)tasks.size() >= 4 * (int64_t)b->n_cu) {
+        double cells = 0.0;
+        for (int r = 0; r < M; r++) cells += (double)b->members[idx[r]].cu->static_set.n_cells;
+        p.force_bs = forcing_block_for(cells / (double)tasks.size());
+    }
+    if (const char* v = std::getenv("TDLB_BATCH_FORCE_BLOCK")) {
+        const int t = std::atoi(v);
+        if (t >= 64 && t <= kForcePlaneBlock && t % 64 == 0) p.force_bs = t;
+    }
+    // What a plane keeps in LDS through its levels (plane_levels) has a share of
+    // the CU's LDS that keeps the workgroups resident together that the registers
+    // allow (at most 128 VGPRs: 1024 lanes per CU); what does not fit stays in HBM.
+    // All batch formats compute in 4-byte floats.  The launch-sized LDS stays
+    // within 64 KB, which needs no kernel attribute.
+    {
+        const int64_t per_cu = std::max<int64_t>(1, kForcePlaneBlock / p.force_bs);
+        const int64_t bytes = (int64_t)std::min<size_t>(kCuLdsBytes / (size_t)per_cu, 64 * 1024) / 16 * 16;
+        p.force_lds_bytes = std::min<int64_t>((most_lds + 15) / 16 * 16, bytes);
+    }
+    for (int r = 0; r < M; r++) {
+        tdlb_cu* cu = b->members[idx[r]].cu;
+        CHK(ensure_force_scratch(cu->static_set, cu->tsize, p.force_lds_bytes));
+        mem[r].fg.fscr = cu->static_set.fscr;
+    }
 
     int moved = 0;
     int g;
@@ -374,49 +398,24 @@ int build_plan(tdlb_batch* b, int64_t K, bool* structure_changed) {
                               b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));  // host vectors go out of scope
 
-    BatchPlan& p = b->plan;
     p.mem = b->d_mem.p;
     p.mem_rw = b->d_mem.p;
     p.n_members = M;
     p.off_coll = b->d_tab.p;
     p.coll_member = b->d_bm.p;
-    p.off_rot = b->d_tab.p + (M + 1);
-    p.off_words = b->d_tab.p + 2 * (M + 1);
+    p.off_gather = b->d_tab.p + (M + 1);
+    p.gather_member = b->d_bm.p + tot_coll;
     p.tasks = b->d_tasks.p;
-    // small forcing workgroups only with enough tasks to keep every CU busy
-    // several times over (a batch of one tank runs faster with 1024 lanes)
-    p.force_bs = kForcePlaneBlock;
-    if ((int64_t)tasks.size() >= 4 * (int64_t)b->n_cu) {
-        double cells = 0.0;
-        for (int r = 0; r < M; r++) cells += (double)b->members[idx[r]].cu->static_set.n_cells;
-        p.force_bs = forcing_block_for(cells / (double)tasks.size());
-    }
-    if (const char* v = std::getenv("TDLB_BATCH_FORCE_BLOCK")) {
-        const int t = std::atoi(v);
-        if (t >= 64 && t <= kForcePlaneBlock && t % 64 == 0) p.force_bs = t;
-    }
-    // The force values (and moments) of a solo plane stay in LDS through its
-    // levels when they fit a share of the CU's LDS that keeps the workgroups
-    // resident together that the registers allow (at most 128 VGPRs: 1024 lanes
-    // per CU); larger planes keep them in HBM.  All batch formats compute in
-    // 4-byte floats.  The launch-sized LDS stays within 64 KB, which needs no
-    // kernel attribute.
-    {
-        const int64_t per_cu = std::max<int64_t>(1, kForcePlaneBlock / p.force_bs);
-        const int64_t bytes = (int64_t)std::min<size_t>({kPlaneLdsBytes, kCuLdsBytes / (size_t)per_cu, 64 * 1024});
-        p.force_lds_bytes = std::min<int64_t>(solo_cells * 7 * (int64_t)sizeof(float), bytes) / 16 * 16;
-    }
     p.tot_coll = tot_coll;
-    p.tot_rot = tot_rot;
-    p.tot_words = tot_words;
+    p.tot_gather = tot_gather;
     p.n_tasks = (int64_t)tasks.size();
     p.bs = b->bs;
-    // launches: blades, fused, mask, forcing planes, advance
-    b->launches_per_step = 5;
+    // launches: fused, forcing gather, forcing levels, advance
+    b->launches_per_step = 4;
     // A captured step bakes in every launch size and kernel argument: recapture
     // whenever any of them differs (member identity alone is not enough, a freed
     // handle's address can come back for a tank of another size).
-    std::vector<int64_t> sig = {M, tot_coll, tot_rot, tot_words, p.n_tasks, p.bs, p.force_bs, p.force_lds_bytes,
+    std::vector<int64_t> sig = {M, tot_coll, tot_gather, p.n_tasks, p.bs, p.force_bs, p.force_lds_bytes,
                                 (int64_t)(uintptr_t)b->d_mem.p, (int64_t)(uintptr_t)b->d_tab.p,
                                 (int64_t)(uintptr_t)b->d_tasks.p, (int64_t)(uintptr_t)b->d_bm.p};
     *structure_changed = moved || sig != b->launch_sig || key != b->key || b->buffers_moved;

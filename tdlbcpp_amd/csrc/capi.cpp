@@ -369,15 +369,91 @@ int forcing_pass(tdlb_cu* cu, const DevPoints& dp, const std::vector<ForceSegmen
     return TDLB_OK;
 }
 
-// cost (estimated microseconds) above which a plane gets a team of workgroups,
-// one per this much; a wall plane of a 512^3 tank is ~100
-constexpr double kTeamCost = 120.0;
-constexpr int32_t kMaxTeam = 16;
-// TDLB_FORCE_TEAM_COST overrides kTeamCost (tests give small tanks teams)
-double team_cost() {
-    const char* v = std::getenv("TDLB_FORCE_TEAM_COST");
-    const double c = v ? std::atof(v) : 0.0;
-    return c > 0.0 ? c : kTeamCost;
+// Workgroup of a tank's levels launch, from all but the few largest planes (the
+// impeller disk's).  lanes: a lane per static cell for the copies in and out,
+// which is more than a quad per point of a level (96^3: 192 lanes 43 us a pass,
+// 1024 lanes 38).  LDS: what holds everything of every plane, at most a CU's (a
+// workgroup's registers leave room for one a CU anyway); what a plane cannot hold
+// there stays in HBM.
+void level_shape(const Grid& g, const std::vector<PlaneDesc>& planes, const std::vector<int32_t>& widest,
+                 int64_t blade_points, size_t tsize, IndexedSet& set) {
+    if (planes.empty()) return;
+    const size_t at = planes.size() - 1 - planes.size() / 32;
+    std::vector<int64_t> cells;
+    for (const PlaneDesc& pd : planes) cells.push_back(pd.cell_end - pd.cell_begin);
+    std::vector<int32_t> wide(widest);
+    const int64_t most = *std::max_element(cells.begin(), cells.end());
+    std::nth_element(cells.begin(), cells.begin() + at, cells.end());
+    std::nth_element(wide.begin(), wide.begin() + at, wide.end());
+    // static cells: moments and force values; blades: rows and moments of a plane's points and, if it fits, the
+    // plane's force values
+    const int64_t per = 7 * (int64_t)tsize, rows = blade_points * blade_row_bytes(tsize);
+    int64_t want = std::max(most * per, rows + plane_force_bytes(g, tsize));
+    if (want > (int64_t)kCuLdsBytes) want = std::min<int64_t>(std::max(most * per, rows), kCuLdsBytes);
+    set.level_lds = (int32_t)((want + 15) / 16 * 16);
+    const int most_lanes = tsize > 4 ? level_block<double>() : level_block<float>();
+    set.level_lanes = (int32_t)std::min<int64_t>(most_lanes, std::max<int64_t>(4 * wide[at], cells[at]) / 64 * 64 + 64);
+}
+
+bool pipe_wanted() {
+    const char* env = std::getenv("TDLB_PIPE");
+    return env && std::atoi(env) == 1;
+}
+
+// Parts of a plane that its levels may run apart: 1 for the points of components
+// (points linked by shared stencil cells) that no blade ever touches, in planes
+// whose static cells a CU's LDS cannot hold with their moments; 0 for all others.
+// The impeller disk's plane splits into the disk and the tank wall with its
+// baffles (from about 230^3).
+std::vector<uint8_t> plane_parts(const tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat) {
+    const int64_t n = (int64_t)stat.size(), gh = cu->prm.ghost;
+    std::vector<uint8_t> part((size_t)n, 0);
+    if (pipe_wanted()) return part;  // the one-launch step takes a plane's cells as one range
+    std::vector<int64_t> per_plane((size_t)cu->yg, 0);
+    for (const tdlb_ib_point& q : stat) per_plane[q.j + gh]++;
+    // a plane's cells are at most 9 a point; a filled disk has little more than one a point
+    const int64_t room = (int64_t)kCuLdsBytes / (7 * (int64_t)cu->tsize);
+    std::vector<std::vector<int64_t>> of((size_t)cu->yg);
+    for (int64_t q = 0; q < n; q++)
+        if (9 * per_plane[stat[q].j + gh] > room) of[stat[q].j + gh].push_back(q);
+    std::vector<int32_t> owner((size_t)cu->xg * cu->zg, -1);  // of a cell of the plane: a point that covers it
+    uint64_t sc[9];
+    for (const std::vector<int64_t>& pts : of) {
+        if (pts.empty()) continue;
+        std::vector<int32_t> up(pts.size());
+        std::iota(up.begin(), up.end(), 0);
+        auto root = [&](int32_t a) {
+            while (up[a] != a) a = up[a] = up[up[a]];
+            return a;
+        };
+        std::vector<size_t> covered;
+        for (size_t t = 0; t < pts.size(); t++) {
+            const tdlb_ib_point& q = stat[pts[t]];
+            stencil_cells(cu, q.i + gh, q.j + gh, q.k + gh, sc);
+            for (uint64_t c : sc) {
+                const size_t at = (size_t)(c / cu->g.yz) * cu->zg + (size_t)(c % cu->zg);
+                if (owner[at] < 0) {
+                    owner[at] = (int32_t)t;
+                    covered.push_back(at);
+                } else {
+                    up[root((int32_t)t)] = root(owner[at]);
+                }
+            }
+        }
+        if ((int64_t)covered.size() > room) {
+            // blade points round to at most outer + sqrt(1/2), stencils reach sqrt(2) further
+            const double reach = cu->rp.blade_outer_radius + 3.0;
+            std::vector<uint8_t> touched(pts.size(), cu->blade_wraps ? 1 : 0);
+            for (size_t at : covered) {
+                const double x = (double)(at / cu->zg) - (double)gh - cu->rp.center_x;
+                const double z = (double)(at % cu->zg) - (double)gh - cu->rp.center_z;
+                if (x * x + z * z <= reach * reach) touched[root(owner[at])] = 1;
+            }
+            for (size_t t = 0; t < pts.size(); t++) part[pts[t]] = touched[root((int32_t)t)] ? 0 : 1;
+        }
+        for (size_t at : covered) owner[at] = -1;
+    }
+    return part;
 }
 
 // Plane tasks of a bound tank's static list (ForceGeom, kernels.h).  Levels as
@@ -396,13 +472,14 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
     std::vector<int32_t> lev(n);
     for (size_t l = 0; l + 1 < loffs.size(); l++)
         for (int64_t a = loffs[l]; a < loffs[l + 1]; a++) lev[lorder[a]] = (int32_t)l;
+    const std::vector<uint8_t> part = plane_parts(cu, stat);
     order.resize(n);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) {
-        return stat[a].j != stat[b].j ? stat[a].j < stat[b].j : lev[a] < lev[b];
+        return stat[a].j != stat[b].j ? stat[a].j < stat[b].j : part[a] != part[b] ? part[a] < part[b] : lev[a] < lev[b];
     });
     const int n_classes = be.n_blades > 0 ? 5 * be.n_bcol : 0;
-    const int64_t blade_pts = (int64_t)be.n_blades * be.n_radial;  // per blade plane
+    std::vector<int32_t> widest;  // points of the largest level of each plane
     std::vector<PlaneDesc> planes;
     std::vector<double> cost;
     std::vector<int64_t> lev_off;
@@ -412,16 +489,20 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
     uint64_t sc[9];
     int32_t max_levels = 0;
     int64_t a0 = 0;
-    for (int64_t j = 1; j <= cu->g.yg1; j++) {
+    // a task per plane and part: part 0 (which the blades belong to), then part 1
+    for (int64_t jp = 2; jp <= 2 * cu->g.yg1 + 1; jp++) {
+        const int64_t j = jp / 2;
+        const uint8_t pt = (uint8_t)(jp & 1);
         int64_t a1 = a0;
-        while (a1 < n && stat[order[a1]].j + gh == j) a1++;
-        const bool blades = n_classes > 0 && j >= blade_j0 && j < blade_j0 + be.n_planes;
+        while (a1 < n && stat[order[a1]].j + gh == j && part[order[a1]] == pt) a1++;
+        const bool blades = pt == 0 && n_classes > 0 && j >= blade_j0 && j < blade_j0 + be.n_planes;
         if (a1 == a0 && !blades) {
             a0 = a1;
             continue;
         }
         PlaneDesc pd{};
         pd.j = (int32_t)j;
+        pd.blades = blades ? 1 : 0;
         pd.cell_begin = (int64_t)cells.size();
         pc.clear();
         for (int64_t a = a0; a < a1; a++) {
@@ -433,89 +514,43 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
         std::sort(uq.begin(), uq.end());
         uq.erase(std::unique(uq.begin(), uq.end()), uq.end());
         for (size_t e = 0; e < pc.size(); e++)
-            sidx[9 * (size_t)a0 + e] =
-                (int32_t)(pd.cell_begin + (std::lower_bound(uq.begin(), uq.end(), pc[e]) - uq.begin()));
+            sidx[9 * (size_t)a0 + e] = (int32_t)(std::lower_bound(uq.begin(), uq.end(), pc[e]) - uq.begin());
         cells.insert(cells.end(), uq.begin(), uq.end());
         pd.cell_end = (int64_t)cells.size();
         const int32_t nl = a1 > a0 ? lev[order[a1 - 1]] + 1 : 0;
         pd.n_levels = nl;
         pd.lev = (int64_t)lev_off.size();
-        int64_t a = a0, passes = 0;
+        int64_t a = a0, wide = 0;
         for (int32_t l = 0; l < nl; l++) {
             lev_off.push_back(a);
             const int64_t b = a;
             while (a < a1 && lev[order[a]] == l) a++;
-            passes += (a - b + kForcePlanePoints - 1) / kForcePlanePoints;
+            wide = std::max(wide, a - b);
         }
         lev_off.push_back(a1);
         max_levels = std::max(max_levels, nl);
-        int64_t gather = pd.cell_end - pd.cell_begin;
-        if (blades) {
-            for (int c = 0; c < n_classes; c++) {
-                const int64_t cls = blade_class_size(be, c) / std::max(be.n_planes, 1);
-                passes += (cls + kForcePlanePoints - 1) / kForcePlanePoints;
-            }
-            gather += 9 * blade_pts;
-        }
         planes.push_back(pd);
-        cost.push_back(3.0 * (double)(passes + n_classes) + (double)gather / 1024.0);
+        widest.push_back((int32_t)wide);
+        // about 1 us a level, 2 us a blade level, and the copies of cells and passes
+        cost.push_back(nl + 2.0 * (blades ? n_classes : 0) + (double)(a1 - a0) / 256.0 +
+                       (double)(pd.cell_end - pd.cell_begin) / 1024.0);
         a0 = a1;
     }
     if (a0 != n) return fail(TDLB_ERR_INVALID, "static IB points outside the interior planes");
-    // A plane whose passes would keep one workgroup far longer than a wall
-    // plane (the impeller disk's) runs on a team; teams come first in the
-    // launch, then the solo planes, longest first.
+    level_shape(cu->g, planes, widest, (int64_t)be.n_blades * be.n_radial, cu->tsize, set);
     std::vector<size_t> by(planes.size());
     std::iota(by.begin(), by.end(), 0);
     std::stable_sort(by.begin(), by.end(), [&](size_t x, size_t y) { return cost[x] > cost[y]; });
     std::vector<PlaneDesc> sorted(planes.size());
-    std::vector<PlaneBlock> blocks;
-    const double tcost = team_cost();
     set.plane_cost.resize(planes.size());
-    int32_t n_teams = 0;
     for (size_t t = 0; t < by.size(); t++) {
-        PlaneDesc pd = planes[by[t]];
-        const double c = cost[by[t]];
-        pd.team = (int32_t)std::min<double>(kMaxTeam, std::max(1.0, std::ceil(c / tcost)));
-        pd.bar = pd.team > 1 ? n_teams++ : -1;
-        sorted[t] = pd;
-        set.plane_cost[t] = (float)(c / pd.team);
-    }
-    // a team's workgroups go kXcds apart (launches dispatch workgroup b to XCD
-    // b mod kXcds), so one XCD runs the whole team; the other slots take the
-    // solo planes, longest first
-    {
-        int64_t row[kXcds] = {0};
-        std::vector<PlaneBlock> slot;
-        for (size_t t = 0; t < sorted.size(); t++) {
-            if (sorted[t].team == 1) continue;
-            int x = 0;
-            for (int y = 1; y < kXcds; y++)
-                if (row[y] < row[x]) x = y;
-            for (int32_t r = 0; r < sorted[t].team; r++) {
-                const size_t at = (size_t)x + (size_t)kXcds * (size_t)(row[x] + r);
-                if (slot.size() <= at) slot.resize(at + 1, PlaneBlock{-1, 0});
-                slot[at] = PlaneBlock{(int32_t)t, r};
-            }
-            row[x] += sorted[t].team;
-        }
-        size_t next_solo = 0;
-        auto solo = [&]() -> PlaneBlock {
-            while (next_solo < sorted.size() && sorted[next_solo].team != 1) next_solo++;
-            return next_solo < sorted.size() ? PlaneBlock{(int32_t)next_solo++, 0} : PlaneBlock{-1, 0};
-        };
-        for (auto& b : slot)
-            if (b.plane < 0) b = solo();
-        for (PlaneBlock b = solo(); b.plane >= 0; b = solo()) slot.push_back(b);
-        blocks = slot;
+        sorted[t] = planes[by[t]];
+        set.plane_cost[t] = (float)cost[by[t]];
     }
     set.n_cells = (int64_t)cells.size();
     set.n_points = n;
     set.n_planes = (int32_t)sorted.size();
-    set.n_blocks = (int32_t)blocks.size();
-    set.n_teams = n_teams;
     set.max_levels = max_levels;
-    set.block_list = blocks;
     set.plane_list = sorted;
     auto upload = [&](void** dst, const void* src, size_t bytes) -> int {
         if (bytes == 0) return TDLB_OK;
@@ -527,14 +562,9 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
     CHK(upload((void**)&set.sidx, sidx.data(), sidx.size() * 4));
     CHK(upload((void**)&set.planes, sorted.data(), sorted.size() * sizeof(PlaneDesc)));
     CHK(upload((void**)&set.lev_off, lev_off.data(), lev_off.size() * sizeof(int64_t)));
-    CHK(upload((void**)&set.blocks, blocks.data(), blocks.size() * sizeof(PlaneBlock)));
-    if (n_teams > 0) {
-        const size_t bb = (size_t)n_teams * kBarWords * sizeof(uint32_t);
-        if (hipMalloc((void**)&set.bar, bb) != hipSuccess) return fail(TDLB_ERR_NOMEM, "IB team barriers");
-        HIPCHK(launch_zero(set.bar, bb, cu->stream));
-    }
     if (!cells.empty() && hipMalloc(&set.cache, cells.size() * 4 * cu->tsize) != hipSuccess)
         return fail(TDLB_ERR_NOMEM, "IB moment cache");
+    CHK(ensure_force_scratch(set, cu->tsize, set.level_lds));
     HIPCHK(hipStreamSynchronize(cu->stream));  // host tables go out of scope
     return TDLB_OK;
 }
@@ -546,17 +576,9 @@ int build_rows(tdlb_cu* cu) {
     const size_t row = cu->tsize == 4 ? sizeof(ForceRow<float>) : sizeof(ForceRow<double>);
     const size_t n = (size_t)(cu->n_static + cu->n_rot);
     if (n == 0) return TDLB_OK;
-    std::vector<int32_t> plane_of_j((size_t)cu->yg, 0);
-    for (size_t t = 0; t < set.plane_list.size(); t++) plane_of_j[set.plane_list[t].j] = (int32_t)t;
-    int32_t* dj = nullptr;
     if (hipMalloc(&set.rows, 3 * n * row) != hipSuccess) return fail(TDLB_ERR_NOMEM, "IB stencil rows");
-    if (hipMalloc((void**)&dj, plane_of_j.size() * 4) != hipSuccess) return fail(TDLB_ERR_NOMEM, "IB stencil rows");
-    hipError_t e = hipMemcpyAsync(dj, plane_of_j.data(), plane_of_j.size() * 4, hipMemcpyHostToDevice, cu->stream);
-    if (e == hipSuccess)
-        e = launch_static_rows(cu->eprec(), cu->pts.d, cu->n_static, set.sidx, set.planes, dj, set.rows, cu->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
-    (void)hipFree(dj);
-    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("IB stencil rows: ") + hipGetErrorString(e));
+    HIPCHK(launch_static_rows(cu->eprec(), cu->pts.d, cu->n_static, set.sidx, set.rows, cu->stream));
+    HIPCHK(hipStreamSynchronize(cu->stream));
     if (set.sidx) (void)hipFree(set.sidx);
     set.sidx = nullptr;
     return TDLB_OK;
@@ -566,11 +588,10 @@ int build_rows(tdlb_cu* cu) {
 // launch must see every XCC id (each XCD's work queue needs workers); checked
 // once per device.  The step is opt-in (TDLB_PIPE=1): at 512^3 its rows run
 // slower than the separate stream-collide kernel.
-bool pipe_device_ok(tdlb_cu* cu, bool honour_env = true) {
+bool pipe_device_ok(tdlb_cu* cu) {
     static std::mutex mu;
     static std::unordered_map<int, bool> known;
-    const char* env = std::getenv("TDLB_PIPE");
-    if (honour_env && !(env && std::atoi(env) == 1)) return false;
+    if (!pipe_wanted()) return false;
     std::lock_guard<std::mutex> lk(mu);
     auto it = known.find(cu->device);
     if (it != known.end()) return it->second;
@@ -580,8 +601,7 @@ bool pipe_device_ok(tdlb_cu* cu, bool honour_env = true) {
 }
 
 // Tables of the one-launch step (PipeArgs): the first static stencil cell of
-// every row in the plane-grouped cell list, and the forcing-level workgroups
-// of each XCD's plane range, teams first.
+// every row in the plane-grouped cell list.
 int setup_pipe(tdlb_cu* cu) {
     cu->pipe = false;
     for (void* p : {(void*)cu->rowcell, (void*)cu->pctr})
@@ -624,10 +644,10 @@ int setup_pipe(tdlb_cu* cu) {
     return TDLB_OK;
 }
 
-// One step of a bound Esotwist tank in one launch: blade points of the step
-// generated before, static stencil cells prepared when the previous mask may
-// lack them.  Same arithmetic and order as launch_esotwist + bound_forcing.
-int pipe_step(tdlb_cu* cu) {
+// One step of a bound Esotwist tank with stream-collide and static gather in one
+// launch, static stencil cells prepared when the previous mask may lack them.
+// Same arithmetic and order as launch_esotwist + bound_forcing.
+int pipe_step(tdlb_cu* cu, const BladeStep& st) {
     uint64_t* prev = cu->fmask[cu->fm];
     uint64_t* next = cu->fmask[1 - cu->fm];
     if (!cu->static_in_prev)
@@ -646,6 +666,11 @@ int pipe_step(tdlb_cu* cu) {
     const int hint = line_rows_bytes(cu->g, cu->ssize) ? 1 : 0;
     HIPCHK(launch_eso_pipe(cu->prec(), cu->even ? 1 : 0, hint, a, cu->g, cu->cargs(), cu->rho0, cu->alfa, cu->beta,
                            0, row_lanes(cu->g), cu->stream));
+    // the levels read the populations of the next step's collision
+    const GatherBlocks gb = gather_blocks(cu->n_rot, 0, 0);
+    HIPCHK(launch_force_gather(cu->prec(), cu->dlay(), cu->prm.streaming, MOMSRC_ESO_POPS, cu->even ? 0 : 1, a.fg, st,
+                               gb, cu->Q[0], cu->F, prev, next, cu->static_base, cu->g, cu->rho0, cu->stream));
+    HIPCHK(launch_force_levels(cu->eprec(), a.fg, cu->F, next, cu->g, cu->alfa, cu->beta, cu->stream));
     if (cu->o_dirty) {
         HIPCHK(launch_zero_interior_o(cu->O, cu->g, cu->stream));
         cu->o_dirty = false;
@@ -656,10 +681,10 @@ int pipe_step(tdlb_cu* cu) {
     return TDLB_OK;
 }
 
-// A team barrier of the forcing planes that gave up waiting leaves its flag
-// set (kBarSpinLimit): report it once and clear it.  Never expected (teams are
-// resident together); results after it are not the reference's.
-int check_team_barriers(tdlb_cu* cu) {
+// A wait of the one-launch step that gave up leaves its flag set
+// (kBarSpinLimit): report it once and clear it.  Never expected; results after
+// it are not the reference's.
+int check_pipe_waits(tdlb_cu* cu) {
     if (cu->pctr) {
         uint32_t f[kXcds];
         for (int x = 0; x < kXcds; x++)
@@ -671,54 +696,40 @@ int check_team_barriers(tdlb_cu* cu) {
                 return fail(TDLB_ERR_HIP, "one-launch step: a wait timed out (results are invalid)");
             }
     }
-    const IndexedSet& set = cu->static_set;
-    if (!set.bar || set.n_teams <= 0) return TDLB_OK;
-    std::vector<uint32_t> w((size_t)set.n_teams * kBarWords);
-    HIPCHK(hipMemcpy(w.data(), set.bar, w.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    uint32_t bad = 0;
-    for (int32_t t = 0; t < set.n_teams; t++) bad |= w[(size_t)t * kBarWords + 2];
-    if (!bad) return TDLB_OK;
-    if (bad & 2u) {
-        HIPCHK(launch_zero(set.bar, w.size() * sizeof(uint32_t), cu->stream));
-        HIPCHK(hipStreamSynchronize(cu->stream));
-        return fail(TDLB_ERR_HIP, "IB forcing: a plane team ran on more than one XCD (forcing results are invalid)");
-    }
-    // a workgroup that gave up left the arrival count behind: restart every barrier
-    HIPCHK(launch_zero(set.bar, w.size() * sizeof(uint32_t), cu->stream));
-    HIPCHK(hipStreamSynchronize(cu->stream));
-    return fail(TDLB_ERR_HIP, "IB forcing: a plane team barrier timed out (forcing results are invalid)");
+    return TDLB_OK;
 }
 
-// One forcing pass of the bound tank: the next occupancy mask starts from the
-// static bits (static_base), the static stencil cells are prepared only when
-// the previous mask may lack them, and every plane task runs in one launch.
-int bound_forcing(tdlb_cu* cu, int momsrc, bool prepare_static) {
+// blade orientation of a step
+BladeStep blade_step(const tdlb_cu* cu, double angle, double omega) {
+    BladeStep st{};
+    Rushton(cu->rp).blade_trig(angle, st.cosb, st.sinb);
+    st.omega = omega;
+    return st;
+}
+
+// One forcing pass of the bound tank: the gather starts the next occupancy mask
+// from the static bits (static_base) and generates the step's blades; the static
+// stencil cells are prepared only when the previous mask may lack them (their
+// bits are in static_base).
+int bound_forcing(tdlb_cu* cu, int momsrc, bool prepare_static, const BladeStep& st) {
     uint64_t* prev = cu->fmask[cu->fm];
     uint64_t* next = cu->fmask[1 - cu->fm];
     const bool stored = momsrc == MOMSRC_STORED;
     const void* Qsrc = stored ? cu->eq() : cu->Q[cu->cur];
     const int qp = stored ? cu->eprec() : cu->prec();
-    HIPCHK(launch_copy(next, cu->static_base, cu->mask_bytes(), cu->stream));
+    const ForceGeom fg = cu->fgeom();
     if (prepare_static)
         HIPCHK(launch_force_prepare(cu->eprec(), cu->pts.d, 0, cu->n_static, cu->F, prev, next, cu->g, cu->stream));
-    HIPCHK(launch_force_planes(qp, cu->dlay(), cu->prm.streaming, momsrc, cu->even ? 1 : 0, cu->fgeom(), Qsrc, cu->F,
-                               prev, next, cu->g, cu->alfa, cu->beta, cu->rho0, cu->stream));
+    HIPCHK(launch_force_gather(qp, cu->dlay(), cu->prm.streaming, momsrc, cu->even ? 1 : 0, fg, st,
+                               gather_blocks(cu->n_rot, fg.n_cells, (int64_t)cu->mask_words), Qsrc, cu->F, prev, next,
+                               cu->static_base, cu->g, cu->rho0, cu->stream));
+    HIPCHK(launch_force_levels(cu->eprec(), fg, cu->F, next, cu->g, cu->alfa, cu->beta, cu->stream));
     if (cu->o_dirty) {
         HIPCHK(launch_zero_interior_o(cu->O, cu->g, cu->stream));
         cu->o_dirty = false;
     }
     cu->fm = 1 - cu->fm;
     cu->static_in_prev = true;
-    return TDLB_OK;
-}
-
-int gen_blades(tdlb_cu* cu, double angle, double omega) {
-    BladeStep st{};
-    Rushton R(cu->rp);
-    R.blade_trig(angle, st.cosb, st.sinb);
-    st.omega = omega;
-    HIPCHK(launch_gen_blades(cu->prec(), cu->blade, st, cu->pts.d, cu->static_set.rows, cu->g, cu->n_static,
-                             cu->stream));
     return TDLB_OK;
 }
 
@@ -1159,7 +1170,7 @@ int tdlb_cu_synchronize(tdlb_cu_t cu) {
     if (!cu) return fail(TDLB_ERR_INVALID, "null handle");
     CHK(set_device(cu));
     HIPCHK(hipStreamSynchronize(cu->stream));
-    return check_team_barriers(cu);
+    return check_pipe_waits(cu);
 }
 
 int tdlb_cu_stream(tdlb_cu_t cu, void** s) {
@@ -1303,6 +1314,8 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     cu->n_static = (int64_t)stat.size();
     cu->n_rot = (int64_t)rot.size();
     cu->n_blade_classes = cu->n_rot > 0 ? 5 * be.n_bcol : 0;
+    cu->rp = *p;
+    cu->blade_wraps = wraps;
     std::vector<int64_t> order;
     CHK(build_plane_set(cu, stat, be, p->blade_plane_lo + cu->prm.ghost, order, cu->static_set));
     HostPoints hs;
@@ -1325,7 +1338,6 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     cu->blade.cz = p->center_z;
     cu->blade.ghost = (int32_t)cu->prm.ghost;
     cu->blade.merged = !wraps && blades_apart(p->n_blades, p->blade_inner_radius) ? 1 : 0;
-    cu->rp = *p;
 
     // static occupancy bits: run the prepare kernel on an empty mask
     if (!cu->static_bits && hipMalloc((void**)&cu->static_bits, cu->mask_bytes()) != hipSuccess)
@@ -1356,12 +1368,11 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     cu->bound = true;
     cu->alfa = alfa;
     cu->beta = beta;
-    cu->xcc_rr = pipe_device_ok(cu, false);
+    HIPCHK(allow_level_lds(cu->eprec()));
     CHK(setup_pipe(cu));
 
     // initial forcing of main.cpp:305 on the current density and momentum
-    CHK(gen_blades(cu, angle, delta));
-    CHK(bound_forcing(cu, cell_source(cu).momsrc, true));
+    CHK(bound_forcing(cu, cell_source(cu).momsrc, true, blade_step(cu, angle, delta)));
     return TDLB_OK;
 }
 
@@ -1375,10 +1386,10 @@ int tdlb_cu_run(tdlb_cu_t cu, int64_t nsteps, uint64_t* step, double* angle) {
         *step += 1;                                             // running.incrementStep()
         const double delta = to_prec(cu, R.step_increment(*step));
         *angle += delta;                                        // running.angle += delta
-        CHK(gen_blades(cu, *angle, delta));                     // updateRotatingGeometry
+        const BladeStep st = blade_step(cu, *angle, delta);     // updateRotatingGeometry
         if (cu->pipe && cu->phase == PH_LAZY) {
             const int c0 = prof_mark(cu);
-            CHK(pipe_step(cu));
+            CHK(pipe_step(cu, st));
             const int c1 = prof_mark(cu);
             if (c0 >= 0 && c1 >= 0) {
                 cu->coll.push_back({c0, c1});
@@ -1416,7 +1427,7 @@ int tdlb_cu_run(tdlb_cu_t cu, int64_t nsteps, uint64_t* step, double* angle) {
             }
         }
         const int c1 = prof_mark(cu);
-        CHK(bound_forcing(cu, cu->simple() ? MOMSRC_PULL_POPS : MOMSRC_ESO_POPS, !cu->static_in_prev));
+        CHK(bound_forcing(cu, cu->simple() ? MOMSRC_PULL_POPS : MOMSRC_ESO_POPS, !cu->static_in_prev, st));
         const int c2 = prof_mark(cu);
         if (c0 >= 0 && c1 >= 0) cu->coll.push_back({c0, c1});
         if (c1 >= 0 && c2 >= 0) cu->force.push_back({c1, c2});

@@ -97,34 +97,43 @@ struct IndexedSet {
     int32_t* sidx = nullptr;
     void* rows = nullptr;  // bound tank: ForceRow x 3 per static and blade point
     void* cache = nullptr;
+    void* fscr = nullptr;  // bound tank: force scratch of planes beyond the LDS
     PlaneDesc* planes = nullptr;
     int64_t* lev_off = nullptr;
-    PlaneBlock* blocks = nullptr;
-    uint32_t* bar = nullptr;
     int64_t n_cells = 0, n_points = 0;
-    int32_t n_planes = 0, n_blocks = 0, n_teams = 0, max_levels = 0;
-    std::vector<float> plane_cost;  // host: duration estimate of each plane's workgroups (planes order)
-    std::vector<PlaneBlock> block_list;  // host copy of blocks
+    int32_t n_planes = 0, max_levels = 0;
+    int32_t level_lanes = 64, level_lds = 0;  // workgroup of the levels launch
+    std::vector<float> plane_cost;       // host: duration estimate of each plane (planes order)
     std::vector<PlaneDesc> plane_list;   // host copy of planes
     void release() {
-        void* ptrs[] = {cells, sidx, rows, cache, planes, lev_off, blocks, bar};
+        void* ptrs[] = {cells, sidx, rows, cache, fscr, planes, lev_off};
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
         cells = nullptr;
         sidx = nullptr;
         rows = nullptr;
         cache = nullptr;
+        fscr = nullptr;
         planes = nullptr;
         lev_off = nullptr;
-        blocks = nullptr;
-        bar = nullptr;
         n_cells = n_points = 0;
-        n_planes = n_blocks = n_teams = max_levels = 0;
+        n_planes = max_levels = 0;
         plane_cost.clear();
-        block_list.clear();
         plane_list.clear();
     }
 };
+
+// Room for the force values of planes that a levels launch with lds_bytes cannot hold in LDS.
+inline int ensure_force_scratch(IndexedSet& set, size_t tsize, int64_t lds_bytes) {
+    if (set.fscr) return TDLB_OK;
+    for (const PlaneDesc& pd : set.plane_list)
+        if ((pd.cell_end - pd.cell_begin) * 3 * (int64_t)tsize > lds_bytes) {
+            if (hipMalloc(&set.fscr, (size_t)set.n_cells * 4 * tsize) == hipSuccess) return TDLB_OK;
+            set.fscr = nullptr;
+            return fail(TDLB_ERR_NOMEM, "IB force scratch");
+        }
+    return TDLB_OK;
+}
 
 // Host-side copy of points in the CU's type, structure of arrays.
 struct HostPoints {
@@ -180,6 +189,7 @@ struct tdlb_cu {
 
     // bound Rushton tank
     bool bound = false;
+    bool blade_wraps = false;            // a blade stencil may wrap to the other side of the tank
     tdlb_rushton_params rp{};
     DevPoints pts;                       // static points [0, n_static), blades after
     IndexedSet static_set;               // stencil cells of the static points
@@ -191,7 +201,6 @@ struct tdlb_cu {
 
     // one-launch Esotwist step (launch_eso_pipe), set up at bind when the tank allows it
     bool pipe = false;
-    bool xcc_rr = false;  // launches dispatch workgroup b to XCD b mod kXcds (checked at bind)
     int32_t* rowcell = nullptr;
     uint32_t* pctr = nullptr;
 
@@ -240,13 +249,13 @@ struct tdlb_cu {
         f.rows = static_set.rows;
         f.scache = static_set.cache;
         f.rcache = rot_cache;
+        f.fscr = static_set.fscr;
+        f.n_cells = static_set.n_cells;
         f.planes = static_set.planes;
         f.n_planes = static_set.n_planes;
+        f.level_lanes = static_set.level_lanes;
+        f.level_lds = static_set.level_lds;
         f.lev_off = static_set.lev_off;
-        f.blocks = static_set.blocks;
-        f.n_blocks = static_set.n_blocks;
-        f.bar = static_set.bar;
-        f.local_teams = xcc_rr ? 1 : 0;
         f.blade = blade;
         return f;
     }

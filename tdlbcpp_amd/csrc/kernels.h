@@ -121,22 +121,17 @@ hipError_t launch_force_level_cached(int prec, const PointsDev& p, int64_t begin
                                      const Grid& g, double alfa, double beta, hipStream_t s);
 // ---- IB forcing of a bound tank by j planes.  Stencils span i and k at the
 // point's j, so points of different planes never share a cell and each plane
-// is an independent task: a workgroup (or a team of workgroups for a plane
-// with many points, such as the impeller disk's) runs a plane's blade
-// occupancy bits, the density and momentum of its stencil cells, then its
-// static levels and blade colour classes in list order, with a barrier
-// between levels instead of a kernel launch.
+// is an independent task.  A pass is two launches: the gather (blade points,
+// occupancy, density and momentum of every stencil cell) over the whole chip,
+// then one workgroup per plane that runs the plane's static levels and blade
+// levels in list order, with a barrier between levels instead of a launch.
 struct PlaneDesc {
     int32_t j;                     // plane index including the ghost offset
-    int32_t n_levels;              // static levels of the plane
+    int32_t n_levels;              // static levels of the plane (none of them empty)
     int64_t cell_begin, cell_end;  // its unique static stencil cells in ForceGeom::cells / scache
     int64_t lev;                   // ForceGeom::lev_off[lev .. lev + n_levels]: point offsets of its levels
-    int32_t team;                  // workgroups running the plane together
-    int32_t bar;                   // its barrier in ForceGeom::bar (team > 1), else -1
-};
-// workgroup -> (plane, rank in the plane's team); plane -1: an empty slot
-struct PlaneBlock {
-    int32_t plane, rank;
+    int32_t blades;                // 1: runs the plane's blade levels (a plane may be two tasks, plane_parts)
+    int32_t pad;
 };
 // One row (k1 = c - 1) of a point's 3 x 3 stencil: what the forcing of a point
 // needs besides the flow, 32 bytes in FP32.  lane c of the point's quad loads
@@ -152,27 +147,36 @@ struct ForceGeom {
     PointsDev pts;           // static points [0, n_static) plane by plane, level by level; blades after
     int64_t n_static, n_rot;
     const uint32_t* cells;   // unique static stencil cells, grouped by plane
+    int64_t n_cells;
     void* rows;              // ForceRow x 3 per point, static points first, blades after
     void* scache;            // {rho, jx, jy, jz} in T per entry of cells
     void* rcache;            // {rho, jx, jy, jz} in T x 9 per blade point
-    const PlaneDesc* planes;
+    void* fscr;              // 4 T per entry of cells, for planes whose force values exceed the LDS (or null)
+    const PlaneDesc* planes;  // longest first
     int32_t n_planes;
-    const PlaneBlock* blocks;  // team workgroups first, then the longest tasks first
-    int32_t n_blocks;
+    int32_t level_lanes, level_lds;  // workgroup of the levels launch: lanes and bytes of LDS
     const int64_t* lev_off;
-    uint32_t* bar;           // kBarWords words per team: arrivals, generation, flags, XCC ids seen
     BladeLayout blade;       // n_blades 0: no blades
-    int32_t local_teams;     // 1: a team's workgroups sit kXcds apart in blocks, so one XCD runs them
-                             // (launches deal workgroups to the XCDs in turn)
 };
-constexpr int kBarWords = 4;
-// points one pass of a plane task handles: a quad of lanes per point
-constexpr int kForcePlanePoints = 256;
-constexpr int kForcePlaneBlock = 1024;  // threads of a plane task's workgroup, at most
-// LDS of a single tank's plane-task workgroup for the force values of a solo
-// plane's static cells: 8192 cells in FP32 (6570 per plane at 512^3).  The
-// workgroup's registers already hold a CU to one workgroup.
-constexpr size_t kPlaneLdsBytes = 96 * 1024;
+// Blocks of a tank's gather launch: blade stencil cells, static stencil cells, mask words.
+constexpr int kGatherBlock = 256;
+struct GatherBlocks {
+    uint32_t blades, cells, words;
+};
+inline GatherBlocks gather_blocks(int64_t n_rot, int64_t n_cells, int64_t mask_words) {
+    auto nb = [](int64_t n) { return (uint32_t)((n + kGatherBlock - 1) / kGatherBlock); };
+    return {nb(9 * n_rot), nb(n_cells), nb(mask_words)};
+}
+// lanes of a plane's workgroup, at most (a quad per point); FP64 rows need the registers of half as many
+constexpr int kForcePlaneBlock = 1024;
+template <typename T>
+constexpr int level_block() { return sizeof(T) > 4 ? kForcePlaneBlock / 2 : kForcePlaneBlock; }
+// LDS of a blade point's three rows with their moments (BladeRow)
+constexpr int64_t blade_row_bytes(size_t tsize) { return 3 * (tsize > 4 ? 160 : 80); }
+// force values of a whole plane
+TDLB_HD inline int64_t plane_force_bytes(const Grid& g, size_t tsize) {
+    return 3 * (int64_t)g.xg1 * g.zg1 * (int64_t)tsize;
+}
 constexpr size_t kCuLdsBytes = 160 * 1024;  // LDS of a gfx950 CU
 // Workgroup of a batch's forcing planes for a mean of `cells` static stencil
 // cells per task: a lane per ~4 cells, a power of two from 128 to
@@ -186,17 +190,23 @@ inline int forcing_block_for(double cells) {
     while (t < kForcePlaneBlock && 2.0 * t <= cells / 4.0) t *= 2;
     return t;
 }
-// One forcing pass of a bound tank (every plane of fg): next must already hold
-// the static occupancy bits; blade stencil cells missing from prev get F = 0
-// and their bit in next.
-hipError_t launch_force_planes(int prec, int layout, int streaming, int momsrc, int even, const ForceGeom& fg,
-                               const void* Q, void* F, const uint64_t* prev, uint64_t* next, const Grid& g,
-                               double alfa, double beta, float rho0, hipStream_t s);
+// The gather of a bound tank's forcing pass (gb: which parts), then the levels of
+// every plane.  The gather starts next from static_base, the levels add the
+// blades' bits; blade stencil cells missing from prev get F = 0.
+hipError_t launch_force_gather(int prec, int layout, int streaming, int momsrc, int even, const ForceGeom& fg,
+                               const BladeStep& st, const GatherBlocks& gb, const void* Q, void* F,
+                               const uint64_t* prev, uint64_t* next, const uint64_t* static_base, const Grid& g,
+                               float rho0, hipStream_t s);
+hipError_t launch_force_levels(int prec, const ForceGeom& fg, void* F, uint64_t* next, const Grid& g, double alfa,
+                               double beta, hipStream_t s);
+// once per device before the first launch_force_levels
+hipError_t allow_level_lds(int prec);
 
 // ---- One Esotwist main-loop step in one persistent launch (LIJK, float
 // arithmetic): the fused stream-collide of every row, the forcing gather of
 // each row soon after the rows it reads are written (lines still in L2 or the
-// memory-side cache), then the forcing levels of every plane.  Each XCD takes
+// memory-side cache); the blade gather and the levels of every plane follow as in
+// the separate launches.  Each XCD takes
 // a contiguous range of j planes from its own work queue (the hardware XCC id
 // picks the queue), so the rows a gather reads were written through the same
 // L2; only the two edge planes of a range wait for the neighbouring XCDs.
@@ -276,13 +286,9 @@ hipError_t launch_plane_xz(int prec, int layout, const void* Q, const void* F, c
 hipError_t launch_vorticity(int prec, int layout, int streaming, int momsrc, int even, const void* Q, const Grid& g,
                             int axis, int cut, const uint8_t* exclude, void* out, float rho0, hipStream_t s);
 
-// blade points of a step into out[offset ..], their stencil rows into rows[3 offset ..]
-hipError_t launch_gen_blades(int prec, const BladeLayout& bl, const BladeStep& st, const PointsDev& out, void* rows,
-                             const Grid& g, int64_t offset, hipStream_t s);
 // stencil rows of the n static points p, from the positions sidx (9 per point) of
-// their cells in the plane-grouped list; plane_of_j: index into planes of plane j
-hipError_t launch_static_rows(int prec, const PointsDev& p, int64_t n, const int32_t* sidx, const PlaneDesc* planes,
-                              const int32_t* plane_of_j, void* rows, hipStream_t s);
+// their cells in their plane's list
+hipError_t launch_static_rows(int prec, const PointsDev& p, int64_t n, const int32_t* sidx, void* rows, hipStream_t s);
 hipError_t launch_solid_mask(double cx, double cz, double radius, uint8_t* out, const Grid& g, int ghost,
                              hipStream_t s);
 
@@ -312,6 +318,7 @@ struct MemberDev {
     uint64_t* fmask[2];
     const uint64_t* static_base;
     ForceGeom fg;            // IB points, stencil caches and plane tasks of the member
+    GatherBlocks gb;         // its blocks in the gather launch
     const BladeStep* steps;  // blade orientation of step done + 1, done + 2, ...
     int64_t n_steps;         // steps this member may still take in the batch
     // advanced on the device after every step
@@ -319,9 +326,9 @@ struct MemberDev {
     int64_t done;
 };
 
-// one workgroup of the batch's forcing launch: member and its PlaneBlock
+// one workgroup of the batch's levels launch
 struct PlaneTask {
-    int32_t member, block;
+    int32_t member, plane;
 };
 
 // Device tables of one batch step.  off_* are member prefix sums (n_members + 1
@@ -333,18 +340,17 @@ struct BatchPlan {
     int32_t n_members;
     const int64_t* off_coll;   // blocks of the fused kernel
     const int32_t* coll_member;  // member of each block of the fused kernel (or null: search off_coll)
-    const int64_t* off_rot;    // blade points
-    const int64_t* off_words;  // occupancy-mask words
+    const int64_t* off_gather;     // blocks of the gather
+    const int32_t* gather_member;  // member of each of them
     const PlaneTask* tasks;
-    int64_t tot_coll, tot_rot, tot_words, n_tasks;
+    int64_t tot_coll, tot_gather, n_tasks;
     int32_t bs;  // threads per block of the fused kernel (256 or 512)
-    int32_t force_bs;  // threads per workgroup of the forcing pass (64 .. kForcePlaneBlock, a multiple of 64)
+    int32_t force_bs;  // lanes per workgroup of the levels (64 .. kForcePlaneBlock, a multiple of 64)
     int64_t force_lds_bytes;  // LDS of a plane task's workgroup for force values and moments (0: none)
 };
 
-// Enqueue `steps` main-loop steps of every active member: per step blade
-// generation, the fused stream-collide, the static occupancy bits, the forcing
-// planes, advance.
+// Enqueue `steps` main-loop steps of every active member: per step the fused
+// stream-collide, the forcing gather, the forcing levels, advance.
 hipError_t launch_batch_step(int prec, int layout, int streaming, const BatchPlan& plan, int steps, hipStream_t s);
 // blocks of the fused kernel for one member with the given tile and block size
 int64_t batch_coll_blocks(const Grid& g, int tile, int bs);

@@ -1328,78 +1328,22 @@ __global__ __launch_bounds__(kBlock) void k_force_level_cached(PointsDev p, int6
 }
 
 // ------------------------------------------------------------------ IB forcing by planes
-// A bound tank's forcing pass as independent plane tasks (ForceGeom in
-// kernels.h).  A task first clears F and sets the occupancy bit of the blade
-// stencil cells missing from the previous mask (prepare_point) and computes the
-// density and momentum of its static and blade stencil cells; then it runs its
-// static levels and its blade levels in order, passes of up to kPlanePoints
-// points per workgroup, a quad of lanes per point (force_row), with a barrier
-// after every level: the sequential list order of Forcing.hpp:73-135 within the
-// plane, without a kernel launch per level.  A plane with many
-// points runs on a team of workgroups that meet at a barrier in global memory
-// (team_barrier); teams are the first workgroups of the launch, so they are
-// dispatched, and resident, before any other workgroup of it.
-constexpr int kPlaneBlock = kForcePlaneBlock;
-constexpr int kPlanePoints = kPlaneBlock / 4;
-static_assert(kPlanePoints == kForcePlanePoints, "points per pass of a plane task");
-// polls of a team barrier before it gives up and flags a time-out (about a
-// second; every member of a team is resident, so a healthy barrier takes
-// microseconds)
-constexpr uint32_t kBarSpinLimit = 1u << 20;
-
-// Sense-reversing barrier of a team of workgroups: bar[0] counts arrivals,
-// bar[1] is the generation, bar[2] the time-out flag.  The last arrival resets
-// the count (waiting for that reset to complete) and then advances the
-// generation, so the barrier is ready for the next level and the next launch.
-// Every wave waits for its own stores before the workgroup barrier that
-// precedes the arrival: the barrier itself does not wait for them, and the
-// arriving thread's fence covers only its own wave's stores, so a store of
-// another wave could otherwise still be on its way to another L2 channel when
-// the arrival is seen.  Local teams (every member on one XCD,
-// ForceGeom::local_teams) exchange F and the caches through that XCD's L2, and
-// each CU drops its L1 after the wait, with an invalidate at device scope (at
-// work-group scope it leaves the L1 alone when work-groups are not split across
-// CUs, and a member would read back F lines it cached before another member
-// wrote them); the last arrival checks that every member reported the same XCC
-// id (bar[2] bit 2 otherwise).  Other teams fence at agent scope (L2
-// write-back before the arrival, invalidation after the wait).  The wait polls
-// with relaxed loads (an acquire load would invalidate the L2 on every poll).
-__device__ __forceinline__ void team_barrier(uint32_t* bar, int team, bool local) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        if (!local) __threadfence();
-        if (local) {
-            // bar[3] collects the XCC ids of the arrivals: one XCD must run the team
-            uint32_t x;
-            asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(x));
-            (void)__hip_atomic_fetch_or(&bar[3], 1u << (x & 15u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
-        const uint32_t gen = __hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (__hip_atomic_fetch_add(&bar[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)team - 1) {
-            if (local) {
-                const uint32_t seen = __hip_atomic_exchange(&bar[3], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (__builtin_popcount(seen) != 1) atomicOr(&bar[2], 2u);
-            }
-            __hip_atomic_exchange(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __hip_atomic_store(&bar[1], gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            uint32_t spins = 0;
-            while (__hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen) {
-                if (++spins >= kBarSpinLimit) {
-                    atomicOr(&bar[2], 1u);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(2);
-            }
-        }
-        if (!local) __threadfence();
-    }
-    __syncthreads();
-    if (local) asm volatile("buffer_inv sc1" ::: "memory");
-}
+// A bound tank's forcing pass in two launches (ForceGeom in kernels.h).  The
+// gather (force_gather) spreads over the whole chip: it generates the step's
+// blade points and their stencil rows, starts the next occupancy mask from the
+// static bits, clears F of blade cells missing from the previous mask
+// (prepare_point), and writes density and momentum of every static and blade
+// stencil cell to their caches.  It is bound by the lines of its scattered
+// population reads.  The levels (plane_levels) are one workgroup per j plane,
+// the sequential list order of Forcing.hpp:73-135 within the plane: static
+// levels, then blade levels, passes of a point per quad of lanes with a barrier
+// after every level, bound by the latency of that chain.  Gathering inside the
+// plane's workgroup instead left the gather to one CU per plane (96 of 256 CUs
+// at 96^3: 12 us) and, beyond 256 planes, to rounds of workgroups; a plane with
+// many points then needed several workgroups meeting at barriers in HBM (24^3: 205
+// us).  Whole pass, gather and levels in one -> two launches: 24^3 205 -> 33 us,
+// 60^3 41 -> 29, 96^3 47 -> 37, 192^3 FP64 219 -> 132, 256^3 226 -> 166, 512^3
+// 597 -> 549 (gather 390, 5.1 TB/s of lines; levels 140).
 
 // ---- A point of a plane task on a quad of lanes: lane c = 0..2 of the quad
 // takes stencil row k1 = c - 1 (cells s = 3c + m for i1 = m - 1), lane 3 repeats
@@ -1481,20 +1425,16 @@ __device__ __forceinline__ ForceRow<T> make_row(T ifr, T kfr, int c, T vel) {
 }
 
 // ForceRow of every static point: e[m] = the cell's entry in its plane's list
-// (cell_of maps the point to its plane's first entry)
 template <typename T>
-__global__ void k_static_rows(PointsDev p, int64_t n, const int32_t* __restrict__ sidx,
-                              const PlaneDesc* __restrict__ planes, const int32_t* __restrict__ plane_of_j,
-                              ForceRow<T>* __restrict__ rows) {
+__global__ void k_static_rows(PointsDev p, int64_t n, const int32_t* __restrict__ sidx, ForceRow<T>* __restrict__ rows) {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (t >= 3 * n) return;
     const int64_t q = t / 3;
     const int c = (int)(t - 3 * q);
     const T* vel = static_cast<const T*>(c == 0 ? p.u : c == 1 ? p.v : p.w);
     ForceRow<T> r = make_row<T>(static_cast<const T*>(p.ifrac)[q], static_cast<const T*>(p.kfrac)[q], c, vel[q]);
-    const int64_t first = planes[plane_of_j[p.j[q]]].cell_begin;
 #pragma unroll
-    for (int m = 0; m < 3; m++) r.e[m] = (int32_t)(sidx[9 * q + 3 * c + m] - first);
+    for (int m = 0; m < 3; m++) r.e[m] = sidx[9 * q + 3 * c + m];
     rows[t] = r;
 }
 
@@ -1543,6 +1483,17 @@ __device__ __forceinline__ int level_index(const BladeLevel& v, int t, int bp) {
     const int s = t / v.nr, ri = t - s * v.nr;
     return blade_index(v.e, v.first + s * v.stride, v.rmod + 5 * ri, bp);
 }
+// position of radial point r of blade b among the plane's points in level order
+__device__ __forceinline__ int level_slot(const BladeLayout& bl, int b, int r) {
+    const BladeEnum e = blade_enum_of(bl);
+    const int groups = bl.merged ? 1 : e.n_bcol, grp = b % groups, bi = b / groups, rmod = r % 5;
+    const int nb = (e.n_blades - grp + groups - 1) / groups;
+    int before = 0;
+    for (int a = 0; a < grp; a++) before += (e.n_blades - a + groups - 1) / groups;
+    before *= e.n_radial;
+    for (int a = 0; a < rmod; a++) before += nb * (e.n_radial > a ? (e.n_radial - a + 4) / 5 : 0);
+    return before + bi * ((e.n_radial - rmod + 4) / 5) + r / 5;
+}
 // blade plane index of plane j and its blade levels (0: no blades)
 __device__ __forceinline__ int blade_plane(const ForceGeom& fg, int j, int& nlev) {
     const BladeLayout& bl = fg.blade;
@@ -1559,288 +1510,416 @@ __device__ __forceinline__ void gather_cells(const ForceGeom& fg, int64_t c0, in
                                              float rho0) {
     auto* scache = static_cast<Mom4<typename PR::T>*>(fg.scache);
     for (int64_t e = c0 + t; e < c1; e += threads) {
-        int i, j, k;
-        decode_cell(g, fg.cells[e], i, j, k);
+        const uint32_t n = fg.cells[e];  // below 2^31: 32-bit divisions
+        const int i = (int)(n / g.yz);
+        const uint32_t r = n - (uint32_t)i * g.yz;
+        const int j = (int)(r / (uint32_t)g.zg), k = (int)(r - (uint32_t)j * (uint32_t)g.zg);
         Mom4<typename PR::T> m;
         cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, m.r, m.x, m.y, m.z, rho0);
         scache[e] = m;
     }
 }
 
-// Blade stencil cells of plane j: occupancy bit in next, F = 0 where the
-// previous mask lacks the cell (prepare_point), density and momentum into the
-// blade cache.
+// Stencil cell s of blade point t / 9 (s = t % 9; points blade by blade, plane by
+// plane): the point from the step's blade orientation (blade_point, the host
+// generator's arithmetic), by its first lanes also to the point list and the
+// stencil rows; F = 0 where the previous mask lacks the cell; density and
+// momentum into the blade cache.
 template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
-__device__ void gather_blades(const ForceGeom& fg, int j, int t0, int threads,
-                              const typename PR::S* __restrict__ Q, typename PR::T* __restrict__ F,
-                              const uint64_t* __restrict__ prev, uint64_t* __restrict__ next, const Grid& g,
-                              float rho0) {
+__device__ __forceinline__ void gather_blade_cell(const ForceGeom& fg, const BladeStep& st, int t,
+                                                  const typename PR::S* __restrict__ Q,
+                                                  typename PR::T* __restrict__ F, const uint64_t* __restrict__ prev,
+                                                  const Grid& g, float rho0) {
     using T = typename PR::T;
-    auto* rcache = static_cast<Mom4<T>*>(fg.rcache);
-    int nlev;
-    const int bp = blade_plane(fg, j, nlev);
-    if (nlev == 0) return;
-    const BladeEnum be = blade_enum_of(fg.blade);
-    const int n9 = 9 * be.n_blades * be.n_radial;
-    for (int t = t0; t < n9; t += threads) {
-        const int pt = t / 9, s = t - 9 * pt;
-        const int b = pt / be.n_radial, e = blade_index(be, b, pt - b * be.n_radial, bp);
-        const int64_t q = fg.n_static + e;
-        const int i2 = wrap_ik(fg.pts.i[q] + (s % 3) - 1, g.xg1), k2 = wrap_ik(fg.pts.k[q] + (s / 3) - 1, g.zg1);
-        if (!mask_test(prev, g, i2, j, k2)) {
-            const uint64_t cc = cell_index(g, i2, j, k2);
-            F[3 * cc + 0] = T(0);
-            F[3 * cc + 1] = T(0);
-            F[3 * cc + 2] = T(0);
-        }
-        atomicOr((unsigned long long*)&next[mask_word_index(g, i2, j, k2)], 1ull << (k2 & 63));
-        Mom4<T> m;
-        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i2, j, k2, m.r, m.x, m.y, m.z, rho0);
-        rcache[9 * (int64_t)e + s] = m;
+    const BladeLayout& bl = fg.blade;
+    const BladeEnum be = blade_enum_of(bl);
+    const int pt = t / 9, s = t - 9 * pt, c = s / 3;
+    const int u = pt / be.n_radial, r = pt - u * be.n_radial, b = u / be.n_planes, pl = u - b * be.n_planes;
+    const int e = blade_index(be, b, r, pl);
+    tdlb_ib_point p;
+    blade_point(bl.cx, bl.cz, bl.r_inner, bl.j_lo + pl, r, st.cosb[b], st.sinb[b], st.omega, &p);
+    const int i = (int)p.i + bl.ghost, j = (int)p.j + bl.ghost, k = (int)p.k + bl.ghost;
+    const int64_t q = fg.n_static + e;
+    if (s == 0) {
+        fg.pts.i[q] = i;
+        fg.pts.j[q] = j;
+        fg.pts.k[q] = k;
+        static_cast<T*>(fg.pts.ifrac)[q] = (T)p.i_frac;
+        static_cast<T*>(fg.pts.kfrac)[q] = (T)p.k_frac;
+        static_cast<T*>(fg.pts.u)[q] = (T)p.u_delta;
+        static_cast<T*>(fg.pts.v)[q] = (T)p.v_delta;
+        static_cast<T*>(fg.pts.w)[q] = (T)p.w_delta;
     }
+    if (s == 3 * c) {
+        ForceRow<T> row = make_row<T>((T)p.i_frac, (T)p.k_frac, c,
+                                      (T)(c == 0 ? p.u_delta : c == 1 ? p.v_delta : p.w_delta));
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+            row.e[m] = (int32_t)cell_index(g, wrap_ik(i + m - 1, g.xg1), j, wrap_ik(k + c - 1, g.zg1));
+        static_cast<ForceRow<T>*>(fg.rows)[3 * q + c] = row;
+    }
+    const int i2 = wrap_ik(i + (s - 3 * c) - 1, g.xg1), k2 = wrap_ik(k + c - 1, g.zg1);
+    if (!mask_test(prev, g, i2, j, k2)) {
+        const uint64_t cc = cell_index(g, i2, j, k2);
+        F[3 * cc + 0] = T(0);
+        F[3 * cc + 1] = T(0);
+        F[3 * cc + 2] = T(0);
+    }
+    Mom4<T> m;
+    cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i2, j, k2, m.r, m.x, m.y, m.z, rho0);
+    static_cast<Mom4<T>*>(fg.rcache)[9 * (int64_t)e + s] = m;
 }
 
-// The plane's static levels by workgroup `rank` of a team of `team`, passes of a
-// point per quad of lanes, with sync() after every level.  Each pass loads the
-// next pass's rows before it computes (the rows do not change during the pass).
-// lm: the moments, by entry of the plane, in LDS or the cache in HBM; lf: the
-// force values by entry in LDS, or null: in F.
-template <typename T, typename Sync>
-__device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDesc& pd, int rank, int team,
-                                              const Mom4<T>* lm, T* lf, T* __restrict__ F, T alfa, T beta,
-                                              Sync&& sync) {
-    const ForceRow<T>* __restrict__ rows = static_cast<const ForceRow<T>*>(fg.rows);
+// Block b of a tank's gather: the blades' blocks first (their points cost the
+// most arithmetic), then the static cells', then the mask words'.
+template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+__device__ __forceinline__ void force_gather(const ForceGeom& fg, const BladeStep& st, uint32_t b,
+                                             const GatherBlocks& gb, const typename PR::S* __restrict__ Q,
+                                             typename PR::T* __restrict__ F, const uint64_t* __restrict__ prev,
+                                             uint64_t* __restrict__ next, const uint64_t* __restrict__ static_base,
+                                             const Grid& g, float rho0) {
+    if (b < gb.blades) {
+        const int64_t t = (int64_t)b * kGatherBlock + threadIdx.x;
+        if (t < 9 * fg.n_rot)
+            gather_blade_cell<PR, L, STREAM, MOMSRC, EVEN>(fg, st, (int)t, Q, F, prev, g, rho0);
+        return;
+    }
+    b -= gb.blades;
+    if (b < gb.cells) {
+        const int64_t e = (int64_t)b * kGatherBlock + threadIdx.x;
+        gather_cells<PR, L, STREAM, MOMSRC, EVEN>(fg, e, min(e + 1, fg.n_cells), 0, 1, Q, g, rho0);
+        return;
+    }
+    const uint64_t w = (uint64_t)(b - gb.cells) * kGatherBlock + threadIdx.x;
+    if (w < (uint64_t)g.xg * g.yg * g.mask_w) next[w] = static_base[w];
+}
+
+template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+__global__ __launch_bounds__(kGatherBlock) void k_force_gather(ForceGeom fg, BladeStep st, GatherBlocks gb,
+                                                               const typename PR::S* __restrict__ Q,
+                                                               typename PR::T* __restrict__ F,
+                                                               const uint64_t* __restrict__ prev,
+                                                               uint64_t* __restrict__ next,
+                                                               const uint64_t* __restrict__ static_base, Grid g,
+                                                               float rho0) {
+    force_gather<PR, L, STREAM, MOMSRC, EVEN>(fg, st, blockIdx.x, gb, Q, F, prev, next, static_base, g, rho0);
+}
+
+// a copy that every lane knows to be the same for the whole wave (scalar registers)
+template <typename X>
+__device__ __forceinline__ X uniform_copy(const X& x) {
+    static_assert(sizeof(X) % 4 == 0, "words");
+    struct Words {
+        int w[sizeof(X) / 4];
+    };
+    Words a = __builtin_bit_cast(Words, x);
+#pragma unroll
+    for (size_t t = 0; t < sizeof(X) / 4; t++) a.w[t] = __builtin_amdgcn_readfirstlane(a.w[t]);
+    return __builtin_bit_cast(X, a);
+}
+
+// The plane's static levels, passes of a point per quad of lanes, with a barrier
+// after every level.  Rows are loaded two passes ahead and moments in HBM one
+// pass ahead: neither changes during the pass.  lm: the moments by entry of the
+// plane, in LDS (MOM_LDS) or the cache in HBM; the force values by entry: lf in
+// LDS (F_LDS), else four T an entry in the plane's scratch fs.  Loads return in
+// order, so in HBM a pass asks for its force values before the rows and moments
+// of later passes, and within a level for the next pass's before it stores its own.
+template <typename T, bool MOM_LDS, bool F_LDS>
+__device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDesc& pd, const Mom4<T>* lm, T* lf,
+                                              Mom4<T>* fs, T alfa, T beta) {
+    const ForceRow<T>* rows = static_cast<const ForceRow<T>*>(fg.rows);
     const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), c = min(lane, 2);
-    const int per = (int)(blockDim.x >> 2), p0 = rank * per, pstride = team * per;
-    const int nlev = pd.n_levels;
-    const int64_t* __restrict__ off = fg.lev_off + pd.lev;
+    const int per = (int)(blockDim.x >> 2), nlev = pd.n_levels;
+    // Level ends without a load in the loop, whose wait would include every load
+    // before it: lane i of the wave holds the end of level base + i.
+    const int64_t* off = fg.lev_off + pd.lev;
+    const int64_t q0 = off[0];
+    int base = 0, ends = 0;
+    auto hold = [&](int l) {
+        base = l;
+        ends = (int)(off[min(l + (int)(threadIdx.x & 63), nlev - 1) + 1] - q0);
+    };
+    auto level_end = [&](int l) {
+        if (l - base >= 64) hold(l);
+        return __builtin_amdgcn_readlane(ends, l - base);
+    };
+    if (nlev > 0) hold(0);
+    rows += 3 * q0;
     struct Pass {
+        int l;       // level, nlev after the last
+        int q, end;  // first point, end of the level
+    };
+    auto next = [&](Pass a) {
+        if (a.l >= nlev) return a;
+        if (a.q + per < a.end) return Pass{a.l, a.q + per, a.end};
+        return Pass{a.l + 1, a.end, a.l + 1 < nlev ? level_end(a.l + 1) : a.end};
+    };
+    struct Row {
         ForceRow<T> r;
-        uint32_t cell[3];  // cell_index of the entries (force values in F only)
+        Mom4<T> mo[MOM_LDS ? 1 : 3];
         bool ok;
     };
-    auto load = [&](int l, int64_t q) {
-        Pass a{};
-        a.ok = l < nlev && q + slot < off[l + 1];
-        if (a.ok) {
-            a.r = rows[3 * (q + slot) + c];
-            if (!lf)
+    auto load = [&](Pass a) {
+        Row x{};
+        x.ok = a.l < nlev && a.q + slot < a.end;
+        if (x.ok) x.r = rows[3 * (int64_t)(a.q + slot) + c];
+        return x;
+    };
+    auto complete = [&](Row& x) {
+        if constexpr (!MOM_LDS)
+            if (x.ok)
 #pragma unroll
-                for (int m = 0; m < 3; m++) a.cell[m] = fg.cells[pd.cell_begin + a.r.e[m]];
-        }
-        return a;
+                for (int m = 0; m < 3; m++) x.mo[m] = lm[x.r.e[m]];
     };
-    // the first pass of this workgroup at or after level l: empty levels still end with a sync
-    auto skip = [&](int l) {
-        while (l < nlev && off[l] + p0 >= off[l + 1]) l++;
-        return l;
+    struct Force {
+        T f[3][3];
     };
-    int l = skip(0);
-    for (int k = 0; k < l; k++) sync();
-    int64_t q = l < nlev ? off[l] + p0 : 0;
-    Pass cur = load(l, q);
-    while (l < nlev) {
-        int nl = l;
-        int64_t nq = q + pstride;
-        if (nq >= off[l + 1]) {
-            nl = skip(l + 1);
-            nq = nl < nlev ? off[nl] + p0 : 0;
+    auto fetch = [&](const Row& x, Force& v) {
+        if (!x.ok) return;
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            const int e = x.r.e[m];
+            if constexpr (F_LDS) {
+#pragma unroll
+                for (int a = 0; a < 3; a++) v.f[m][a] = lf[3 * e + a];
+            } else {
+                const Mom4<T> w = fs[e];
+                v.f[m][0] = w.r;
+                v.f[m][1] = w.x;
+                v.f[m][2] = w.y;
+            }
         }
-        const Pass nxt = load(nl, nq);
-        if (cur.ok) {
+    };
+    Pass a0{0, 0, nlev > 0 ? level_end(0) : 0}, a1 = next(a0);
+    Row r0 = load(a0), r1 = load(a1);
+    complete(r0);
+    Force v0{}, v1{};
+    bool have = false;  // v0 was asked for in the pass before
+    while (a0.l < nlev) {
+        if (F_LDS || !have) fetch(r0, v0);
+        const Pass a2 = next(a1);
+        const bool same = a1.l == a0.l;
+        if constexpr (!F_LDS) {
+            if (same) fetch(r1, v1);
+        }
+        complete(r1);
+        __builtin_amdgcn_sched_barrier(0);  // the rows behind them: no wait for moments or forces includes theirs
+        Row r2 = load(a2);
+        if (r0.ok) {
             Mom4<T> mo[3];
-            T f[3][3];
 #pragma unroll
             for (int m = 0; m < 3; m++) {
-                const T* fp = lf ? lf + 3 * cur.r.e[m] : F + 3 * (uint64_t)cur.cell[m];
-                mo[m] = lm[cur.r.e[m]];
-                f[m][0] = fp[0];
-                f[m][1] = fp[1];
-                f[m][2] = fp[2];
+                if constexpr (MOM_LDS) mo[m] = lm[r0.r.e[m]];
+                else mo[m] = r0.mo[m];
             }
-            force_row(cur.r, mo, f, alfa, beta);
+            force_row(r0.r, mo, v0.f, alfa, beta);
             if (lane < 3)
 #pragma unroll
                 for (int m = 0; m < 3; m++) {
-                    T* fp = lf ? lf + 3 * cur.r.e[m] : F + 3 * (uint64_t)cur.cell[m];
-                    fp[0] = f[m][0];
-                    fp[1] = f[m][1];
-                    fp[2] = f[m][2];
+                    const int e = r0.r.e[m];
+                    if constexpr (F_LDS) {
+#pragma unroll
+                        for (int a = 0; a < 3; a++) lf[3 * e + a] = v0.f[m][a];
+                    } else {
+                        fs[e] = Mom4<T>{v0.f[m][0], v0.f[m][1], v0.f[m][2], T(0)};
+                    }
                 }
         }
-        for (int k = l; k < nl; k++) sync();  // levels l .. nl - 1 are done
-        l = nl;
-        q = nq;
-        cur = nxt;
+        if (!same) __syncthreads();
+        a0 = a1;
+        a1 = a2;
+        r0 = r1;
+        r1 = r2;
+        if constexpr (!F_LDS) {
+            v0 = v1;
+            have = same;
+        }
     }
 }
 
-// The plane's blade levels, as static_levels: force values in F, moments in the
-// blade cache, the next level's rows and moments loaded a level ahead.
-template <typename T, typename Sync>
-__device__ __forceinline__ void blade_levels(const ForceGeom& fg, int j, int rank, int team, T* __restrict__ F,
-                                             T alfa, T beta, Sync&& sync) {
-    int nlev;
-    const int bp = blade_plane(fg, j, nlev);
-    if (nlev == 0) return;
+// cell n of plane j in the plane's own (i, k) order
+__device__ __forceinline__ int plane_index(const Grid& g, uint32_t n, int j) {
+    const int i = (int)(n / g.yz), k = (int)(n - (uint32_t)i * g.yz - (uint32_t)j * (uint32_t)g.zg);
+    return (i - 1) * g.zg1 + k - 1;
+}
+
+// The blade levels of a plane.  With room in LDS the rows and moments of all its
+// points come there first, in level order, and if a copy of the whole plane's
+// force values fits beside them the stencil cells' too: a level then waits on
+// LDS alone (1.7 us a level from the caches, most of it the latency of the next
+// rows).  Otherwise the force values stay in F, and without any room the rows and
+// moments in the caches.
+template <typename T>
+struct BladeRow {
+    ForceRow<T> r;
+    Mom4<T> mo[3];
+};
+static_assert(3 * sizeof(BladeRow<float>) == blade_row_bytes(4) && 3 * sizeof(BladeRow<double>) == blade_row_bytes(8), "LDS");
+template <typename T, bool ROWS_LDS, bool F_LDS>
+__device__ __forceinline__ void blade_levels(const ForceGeom& fg, const Grid& g, int j, int bp, int nlev,
+                                             T* __restrict__ F, uint64_t* __restrict__ next, BladeRow<T>* lr, T* ld,
+                                             T alfa, T beta) {
     const ForceRow<T>* __restrict__ rows = static_cast<const ForceRow<T>*>(fg.rows) + 3 * fg.n_static;
     const Mom4<T>* __restrict__ cache = static_cast<const Mom4<T>*>(fg.rcache);
     const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), c = min(lane, 2);
-    const int per = (int)(blockDim.x >> 2), p0 = rank * per, pstride = team * per;
+    const int per = (int)(blockDim.x >> 2);
+    // the occupancy bits of the rows' cells, and what the levels need in LDS, rows in level order
+    const BladeEnum be = blade_enum_of(fg.blade);
+    const int n3 = 3 * be.n_blades * be.n_radial;
+    for (int t = (int)threadIdx.x; t < n3; t += (int)blockDim.x) {
+        const int pt = t / 3, row = t - 3 * pt, b = pt / be.n_radial, r = pt - b * be.n_radial;
+        const int64_t e = blade_index(be, b, r, bp);
+        BladeRow<T> x;
+        x.r = rows[3 * e + row];
+        if constexpr (ROWS_LDS)
+#pragma unroll
+            for (int m = 0; m < 3; m++) x.mo[m] = cache[9 * e + 3 * row + m];
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            const uint32_t n = (uint32_t)x.r.e[m];
+            const int i = (int)(n / g.yz), k = (int)(n - (uint32_t)i * g.yz - (uint32_t)j * (uint32_t)g.zg);
+            atomicOr((unsigned long long*)&next[mask_word_index(g, i, j, k)], 1ull << (k & 63));
+            if constexpr (F_LDS) {
+                x.r.e[m] = (i - 1) * g.zg1 + k - 1;
+#pragma unroll
+                for (int a = 0; a < 3; a++) ld[3 * x.r.e[m] + a] = F[3 * (uint64_t)n + a];
+            }
+        }
+        if constexpr (ROWS_LDS) lr[3 * level_slot(fg.blade, b, r) + row] = x;
+    }
+    if constexpr (ROWS_LDS) __syncthreads();
     struct Pass {
         ForceRow<T> r;
         Mom4<T> mo[3];
         bool ok;
     };
-    auto load = [&](int l, int t) {
+    auto load = [&](int l, int at, int t) {
         Pass a{};
         if (l >= nlev) return a;
         const BladeLevel v = blade_level(fg.blade, l);
         a.ok = t < v.count;
         if (a.ok) {
-            const int64_t e = level_index(v, t, bp);
-            a.r = rows[3 * e + c];
+            if constexpr (ROWS_LDS) {
+                const BladeRow<T>& x = lr[3 * (at + t) + c];
+                a.r = x.r;
 #pragma unroll
-            for (int m = 0; m < 3; m++) a.mo[m] = cache[9 * e + 3 * c + m];
+                for (int m = 0; m < 3; m++) a.mo[m] = x.mo[m];
+            } else {
+                const int64_t e = level_index(v, t, bp);
+                a.r = rows[3 * e + c];
+#pragma unroll
+                for (int m = 0; m < 3; m++) a.mo[m] = cache[9 * e + 3 * c + m];
+            }
         }
         return a;
     };
-    auto count = [&](int l) { return blade_level(fg.blade, l).count; };
-    int l = 0, u = p0;
-    Pass cur = load(0, u + slot);
-    while (l < nlev) {
-        int nl = l, nu = u + pstride;
-        if (nu >= count(l)) {
-            nl = l + 1;
-            nu = p0;
-        }
-        const Pass nxt = load(nl, nu + slot);
-        if (cur.ok) {
-            T f[3][3];
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                const T* fp = F + 3 * (uint64_t)(uint32_t)cur.r.e[m];
-                f[m][0] = fp[0];
-                f[m][1] = fp[1];
-                f[m][2] = fp[2];
-            }
-            force_row(cur.r, cur.mo, f, alfa, beta);
-            if (lane < 3)
+    for (int l = 0, at = 0; l < nlev; l++) {
+        const int count = blade_level(fg.blade, l).count;  // 0 with fewer than 5 radial points
+        for (int u = 0; u < count; u += per) {
+            const Pass cur = load(l, at, u + slot);
+            if (cur.ok) {
+                T f[3][3];
+                uint64_t p[3];
 #pragma unroll
                 for (int m = 0; m < 3; m++) {
-                    T* fp = F + 3 * (uint64_t)(uint32_t)cur.r.e[m];
-                    fp[0] = f[m][0];
-                    fp[1] = f[m][1];
-                    fp[2] = f[m][2];
+                    p[m] = 3 * (uint64_t)(uint32_t)cur.r.e[m];
+#pragma unroll
+                    for (int a = 0; a < 3; a++) f[m][a] = F_LDS ? ld[(int)p[m] + a] : F[p[m] + a];
                 }
+                force_row(cur.r, cur.mo, f, alfa, beta);
+                if (lane < 3)
+#pragma unroll
+                    for (int m = 0; m < 3; m++)
+#pragma unroll
+                        for (int a = 0; a < 3; a++) {
+                            if constexpr (F_LDS) ld[(int)p[m] + a] = f[m][a];
+                            else F[p[m] + a] = f[m][a];
+                        }
+            }
         }
-        if (nl != l) sync();
-        l = nl;
-        u = nu;
-        cur = nxt;
+        if (count > 0) __syncthreads();
+        at += count;
+    }
+    if constexpr (F_LDS) {
+        // back to F, once per point and cell: points that share a cell write the same value
+        const int n9 = 9 * fg.blade.n_blades * fg.blade.n_radial;
+        for (int t = (int)threadIdx.x; t < n9; t += (int)blockDim.x) {
+            const int pr = t / 3, p = lr[pr].r.e[t - 3 * pr];
+            const int i = p / g.zg1, k = p - i * g.zg1;
+            const uint64_t n = cell_index(g, i + 1, j, k + 1);
+#pragma unroll
+            for (int a = 0; a < 3; a++) F[3 * n + a] = ld[3 * p + a];
+        }
     }
 }
 
-// Workgroup `rank` of the plane's team.  A solo plane whose static cells fit
-// keeps their force values in LDS through the static levels, and their moments
-// too when both fit (every stencil cell of a plane task lies in its own plane,
-// which no other task touches): a level then waits on LDS alone.  The blade
-// cells' zeroing does not reach a static cell that holds a force value: the
-// static cells are in the previous mask, or were cleared before the pass.
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
-__device__ void force_plane(const ForceGeom& fg, const PlaneDesc& pd, int rank,
-                            const typename PR::S* __restrict__ Q, typename PR::T* __restrict__ F,
-                            const uint64_t* __restrict__ prev, uint64_t* __restrict__ next, const Grid& g,
-                            typename PR::T alfa, typename PR::T beta, float rho0, void* lds_buf, int64_t lds_bytes) {
-    using T = typename PR::T;
-    const int team = pd.team;
-    uint32_t* bar = team > 1 ? fg.bar + kBarWords * pd.bar : nullptr;
-    const int t0 = rank * (int)blockDim.x + (int)threadIdx.x, threads = team * (int)blockDim.x;
-    const bool local = fg.local_teams != 0;
-    auto sync = [&]() {
-        if (team > 1) team_barrier(bar, team, local);
-        else __syncthreads();
-    };
-    const int nc = (int)(pd.cell_end - pd.cell_begin);
+// The levels of one plane by one workgroup.  Every stencil cell of a plane lies
+// in the plane, which no other workgroup touches, so the force values of the
+// static cells leave F for the static levels: to LDS, with the moments when both
+// fit, else to the plane's scratch in HBM.
+template <typename T>
+__device__ __forceinline__ void plane_levels(const ForceGeom& fg, const PlaneDesc* plane, T* __restrict__ F,
+                                             uint64_t* __restrict__ next, const Grid& g, T alfa, T beta, void* lds,
+                                             int64_t lds_bytes) {
+    const PlaneDesc pd = uniform_copy(*plane);
+    const int tid = (int)threadIdx.x, nt = (int)blockDim.x, nc = (int)(pd.cell_end - pd.cell_begin);
     const int64_t mom_bytes = (int64_t)nc * sizeof(Mom4<T>), f_bytes = (int64_t)nc * 3 * sizeof(T);
-    const bool in_lds = lds_buf && team == 1 && f_bytes <= lds_bytes;
-    const bool mom_lds = in_lds && mom_bytes + f_bytes <= lds_bytes;
-    auto* gm = static_cast<Mom4<T>*>(fg.scache) + pd.cell_begin;
-    auto* lm = static_cast<Mom4<T>*>(lds_buf);
-    T* lf = mom_lds ? reinterpret_cast<T*>(lm + nc) : static_cast<T*>(lds_buf);
+    const bool f_lds = f_bytes <= lds_bytes, mom_lds = mom_bytes + f_bytes <= lds_bytes;
+    const auto* gm = static_cast<const Mom4<T>*>(fg.scache) + pd.cell_begin;
+    auto* fs = static_cast<Mom4<T>*>(fg.fscr) + pd.cell_begin;
+    auto* lm = static_cast<Mom4<T>*>(lds);
+    T* lf = mom_lds ? reinterpret_cast<T*>(lm + nc) : static_cast<T*>(lds);
     const uint32_t* __restrict__ cells = fg.cells + pd.cell_begin;
-    for (int e = t0; e < nc; e += threads) {
-        const uint32_t n = cells[e];
-        const int i = (int)(n / g.yz), k = (int)(n - (uint32_t)i * g.yz - (uint32_t)pd.j * (uint32_t)g.zg);
+    for (int e = tid; e < nc; e += nt) {
+        const uint64_t n = cells[e];
         T f[3];
-        if (in_lds)
 #pragma unroll
-            for (int a = 0; a < 3; a++) f[a] = F[3 * (uint64_t)n + a];
-        Mom4<T> m;
-        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i, pd.j, k, m.r, m.x, m.y, m.z, rho0);
-        if (mom_lds) lm[e] = m;
-        else gm[e] = m;
-        if (in_lds)
+        for (int a = 0; a < 3; a++) f[a] = F[3 * n + a];
+        if (mom_lds) lm[e] = gm[e];
+        if (f_lds)
 #pragma unroll
             for (int a = 0; a < 3; a++) lf[3 * e + a] = f[a];
+        else fs[e] = Mom4<T>{f[0], f[1], f[2], T(0)};
     }
-    gather_blades<PR, L, STREAM, MOMSRC, EVEN>(fg, pd.j, t0, threads, Q, F, prev, next, g, rho0);
-    sync();
-    // the three homes of moments and force values are loops of their own, each with one address space
-    if (mom_lds) static_levels<T>(fg, pd, 0, 1, lm, lf, F, alfa, beta, sync);
-    else if (in_lds) static_levels<T>(fg, pd, 0, 1, gm, lf, F, alfa, beta, sync);
-    else static_levels<T>(fg, pd, rank, team, gm, (T*)nullptr, F, alfa, beta, sync);
-    if (in_lds) {
-        // every static level ended with a barrier: the force values back to F before the blade levels read it
-        for (int e = (int)threadIdx.x; e < nc; e += (int)blockDim.x) {
-            const uint64_t n = cells[e];
+    __syncthreads();
+    if (mom_lds) static_levels<T, true, true>(fg, pd, lm, lf, nullptr, alfa, beta);
+    else if (f_lds) static_levels<T, false, true>(fg, pd, gm, lf, nullptr, alfa, beta);
+    else static_levels<T, false, false>(fg, pd, gm, nullptr, fs, alfa, beta);
+    // every static level ended with a barrier: the force values back to F before the blade levels read it
+    for (int e = tid; e < nc; e += nt) {
+        const uint64_t n = cells[e];
+        if (f_lds) {
 #pragma unroll
             for (int a = 0; a < 3; a++) F[3 * n + a] = lf[3 * e + a];
+        } else {
+            const Mom4<T> v = fs[e];
+            F[3 * n + 0] = v.r;
+            F[3 * n + 1] = v.x;
+            F[3 * n + 2] = v.y;
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
     }
-    blade_levels<T>(fg, pd.j, rank, team, F, alfa, beta, sync);
+    int nlev;
+    const int bp = blade_plane(fg, pd.j, nlev);
+    if (nlev == 0 || !pd.blades) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const int64_t row_bytes = 3 * (int64_t)fg.blade.n_blades * fg.blade.n_radial * sizeof(BladeRow<T>);
+    auto* lr = static_cast<BladeRow<T>*>(lds);
+    T* ld = reinterpret_cast<T*>(static_cast<char*>(lds) + row_bytes);
+    if (row_bytes + plane_force_bytes(g, sizeof(T)) <= lds_bytes)
+        blade_levels<T, true, true>(fg, g, pd.j, bp, nlev, F, next, lr, ld, alfa, beta);
+    else if (row_bytes <= lds_bytes)
+        blade_levels<T, true, false>(fg, g, pd.j, bp, nlev, F, next, lr, nullptr, alfa, beta);
+    else blade_levels<T, false, false>(fg, g, pd.j, bp, nlev, F, next, nullptr, nullptr, alfa, beta);
 }
 
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
-__global__ __launch_bounds__(kPlaneBlock) void k_force_planes(ForceGeom fg, const typename PR::S* __restrict__ Q,
-                                                              typename PR::T* __restrict__ F,
-                                                              const uint64_t* __restrict__ prev,
-                                                              uint64_t* __restrict__ next, Grid g,
-                                                              typename PR::T alfa, typename PR::T beta, float rho0) {
-    __shared__ float4 lds[kPlaneLdsBytes / sizeof(float4)];
-    const PlaneBlock pb = fg.blocks[blockIdx.x];
-    if (pb.plane < 0) return;
-    force_plane<PR, L, STREAM, MOMSRC, EVEN>(fg, fg.planes[pb.plane], pb.rank, Q, F, prev, next, g, alfa, beta,
-                                             rho0, lds, (int64_t)kPlaneLdsBytes);
-}
-
-// The levels of every plane after the gathers of the one-launch step: a
-// workgroup (or team) per plane runs its blade stencil cells (occupancy, F,
-// moments) and then its static levels and blade classes.
-constexpr int kLevelBlock = 1024;
-template <typename PR, int EVEN>
-__global__ __launch_bounds__(kLevelBlock) void k_force_levels(ForceGeom fg, const typename PR::S* __restrict__ Q,
-                                                              float* __restrict__ F, const uint64_t* __restrict__ prev,
-                                                              uint64_t* __restrict__ next, Grid g, float alfa,
-                                                              float beta, float rho0) {
-    const PlaneBlock pb = fg.blocks[blockIdx.x];
-    if (pb.plane < 0) return;
-    const PlaneDesc& pd = fg.planes[pb.plane];
-    const int team = pd.team;
-    uint32_t* bar = team > 1 ? fg.bar + kBarWords * pd.bar : nullptr;
-    const bool local = fg.local_teams != 0;
-    auto sync = [&]() {
-        if (team > 1) team_barrier(bar, team, local);
-        else __syncthreads();
-    };
-    gather_blades<PR, LayoutLIJK, StreamEsotwist, MOMSRC_ESO_POPS, EVEN>(
-        fg, pd.j, pb.rank * (int)blockDim.x + (int)threadIdx.x, team * (int)blockDim.x, Q, F, prev, next, g, rho0);
-    sync();
-    static_levels<float>(fg, pd, pb.rank, team, static_cast<const Mom4<float>*>(fg.scache) + pd.cell_begin,
-                         (float*)nullptr, F, alfa, beta, sync);
-    blade_levels<float>(fg, pd.j, pb.rank, team, F, alfa, beta, sync);
+template <typename T>
+__global__ __launch_bounds__(level_block<T>()) void k_force_levels(ForceGeom fg, T* __restrict__ F,
+                                                                   uint64_t* __restrict__ next, Grid g, T alfa, T beta,
+                                                                   int64_t lds_bytes) {
+    extern __shared__ float4 levels_lds[];  // lds_bytes, launch-sized
+    plane_levels<T>(fg, fg.planes + blockIdx.x, F, next, g, alfa, beta, levels_lds, lds_bytes);
 }
 
 // ------------------------------------------------------------------ pipelined Esotwist step
@@ -1852,8 +1931,8 @@ __global__ __launch_bounds__(kLevelBlock) void k_force_levels(ForceGeom fg, cons
 //      the gathers of xg1 - 1, xg1 and 1
 //   B  the edge planes jlo and jhi (their gathers read rows of the
 //      neighbouring XCDs), in chunks, once those XCDs have released their rows
-//   C  the forcing levels of the range's planes (PlaneDesc), teams first
-// A row item also copies its rows' static occupancy words into next.  Items
+// (The blade cells and the forcing levels follow in launches of their own.)  A row
+// item also copies its rows' static occupancy words into next.  Items
 // wait only for earlier items, so every wait ends; spins are bounded anyway
 // (kBarSpinLimit, flag in the XCD's counters).
 //
@@ -1864,6 +1943,8 @@ __global__ __launch_bounds__(kLevelBlock) void k_force_levels(ForceGeom fg, cons
 // written through this XCD's L2, and each row's stores are complete
 // (s_waitcnt) before its count.  The release of a range for the neighbours is
 // an agent-scope fence pair.
+// polls of a wait before it gives up and flags a time-out (about a second)
+constexpr uint32_t kBarSpinLimit = 1u << 20;
 __device__ __forceinline__ uint32_t xcc_id() {
     uint32_t x;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(x));
@@ -2277,49 +2358,6 @@ __global__ void k_vorticity(const typename PR::S* __restrict__ Q, Grid g, int ax
 }
 
 // ------------------------------------------------------------------ geometry on the device
-template <typename T>
-__device__ __forceinline__ void blade_gen_point(const BladeLayout& bl, const BladeStep& st, const PointsDev& out,
-                                                ForceRow<T>* __restrict__ rows, const Grid& g, int64_t offset,
-                                                int64_t t) {
-    BladeEnum e;
-    e.n_blades = bl.n_blades;
-    e.n_planes = bl.n_planes;
-    e.n_radial = bl.n_radial;
-    e.n_bcol = bl.n_bcol;
-    int b, pl, r, cls;
-    blade_decode(e, t, b, pl, r, cls);
-    tdlb_ib_point pt;
-    blade_point(bl.cx, bl.cz, bl.r_inner, bl.j_lo + pl, r, st.cosb[b], st.sinb[b], st.omega, &pt);
-    const int64_t q = offset + t;
-    out.i[q] = (int32_t)(pt.i + bl.ghost);
-    out.j[q] = (int32_t)(pt.j + bl.ghost);
-    out.k[q] = (int32_t)(pt.k + bl.ghost);
-    static_cast<T*>(out.ifrac)[q] = (T)pt.i_frac;
-    static_cast<T*>(out.kfrac)[q] = (T)pt.k_frac;
-    static_cast<T*>(out.u)[q] = (T)pt.u_delta;
-    static_cast<T*>(out.v)[q] = (T)pt.v_delta;
-    static_cast<T*>(out.w)[q] = (T)pt.w_delta;
-    // its three stencil rows for the blade levels (e: cell_index of the cells)
-    const T vel[3] = {(T)pt.u_delta, (T)pt.v_delta, (T)pt.w_delta};
-    const int i = (int)pt.i + bl.ghost, j = (int)pt.j + bl.ghost, k = (int)pt.k + bl.ghost;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        ForceRow<T> row = make_row<T>((T)pt.i_frac, (T)pt.k_frac, c, vel[c]);
-#pragma unroll
-        for (int m = 0; m < 3; m++)
-            row.e[m] = (int32_t)cell_index(g, wrap_ik(i + m - 1, g.xg1), j, wrap_ik(k + c - 1, g.zg1));
-        rows[3 * q + c] = row;
-    }
-}
-
-template <typename T>
-__global__ void k_gen_blades(BladeLayout bl, BladeStep st, PointsDev out, ForceRow<T>* __restrict__ rows, Grid g,
-                             int64_t offset, int64_t count) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    blade_gen_point<T>(bl, st, out, rows, g, offset, t);
-}
-
 // getExternalPoints as a mask: a cell is outside when its centre lies beyond the
 // tank radius from the axis (exact: integer and half-integer coordinates).
 __global__ void k_solid_mask(double cx, double cz, double radius, uint8_t* __restrict__ out, Grid g, int ghost) {
@@ -2834,23 +2872,45 @@ hipError_t with_cell_source(int layout, int streaming, int momsrc, int even, Fn&
 }
 }  // namespace
 
-hipError_t launch_force_planes(int prec, int layout, int streaming, int momsrc, int even, const ForceGeom& fg,
-                               const void* Q, void* F, const uint64_t* prev, uint64_t* next, const Grid& g,
-                               double alfa, double beta, float rho0, hipStream_t s) {
-    if (fg.n_blocks <= 0) return hipSuccess;
+hipError_t launch_force_gather(int prec, int layout, int streaming, int momsrc, int even, const ForceGeom& fg,
+                               const BladeStep& st, const GatherBlocks& gb, const void* Q, void* F,
+                               const uint64_t* prev, uint64_t* next, const uint64_t* static_base, const Grid& g,
+                               float rho0, hipStream_t s) {
+    const uint32_t nb = gb.blades + gb.cells + gb.words;
+    if (nb == 0) return hipSuccess;
     hipError_t e = hipErrorInvalidValue;
     TDLB_WITH_PREC(prec, {
         using S = typename PR::S;
         using T = typename PR::T;
         e = with_cell_source<PR>(layout, streaming, momsrc, even, [&](auto Lc, auto Sc, auto Mc, auto Ec) {
-            hipLaunchKernelGGL((k_force_planes<PR, decltype(Lc)::value, decltype(Sc)::value, decltype(Mc)::value,
+            hipLaunchKernelGGL((k_force_gather<PR, decltype(Lc)::value, decltype(Sc)::value, decltype(Mc)::value,
                                                decltype(Ec)::value>),
-                               dim3((uint32_t)fg.n_blocks), dim3(kPlaneBlock), 0, s, fg, (const S*)Q, (T*)F, prev,
-                               next, g, (T)alfa, (T)beta, rho0);
+                               dim3(nb), dim3(kGatherBlock), 0, s, fg, st, gb, (const S*)Q, (T*)F, prev, next,
+                               static_base, g, rho0);
             return hipGetLastError();
         });
     });
     return e;
+}
+
+hipError_t launch_force_levels(int prec, const ForceGeom& fg, void* F, uint64_t* next, const Grid& g, double alfa,
+                               double beta, hipStream_t s) {
+    if (fg.n_planes <= 0) return hipSuccess;
+    const dim3 grid((uint32_t)fg.n_planes), block((uint32_t)fg.level_lanes);
+    if (prec == 1)
+        hipLaunchKernelGGL(k_force_levels<double>, grid, block, fg.level_lds, s, fg, (double*)F, next, g, alfa, beta,
+                           (int64_t)fg.level_lds);
+    else
+        hipLaunchKernelGGL(k_force_levels<float>, grid, block, fg.level_lds, s, fg, (float*)F, next, g, (float)alfa,
+                           (float)beta, (int64_t)fg.level_lds);
+    return hipGetLastError();
+}
+
+// Launches may ask for up to the whole LDS of a CU.
+hipError_t allow_level_lds(int prec) {
+    const void* k = prec == 1 ? reinterpret_cast<const void*>(&k_force_levels<double>)
+                              : reinterpret_cast<const void*>(&k_force_levels<float>);
+    return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCuLdsBytes);
 }
 
 bool line_rows_bytes(const Grid& g, size_t ssize) {
@@ -2873,7 +2933,6 @@ hipError_t launch_eso_pipe(int prec, int even, int hint, const PipeArgs& a, cons
     if (lanes != bk) return hipErrorInvalidValue;
     auto go = [&](auto pr) -> hipError_t {
         using PR = decltype(pr);
-        using S = typename PR::S;
         const auto P = to_params<float, typename PR::D>(c);
 #define TDLB_PIPE(E, H)                                                                                         \
     hipLaunchKernelGGL((k_eso_pipe<PR, E, H>), dim3(blocks), dim3(bk), 0, s, a, g, P, nkb, rho0, (float)alfa,    \
@@ -2892,16 +2951,6 @@ hipError_t launch_eso_pipe(int prec, int even, int hint, const PipeArgs& a, cons
         if (even) { if (hint) TDLB_PIPE(1, true); else TDLB_PIPE(1, false); }
         else { if (hint) TDLB_PIPE(0, true); else TDLB_PIPE(0, false); }
 #undef TDLB_PIPE
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess || a.fg.n_blocks <= 0) return e;
-        // the levels read the populations of the next step's collision
-        const S* q = static_cast<const S*>(a.Q);
-        if (even)
-            hipLaunchKernelGGL((k_force_levels<PR, 0>), dim3((uint32_t)a.fg.n_blocks), dim3(kLevelBlock), 0, s, a.fg,
-                               q, static_cast<float*>(a.F), a.prev, a.next, g, (float)alfa, (float)beta, rho0);
-        else
-            hipLaunchKernelGGL((k_force_levels<PR, 1>), dim3((uint32_t)a.fg.n_blocks), dim3(kLevelBlock), 0, s, a.fg,
-                               q, static_cast<float*>(a.F), a.prev, a.next, g, (float)alfa, (float)beta, rho0);
         return hipGetLastError();
     };
     switch (prec) {
@@ -3063,22 +3112,11 @@ hipError_t launch_vorticity(int prec, int layout, int streaming, int momsrc, int
     return e;
 }
 
-hipError_t launch_gen_blades(int prec, const BladeLayout& bl, const BladeStep& st, const PointsDev& out, void* rows,
-                             const Grid& g, int64_t offset, hipStream_t s) {
-    const int64_t count = (int64_t)bl.n_blades * bl.n_planes * bl.n_radial;
-    if (count <= 0) return hipSuccess;
-    const uint32_t nb = (uint32_t)((count + kBlock - 1) / kBlock);
-    if (prec != 1) hipLaunchKernelGGL(k_gen_blades<float>, dim3(nb), dim3(kBlock), 0, s, bl, st, out, (ForceRow<float>*)rows, g, offset, count);
-    else hipLaunchKernelGGL(k_gen_blades<double>, dim3(nb), dim3(kBlock), 0, s, bl, st, out, (ForceRow<double>*)rows, g, offset, count);
-    return hipGetLastError();
-}
-
-hipError_t launch_static_rows(int prec, const PointsDev& p, int64_t n, const int32_t* sidx, const PlaneDesc* planes,
-                              const int32_t* plane_of_j, void* rows, hipStream_t s) {
+hipError_t launch_static_rows(int prec, const PointsDev& p, int64_t n, const int32_t* sidx, void* rows, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const uint32_t nb = (uint32_t)((3 * n + kBlock - 1) / kBlock);
-    if (prec != 1) hipLaunchKernelGGL(k_static_rows<float>, dim3(nb), dim3(kBlock), 0, s, p, n, sidx, planes, plane_of_j, (ForceRow<float>*)rows);
-    else hipLaunchKernelGGL(k_static_rows<double>, dim3(nb), dim3(kBlock), 0, s, p, n, sidx, planes, plane_of_j, (ForceRow<double>*)rows);
+    if (prec != 1) hipLaunchKernelGGL(k_static_rows<float>, dim3(nb), dim3(kBlock), 0, s, p, n, sidx, (ForceRow<float>*)rows);
+    else hipLaunchKernelGGL(k_static_rows<double>, dim3(nb), dim3(kBlock), 0, s, p, n, sidx, (ForceRow<double>*)rows);
     return hipGetLastError();
 }
 
@@ -3165,58 +3203,45 @@ __global__ __launch_bounds__(kRowBlock) void k_batch_fused(const MemberDev* __re
     }
 }
 
-__global__ void k_batch_blades(const MemberDev* __restrict__ mem, const int64_t* __restrict__ off, int n,
-                               int64_t total) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= total || t >= off[n]) return;
-    const int m = find_slot(off, n, t);
-    const MemberDev& md = mem[m];
-    if (!md.active) return;
-    blade_gen_point<float>(md.fg.blade, md.steps[md.done], md.fg.pts, static_cast<ForceRow<float>*>(md.fg.rows), md.g,
-                           md.fg.n_static, t - off[m]);
-}
-
-// the new occupancy mask starts from the static stencil bits
-__global__ void k_batch_mask_init(const MemberDev* __restrict__ mem, const int64_t* __restrict__ off, int n,
-                                  int64_t total) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= total || t >= off[n]) return;
-    const int m = find_slot(off, n, t);
-    const MemberDev& md = mem[m];
-    if (!md.active) return;
-    md.fmask[1 - md.fm][t - off[m]] = md.static_base[t - off[m]];
-}
-
-// the forcing planes of every member: one workgroup per (member, plane) task,
-// density and momentum from the populations the fused kernel just wrote
+// the gather of every member (force_gather) from the populations the fused kernel just wrote
 template <typename PR, int L, int STREAM>
-__global__ __launch_bounds__(kPlaneBlock) void k_batch_force_planes(const MemberDev* __restrict__ mem,
-                                                                    const PlaneTask* __restrict__ tasks,
-                                                                    int64_t lds_bytes) {
-    extern __shared__ float4 batch_lds[];  // lds_bytes for force values and moments, launch-sized
-    const PlaneTask tk = tasks[blockIdx.x];
-    const MemberDev& md = mem[tk.member];
+__global__ __launch_bounds__(kGatherBlock) void k_batch_gather(const MemberDev* __restrict__ mem,
+                                                               const int64_t* __restrict__ off,
+                                                               const int32_t* __restrict__ bm) {
+    const int m = bm[blockIdx.x];
+    const MemberDev& md = mem[m];
     if (!md.active) return;
     using S = typename PR::S;
-    void* lds = lds_bytes > 0 ? batch_lds : nullptr;
-    const PlaneBlock pb = md.fg.blocks[tk.block];
-    if (pb.plane < 0) return;
-    const PlaneDesc& pd = md.fg.planes[pb.plane];
+    const uint32_t b = (uint32_t)(blockIdx.x - off[m]);
     const uint64_t* prev = md.fmask[md.fm];
     uint64_t* next = md.fmask[1 - md.fm];
+    const BladeStep& st = md.steps[md.done];
     if constexpr (STREAM == StreamEsotwist) {
         const S* Q = static_cast<const S*>(md.Q[0]);
         if (md.even)
-            force_plane<PR, L, STREAM, MOMSRC_ESO_POPS, 0>(md.fg, pd, pb.rank, Q, md.F, prev, next, md.g, md.alfa, md.beta,
-                                                            md.rho0, lds, lds_bytes);
+            force_gather<PR, L, STREAM, MOMSRC_ESO_POPS, 0>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base,
+                                                            md.g, md.rho0);
         else
-            force_plane<PR, L, STREAM, MOMSRC_ESO_POPS, 1>(md.fg, pd, pb.rank, Q, md.F, prev, next, md.g, md.alfa, md.beta,
-                                                            md.rho0, lds, lds_bytes);
+            force_gather<PR, L, STREAM, MOMSRC_ESO_POPS, 1>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base,
+                                                            md.g, md.rho0);
     } else {
         const S* Q = static_cast<const S*>(md.Q[1 - md.cur]);
-        force_plane<PR, L, STREAM, MOMSRC_PULL_POPS, 1>(md.fg, pd, pb.rank, Q, md.F, prev, next, md.g, md.alfa, md.beta,
-                                                         md.rho0, lds, lds_bytes);
+        force_gather<PR, L, STREAM, MOMSRC_PULL_POPS, 1>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base, md.g,
+                                                         md.rho0);
     }
+}
+
+// the levels of every member's planes: one workgroup per (member, plane) task
+__global__ __launch_bounds__(kForcePlaneBlock) void k_batch_levels(const MemberDev* __restrict__ mem,
+                                                                   const PlaneTask* __restrict__ tasks,
+                                                                   int64_t lds_bytes) {
+    extern __shared__ float4 batch_lds[];  // lds_bytes, launch-sized
+    const PlaneTask tk = tasks[blockIdx.x];
+    const MemberDev& md = mem[tk.member];
+    if (!md.active) return;
+    const ForceGeom fg = uniform_copy(md.fg);
+    const Grid g = uniform_copy(md.g);
+    plane_levels<float>(fg, fg.planes + tk.plane, md.F, md.fmask[1 - md.fm], g, md.alfa, md.beta, batch_lds, lds_bytes);
 }
 
 template <int STREAM>
@@ -3246,18 +3271,14 @@ template <typename PR, int L, int STREAM>
 hipError_t batch_step_t(const BatchPlan& p, hipStream_t s) {
     const int n = p.n_members;
     if (p.bs != 256 && p.bs != 512) return hipErrorInvalidValue;
-    if (p.tot_rot > 0)
-        hipLaunchKernelGGL(k_batch_blades, dim3(nblk(p.tot_rot, kBlock)), dim3(kBlock), 0, s, p.mem, p.off_rot, n,
-                           p.tot_rot);
     hipError_t e = batch_fused_t<PR, L, STREAM>(p, s);
     if (e != hipSuccess) return e;
-    if (p.tot_words > 0)
-        hipLaunchKernelGGL(k_batch_mask_init, dim3(nblk(p.tot_words, kBlock)), dim3(kBlock), 0, s, p.mem,
-                           p.off_words, n, p.tot_words);
+    if (p.tot_gather > 0)
+        hipLaunchKernelGGL((k_batch_gather<PR, L, STREAM>), dim3((uint32_t)p.tot_gather), dim3(kGatherBlock), 0, s, p.mem,
+                           p.off_gather, p.gather_member);
     if (p.n_tasks > 0)
-        hipLaunchKernelGGL((k_batch_force_planes<PR, L, STREAM>), dim3((uint32_t)p.n_tasks),
-                           dim3(p.force_bs > 0 ? p.force_bs : kPlaneBlock),
-                           (uint32_t)p.force_lds_bytes, s, p.mem, p.tasks, p.force_lds_bytes);
+        hipLaunchKernelGGL(k_batch_levels, dim3((uint32_t)p.n_tasks), dim3(p.force_bs), (uint32_t)p.force_lds_bytes, s,
+                           p.mem, p.tasks, p.force_lds_bytes);
     hipLaunchKernelGGL(k_batch_advance<STREAM>, dim3(nblk(n, 64)), dim3(64), 0, s, p.mem_rw, n);
     return hipGetLastError();
 }

@@ -1,8 +1,9 @@
 """The bound tank's forcing against the oracle where its scheduling changes form:
 blade classes merged into one level per radial class or not (by the distance of
 the blades at the inner radius, and not where a blade stencil may wrap), levels
-on a part of a workgroup, planes whose force values stay in LDS or not.  The
-point order of the lists fixes every rounding, so results are bit-identical."""
+on a part of a workgroup, planes whose force values and moments stay in LDS or
+not, and the same in batches, whose workgroups have less LDS.  The point order of
+the lists fixes every rounding, so results are bit-identical."""
 import numpy as np
 import pytest
 
@@ -51,3 +52,51 @@ def test_blades_reaching_the_walls_are_not_merged():
     rp.blade_outer_radius, rp.blade_inner_radius = 23.0, 12.0
     print(f"[gpu case] blades to the walls T={T}", flush=True)
     compare(T, 4, td.PREC_F32, rp=rp)
+
+
+def wide_disk(T, radius):
+    rp = td.rushton_defaults(T, startup_steps=2)
+    rp.disk_radius = radius
+    return rp
+
+
+# static cells of the disk plane: about 8500 (force values in LDS, moments not), 16500 (neither)
+@pytest.mark.parametrize("T,radius", [(110, 50.0), (150, 70.0)])
+def test_planes_beyond_the_lds_match_oracle(T, radius):
+    print(f"[gpu case] disk of radius {radius} in {T}^3", flush=True)
+    compare(T, 2, td.PREC_F32, rp=wide_disk(T, radius))
+
+
+def test_fp64_plane_beyond_the_lds_matches_oracle():
+    print("[gpu case] disk of radius 50 in 110^3, fp64", flush=True)
+    compare(110, 2, td.PREC_F64, rp=wide_disk(110, 50.0))
+
+
+# workgroups of 64 lanes leave a plane 10 KB of LDS: no room for the blades' rows of the 97^3 tank
+@pytest.mark.parametrize("block", [None, "64", "1024"])
+def test_batch_levels_match_solo_runs(block, monkeypatch):
+    if block:
+        monkeypatch.setenv("TDLB_BATCH_FORCE_BLOCK", block)
+    print(f"[gpu case] batch levels, block {block}", flush=True)
+    specs = [(24, None), (51, None), (97, None), (110, 50.0), (150, 70.0)]
+
+    def tank(T, radius):
+        cu = td.ComputeUnit(T, precision=td.PREC_F16, **td.flow_for_tank(T))
+        cu.initialise(1.0)
+        cu.bind_rushton(wide_disk(T, radius) if radius else td.rushton_defaults(T, startup_steps=2))
+        return cu
+
+    batch = td.Batch(td.PREC_F16)
+    members = [tank(*s) for s in specs]
+    for cu in members:
+        batch.add(cu, 5)
+    batch.run(5)
+    for cu, s in zip(members, specs):
+        solo = tank(*s)
+        solo.run(5)
+        assert np.array_equal(cu.get(td.FIELD_F), solo.get(td.FIELD_F)), s
+        assert np.array_equal(cu.get(td.FIELD_Q), solo.get(td.FIELD_Q)), s
+        solo.close()
+    batch.close()
+    for cu in members:
+        cu.close()
