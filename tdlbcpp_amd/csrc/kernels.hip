@@ -2208,10 +2208,19 @@ __global__ __launch_bounds__(kBlock) void k_reduce_cells(const typename PR::S* _
     }
 }
 
-__global__ void k_reduce_final(const double* __restrict__ partial, int nblocks, double* __restrict__ out) {
+// The partials added in block order, one lane per value.  The chain of 1024
+// dependent adds is the least this order allows (about 5 us); loading each
+// partial inside the chain took 150 us, so a workgroup brings them to LDS first.
+constexpr int kReduceFinalBlock = 1024;
+__global__ __launch_bounds__(kReduceFinalBlock) void k_reduce_final(const double* __restrict__ partial,
+                                                                    double* __restrict__ out) {
+    __shared__ double p[kReduceBlocks * kReduceVals];
+    for (int t = (int)threadIdx.x; t < kReduceBlocks * kReduceVals; t += kReduceFinalBlock) p[t] = partial[t];
+    __syncthreads();
     if (threadIdx.x >= kReduceVals) return;
     double a = 0.0;
-    for (int b = 0; b < nblocks; b++) a += partial[(uint64_t)b * kReduceVals + threadIdx.x];
+#pragma unroll 32
+    for (int b = 0; b < kReduceBlocks; b++) a += p[b * kReduceVals + (int)threadIdx.x];
     out[threadIdx.x] = a;
 }
 
@@ -2999,7 +3008,7 @@ hipError_t launch_reduce(int prec, int layout, int streaming, int momsrc, int ev
         });
     });
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(64), 0, s, partial, kReduceBlocks, out);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kReduceFinalBlock), 0, s, partial, out);
     return hipGetLastError();
 }
 
