@@ -32,13 +32,13 @@ extern "C" {
 #define TDLB_ERR_IO (-5)          /* file read or write failed */
 #define TDLB_ERR_UNSUPPORTED (-6) /* combination not implemented */
 
-/* MemoryLayoutType (Header.h:38) */
+/* MemoryLayoutType (Header.h:38): the order of Q at the boundary (download,
+ * upload, checkpoint files).  In HBM the lattice of every handle is LIJK, where
+ * the 18 slots of a wavefront's cells are 18 contiguous runs instead of 72-byte
+ * strided gathers. */
 #define TDLB_LAYOUT_IJKL 0 /* slot l of cell n at q[n*18 + l] */
 #define TDLB_LAYOUT_LIJK 1 /* slot l of cell n at q[l*size + n] */
-/* No counterpart in the reference: Q is IJKL at the boundary (download, upload,
- * checkpoint files), while the lattice stays LIJK in HBM, where the 18 slots of
- * a wavefront's cells are 18 contiguous runs instead of 72-byte strided
- * gathers.  Every result equals TDLB_LAYOUT_IJKL's. */
+/* no counterpart in the reference: as TDLB_LAYOUT_IJKL */
 #define TDLB_LAYOUT_IJKL_SOA 2
 /* Streaming (Header.h:37) */
 #define TDLB_STREAM_SIMPLE 0

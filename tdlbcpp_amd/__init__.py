@@ -14,7 +14,7 @@ import numpy as np
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libtdlb_hip.so")
 
-LAYOUT_IJKL, LAYOUT_LIJK, LAYOUT_IJKL_SOA = 0, 1, 2  # IJKL_SOA: IJKL at the boundary, LIJK in HBM
+LAYOUT_IJKL, LAYOUT_LIJK, LAYOUT_IJKL_SOA = 0, 1, 2  # order of Q at the boundary; IJKL_SOA as IJKL
 STREAM_SIMPLE, STREAM_ESOTWIST = 0, 1
 PREC_F32, PREC_F64, PREC_F16, PREC_BF16, PREC_E3M12 = 0, 1, 2, 3, 4
 FIELD_Q, FIELD_F, FIELD_NU, FIELD_O = 0, 1, 2, 3

@@ -67,12 +67,12 @@ struct DevBuf {
     }
 };
 
-using TileKey = std::tuple<int64_t, int64_t, int64_t, int, int, int>;
+using TileKey = std::tuple<int64_t, int64_t, int64_t, int, int>;
 struct TileTimes {
     float ms[2][kTiles];
 };
 std::mutex g_tile_mu;
-std::map<TileKey, TileTimes> g_tiles;  // fused-kernel timings per grid shape, precision, layout, streaming
+std::map<TileKey, TileTimes> g_tiles;  // fused-kernel timings per grid shape, precision, streaming
 constexpr int kBlockSizes[2] = {256, 512};
 constexpr int kGraphSteps = 8;  // steps in one replay of the long graph
 
@@ -82,7 +82,6 @@ struct tdlb_batch {
     int prec = 0, layout = 0, streaming = 0, device = 0;
     hipStream_t stream = nullptr;
     std::vector<Member> members;
-    int dlayout() const { return layout == TDLB_LAYOUT_IJKL ? LayoutIJKL : LayoutLIJK; }  // layout in HBM
     bool use_graph = true;
     bool autotune = true;
 
@@ -158,7 +157,7 @@ MemberDev describe(const tdlb_batch* b, const Member& m) {
 // is about to be initialised).  Zero timings (autotuning off) select the row
 // tile at 256 threads.
 int tune_shape(tdlb_batch* b, tdlb_cu* cu, bool own, TileTimes* out, hipStream_t s) {
-    const TileKey key{cu->g.xg1, cu->g.yg1, cu->g.zg1, b->prec, b->layout, b->streaming};
+    const TileKey key{cu->g.xg1, cu->g.yg1, cu->g.zg1, b->prec, b->streaming};
     {
         std::lock_guard<std::mutex> lk(g_tile_mu);
         auto it = g_tiles.find(key);
@@ -231,11 +230,11 @@ int tune_shape(tdlb_batch* b, tdlb_cu* cu, bool own, TileTimes* out, hipStream_t
             ok = hipMemcpyAsync(dmem, &md, sizeof(md), hipMemcpyHostToDevice, s) == hipSuccess &&
                  hipMemcpyAsync(dtab, tab, sizeof(tab), hipMemcpyHostToDevice, s) == hipSuccess;
             for (int w = 0; w < 2 && ok; w++)
-                ok = launch_batch_fused(b->prec, b->dlayout(), b->streaming, p, s) == hipSuccess;
+                ok = launch_batch_fused(b->prec, b->streaming, p, s) == hipSuccess;
             ok = ok && hipEventRecord(e0, s) == hipSuccess;
             constexpr int reps = 5;
             for (int w = 0; w < reps && ok; w++)
-                ok = launch_batch_fused(b->prec, b->dlayout(), b->streaming, p, s) == hipSuccess;
+                ok = launch_batch_fused(b->prec, b->streaming, p, s) == hipSuccess;
             ok = ok && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
             float ms = 0.f;
             ok = ok && hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
@@ -427,7 +426,7 @@ int build_plan(tdlb_batch* b, int64_t K, bool* structure_changed) {
 }
 
 int record_steps(tdlb_batch* b, int steps) {
-    HIPCHK(launch_batch_step(b->prec, b->dlayout(), b->streaming, b->plan, steps, b->stream));
+    HIPCHK(launch_batch_step(b->prec, b->streaming, b->plan, steps, b->stream));
     return TDLB_OK;
 }
 

@@ -1,8 +1,8 @@
 // C ABI of the MI355X ComputeUnit (declared in include/tdlb.h).
 //
-// State of a handle.  Q[cur] holds the ComputeUnit's Q array in the reference's
-// layout.  Two phases:
-//   explicit  Q[cur] is byte for byte what the reference's Q would hold;
+// State of a handle.  Q[cur] holds the ComputeUnit's Q array in the kernels' own
+// order (device.h), converted at the boundary.  Two phases:
+//   explicit  Q[cur] is value for value what the reference's Q would hold;
 //   lazy      left by the fused main-loop path: Q[cur] holds post-collision
 //             populations (Simple) or streamed populations (Esotwist) and the
 //             forcing of the step has been applied; the reference's Q is
@@ -140,8 +140,8 @@ int ensure_m(tdlb_cu* cu) {
         cu->M = nullptr;
         return fail(TDLB_ERR_NOMEM, "explicit Q of the 16-bit storage");
     }
-    HIPCHK(launch_fill_q(cu->eprec(), cu->dlay(), cu->M, cu->g, cu->rho0, cu->stream));
-    if (cu->simple()) HIPCHK(launch_bounce_back((int)cu->tsize, cu->dlay(), cu->M, cu->g, cu->stream));
+    HIPCHK(launch_fill_q(cu->eprec(), cu->M, cu->g, cu->rho0, cu->stream));
+    if (cu->simple()) HIPCHK(launch_bounce_back((int)cu->tsize, cu->M, cu->g, cu->stream));
     return TDLB_OK;
 }
 
@@ -152,16 +152,16 @@ int materialise(tdlb_cu* cu) {
     if (cu->simple()) {
         void* src = cu->Q[cu->cur];
         void* dst = cu->shifted() ? cu->M : cu->Q[1 - cu->cur];
-        HIPCHK(launch_simple(cu->prec(), cu->dlay(), MODE_MOM_PULL, src, dst, dst, cu->F, cu->Nu,
+        HIPCHK(launch_simple(cu->prec(), MODE_MOM_PULL, src, dst, dst, cu->F, cu->Nu,
                              cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
         if (cu->shifted()) {
-            HIPCHK(launch_ghost_fill_decode(cu->prec(), cu->dlay(), src, dst, cu->g, cu->rho0, cu->stream));
+            HIPCHK(launch_ghost_fill_decode(cu->prec(), src, dst, cu->g, cu->rho0, cu->stream));
         } else {
-            HIPCHK(launch_ghost_fill((int)cu->ssize, cu->dlay(), src, dst, cu->g, cu->stream));
+            HIPCHK(launch_ghost_fill((int)cu->ssize, src, dst, cu->g, cu->stream));
             cu->cur = 1 - cu->cur;
         }
     } else {
-        HIPCHK(launch_esotwist(cu->prec(), cu->dlay(), MODE_MOM, cu->even ? 1 : 0, cu->Q[0], cu->eq(), cu->F,
+        HIPCHK(launch_esotwist(cu->prec(), MODE_MOM, cu->even ? 1 : 0, cu->Q[0], cu->eq(), cu->F,
                                cu->Nu, cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
     }
     cu->phase = PH_EXPLICIT;
@@ -341,10 +341,10 @@ int forcing_pass(tdlb_cu* cu, const DevPoints& dp, const std::vector<ForceSegmen
     if (!tiny) {
         for (auto& sg : segs) {
             if (sg.set)
-                HIPCHK(launch_ib_moments_cells(qp, cu->dlay(), cu->prm.streaming, momsrc, even, sg.set->cells,
+                HIPCHK(launch_ib_moments_cells(qp, cu->prm.streaming, momsrc, even, sg.set->cells,
                                                sg.set->n_cells, sg.set->cache, Qsrc, cu->g, cu->rho0, cu->stream));
             else
-                HIPCHK(launch_ib_moments_points(qp, cu->dlay(), cu->prm.streaming, momsrc, even, dp.d,
+                HIPCHK(launch_ib_moments_points(qp, cu->prm.streaming, momsrc, even, dp.d,
                                                 sg.cache_base, sg.n_points, sg.direct_cache, Qsrc, cu->g, cu->rho0,
                                                 cu->stream));
         }
@@ -352,7 +352,7 @@ int forcing_pass(tdlb_cu* cu, const DevPoints& dp, const std::vector<ForceSegmen
     for (auto& sg : segs)
         for (auto& r : sg.levels) {
             if (tiny)
-                HIPCHK(launch_force_level(qp, cu->dlay(), cu->prm.streaming, momsrc, even, dp.d, r.first,
+                HIPCHK(launch_force_level(qp, cu->prm.streaming, momsrc, even, dp.d, r.first,
                                           r.second - r.first, cu->F, Qsrc, cu->g, cu->alfa, cu->beta, cu->rho0,
                                           cu->stream));
             else
@@ -609,7 +609,7 @@ int setup_pipe(tdlb_cu* cu) {
     cu->rowcell = nullptr;
     cu->pctr = nullptr;
     const Grid& g = cu->g;
-    const bool shape = !cu->simple() && cu->dlay() == LayoutLIJK && cu->prm.precision != TDLB_PREC_F64 &&
+    const bool shape = !cu->simple() && cu->prm.layout != TDLB_LAYOUT_IJKL && cu->prm.precision != TDLB_PREC_F64 &&
                        g.xg1 >= 4 && g.yg1 >= 3 * kXcds && g.zg1 >= 64;
     if (!shape || !pipe_device_ok(cu)) return TDLB_OK;
     const IndexedSet& set = cu->static_set;
@@ -668,7 +668,7 @@ int pipe_step(tdlb_cu* cu, const BladeStep& st) {
                            0, row_lanes(cu->g), cu->stream));
     // the levels read the populations of the next step's collision
     const GatherBlocks gb = gather_blocks(cu->n_rot, 0, 0);
-    HIPCHK(launch_force_gather(cu->prec(), cu->dlay(), cu->prm.streaming, MOMSRC_ESO_POPS, cu->even ? 0 : 1, a.fg, st,
+    HIPCHK(launch_force_gather(cu->prec(), cu->prm.streaming, MOMSRC_ESO_POPS, cu->even ? 0 : 1, a.fg, st,
                                gb, cu->Q[0], cu->F, prev, next, cu->static_base, cu->g, cu->rho0, cu->stream));
     HIPCHK(launch_force_levels(cu->eprec(), a.fg, cu->F, next, cu->g, cu->alfa, cu->beta, cu->stream));
     if (cu->o_dirty) {
@@ -720,7 +720,7 @@ int bound_forcing(tdlb_cu* cu, int momsrc, bool prepare_static, const BladeStep&
     const ForceGeom fg = cu->fgeom();
     if (prepare_static)
         HIPCHK(launch_force_prepare(cu->eprec(), cu->pts.d, 0, cu->n_static, cu->F, prev, next, cu->g, cu->stream));
-    HIPCHK(launch_force_gather(qp, cu->dlay(), cu->prm.streaming, momsrc, cu->even ? 1 : 0, fg, st,
+    HIPCHK(launch_force_gather(qp, cu->prm.streaming, momsrc, cu->even ? 1 : 0, fg, st,
                                gather_blocks(cu->n_rot, fg.n_cells, (int64_t)cu->mask_words), Qsrc, cu->F, prev, next,
                                cu->static_base, cu->g, cu->rho0, cu->stream));
     HIPCHK(launch_force_levels(cu->eprec(), fg, cu->F, next, cu->g, cu->alfa, cu->beta, cu->stream));
@@ -840,7 +840,7 @@ int tdlb_cu_create(const tdlb_cu_params* p, const tdlb_flow* f, tdlb_cu_t* out) 
     cu->g.size = size;
     cu->tsize = p->precision == TDLB_PREC_F64 ? 8 : 4;
     cu->ssize = p->precision == TDLB_PREC_F64 ? 8 : p->precision == TDLB_PREC_F32 ? 4 : 2;
-    set_q_geometry(cu->g, cu->dlay(), cu->ssize);
+    set_q_geometry(cu->g, cu->ssize);
     if (cu->q_cells() >= (1ull << 32)) {
         delete cu;
         return fail(TDLB_ERR_UNSUPPORTED, "grid too large for 32-bit cell indexing");
@@ -924,7 +924,7 @@ int tdlb_cu_initialise(tdlb_cu_t cu, double rho) {
     } else {
         const int nq = cu->simple() ? 2 : 1;
         for (int b = 0; b < nq; b++)
-            HIPCHK(launch_fill_q(cu->prec(), cu->dlay(), cu->Q[b], cu->g, r, cu->stream));
+            HIPCHK(launch_fill_q(cu->prec(), cu->Q[b], cu->g, r, cu->stream));
     }
     HIPCHK(launch_zero(cu->F, cu->f_bytes(), cu->stream));
     HIPCHK(launch_zero(cu->Nu, cu->nu_bytes(), cu->stream));
@@ -949,10 +949,10 @@ int tdlb_cu_collision(tdlb_cu_t cu) {
     const auto c = cu->cargs();
     void* q = cu->Q[cu->cur];
     if (cu->simple())
-        HIPCHK(launch_simple(cu->prec(), cu->dlay(), MODE_COLL, q, q, q, cu->F, cu->Nu, cu->fmask[cu->fm],
+        HIPCHK(launch_simple(cu->prec(), MODE_COLL, q, q, q, cu->F, cu->Nu, cu->fmask[cu->fm],
                              cu->g, c, cu->rho0, cu->stream));
     else
-        HIPCHK(launch_esotwist(cu->prec(), cu->dlay(), MODE_COLL, cu->even ? 1 : 0, q, q, cu->F, cu->Nu,
+        HIPCHK(launch_esotwist(cu->prec(), MODE_COLL, cu->even ? 1 : 0, q, q, cu->F, cu->Nu,
                                cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
     return TDLB_OK;
 }
@@ -965,10 +965,10 @@ int tdlb_cu_moments(tdlb_cu_t cu) {
     const auto c = cu->cargs();
     void* q = cu->Q[cu->cur];
     if (cu->simple())
-        HIPCHK(launch_simple(cu->prec(), cu->dlay(), MODE_MOM, q, q, q, cu->F, cu->Nu, cu->fmask[cu->fm], cu->g,
+        HIPCHK(launch_simple(cu->prec(), MODE_MOM, q, q, q, cu->F, cu->Nu, cu->fmask[cu->fm], cu->g,
                              c, cu->rho0, cu->stream));
     else
-        HIPCHK(launch_esotwist(cu->prec(), cu->dlay(), MODE_MOM, cu->even ? 1 : 0, q, q, cu->F, cu->Nu,
+        HIPCHK(launch_esotwist(cu->prec(), MODE_MOM, cu->even ? 1 : 0, q, q, cu->F, cu->Nu,
                                cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
     return TDLB_OK;
 }
@@ -982,7 +982,7 @@ int tdlb_cu_stream_push(tdlb_cu_t cu) {
         cu->even = !cu->even;
         return TDLB_OK;
     }
-    HIPCHK(launch_push_all((int)cu->tsize, cu->dlay(), cu->Q[cu->cur], cu->Q[1 - cu->cur], cu->g, cu->stream));
+    HIPCHK(launch_push_all((int)cu->tsize, cu->Q[cu->cur], cu->Q[1 - cu->cur], cu->g, cu->stream));
     cu->cur = 1 - cu->cur;
     return TDLB_OK;
 }
@@ -996,7 +996,7 @@ int tdlb_cu_stream_pull(tdlb_cu_t cu) {
         cu->even = !cu->even;
         return TDLB_OK;
     }
-    HIPCHK(launch_pull_all((int)cu->tsize, cu->dlay(), cu->Q[cu->cur], cu->Q[1 - cu->cur], cu->g, cu->stream));
+    HIPCHK(launch_pull_all((int)cu->tsize, cu->Q[cu->cur], cu->Q[1 - cu->cur], cu->g, cu->stream));
     cu->cur = 1 - cu->cur;
     return TDLB_OK;
 }
@@ -1007,7 +1007,7 @@ int tdlb_cu_bounce_back(tdlb_cu_t cu) {
     CHK(set_device(cu));
     CHK(materialise(cu));
     if (!cu->simple()) return TDLB_OK;  // Boundary.hpp:13-14
-    HIPCHK(launch_bounce_back((int)cu->tsize, cu->dlay(), cu->Q[cu->cur], cu->g, cu->stream));
+    HIPCHK(launch_bounce_back((int)cu->tsize, cu->Q[cu->cur], cu->g, cu->stream));
     return TDLB_OK;
 }
 
@@ -1052,6 +1052,29 @@ int tdlb_cu_field_bytes(tdlb_cu_t cu, int field, size_t* bytes) {
     return TDLB_OK;
 }
 
+// The explicit Q to `out` or from `in` (one of them null), converted between the
+// kernels' array and the boundary's in pieces, so that a lattice of more than half
+// the memory still moves.
+static int move_q(tdlb_cu* cu, void* out, const void* in, size_t bytes) {
+    constexpr size_t kPiece = (size_t)1 << 29;
+    const size_t piece = std::min(bytes, kPiece);
+    void* tmp = nullptr;
+    if (hipMalloc(&tmp, piece) != hipSuccess) return fail(TDLB_ERR_NOMEM, "Q staging");
+    hipError_t e = hipSuccess;
+    for (size_t at = 0; at < bytes && e == hipSuccess; at += piece) {
+        const size_t n = std::min(piece, bytes - at);
+        if (in) e = hipMemcpyAsync(tmp, (const char*)in + at, n, hipMemcpyHostToDevice, cu->stream);
+        if (e == hipSuccess)
+            e = launch_q_boundary((int)cu->tsize, cu->blay(), out ? 1 : 0, cu->eq(), tmp, at / cu->tsize,
+                                  (at + n) / cu->tsize, cu->g, cu->stream);
+        if (e == hipSuccess && out) e = hipMemcpyAsync((char*)out + at, tmp, n, hipMemcpyDeviceToHost, cu->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
+    }
+    (void)hipFree(tmp);
+    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string(out ? "download" : "upload") + " Q: " + hipGetErrorString(e));
+    return TDLB_OK;
+}
+
 int tdlb_cu_download(tdlb_cu_t cu, int field, void* host, size_t bytes) {
     size_t need = 0;
     CHK(tdlb_cu_field_bytes(cu, field, &need));
@@ -1068,16 +1091,7 @@ int tdlb_cu_download(tdlb_cu_t cu, int field, void* host, size_t bytes) {
         if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("download F: ") + hipGetErrorString(e));
         return TDLB_OK;
     }
-    if (field == TDLB_FIELD_Q && cu->q_converted()) {
-        void* tmp = nullptr;
-        if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "download Q staging");
-        hipError_t e = launch_q_boundary((int)cu->tsize, cu->dlay(), cu->blay(), 1, cu->eq(), tmp, cu->g, cu->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(host, tmp, need, hipMemcpyDeviceToHost, cu->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
-        (void)hipFree(tmp);
-        if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("download Q: ") + hipGetErrorString(e));
-        return TDLB_OK;
-    }
+    if (field == TDLB_FIELD_Q) return move_q(cu, host, nullptr, need);
     if (field == TDLB_FIELD_NU && cu->shifted()) {
         void* tmp = nullptr;
         if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "download Nu staging");
@@ -1088,7 +1102,7 @@ int tdlb_cu_download(tdlb_cu_t cu, int field, void* host, size_t bytes) {
         if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("download Nu: ") + hipGetErrorString(e));
         return TDLB_OK;
     }
-    const void* src = field == TDLB_FIELD_Q ? cu->eq() : field == TDLB_FIELD_NU ? cu->Nu : (const void*)cu->O;
+    const void* src = field == TDLB_FIELD_NU ? cu->Nu : (const void*)cu->O;
     HIPCHK(hipMemcpyAsync(host, src, need, hipMemcpyDeviceToHost, cu->stream));
     HIPCHK(hipStreamSynchronize(cu->stream));
     return TDLB_OK;
@@ -1100,18 +1114,8 @@ int tdlb_cu_upload(tdlb_cu_t cu, int field, const void* host, size_t bytes) {
     if (!host || bytes != need) return fail(TDLB_ERR_INVALID, "upload: buffer size must be " + std::to_string(need));
     CHK(set_device(cu));
     CHK(materialise(cu));
-    void* dst = field == TDLB_FIELD_Q ? cu->eq() : field == TDLB_FIELD_F ? cu->F
-              : field == TDLB_FIELD_NU ? cu->Nu : (void*)cu->O;
-    if (field == TDLB_FIELD_Q && cu->q_converted()) {
-        void* tmp = nullptr;
-        if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "upload Q staging");
-        hipError_t e = hipMemcpyAsync(tmp, host, need, hipMemcpyHostToDevice, cu->stream);
-        if (e == hipSuccess) e = launch_q_boundary((int)cu->tsize, cu->dlay(), cu->blay(), 0, tmp, dst, cu->g, cu->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
-        (void)hipFree(tmp);
-        if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("upload Q: ") + hipGetErrorString(e));
-        return TDLB_OK;
-    }
+    void* dst = field == TDLB_FIELD_F ? cu->F : field == TDLB_FIELD_NU ? cu->Nu : (void*)cu->O;
+    if (field == TDLB_FIELD_Q) return move_q(cu, nullptr, host, need);
     if (field == TDLB_FIELD_NU && cu->shifted()) {
         void* tmp = nullptr;
         if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "upload Nu staging");
@@ -1403,25 +1407,25 @@ int tdlb_cu_run(tdlb_cu_t cu, int64_t nsteps, uint64_t* step, double* angle) {
             void* e = cu->eq();
             if (cu->simple()) {
                 // settle the ghost layer once (bounce-back rims); the 16-bit lattices never read theirs
-                HIPCHK(launch_bounce_back((int)cu->tsize, cu->dlay(), e, cu->g, cu->stream));
+                HIPCHK(launch_bounce_back((int)cu->tsize, e, cu->g, cu->stream));
                 if (!cu->shifted())
-                    HIPCHK(launch_ghost_copy((int)cu->ssize, cu->dlay(), q, cu->Q[1 - cu->cur], cu->g,
+                    HIPCHK(launch_ghost_copy((int)cu->ssize, q, cu->Q[1 - cu->cur], cu->g,
                                              cu->stream));
-                HIPCHK(launch_simple(cu->prec(), cu->dlay(), MODE_COLL, q, q, e, cu->F, cu->Nu,
+                HIPCHK(launch_simple(cu->prec(), MODE_COLL, q, q, e, cu->F, cu->Nu,
                                      cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
             } else {
-                HIPCHK(launch_esotwist(cu->prec(), cu->dlay(), MODE_COLL, cu->even ? 1 : 0, q, e, cu->F, cu->Nu,
+                HIPCHK(launch_esotwist(cu->prec(), MODE_COLL, cu->even ? 1 : 0, q, e, cu->F, cu->Nu,
                                        cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
                 cu->even = !cu->even;
             }
             cu->phase = PH_LAZY;
         } else {
             if (cu->simple()) {
-                HIPCHK(launch_simple(cu->prec(), cu->dlay(), MODE_FUSED, cu->Q[cu->cur], cu->Q[1 - cu->cur],
+                HIPCHK(launch_simple(cu->prec(), MODE_FUSED, cu->Q[cu->cur], cu->Q[1 - cu->cur],
                                      nullptr, cu->F, cu->Nu, cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
                 cu->cur = 1 - cu->cur;
             } else {
-                HIPCHK(launch_esotwist(cu->prec(), cu->dlay(), MODE_FUSED, cu->even ? 1 : 0, cu->Q[0], nullptr,
+                HIPCHK(launch_esotwist(cu->prec(), MODE_FUSED, cu->even ? 1 : 0, cu->Q[0], nullptr,
                                        cu->F, cu->Nu, cu->fmask[cu->fm], cu->g, c, cu->rho0, cu->stream));
                 cu->even = !cu->even;
             }
@@ -1529,7 +1533,7 @@ int tdlb_cu_reductions(tdlb_cu_t cu, double* out) {
     const ReduceArgs ra = reduce_args(cu);
     const CellSource cs = cell_source(cu);
     double* res = cu->red + (size_t)kReduceBlocks * kReduceVals;
-    HIPCHK(launch_reduce(cs.prec, cu->dlay(), cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F,
+    HIPCHK(launch_reduce(cs.prec, cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F,
                          cu->fmask[cu->fm], cu->g, ra, cu->rho0, cu->red, res, cu->stream));
     HIPCHK(hipMemcpyAsync(out, res, sizeof(double) * kReduceVals, hipMemcpyDeviceToHost, cu->stream));
     HIPCHK(hipStreamSynchronize(cu->stream));
@@ -1548,7 +1552,7 @@ int tdlb_cu_reductions_noalloc(tdlb_cu_t cu, double* out_device) {
     // the shared scratch needs no clearing between calls
     double* partial = g_scratch[cu->device];
     const CellSource cs = cell_source(cu);
-    HIPCHK(launch_reduce(cs.prec, cu->dlay(), cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F,
+    HIPCHK(launch_reduce(cs.prec, cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F,
                          cu->fmask[cu->fm], cu->g, ra, cu->rho0, partial, out_device, cu->stream));
     return TDLB_OK;
 }
@@ -1561,7 +1565,7 @@ int tdlb_cu_macroscopic(tdlb_cu_t cu, void* out, size_t bytes) {
     void* tmp = nullptr;
     if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "macroscopic staging");
     const CellSource cs = cell_source(cu);
-    hipError_t e = launch_macroscopic(cs.prec, cu->dlay(), cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F,
+    hipError_t e = launch_macroscopic(cs.prec, cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F,
                                       cu->fmask[cu->fm], cu->g, cu->rho0, tmp, cu->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, need, hipMemcpyDeviceToHost, cu->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
@@ -1595,7 +1599,7 @@ int tdlb_cu_double_resolution(tdlb_cu_t cu) {
     }
     hipError_t e = hipStreamSynchronize(cu->stream);
     if (e == hipSuccess)
-        e = launch_regrid((int)cu->tsize, cu->dlay(), cu->eq(), n->eq(), (int)(cu->nu_bytes() / cu->g.size), cu->Nu,
+        e = launch_regrid((int)cu->tsize, cu->eq(), n->eq(), (int)(cu->nu_bytes() / cu->g.size), cu->Nu,
                           n->Nu, cu->g, n->g, n->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(n->stream);
     if (e != hipSuccess) return drop(fail(TDLB_ERR_HIP, std::string("regrid: ") + hipGetErrorString(e)));
@@ -1658,7 +1662,7 @@ int tdlb_cu_plane_xz(tdlb_cu_t cu, int64_t cut, const uint8_t* exclude, void* qv
     if (e == hipSuccess) e = hipMalloc((void**)&df, cells * sizeof(PlaneRec3));
     if (e == hipSuccess) e = hipMalloc((void**)&dflag, cells);
     if (e == hipSuccess)
-        e = launch_plane_xz(cu->eprec(), cu->dlay(), cu->eq(), cu->F, cu->fmask[cu->fm], ex, cu->g, (int)cut,
+        e = launch_plane_xz(cu->eprec(), cu->eq(), cu->F, cu->fmask[cu->fm], ex, cu->g, (int)cut,
                             cu->prm.i0, cu->prm.k0, dq, df, dflag, cu->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(hq.data(), dq, cells * sizeof(PlaneRec4), hipMemcpyDeviceToHost, cu->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(hf.data(), df, cells * sizeof(PlaneRec3), hipMemcpyDeviceToHost, cu->stream);
@@ -1693,7 +1697,7 @@ int tdlb_cu_vorticity(tdlb_cu_t cu, int32_t axis, int64_t cut, const uint8_t* ex
     void* tmp = nullptr;
     hipError_t e = hipMalloc(&tmp, need);
     if (e == hipSuccess)
-        e = launch_vorticity(cu->eprec(), cu->dlay(), cu->prm.streaming, MOMSRC_STORED, cu->even ? 1 : 0, cu->eq(),
+        e = launch_vorticity(cu->eprec(), cu->prm.streaming, MOMSRC_STORED, cu->even ? 1 : 0, cu->eq(),
                              cu->g, axis, (int)cut, ex, tmp, cu->rho0, cu->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, need, hipMemcpyDeviceToHost, cu->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);

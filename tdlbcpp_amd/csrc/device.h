@@ -4,13 +4,13 @@
 // (tdlbcpp/src/ComputeUnit.hpp:454-463): F is an array of {x,y,z} per cell, Nu
 // one value per cell, O one byte per cell, all indexed by n.
 //
-// The population arrays have their own cell index qn = qcell(i,j,k):
-//   IJKL: Q[qn*18 + l], qn = n                          (tdlbcpp/src/Field.hpp:18-144)
-//   LIJK: Q[l*qsize + qn], qn = i*qyz + j*qz + (k-1) for interior k: k-rows of
-//         the zg1 interior cells back to back, the k-ghost cells of each row in
-//         a side region (qside), so the lines the stream-collide kernels move
-//         hold interior cells only.
-// At the boundary (download, upload, checkpoint) Q is the reference's dense array.
+// The population arrays have their own cell index qn = qcell(i,j,k) and are
+// structures of arrays: Q[l*qsize + qn], qn = i*qyz + j*qz + (k-1) for interior k:
+// k-rows of the zg1 interior cells back to back, the k-ghost cells of each row in a
+// side region (qside), so the lines the stream-collide kernels move hold interior
+// cells only.  At the boundary (download, upload, checkpoint) Q is the reference's
+// dense array in the handle's layout: IJKL n*18 + l or LIJK l*size + n
+// (tdlbcpp/src/Field.hpp:18-144).
 //
 // The F-occupancy bitmask has one bit per cell, rows of k padded to 64-bit
 // words: word (i*yg + j)*mask_w + k/64, bit k%64.  A set bit means F of that
@@ -31,14 +31,13 @@ struct Grid {
     uint64_t size;          // xg*yg*zg
     uint32_t qz, qyz;       // population arrays: row pitch and i-plane pitch in cells
     uint32_t qoff;          // population index of cell (0,0,0) (modulo 2^32)
-    uint32_t qside;         // first cell of the k-ghost side region, 0: none
-    uint64_t qsize;         // cells per slot plane (LIJK)
+    uint32_t qside;         // first cell of the k-ghost side region
+    uint64_t qsize;         // cells per slot plane
 };
 
 // slot l of the population cell qn
-template <int L>
 __device__ __forceinline__ uint64_t qaddr(const Grid& g, uint32_t qn, int l) {
-    return L == LayoutIJKL ? (uint64_t)qn * kQ + (uint64_t)l : (uint64_t)l * g.qsize + (uint64_t)qn;
+    return (uint64_t)l * g.qsize + (uint64_t)qn;
 }
 
 __host__ __device__ __forceinline__ uint32_t cell_index(const Grid& g, int i, int j, int k) {
@@ -53,10 +52,10 @@ __device__ __forceinline__ void decode_cell(const Grid& g, uint64_t n, int& i, i
     k = (int)(r - (uint32_t)j * (uint32_t)g.zg);
 }
 
-// population cell of (i,j,k); with a side region the rows hold the interior
-// k = 1..zg1 only and the two k-ghost cells of row (i,j) sit at qside + 2(i*yg + j)
+// population cell of (i,j,k): the rows hold the interior k = 1..zg1 only, the two
+// k-ghost cells of row (i,j) sit at qside + 2(i*yg + j)
 __host__ __device__ __forceinline__ uint32_t qcell(const Grid& g, int i, int j, int k) {
-    if (g.qside && (k == 0 || k > g.zg1))
+    if (k == 0 || k > g.zg1)
         return g.qside + 2u * ((uint32_t)i * (uint32_t)g.yg + (uint32_t)j) + (k != 0 ? 1u : 0u);
     return g.qoff + (uint32_t)i * g.qyz + (uint32_t)j * g.qz + (uint32_t)k;
 }

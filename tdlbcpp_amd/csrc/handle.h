@@ -60,24 +60,15 @@ struct DevPoints {
     }
 };
 
-// Population arrays in LIJK: a k-row holds the interior cells k = 1..zg1 only,
-// rows back to back (ghost rows in i and j included), and the two k-ghost
-// cells of every row sit in a side region after the rows.  The stream-collide
-// kernels never touch a k-ghost (Esotwist wraps periodically, the Simple pull
-// reads interior neighbours only), so every line they move holds interior
-// cells only, and at zg1 = 512 every row starts a 128 B line.  Slot planes of
-// 16 MiB and more start on 1 MiB boundaries (planes of 18 concurrent streams
-// whose starts fall at arbitrary offsets measured 4 % slower at 512^3), smaller
-// ones on 128 B lines.  IJKL keeps the dense index.
-inline void set_q_geometry(Grid& g, int dlay, size_t ssize) {
-    g.qside = 0;
-    if (dlay == LayoutIJKL) {
-        g.qz = (uint32_t)g.zg;
-        g.qyz = g.yz;
-        g.qoff = 0;
-        g.qsize = g.size;
-        return;
-    }
+// Population arrays: a k-row holds the interior cells k = 1..zg1 only, rows back
+// to back (ghost rows in i and j included), and the two k-ghost cells of every row
+// sit in a side region after the rows.  The stream-collide kernels never touch a
+// k-ghost (Esotwist wraps periodically, the Simple pull reads interior neighbours
+// only), so every line they move holds interior cells only, and at zg1 = 512 every
+// row starts a 128 B line.  Slot planes of 16 MiB and more start on 1 MiB
+// boundaries (planes of 18 concurrent streams whose starts fall at arbitrary
+// offsets measured 4 % slower at 512^3), smaller ones on 128 B lines.
+inline void set_q_geometry(Grid& g, size_t ssize) {
     g.qz = (uint32_t)g.zg1;
     g.qyz = (uint32_t)((uint64_t)g.yg * g.qz);
     g.qoff = 0xffffffffu;  // (i, j, k) at i*qyz + j*qz + k - 1 (modulo 2^32)
@@ -213,24 +204,20 @@ struct tdlb_cu {
     std::vector<std::pair<int, int>> coll, force;
     size_t ev_used = 0;
 
-    // cells per slot of the kernels' population arrays (rows padded in LIJK)
-    size_t q_cells() const { return dlay() == LayoutIJKL ? (size_t)g.size : (size_t)g.qsize; }
+    size_t q_cells() const { return (size_t)g.qsize; }  // cells per slot of the kernels' population arrays
     size_t qb_bytes() const { return (size_t)g.size * kQ * tsize; }  // Q as the reference holds it (boundary)
     size_t q_bytes() const { return q_cells() * kQ * tsize; }        // explicit Q on the device
     size_t qs_bytes() const { return q_cells() * kQ * ssize; }       // one population lattice
-    // Q at the boundary differs from the device array (layout or row padding)
-    bool q_converted() const {
-        return blay() != dlay() || g.qz != (uint32_t)g.zg || g.qoff != 0 || g.qside != 0 ||
-               (size_t)g.qsize != (size_t)g.size;
-    }
     size_t f_bytes() const { return (size_t)g.size * 3 * tsize; }
     size_t nu_bytes() const { return (size_t)g.size * (shifted() ? ssize : tsize); }  // Nu on the device
     size_t nub_bytes() const { return (size_t)g.size * tsize; }                       // Nu at the boundary
     size_t mask_bytes() const { return mask_words * sizeof(uint64_t); }
     bool simple() const { return prm.streaming == TDLB_STREAM_SIMPLE; }
-    // layout of the lattice in HBM (what the kernels address) and of Q at the
-    // boundary (download, upload, checkpoint); they differ for TDLB_LAYOUT_IJKL_SOA
-    int dlay() const { return prm.layout == TDLB_LAYOUT_IJKL ? LayoutIJKL : LayoutLIJK; }
+    // layout of Q at the boundary (download, upload, checkpoint).  In HBM the
+    // lattice is LIJK for every handle: in IJKL a cell's slots are one 72-byte
+    // record, of which a wavefront's step reads and writes single slots in the
+    // records of four rows (256^3 FP32 Esotwist: 0.86 ms a step even staged through
+    // LDS, 0.45 in LIJK).
     int blay() const { return prm.layout == TDLB_LAYOUT_LIJK ? LayoutLIJK : LayoutIJKL; }
     bool shifted() const {
         return prm.precision == TDLB_PREC_F16 || prm.precision == TDLB_PREC_BF16 || prm.precision == TDLB_PREC_E3M12;

@@ -2,8 +2,7 @@
 // Pointers are device pointers; every launcher enqueues on `s` and returns the
 // launch status.  prec: 0 float, 1 double, 2 fp16 storage, 3 bf16 storage (the
 // last two compute in float and store Nu in their 16-bit format; F and point
-// arrays are float).
-// layout: LayoutIJKL/LayoutLIJK.
+// arrays are float).  Population arrays are LIJK (device.h) whatever the layout at the boundary.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -60,7 +59,7 @@ struct BladeStep {
     double omega;               // angular increment this step (rad / step)
 };
 
-hipError_t launch_fill_q(int prec, int layout, void* Q, const Grid& g, double rho, hipStream_t s);
+hipError_t launch_fill_q(int prec, void* Q, const Grid& g, double rho, hipStream_t s);
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t s);
 // One pass of the access-pattern probe: `planes` (1..20) planes of n values of
 // elem_bytes (2, 4, 8) bytes, `stride` values apart from base, each value read
@@ -74,26 +73,26 @@ hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 // storage (prec 2 fp16, 3 bf16: populations kept as k_d (f_d - w_d rho0))
 // MODE_COLL reads the moments from mout and MODE_MOM / MODE_MOM_PULL write them
 // there; F is float, Nu in the 16-bit format.
-hipError_t launch_esotwist(int prec, int layout, int mode, int even, void* Q, void* mout, const void* F, void* Nu,
+hipError_t launch_esotwist(int prec, int mode, int even, void* Q, void* mout, const void* F, void* Nu,
                            const uint64_t* fmask, const Grid& g, const CollideArgs& c, float rho0, hipStream_t s);
-hipError_t launch_simple(int prec, int layout, int mode, const void* src, void* dst, void* mout, const void* F,
+hipError_t launch_simple(int prec, int mode, const void* src, void* dst, void* mout, const void* F,
                          void* Nu, const uint64_t* fmask, const Grid& g, const CollideArgs& c, float rho0,
                          hipStream_t s);
 
 // element size 4 or 8: pure data movement on every cell
-hipError_t launch_push_all(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s);
-hipError_t launch_pull_all(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s);
-hipError_t launch_bounce_back(int esize, int layout, void* Q, const Grid& g, hipStream_t s);
-hipError_t launch_ghost_fill(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s);
-// Q (elements of esize bytes, 4 or 8) between the kernels' population array
-// (layout dlayout, padded rows) and the dense size x 18 array of the boundary
-// (layout blayout): to_boundary != 0 reads the former and writes the latter.
-hipError_t launch_q_boundary(int esize, int dlayout, int blayout, int to_boundary, const void* src, void* dst,
-                             const Grid& g, hipStream_t s);
+hipError_t launch_push_all(int esize, const void* src, void* dst, const Grid& g, hipStream_t s);
+hipError_t launch_pull_all(int esize, const void* src, void* dst, const Grid& g, hipStream_t s);
+hipError_t launch_bounce_back(int esize, void* Q, const Grid& g, hipStream_t s);
+hipError_t launch_ghost_fill(int esize, const void* src, void* dst, const Grid& g, hipStream_t s);
+// Elements [begin, end) of the dense size x 18 array of the boundary (layout
+// blayout; dense points at element begin) from (to_boundary != 0) or to the
+// kernels' population array Q; elements of esize bytes, 4 or 8.
+hipError_t launch_q_boundary(int esize, int blayout, int to_boundary, void* Q, void* dense, uint64_t begin,
+                             uint64_t end, const Grid& g, hipStream_t s);
 // ghost fill from reduced-precision populations (prec 2/3) into a float array
-hipError_t launch_ghost_fill_decode(int prec, int layout, const void* src, void* dst, const Grid& g, float rho0,
+hipError_t launch_ghost_fill_decode(int prec, const void* src, void* dst, const Grid& g, float rho0,
                                     hipStream_t s);
-hipError_t launch_ghost_copy(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s);
+hipError_t launch_ghost_copy(int esize, const void* src, void* dst, const Grid& g, hipStream_t s);
 
 hipError_t launch_mask_from_f(int prec, const void* F, uint64_t* mask, uint64_t* gmask, const Grid& g,
                               hipStream_t s);
@@ -102,16 +101,16 @@ hipError_t launch_zero_interior_o(uint8_t* O, const Grid& g, hipStream_t s);
 
 hipError_t launch_force_prepare(int prec, const PointsDev& p, int64_t begin, int64_t count, void* F,
                                 const uint64_t* prev, uint64_t* next, const Grid& g, hipStream_t s);
-hipError_t launch_force_level(int prec, int layout, int streaming, int momsrc, int even, const PointsDev& p,
+hipError_t launch_force_level(int prec, int streaming, int momsrc, int even, const PointsDev& p,
                               int64_t begin, int64_t count, void* F, const void* Q, const Grid& g, double alfa,
                               double beta, float rho0, hipStream_t s);
 
 // Density and momentum of IB stencil cells, 4 values of T per entry {rho, jx, jy, jz}.
 // cells: sorted cell indices (one entry per cell).
-hipError_t launch_ib_moments_cells(int prec, int layout, int streaming, int momsrc, int even, const uint32_t* cells,
+hipError_t launch_ib_moments_cells(int prec, int streaming, int momsrc, int even, const uint32_t* cells,
                                    int64_t n, void* cache, const void* Q, const Grid& g, float rho0, hipStream_t s);
 // one entry per (point, stencil cell): entry 9*t + s for point begin + t
-hipError_t launch_ib_moments_points(int prec, int layout, int streaming, int momsrc, int even, const PointsDev& p,
+hipError_t launch_ib_moments_points(int prec, int streaming, int momsrc, int even, const PointsDev& p,
                                     int64_t begin, int64_t count, void* cache, const void* Q, const Grid& g,
                                     float rho0, hipStream_t s);
 // One forcing level reading stencil moments from a cache.  sidx: per point 9 cache
@@ -193,7 +192,7 @@ inline int forcing_block_for(double cells) {
 // The gather of a bound tank's forcing pass (gb: which parts), then the levels of
 // every plane.  The gather starts next from static_base, the levels add the
 // blades' bits; blade stencil cells missing from prev get F = 0.
-hipError_t launch_force_gather(int prec, int layout, int streaming, int momsrc, int even, const ForceGeom& fg,
+hipError_t launch_force_gather(int prec, int streaming, int momsrc, int even, const ForceGeom& fg,
                                const BladeStep& st, const GatherBlocks& gb, const void* Q, void* F,
                                const uint64_t* prev, uint64_t* next, const uint64_t* static_base, const Grid& g,
                                float rho0, hipStream_t s);
@@ -251,17 +250,17 @@ struct ReduceArgs {
     int ghost;
 };
 // partial: kReduceBlocks * kReduceVals doubles; out: kReduceVals doubles (device)
-hipError_t launch_reduce(int prec, int layout, int streaming, int momsrc, int even, const void* Q, const void* F,
+hipError_t launch_reduce(int prec, int streaming, int momsrc, int even, const void* Q, const void* F,
                          const uint64_t* fmask, const Grid& g, const ReduceArgs& ra, float rho0, double* partial,
                          double* out, hipStream_t s);
 // {rho, ux, uy, uz} per interior cell in T, interior cells in (i, j, k) order
-hipError_t launch_macroscopic(int prec, int layout, int streaming, int momsrc, int even, const void* Q,
+hipError_t launch_macroscopic(int prec, int streaming, int momsrc, int even, const void* Q,
                               const void* F, const uint64_t* fmask, const Grid& g, float rho0, void* out,
                               hipStream_t s);
 
 // doubleResolutionFullCU: Q (esize 4/8) and a per-cell array (nu_esize 2/4/8)
 // of the old grid og copied into the doubled grid ng
-hipError_t launch_regrid(int esize, int layout, const void* oldQ, void* newQ, int nu_esize, const void* oldNu,
+hipError_t launch_regrid(int esize, const void* oldQ, void* newQ, int nu_esize, const void* oldNu,
                          void* newNu, const Grid& og, const Grid& ng, hipStream_t s);
 // n Nu values between the 16-bit storage of prec 2/3 and float (to_float != 0:
 // decode src into the float dst; else encode)
@@ -279,11 +278,11 @@ struct PlaneRec3 {
     float q[3];
 };
 // one record slot and one flag byte per plane cell (x * z, i-major); prec 0/1 (explicit Q type)
-hipError_t launch_plane_xz(int prec, int layout, const void* Q, const void* F, const uint64_t* fmask,
+hipError_t launch_plane_xz(int prec, const void* Q, const void* F, const uint64_t* fmask,
                            const uint8_t* exclude, const Grid& g, int cut, int64_t i0, int64_t k0, PlaneRec4* q,
                            PlaneRec3* f, uint8_t* flags, hipStream_t s);
 // vorticity field of plane j = cut (axis 0) or k = cut (axis 1), T per cell
-hipError_t launch_vorticity(int prec, int layout, int streaming, int momsrc, int even, const void* Q, const Grid& g,
+hipError_t launch_vorticity(int prec, int streaming, int momsrc, int even, const void* Q, const Grid& g,
                             int axis, int cut, const uint8_t* exclude, void* out, float rho0, hipStream_t s);
 
 // stencil rows of the n static points p, from the positions sidx (9 per point) of
@@ -351,10 +350,10 @@ struct BatchPlan {
 
 // Enqueue `steps` main-loop steps of every active member: per step the fused
 // stream-collide, the forcing gather, the forcing levels, advance.
-hipError_t launch_batch_step(int prec, int layout, int streaming, const BatchPlan& plan, int steps, hipStream_t s);
+hipError_t launch_batch_step(int prec, int streaming, const BatchPlan& plan, int steps, hipStream_t s);
 // blocks of the fused kernel for one member with the given tile and block size
 int64_t batch_coll_blocks(const Grid& g, int tile, int bs);
 // The fused kernel alone over every member (autotuning; advances no state).
-hipError_t launch_batch_fused(int prec, int layout, int streaming, const BatchPlan& plan, hipStream_t s);
+hipError_t launch_batch_fused(int prec, int streaming, const BatchPlan& plan, hipStream_t s);
 
 }  // namespace tdlb

@@ -42,22 +42,9 @@ inline uint32_t blocks_for(uint64_t n, int bs = kBlock) {
     return (uint32_t)(b > 0x7fffffffull ? 0x7fffffffull : (b ? b : 1));
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs (block b to XCD b % 8),
-// each XCD with its own L2.  xcd_block renumbers blocks so that each XCD takes
-// one contiguous range of rows.  In IJKL a cell's 18 slots share lines with its
-// neighbours', which neighbouring rows then find in the same L2 (measured 13-20 %
-// faster); in LIJK every line is read by one row only and the default order,
-// all XCDs streaming through one region of HBM together, is faster (5 %).
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t n) {
-    constexpr uint32_t nx = kXcds;
-    const uint32_t x = b % nx, q = b / nx;
-    const uint32_t per = n / nx, rem = n % nx;
-    return x * per + min(x, rem) + q;
-}
-template <int L>
-__device__ __forceinline__ uint32_t layout_block() {
-    return L == LayoutIJKL ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-}
+// Blocks take rows in dispatch order (round-robin over the 8 XCDs): every line is
+// read by one row only, and all XCDs streaming through one region of HBM together
+// are 5 % faster than each XCD on a contiguous range of its own.
 
 // ------------------------------------------------------------------ precisions
 // S: stored population type, T: arithmetic and F type, N: stored Nu type, D:
@@ -200,24 +187,21 @@ struct HwOps {
 
 // ------------------------------------------------------------------ fills
 // every slot of the population array, row padding included
-template <typename T, int L>
+template <typename T>
 __global__ void k_fill_q(T* __restrict__ Q, Grid g, T rho) {
-    const uint64_t cells = L == LayoutIJKL ? g.size : g.qsize;
-    const uint64_t total = cells * (uint64_t)kQ;
+    const uint64_t total = g.qsize * (uint64_t)kQ;
     for (uint64_t a = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; a < total;
          a += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t slot = (L == LayoutIJKL) ? a % kQ : a / cells;
-        Q[a] = slot == 0 ? rho : T(0);
+        Q[a] = a < g.qsize ? rho : T(0);
     }
 }
 
-// Between the population array of the kernels (layout DL, padded rows) and the
-// dense array of the boundary (layout BL: IJKL n*18 + l, LIJK l*size + n); one
-// boundary element per thread.
-template <typename W, int DL, int BL, bool TO_BOUNDARY>
-__global__ void k_q_boundary(const W* __restrict__ src, W* __restrict__ dst, Grid g) {
-    const uint64_t total = g.size * (uint64_t)kQ;
-    for (uint64_t a = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; a < total;
+// Between the population array of the kernels and the dense array of the boundary
+// (layout BL: IJKL n*18 + l, LIJK l*size + n), elements [begin, end) of the
+// latter, of which `dense` is element begin; one boundary element per thread.
+template <typename W, int BL, bool TO_BOUNDARY>
+__global__ void k_q_boundary(W* __restrict__ Q, W* __restrict__ dense, uint64_t begin, uint64_t end, Grid g) {
+    for (uint64_t a = begin + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; a < end;
          a += (uint64_t)gridDim.x * blockDim.x) {
         uint64_t n, l;
         if (BL == LayoutLIJK) {
@@ -229,9 +213,9 @@ __global__ void k_q_boundary(const W* __restrict__ src, W* __restrict__ dst, Gri
         }
         int i, j, k;
         decode_cell(g, n, i, j, k);
-        const uint64_t q = qaddr<DL>(g, qcell(g, i, j, k), (int)l);
-        if (TO_BOUNDARY) dst[a] = src[q];
-        else dst[q] = src[a];
+        const uint64_t q = qaddr(g, qcell(g, i, j, k), (int)l);
+        if (TO_BOUNDARY) dense[a - begin] = Q[q];
+        else Q[q] = dense[a - begin];
     }
 }
 
@@ -260,7 +244,7 @@ __global__ void k_copy_bytes(uint8_t* __restrict__ d, const uint8_t* __restrict_
 // where d was read.
 // mout receives the moments of MODE_MOM: Q itself (in place) when populations
 // are stored as T, a separate T array in the reference layout otherwise.
-template <typename PR, int L, int MODE, int EVEN, bool HINT = false>
+template <typename PR, int MODE, int EVEN, bool HINT = false>
 __device__ __forceinline__ void esotwist_cell(typename PR::S* __restrict__ Q, typename PR::T* mout,
                                               const typename PR::T* __restrict__ F, typename PR::N* __restrict__ Nu,
                                               const uint64_t* __restrict__ fmask, const Grid& g,
@@ -282,7 +266,7 @@ __device__ __forceinline__ void esotwist_cell(typename PR::S* __restrict__ Q, ty
     T v[kQ];
 #pragma unroll
     for (int d = 0; d < kQ; d++) {
-        const uint64_t a = qaddr<L>(g, home[d], EVEN ? d : opposite(d));
+        const uint64_t a = qaddr(g, home[d], EVEN ? d : opposite(d));
         // reduced-precision storage keeps the moments of MODE_COLL in mout
         // with HINT, the planes read at the cell's own k take the streaming hint
         if constexpr (PR::kShift && MODE == MODE_COLL) v[d] = mout[a];
@@ -300,7 +284,7 @@ __device__ __forceinline__ void esotwist_cell(typename PR::S* __restrict__ Q, ty
         T m[kQ];
         es_moments<T, D>(v, m);
 #pragma unroll
-        for (int d = 0; d < kQ; d++) mout[qaddr<L>(g, home[d], EVEN ? d : opposite(d))] = m[d];
+        for (int d = 0; d < kQ; d++) mout[qaddr(g, home[d], EVEN ? d : opposite(d))] = m[d];
         return;
     }
 
@@ -332,7 +316,7 @@ __device__ __forceinline__ void esotwist_cell(typename PR::S* __restrict__ Q, ty
     for (int d = 0; d < kQ; d++) {
         const int e = opposite(d);
         const uint32_t h = n2 + (uint32_t)((twist_dx(e) ? di2 : 0) + (twist_dy(e) ? dj2 : 0) + (twist_dz(e) ? dk2 : 0));
-        const uint64_t a = qaddr<L>(g, h, EVEN ? e : opposite(e));
+        const uint64_t a = qaddr(g, h, EVEN ? e : opposite(e));
         if constexpr (MODE == MODE_FUSED) {
             if (!HINT || twist_dz(e)) {
                 if constexpr (PR::kShift) store_dev<PR>(Q, a, d, p[d]);
@@ -346,210 +330,23 @@ __device__ __forceinline__ void esotwist_cell(typename PR::S* __restrict__ Q, ty
     }
 }
 
-template <typename PR, int L, int MODE, int EVEN, bool HINT>
+template <typename PR, int MODE, int EVEN, bool HINT>
 __global__ __launch_bounds__(kRowBlock) void k_esotwist(typename PR::S* __restrict__ Q, typename PR::T* mout,
                                                      const typename PR::T* __restrict__ F,
                                                      typename PR::N* __restrict__ Nu,
                                                      const uint64_t* __restrict__ fmask, Grid g,
                                                      CollideParams<typename PR::T> P, uint32_t nkb, float rho0) {
-    const RowBlock rb = row_block(g, layout_block<L>(), nkb, blockDim.x);
+    const RowBlock rb = row_block(g, blockIdx.x, nkb, blockDim.x);
     const int k = rb.k0 + (int)threadIdx.x;
     if (k > g.zg1) return;
-    esotwist_cell<PR, L, MODE, EVEN, HINT>(Q, mout, F, Nu, fmask, g, P, rho0, rb.i, rb.j, k);
-}
-
-// ------------------------------------------------------------------ Esotwist, IJKL through LDS
-// The fused step in IJKL, where a cell's 18 slots are one 72-byte record and a
-// lane reading single slots spans a line per lane.  A workgroup owns a tile
-// of RI x KT cells in (i, k) and marches along j through a chunk of planes,
-// holding two slabs in LDS: the records of rows i0 .. i0 + RI and cells
-// k0 .. k0 + KT (the extra row and cell are the tile's +1 halo, or the
-// periodic wrap) of plane j and of plane j + 1.  A slab is read from HBM with
-// consecutive lanes on consecutive words (whole records, coalesced), the cells
-// of plane j take their 18 values from the two slabs and put the collided ones
-// back in place, and the slab of plane j is written back, every word whose
-// owner is a cell of this tile that has run: a slot of a record belongs to one
-// cell (home(c, d) = c + twist(d), so the owner is the record - twist), and the
-// words owned by another tile, or by a plane outside the chunk, are neither
-// used nor written.  Two tiles may write disjoint words of one line; no word
-// has two writers.
-constexpr int kSlabPad = kQ + 1;  // LDS words per record: consecutive records start in different banks
-
-template <int EVEN>
-__device__ __forceinline__ uint32_t slot_twist_mask(int axis) {
-    uint32_t m = 0;
-#pragma unroll
-    for (int s = 0; s < kQ; s++) {
-        const int d = EVEN ? s : opposite(s);
-        const int t = axis == 0 ? twist_dx(d) : axis == 1 ? twist_dy(d) : twist_dz(d);
-        m |= (uint32_t)t << s;
-    }
-    return m;
-}
-
-template <typename PR, int EVEN, int RI, int KT>
-__global__ __launch_bounds__(RI * KT) void k_esotwist_ijkl_lds(typename PR::S* __restrict__ Q,
-                                                            const typename PR::T* __restrict__ F,
-                                                            typename PR::N* __restrict__ Nu,
-                                                            const uint64_t* __restrict__ fmask, Grid g,
-                                                            CollideParams<typename PR::T> P, int nti, int ntk,
-                                                            int jchunk, float rho0) {
-    using T = typename PR::T;
-    using D = typename PR::D;
-    using S = typename PR::S;
-    static_assert(!PR::kShift, "whole populations only");
-    constexpr int NR = RI + 1, NK = KT + 1, REC = NR * NK, NT = RI * KT;
-    __shared__ S slab[2][REC * kSlabPad];
-
-    const uint32_t b = blockIdx.x;
-    const int tk = (int)(b % (uint32_t)ntk);
-    const int ti = (int)((b / (uint32_t)ntk) % (uint32_t)nti);
-    const int tj = (int)(b / ((uint32_t)ntk * (uint32_t)nti));
-    const int i0 = 1 + ti * RI, k0 = 1 + tk * KT;
-    const int ri = min(RI, g.xg1 - i0 + 1), rk = min(KT, g.zg1 - k0 + 1);  // cells of the tile
-    const int js = 1 + tj * jchunk;
-    if (js > g.yg1) return;
-    const int je = min(g.yg1, js + jchunk - 1);
-    const int tid = (int)threadIdx.x;
-    const uint32_t txm = slot_twist_mask<EVEN>(0), tym = slot_twist_mask<EVEN>(1), tzm = slot_twist_mask<EVEN>(2);
-
-    // A slab row (records k0 .. k0 + rk of row i in plane j) is RW consecutive
-    // words in HBM, except that the +1 record past the last interior cell is
-    // the wrapped k = 1.  Lane t copies words c * NT + t of every row: its word
-    // offsets, LDS positions and slot bits are fixed for the tile, and only the
-    // row's base address changes with the row and the plane.
-    constexpr int RW = NK * kQ, RC = (RW + NT - 1) / NT, ITER = NR * RC;
-    int goff[RC], loff[RC];
-    uint32_t wbits[RC];  // bit 0: word in the tile's slab, 1: twist in x, 2: in y, 3: owner k inside the tile
-    const bool kwrap = k0 + rk > g.zg1;
-#pragma unroll
-    for (int c = 0; c < RC; c++) {
-        const int wr = c * NT + tid, kk = wr / kQ, sl = wr - kk * kQ;
-        const bool ok = wr < RW && kk <= rk;
-        goff[c] = (kwrap && kk == rk) ? (1 - k0) * kQ + sl : wr;  // the wrapped record sits at k = 1
-        loff[c] = kk * kSlabPad + sl;
-        const int okk = kk - (int)((tzm >> sl) & 1u);
-        wbits[c] = (ok ? 1u : 0u) | (((txm >> sl) & 1u) << 1) | (((tym >> sl) & 1u) << 2) |
-                   ((okk >= 0 && okk < rk) ? 8u : 0u);
-    }
-    // word offset of record (i0 + r, j, k0): the row past the tile wraps to i = 1
-    auto row_base = [&](int r, int j) __attribute__((always_inline)) -> int64_t {
-        int i = i0 + r;
-        if (i > g.xg1) i -= g.xg1;
-        const int jp = j > g.yg1 ? j - g.yg1 : j;
-        return (int64_t)cell_index(g, i, jp, k0) * kQ;
-    };
-    // every load of a slab issued before any is used
-    auto fetch = [&](S (&reg)[ITER], int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            if (r > ri) break;
-            const S* row = Q + row_base(r, j);
-#pragma unroll
-            for (int c = 0; c < RC; c++)
-                if (wbits[c] & 1u) reg[r * RC + c] = row[goff[c]];
-        }
-    };
-    auto put = [&](const S (&reg)[ITER], int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            if (r > ri) break;
-#pragma unroll
-            for (int c = 0; c < RC; c++)
-                if (wbits[c] & 1u) slab[buf][r * NK * kSlabPad + loff[c]] = reg[r * RC + c];
-        }
-    };
-    // write back the words of slab buf (plane j) owned by cells of this tile in
-    // planes js .. last: owner row r - tx inside the tile, owner k inside the
-    // tile, owner plane j - ty inside js .. last
-    auto store = [&](int buf, int j, int last) __attribute__((always_inline)) {
-        const bool pl0 = j >= js && j <= last, pl1 = j - 1 >= js && j - 1 <= last;
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            if (r > ri) break;
-            S* row = Q + row_base(r, j);
-#pragma unroll
-            for (int c = 0; c < RC; c++) {
-                const uint32_t wb = wbits[c];
-                const bool tx = wb & 2u, ty = wb & 4u;
-                const bool rok = r == ri ? tx : (r == 0 ? !tx : true);
-                if ((wb & 1u) && (wb & 8u) && rok && (ty ? pl1 : pl0))
-                    row[goff[c]] = slab[buf][r * NK * kSlabPad + loff[c]];
-            }
-        }
-    };
-
-    const int r = tid / KT, kk = tid - (tid / KT) * KT;
-    const bool active = r < ri && kk < rk;
-    const int ci = i0 + (active ? r : 0), ck = k0 + (active ? kk : 0);
-    // Nu and the F-occupancy word of a cell, fetched a plane ahead
-    auto cell_pre = [&](int j, T& nu, uint64_t& mw) __attribute__((always_inline)) {
-        nu = P.use_les ? load_nu<PR>(Nu, cell_index(g, ci, j, ck)) : T(0);
-        mw = fmask[mask_word_index(g, ci, j, ck)];
-    };
-    auto collide = [&](int j, int A, int B, T nuc, uint64_t mw) __attribute__((always_inline)) {
-        if (!active) return;
-        const uint32_t n = cell_index(g, ci, j, ck);
-        T v[kQ];
-#pragma unroll
-        for (int d = 0; d < kQ; d++) {
-            const int at = ((r + twist_dx(d)) * NK + kk + twist_dz(d)) * kSlabPad + (EVEN ? d : opposite(d));
-            v[d] = twist_dy(d) ? slab[B][at] : slab[A][at];
-        }
-        T fx = T(0), fy = T(0), fz = T(0);
-        if ((mw >> (ck & 63)) & 1ull) {
-            fx = F[3 * (uint64_t)n + 0];
-            fy = F[3 * (uint64_t)n + 1];
-            fz = F[3 * (uint64_t)n + 2];
-        }
-        T m[kQ], p[kQ];
-        es_moments<T, D>(v, m);
-        es_collide<T, D>(m, fx, fy, fz, nuc, P, p);
-        if (P.use_les) store_nu<PR>(Nu, n, nuc);
-#pragma unroll
-        for (int d = 0; d < kQ; d++) {
-            const int e = opposite(d);
-            const int at = ((r + twist_dx(e)) * NK + kk + twist_dz(e)) * kSlabPad + (EVEN ? e : opposite(e));
-            if (twist_dy(e)) slab[B][at] = p[d];
-            else slab[A][at] = p[d];
-        }
-    };
-    // Two slabs in LDS (planes j, j + 1) and one in flight in registers: plane
-    // j + 2 is requested while plane j collides and fills the buffer of plane j
-    // once that is written back.
-    S reg[ITER];
-    fetch(reg, js);
-    put(reg, 0);
-    fetch(reg, js + 1);
-    put(reg, 1);
-    T nu_c, nu_n = T(0);
-    uint64_t mw_c, mw_n = 0;
-    cell_pre(js, nu_c, mw_c);
-    __syncthreads();
-    int A = 0;
-    for (int j = js; j <= je; j++) {
-        const int B = A ^ 1;
-        const bool next = j + 2 <= je + 1;
-        if (next) fetch(reg, j + 2);
-        if (j + 1 <= je) cell_pre(j + 1, nu_n, mw_n);
-        collide(j, A, B, nu_c, mw_c);
-        __syncthreads();
-        store(A, j, je);
-        if (next) put(reg, A);
-        __syncthreads();
-        A = B;
-        nu_c = nu_n;
-        mw_c = mw_n;
-    }
-    // plane je + 1: the words of the chunk's last plane (twist in y)
-    store(A, je + 1, je);
+    esotwist_cell<PR, MODE, EVEN, HINT>(Q, mout, F, Nu, fmask, g, P, rho0, rb.i, rb.j, k);
 }
 
 // ------------------------------------------------------------------ Simple
 // In-place collide / moments, or pull from src (the two-lattice form of the
 // reference's in-place push: slot d of an interior cell c takes src[c-e_d][d]
 // when c-e_d is interior and keeps src[c][d] otherwise).
-template <typename PR, int L, int MODE>
+template <typename PR, int MODE>
 __device__ __forceinline__ void simple_cell(const typename PR::S* src,
                                             typename PR::S* dst,   // equal to src for in-place modes
                                             typename PR::T* mout,  // moments output of the MOM modes
@@ -573,15 +370,15 @@ __device__ __forceinline__ void simple_cell(const typename PR::S* src,
             const bool ok = (ex > 0 ? im : ex < 0 ? ip : true) && (ey > 0 ? jm : ey < 0 ? jp : true) &&
                             (ez > 0 ? km : ez < 0 ? kp : true);
             const int32_t off = -(ex * (int32_t)g.qyz + ey * (int32_t)g.qz + ez);
-            const uint64_t a = qaddr<L>(g, ok ? qn + (uint32_t)off : qn, d);
+            const uint64_t a = qaddr(g, ok ? qn + (uint32_t)off : qn, d);
             if constexpr (PR::kShift && MODE == MODE_FUSED) v[d] = load_dev<PR>(src, a, d);
             else v[d] = load_pop<PR>(src, a, d, rho0);
         }
     } else {
 #pragma unroll
         for (int d = 0; d < kQ; d++) {
-            if constexpr (PR::kShift && MODE == MODE_COLL) v[d] = mout[qaddr<L>(g, qn, d)];
-            else v[d] = load_pop<PR>(src, qaddr<L>(g, qn, d), d, rho0);
+            if constexpr (PR::kShift && MODE == MODE_COLL) v[d] = mout[qaddr(g, qn, d)];
+            else v[d] = load_pop<PR>(src, qaddr(g, qn, d), d, rho0);
         }
     }
 
@@ -589,7 +386,7 @@ __device__ __forceinline__ void simple_cell(const typename PR::S* src,
         T m[kQ];
         es_moments<T, D>(v, m);
 #pragma unroll
-        for (int d = 0; d < kQ; d++) mout[qaddr<L>(g, qn, d)] = m[d];
+        for (int d = 0; d < kQ; d++) mout[qaddr(g, qn, d)] = m[d];
         return;
     }
 
@@ -613,193 +410,27 @@ __device__ __forceinline__ void simple_cell(const typename PR::S* src,
     if (P.use_les) store_nu<PR>(Nu, n, nuc);
 #pragma unroll
     for (int d = 0; d < kQ; d++) {
-        if constexpr (PR::kShift && MODE == MODE_FUSED) store_dev<PR>(dst, qaddr<L>(g, qn, d), d, p[d]);
-        else store_pop<PR>(dst, qaddr<L>(g, qn, d), d, p[d], rho0);
+        if constexpr (PR::kShift && MODE == MODE_FUSED) store_dev<PR>(dst, qaddr(g, qn, d), d, p[d]);
+        else store_pop<PR>(dst, qaddr(g, qn, d), d, p[d], rho0);
     }
 }
 
-template <typename PR, int L, int MODE>
+template <typename PR, int MODE>
 __global__ __launch_bounds__(kRowBlock) void k_simple(const typename PR::S* src, typename PR::S* dst,
                                                    typename PR::T* mout, const typename PR::T* __restrict__ F,
                                                    typename PR::N* __restrict__ Nu,
                                                    const uint64_t* __restrict__ fmask, Grid g,
                                                    CollideParams<typename PR::T> P, uint32_t nkb, float rho0) {
-    const RowBlock rb = row_block(g, layout_block<L>(), nkb, blockDim.x);
+    const RowBlock rb = row_block(g, blockIdx.x, nkb, blockDim.x);
     const int k = rb.k0 + (int)threadIdx.x;
     if (k > g.zg1) return;
-    simple_cell<PR, L, MODE>(src, dst, mout, F, Nu, fmask, g, P, rho0, rb.i, rb.j, k);
-}
-
-// ------------------------------------------------------------------ Simple pull, IJKL through LDS
-// index of direction d among the five with e_y = +1
-TDLB_HD constexpr int ypos_index(int d) {
-    int n = 0;
-    for (int e = 0; e < d; e++)
-        if (dir_y(e) > 0) n++;
-    return n;
-}
-
-// The two-lattice pull in IJKL (src -> dst), staged like k_esotwist_ijkl_lds:
-// a workgroup owns a tile of RI x KT cells in (i, k) and marches along j with
-// two slabs of src records in LDS, rows i0 - 1 .. i0 + RI and cells
-// k0 - 1 .. k0 + KT (the +-1 halo; the ghost layer is real memory and the pull
-// never uses it) of planes j and j + 1.  The five directions with e_y = +1 pull
-// from plane j - 1: a lane reads them for its next cell while plane j - 1 is
-// still in LDS and carries them in registers.  Each cell writes its whole
-// record of dst, so no word of dst has two writers and the slabs are read-only.
-template <typename PR, int RI, int KT>
-__global__ __launch_bounds__(RI * KT) void k_simple_ijkl_lds(const typename PR::S* __restrict__ src,
-                                                          typename PR::S* __restrict__ dst,
-                                                          const typename PR::T* __restrict__ F,
-                                                          typename PR::N* __restrict__ Nu,
-                                                          const uint64_t* __restrict__ fmask, Grid g,
-                                                          CollideParams<typename PR::T> P, int nti, int ntk,
-                                                          int jchunk, float rho0) {
-    using T = typename PR::T;
-    using D = typename PR::D;
-    using S = typename PR::S;
-    static_assert(!PR::kShift, "whole populations only");
-    constexpr int NR = RI + 2, NK = KT + 2, REC = NR * NK, NT = RI * KT;
-    __shared__ S slab[2][REC * kSlabPad];
-
-    const uint32_t b = blockIdx.x;
-    const int tk = (int)(b % (uint32_t)ntk);
-    const int ti = (int)((b / (uint32_t)ntk) % (uint32_t)nti);
-    const int tj = (int)(b / ((uint32_t)ntk * (uint32_t)nti));
-    const int i0 = 1 + ti * RI, k0 = 1 + tk * KT;
-    const int ri = min(RI, g.xg1 - i0 + 1), rk = min(KT, g.zg1 - k0 + 1);
-    const int js = 1 + tj * jchunk;
-    if (js > g.yg1) return;
-    const int je = min(g.yg1, js + jchunk - 1);
-    const int tid = (int)threadIdx.x;
-
-    // slab row r holds records k0 - 1 .. k0 + rk of row i0 - 1 + r: RW words
-    // from the word offset of record (i0 - 1 + r, j, k0 - 1)
-    constexpr int RW = NK * kQ, RC = (RW + NT - 1) / NT, ITER = NR * RC;
-    int loff[RC];
-    bool wok[RC];
-#pragma unroll
-    for (int c = 0; c < RC; c++) {
-        const int wr = c * NT + tid, kk = wr / kQ, sl = wr - kk * kQ;
-        wok[c] = wr < RW && kk <= rk + 1;
-        loff[c] = kk * kSlabPad + sl;
-    }
-    auto row_base = [&](int r, int j) __attribute__((always_inline)) -> int64_t {
-        return (int64_t)cell_index(g, i0 - 1 + r, j, k0 - 1) * kQ;
-    };
-    auto fetch = [&](S (&reg)[ITER], int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            if (r > ri + 1) break;
-            const S* row = src + row_base(r, j);
-#pragma unroll
-            for (int c = 0; c < RC; c++) {
-                int t = c * NT + tid;
-                asm volatile("" : "+v"(t));  // not hoisted across the plane loop
-                if (wok[c]) reg[r * RC + c] = row[t];
-            }
-        }
-    };
-    auto put = [&](const S (&reg)[ITER], int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            if (r > ri + 1) break;
-#pragma unroll
-            for (int c = 0; c < RC; c++)
-                if (wok[c]) slab[buf][r * NK * kSlabPad + loff[c]] = reg[r * RC + c];
-        }
-    };
-
-    const int r = tid / KT, kk = tid - (tid / KT) * KT;
-    const bool active = r < ri && kk < rk;
-    const int ci = i0 + (active ? r : 0), ck = k0 + (active ? kk : 0);
-    const bool im = ci >= 2, ip = ci <= g.xg1 - 1, km = ck >= 2, kp = ck <= g.zg1 - 1;
-    // the source c - e_d of direction d is interior in x and z
-    auto xz_ok = [&](int d) __attribute__((always_inline)) {
-        const int ex = dir_x(d), ez = dir_z(d);
-        return (ex > 0 ? im : ex < 0 ? ip : true) && (ez > 0 ? km : ez < 0 ? kp : true);
-    };
-    // slab position of slot d of the source (i - e_x, k - e_z), or of the cell itself
-    auto src_at = [&](int d, bool shift) __attribute__((always_inline)) -> int {
-        const int dr = shift ? -dir_x(d) : 0, dk = shift ? -dir_z(d) : 0;
-        return ((r + 1 + dr) * NK + kk + 1 + dk) * kSlabPad + d;
-    };
-    // the e_y = +1 values of the next plane's cell (its sources lie in plane buf),
-    // used only where the source is interior
-    constexpr int NY = 5;
-    auto carry_from = [&](int buf, T (&cy)[NY]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int d = 0; d < kQ; d++)
-            if (dir_y(d) > 0) cy[ypos_index(d)] = slab[buf][src_at(d, true)];
-    };
-    auto cell_pre = [&](int j, T& nu, uint64_t& mw) __attribute__((always_inline)) {
-        nu = P.use_les ? load_nu<PR>(Nu, cell_index(g, ci, j, ck)) : T(0);
-        mw = fmask[mask_word_index(g, ci, j, ck)];
-    };
-
-    S reg[ITER];
-    fetch(reg, js - 1);
-    put(reg, 0);
-    fetch(reg, js);
-    put(reg, 1);
-    __syncthreads();
-    T cy[NY];
-    carry_from(0, cy);
-    if (js + 1 <= g.yg1 + 1) fetch(reg, js + 1);
-    __syncthreads();
-    put(reg, 0);
-    T nu_c, nu_n = T(0);
-    uint64_t mw_c, mw_n = 0;
-    cell_pre(js, nu_c, mw_c);
-    __syncthreads();
-    int A = 1;  // plane j; A ^ 1 holds plane j + 1
-    for (int j = js; j <= je; j++) {
-        const int B = A ^ 1;
-        const bool next = j + 2 <= je + 1;
-        if (next) fetch(reg, j + 2);
-        if (j + 1 <= je) cell_pre(j + 1, nu_n, mw_n);
-        if (active) {
-            const bool jm = j >= 2, jp = j <= g.yg1 - 1;
-            T v[kQ];
-#pragma unroll
-            for (int d = 0; d < kQ; d++) {
-                // the pull of simple_cell: the source when it is interior in every axis, else the cell itself
-                const int ey = dir_y(d);
-                const bool ok = xz_ok(d) && (ey > 0 ? jm : ey < 0 ? jp : true);
-                if (!ok) v[d] = slab[A][src_at(d, false)];
-                else if (ey > 0) v[d] = cy[ypos_index(d)];
-                else if (ey < 0) v[d] = slab[B][src_at(d, true)];
-                else v[d] = slab[A][src_at(d, true)];
-            }
-            carry_from(A, cy);  // v holds this cell's values; cy now the next cell's
-            const uint32_t cn = cell_index(g, ci, j, ck);
-            T fx = T(0), fy = T(0), fz = T(0);
-            if ((mw_c >> (ck & 63)) & 1ull) {
-                fx = F[3 * (uint64_t)cn + 0];
-                fy = F[3 * (uint64_t)cn + 1];
-                fz = F[3 * (uint64_t)cn + 2];
-            }
-            T m[kQ], p[kQ];
-            es_moments<T, D>(v, m);
-            es_collide<T, D>(m, fx, fy, fz, nu_c, P, p);
-            if (P.use_les) store_nu<PR>(Nu, cn, nu_c);
-            S* out = dst + (uint64_t)cn * kQ;
-#pragma unroll
-            for (int d = 0; d < kQ; d++) out[d] = p[d];
-        }
-        __syncthreads();
-        if (next) put(reg, A);  // plane j + 2 takes the buffer of plane j
-        __syncthreads();
-        A = B;
-        nu_c = nu_n;
-        mw_c = mw_n;
-    }
+    simple_cell<PR, MODE>(src, dst, mout, F, Nu, fmask, g, P, rho0, rb.i, rb.j, k);
 }
 
 // ------------------------------------------------------------------ data movement on every cell
 
 // push: dst[c][d] = src[c-e_d][d] if c-e_d is interior, else src[c][d] (all cells)
-template <typename W, int L>
+template <typename W>
 __global__ void k_push_all(const W* __restrict__ src, W* __restrict__ dst, Grid g) {
     for (uint64_t n = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; n < g.size;
          n += (uint64_t)gridDim.x * blockDim.x) {
@@ -810,13 +441,13 @@ __global__ void k_push_all(const W* __restrict__ src, W* __restrict__ dst, Grid 
         for (int d = 0; d < kQ; d++) {
             const int si = i - dir_x(d), sj = j - dir_y(d), sk = k - dir_z(d);
             const uint32_t s = is_interior(g, si, sj, sk) ? qcell(g, si, sj, sk) : qc;
-            dst[qaddr<L>(g, qc, d)] = src[qaddr<L>(g, s, d)];
+            dst[qaddr(g, qc, d)] = src[qaddr(g, s, d)];
         }
     }
 }
 
 // pull: interior dst[c][d] = src[c-e_d][d]; ghosts copied
-template <typename W, int L>
+template <typename W>
 __global__ void k_pull_all(const W* __restrict__ src, W* __restrict__ dst, Grid g) {
     for (uint64_t n = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; n < g.size;
          n += (uint64_t)gridDim.x * blockDim.x) {
@@ -827,7 +458,7 @@ __global__ void k_pull_all(const W* __restrict__ src, W* __restrict__ dst, Grid 
 #pragma unroll
         for (int d = 0; d < kQ; d++) {
             const uint32_t s = in ? qcell(g, i - dir_x(d), j - dir_y(d), k - dir_z(d)) : qc;
-            dst[qaddr<L>(g, qc, d)] = src[qaddr<L>(g, s, d)];
+            dst[qaddr(g, qc, d)] = src[qaddr(g, s, d)];
         }
     }
 }
@@ -836,7 +467,7 @@ __global__ void k_pull_all(const W* __restrict__ src, W* __restrict__ dst, Grid 
 // face cell takes slot opp(d) of the neighbour g+e_d.  Faces run in the
 // reference's order as separate launches because face rims read ghosts of
 // faces handled later.
-template <typename W, int L>
+template <typename W>
 __global__ void k_bb_face(W* __restrict__ Q, Grid g, int face) {
     const int axis = face >> 1;        // 0 i, 1 j, 2 k
     const int inward = (face & 1) ? -1 : 1;
@@ -857,14 +488,14 @@ __global__ void k_bb_face(W* __restrict__ Q, Grid g, int face) {
             const int comp = axis == 0 ? dir_x(d) : axis == 1 ? dir_y(d) : dir_z(d);
             if (comp != inward) continue;
             const uint32_t s = qcell(g, i + dir_x(d), j + dir_y(d), k + dir_z(d));
-            Q[qaddr<L>(g, c, d)] = Q[qaddr<L>(g, s, opposite(d))];
+            Q[qaddr(g, c, d)] = Q[qaddr(g, s, opposite(d))];
         }
     }
 }
 
 // The 12 edge lines of the bounce-back (Boundary.hpp:41-132): on an edge the
 // one direction pointing inward on both boundary axes takes opp(d) of g+e_d.
-template <typename W, int L>
+template <typename W>
 __global__ void k_bb_edges(W* __restrict__ Q, Grid g) {
     const int nmax = max(g.xg1, max(g.yg1, g.zg1));
     const uint64_t total = 12ull * nmax;
@@ -891,7 +522,7 @@ __global__ void k_bb_edges(W* __restrict__ Q, Grid g) {
         if (s > lim) continue;
         const uint32_t c = qcell(g, i, j, k);
         const uint32_t src = qcell(g, i + dir_x(d), j + dir_y(d), k + dir_z(d));
-        Q[qaddr<L>(g, c, d)] = Q[qaddr<L>(g, src, opposite(d))];
+        Q[qaddr(g, c, d)] = Q[qaddr(g, src, opposite(d))];
     }
 }
 
@@ -935,7 +566,7 @@ __host__ __device__ inline uint64_t ghost_count(const Grid& g) {
 // into the ghost layer (c-e_d interior) and the bounce-back slots whose source
 // g+e_d is interior.  Rim bounce-back slots (ghost source) and never-written
 // slots are left as they are in dst.
-template <typename PR, int L>
+template <typename PR>
 __global__ void k_ghost_fill(const typename PR::S* __restrict__ src, typename PR::T* __restrict__ dst, Grid g,
                              float rho0) {
     const uint64_t total = ghost_count(g);
@@ -953,7 +584,7 @@ __global__ void k_ghost_fill(const typename PR::S* __restrict__ src, typename PR
             const int ex = dir_x(d), ey = dir_y(d), ez = dir_z(d);
             const int si = i - ex, sj = j - ey, sk = k - ez;
             if (is_interior(g, si, sj, sk)) {
-                dst[qaddr<L>(g, c, d)] = load_pop<PR>(src, qaddr<L>(g, qcell(g, si, sj, sk), d), d, rho0);
+                dst[qaddr(g, c, d)] = load_pop<PR>(src, qaddr(g, qcell(g, si, sj, sk), d), d, rho0);
                 continue;
             }
             bool bb = false;
@@ -967,12 +598,12 @@ __global__ void k_ghost_fill(const typename PR::S* __restrict__ src, typename PR
             const int ti = i + ex, tj = j + ey, tk = k + ez;
             if (!is_interior(g, ti, tj, tk)) continue;
             // opp(d) has the rest weight of d
-            dst[qaddr<L>(g, c, d)] = load_pop<PR>(src, qaddr<L>(g, qcell(g, ti, tj, tk), opposite(d)), d, rho0);
+            dst[qaddr(g, c, d)] = load_pop<PR>(src, qaddr(g, qcell(g, ti, tj, tk), opposite(d)), d, rho0);
         }
     }
 }
 
-template <typename W, int L>
+template <typename W>
 __global__ void k_ghost_copy(const W* __restrict__ src, W* __restrict__ dst, Grid g) {
     const uint64_t total = ghost_count(g);
     for (uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t < total;
@@ -981,7 +612,7 @@ __global__ void k_ghost_copy(const W* __restrict__ src, W* __restrict__ dst, Gri
         if (!ghost_cell(g, t, i, j, k)) continue;
         const uint32_t c = qcell(g, i, j, k);
 #pragma unroll
-        for (int d = 0; d < kQ; d++) dst[qaddr<L>(g, c, d)] = src[qaddr<L>(g, c, d)];
+        for (int d = 0; d < kQ; d++) dst[qaddr(g, c, d)] = src[qaddr(g, c, d)];
     }
 }
 
@@ -1074,7 +705,7 @@ __global__ void k_force_prepare(PointsDev p, int64_t begin, int64_t count, T* __
 }
 
 // density and momentum of cell (i,j,k) as the reference's moments() would leave them
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __device__ __forceinline__ void cell_rho_j(const typename PR::S* __restrict__ Q, const Grid& g, int i, int j, int k,
                                            typename PR::T& rho, typename PR::T& jx, typename PR::T& jy,
                                            typename PR::T& jz, float rho0) {
@@ -1089,7 +720,7 @@ __device__ __forceinline__ void cell_rho_j(const typename PR::S* __restrict__ Q,
 #pragma unroll
             for (int d = 0; d < 4; d++) {
                 const uint32_t h = n + (uint32_t)((twist_dx(d) ? di : 0) + (twist_dy(d) ? dj : 0) + (twist_dz(d) ? dk : 0));
-                m[d] = (T)Q[qaddr<L>(g, h, EVEN ? d : opposite(d))];
+                m[d] = (T)Q[qaddr(g, h, EVEN ? d : opposite(d))];
             }
             rho = m[0]; jx = m[1]; jy = m[2]; jz = m[3];
         } else {
@@ -1097,16 +728,16 @@ __device__ __forceinline__ void cell_rho_j(const typename PR::S* __restrict__ Q,
 #pragma unroll
             for (int d = 0; d < kQ; d++) {
                 const uint32_t h = n + (uint32_t)((twist_dx(d) ? di : 0) + (twist_dy(d) ? dj : 0) + (twist_dz(d) ? dk : 0));
-                f[d] = load_pop<PR>(Q, qaddr<L>(g, h, EVEN ? d : opposite(d)), d, rho0);
+                f[d] = load_pop<PR>(Q, qaddr(g, h, EVEN ? d : opposite(d)), d, rho0);
             }
             es_rho_j(f, rho, jx, jy, jz);
         }
     } else {
         if (MOMSRC == MOMSRC_STORED) {
-            rho = (T)Q[qaddr<L>(g, n, 0)];
-            jx = (T)Q[qaddr<L>(g, n, 1)];
-            jy = (T)Q[qaddr<L>(g, n, 2)];
-            jz = (T)Q[qaddr<L>(g, n, 3)];
+            rho = (T)Q[qaddr(g, n, 0)];
+            jx = (T)Q[qaddr(g, n, 1)];
+            jy = (T)Q[qaddr(g, n, 2)];
+            jz = (T)Q[qaddr(g, n, 3)];
         } else {
             const bool im = i >= 2, ip = i <= g.xg1 - 1;
             const bool jm = j >= 2, jp = j <= g.yg1 - 1;
@@ -1118,7 +749,7 @@ __device__ __forceinline__ void cell_rho_j(const typename PR::S* __restrict__ Q,
                 const bool ok = (ex > 0 ? im : ex < 0 ? ip : true) && (ey > 0 ? jm : ey < 0 ? jp : true) &&
                                 (ez > 0 ? km : ez < 0 ? kp : true);
                 const int32_t off = -(ex * (int32_t)g.qyz + ey * (int32_t)g.qz + ez);
-                f[d] = load_pop<PR>(Q, qaddr<L>(g, ok ? n + (uint32_t)off : n, d), d, rho0);
+                f[d] = load_pop<PR>(Q, qaddr(g, ok ? n + (uint32_t)off : n, d), d, rho0);
             }
             es_rho_j(f, rho, jx, jy, jz);
         }
@@ -1128,7 +759,7 @@ __device__ __forceinline__ void cell_rho_j(const typename PR::S* __restrict__ Q,
 // One level of the forcing: points of a level have pairwise disjoint stencils,
 // so each thread runs the reference's gather / correct / spread for one point
 // (Forcing.hpp:73-135) with the F values left by all earlier levels.
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ __launch_bounds__(kBlock) void k_force_level(PointsDev p, int64_t begin, int64_t count,
                                                         typename PR::T* __restrict__ F,
                                                         const typename PR::S* __restrict__ Q, Grid g,
@@ -1153,7 +784,7 @@ __global__ __launch_bounds__(kBlock) void k_force_level(PointsDev p, int64_t beg
         for (int i1 = -1; i1 <= 1; i1++) {
             const int i2 = wrap_ik(pi + i1, g.xg1), k2 = wrap_ik(pk + k1, g.zg1);
             T rho, jx, jy, jz;
-            cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i2, pj, k2, rho, jx, jy, jz, rho0);
+            cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i2, pj, k2, rho, jx, jy, jz, rho0);
             const uint64_t c = cell_index(g, i2, pj, k2);
             const T ppp = wx[i1 + 1] * wz[k1 + 1];
             const T xx = (T)((D)jx + D(0.5) * (D)F[3 * c + 0]);
@@ -1190,7 +821,7 @@ struct alignas(4 * sizeof(T)) Mom4 {
     T r, x, y, z;
 };
 
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ __launch_bounds__(kBlock) void k_ib_moments_cells(const uint32_t* __restrict__ cells, int64_t n,
                                                              Mom4<typename PR::T>* __restrict__ cache,
                                                              const typename PR::S* __restrict__ Q, Grid g,
@@ -1204,11 +835,11 @@ __global__ __launch_bounds__(kBlock) void k_ib_moments_cells(const uint32_t* __r
     const int j = (int)(r / (uint32_t)g.zg);
     const int k = (int)(r - (uint32_t)j * (uint32_t)g.zg);
     Mom4<T> m;
-    cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, m.r, m.x, m.y, m.z, rho0);
+    cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, m.r, m.x, m.y, m.z, rho0);
     cache[t] = m;
 }
 
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ __launch_bounds__(kBlock) void k_ib_moments_points(PointsDev p, int64_t begin, int64_t count,
                                                               Mom4<typename PR::T>* __restrict__ cache,
                                                               const typename PR::S* __restrict__ Q, Grid g,
@@ -1220,7 +851,7 @@ __global__ __launch_bounds__(kBlock) void k_ib_moments_points(PointsDev p, int64
     const int s = (int)(t % 9);
     const int i2 = wrap_ik(p.i[q] + (s % 3) - 1, g.xg1), k2 = wrap_ik(p.k[q] + (s / 3) - 1, g.zg1);
     Mom4<T> m;
-    cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i2, p.j[q], k2, m.r, m.x, m.y, m.z, rho0);
+    cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i2, p.j[q], k2, m.r, m.x, m.y, m.z, rho0);
     cache[t] = m;
 }
 
@@ -1504,7 +1135,7 @@ __device__ __forceinline__ int blade_plane(const ForceGeom& fg, int j, int& nlev
 
 // Static stencil cells [c0, c1) of fg.cells: density and momentum into the cache,
 // thread t of `threads` taking c0 + t, c0 + t + threads, ...
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __device__ __forceinline__ void gather_cells(const ForceGeom& fg, int64_t c0, int64_t c1, int64_t t,
                                              int64_t threads, const typename PR::S* __restrict__ Q, const Grid& g,
                                              float rho0) {
@@ -1515,7 +1146,7 @@ __device__ __forceinline__ void gather_cells(const ForceGeom& fg, int64_t c0, in
         const uint32_t r = n - (uint32_t)i * g.yz;
         const int j = (int)(r / (uint32_t)g.zg), k = (int)(r - (uint32_t)j * (uint32_t)g.zg);
         Mom4<typename PR::T> m;
-        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, m.r, m.x, m.y, m.z, rho0);
+        cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, m.r, m.x, m.y, m.z, rho0);
         scache[e] = m;
     }
 }
@@ -1525,7 +1156,7 @@ __device__ __forceinline__ void gather_cells(const ForceGeom& fg, int64_t c0, in
 // generator's arithmetic), by its first lanes also to the point list and the
 // stencil rows; F = 0 where the previous mask lacks the cell; density and
 // momentum into the blade cache.
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __device__ __forceinline__ void gather_blade_cell(const ForceGeom& fg, const BladeStep& st, int t,
                                                   const typename PR::S* __restrict__ Q,
                                                   typename PR::T* __restrict__ F, const uint64_t* __restrict__ prev,
@@ -1566,13 +1197,13 @@ __device__ __forceinline__ void gather_blade_cell(const ForceGeom& fg, const Bla
         F[3 * cc + 2] = T(0);
     }
     Mom4<T> m;
-    cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i2, j, k2, m.r, m.x, m.y, m.z, rho0);
+    cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i2, j, k2, m.r, m.x, m.y, m.z, rho0);
     static_cast<Mom4<T>*>(fg.rcache)[9 * (int64_t)e + s] = m;
 }
 
 // Block b of a tank's gather: the blades' blocks first (their points cost the
 // most arithmetic), then the static cells', then the mask words'.
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __device__ __forceinline__ void force_gather(const ForceGeom& fg, const BladeStep& st, uint32_t b,
                                              const GatherBlocks& gb, const typename PR::S* __restrict__ Q,
                                              typename PR::T* __restrict__ F, const uint64_t* __restrict__ prev,
@@ -1581,20 +1212,20 @@ __device__ __forceinline__ void force_gather(const ForceGeom& fg, const BladeSte
     if (b < gb.blades) {
         const int64_t t = (int64_t)b * kGatherBlock + threadIdx.x;
         if (t < 9 * fg.n_rot)
-            gather_blade_cell<PR, L, STREAM, MOMSRC, EVEN>(fg, st, (int)t, Q, F, prev, g, rho0);
+            gather_blade_cell<PR, STREAM, MOMSRC, EVEN>(fg, st, (int)t, Q, F, prev, g, rho0);
         return;
     }
     b -= gb.blades;
     if (b < gb.cells) {
         const int64_t e = (int64_t)b * kGatherBlock + threadIdx.x;
-        gather_cells<PR, L, STREAM, MOMSRC, EVEN>(fg, e, min(e + 1, fg.n_cells), 0, 1, Q, g, rho0);
+        gather_cells<PR, STREAM, MOMSRC, EVEN>(fg, e, min(e + 1, fg.n_cells), 0, 1, Q, g, rho0);
         return;
     }
     const uint64_t w = (uint64_t)(b - gb.cells) * kGatherBlock + threadIdx.x;
     if (w < (uint64_t)g.xg * g.yg * g.mask_w) next[w] = static_base[w];
 }
 
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ __launch_bounds__(kGatherBlock) void k_force_gather(ForceGeom fg, BladeStep st, GatherBlocks gb,
                                                                const typename PR::S* __restrict__ Q,
                                                                typename PR::T* __restrict__ F,
@@ -1602,7 +1233,7 @@ __global__ __launch_bounds__(kGatherBlock) void k_force_gather(ForceGeom fg, Bla
                                                                uint64_t* __restrict__ next,
                                                                const uint64_t* __restrict__ static_base, Grid g,
                                                                float rho0) {
-    force_gather<PR, L, STREAM, MOMSRC, EVEN>(fg, st, blockIdx.x, gb, Q, F, prev, next, static_base, g, rho0);
+    force_gather<PR, STREAM, MOMSRC, EVEN>(fg, st, blockIdx.x, gb, Q, F, prev, next, static_base, g, rho0);
 }
 
 // a copy that every lane knows to be the same for the whole wave (scalar registers)
@@ -1989,7 +1620,6 @@ __global__ __launch_bounds__(kRowBlock) __attribute__((amdgpu_waves_per_eu(pipe_
 void k_eso_pipe(PipeArgs a, Grid g, CollideParams<float> P, uint32_t nkb,
                                                       float rho0, float alfa, float beta) {
     using S = typename PR::S;
-    constexpr int L = LayoutLIJK;
     constexpr int STREAM = StreamEsotwist;
     constexpr int MS = MOMSRC_ESO_POPS;
     // the gathers read the populations of the next step's collision
@@ -2044,7 +1674,7 @@ void k_eso_pipe(PipeArgs a, Grid g, CollideParams<float> P, uint32_t nkb,
                 else hi = mid - 1;
             }
             const int64_t e = s_c0[lo] + (t - s_pre[lo]);
-            gather_cells<PR, L, STREAM, MS, GE>(a.fg, e, e + 1, 0, 1, Q, g, rho0);
+            gather_cells<PR, STREAM, MS, GE>(a.fg, e, e + 1, 0, 1, Q, g, rho0);
         }
     };
     auto wait_rows = [&](int i) {
@@ -2082,7 +1712,7 @@ void k_eso_pipe(PipeArgs a, Grid g, CollideParams<float> P, uint32_t nkb,
                     const int j = jlo + (int)(b / nkb);
                     const int k = (int)((b % nkb) * blockDim.x) + 1 + tid;
                     if (k <= g.zg1)
-                        esotwist_cell<PR, L, MODE_FUSED, EVEN, HINT>(Q, nullptr, F, Nu, a.prev, g, P, rho0, i, j, k);
+                        esotwist_cell<PR, MODE_FUSED, EVEN, HINT>(Q, nullptr, F, Nu, a.prev, g, P, rho0, i, j, k);
                     if (b % nkb == 0) {
                         // static occupancy words of the row, and of the ghost rows beside it
                         const int ia = i == 1 ? 0 : i, ib = i == ni ? ni + 1 : i;
@@ -2130,7 +1760,7 @@ void k_eso_pipe(PipeArgs a, Grid g, CollideParams<float> P, uint32_t nkb,
             __threadfence();
             const int64_t c0 = b < nBl ? cl0 + (int64_t)b * chunk : ch0 + (int64_t)(b - nBl) * chunk;
             const int64_t c1 = b < nBl ? cl1 : ch1;
-            gather_cells<PR, L, STREAM, MS, GE>(a.fg, c0, c0 + chunk < c1 ? c0 + chunk : c1, tid, blockDim.x, Q, g,
+            gather_cells<PR, STREAM, MS, GE>(a.fg, c0, c0 + chunk < c1 ? c0 + chunk : c1, tid, blockDim.x, Q, g,
                                                  rho0);
             gather_done();
         }
@@ -2166,7 +1796,7 @@ __device__ __forceinline__ void cell_force(const T* __restrict__ F, const uint64
 
 // Per block: {sum rho, sum jx, jy, jz, sum Fx, Fy, Fz, torque} in FP64.  The
 // grid is fixed, so the partial sums and their combination are deterministic.
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ __launch_bounds__(kBlock) void k_reduce_cells(const typename PR::S* __restrict__ Q,
                                                          const typename PR::T* __restrict__ F,
                                                          const uint64_t* __restrict__ fmask, Grid g, ReduceArgs ra,
@@ -2180,7 +1810,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_cells(const typename PR::S* _
         int i, j, k;
         interior_cell(g, t, i, j, k);
         T rho, jx, jy, jz, fx, fy, fz;
-        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, rho, jx, jy, jz, rho0);
+        cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, rho, jx, jy, jz, rho0);
         cell_force(F, fmask, g, i, j, k, fx, fy, fz);
         acc[0] += (double)rho;
         acc[1] += (double)jx;
@@ -2226,7 +1856,7 @@ __global__ __launch_bounds__(kReduceFinalBlock) void k_reduce_final(const double
 
 // {rho, ux, uy, uz} per interior cell, u as QVec::velocity(F) forms it
 // (QVec.hpp:125-131: (1.0 / rho) * (j + 0.5 * F), double literals).
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ __launch_bounds__(kBlock) void k_macroscopic(const typename PR::S* __restrict__ Q,
                                                         const typename PR::T* __restrict__ F,
                                                         const uint64_t* __restrict__ fmask, Grid g, float rho0,
@@ -2238,7 +1868,7 @@ __global__ __launch_bounds__(kBlock) void k_macroscopic(const typename PR::S* __
         int i, j, k;
         interior_cell(g, t, i, j, k);
         T rho, jx, jy, jz, fx, fy, fz;
-        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, rho, jx, jy, jz, rho0);
+        cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, rho, jx, jy, jz, rho0);
         cell_force(F, fmask, g, i, j, k, fx, fy, fz);
         const D inv = D(1.0) / (D)rho;
         out[4 * t + 0] = rho;
@@ -2257,7 +1887,7 @@ __device__ __forceinline__ uint32_t regrid_source(const Grid& og, const Grid& ng
     return cell_index(og, i / 2 + (i & 1), j / 2 + (j & 1), k / 2 + (k & 1));
 }
 
-template <typename W, int L>
+template <typename W>
 __global__ void k_regrid_q(const W* __restrict__ old, W* __restrict__ nw, Grid og, Grid ng) {
     for (uint64_t n = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; n < ng.size;
          n += (uint64_t)gridDim.x * blockDim.x) {
@@ -2266,7 +1896,7 @@ __global__ void k_regrid_q(const W* __restrict__ old, W* __restrict__ nw, Grid o
         const uint32_t to = qcell(ng, i, j, k);
         const uint32_t from = qcell(og, i / 2 + (i & 1), j / 2 + (j & 1), k / 2 + (k & 1));
 #pragma unroll
-        for (int l = 0; l < kQ; l++) nw[qaddr<L>(ng, to, l)] = old[qaddr<L>(og, from, l)];
+        for (int l = 0; l < kQ; l++) nw[qaddr(ng, to, l)] = old[qaddr(og, from, l)];
     }
 }
 
@@ -2280,7 +1910,7 @@ __global__ void k_regrid_cells(const W* __restrict__ old, W* __restrict__ nw, Gr
 // savePlaneXZ<float, 4> (ComputeUnitOutput.hpp:354-447) for every plane cell
 // (i-major); flags bit 0: a QVec record (cell not excluded), bit 1: an F3 record
 // (Force::isNotZero: all three components non-zero, QVec.hpp:54-56).
-template <typename T, int L>
+template <typename T>
 __global__ void k_plane_xz(const T* __restrict__ Q, const T* __restrict__ F, const uint64_t* __restrict__ fmask,
                            const uint8_t* __restrict__ exclude, Grid g, int cut, int64_t i0, int64_t k0,
                            PlaneRec4* __restrict__ q, PlaneRec3* __restrict__ f, uint8_t* __restrict__ flags) {
@@ -2297,7 +1927,7 @@ __global__ void k_plane_xz(const T* __restrict__ Q, const T* __restrict__ F, con
         r.k = (uint16_t)(k0 + k - 1);
         r.pad = 0;
 #pragma unroll
-        for (int l = 0; l < 4; l++) r.q[l] = (float)Q[qaddr<L>(g, qcell(g, i, cut, k), l)];
+        for (int l = 0; l < 4; l++) r.q[l] = (float)Q[qaddr(g, qcell(g, i, cut, k), l)];
         q[t] = r;
         if (mask_test(fmask, g, i, cut, k)) {
             const T fx = F[3 * (uint64_t)n], fy = F[3 * (uint64_t)n + 1], fz = F[3 * (uint64_t)n + 2];
@@ -2323,7 +1953,7 @@ __global__ void k_plane_xz(const T* __restrict__ Q, const T* __restrict__ F, con
 // no force term) read through the streaming accessor; excluded cells NaN.  The
 // twisted read of a far-side ghost cell leaves the array in the reference, so
 // such neighbours give NaN here.  axis 0: plane j = cut, (x, z); 1: k = cut, (x, y).
-template <typename PR, int L, int STREAM, int MOMSRC, int EVEN>
+template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ void k_vorticity(const typename PR::S* __restrict__ Q, Grid g, int axis, int cut,
                             const uint8_t* __restrict__ exclude, typename PR::T* __restrict__ out, float rho0) {
     using T = typename PR::T;
@@ -2342,7 +1972,7 @@ __global__ void k_vorticity(const typename PR::S* __restrict__ Q, Grid g, int ax
             return;
         }
         T rho, jx, jy, jz;
-        cell_rho_j<PR, L, STREAM, MOMSRC, EVEN>(Q, g, a, b, e, rho, jx, jy, jz, rho0);
+        cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, a, b, e, rho, jx, jy, jz, rho0);
         ux = jx / rho;
         uy = jy / rho;
         uz = jz / rho;
@@ -2403,22 +2033,7 @@ inline void row_launch(const Grid& g, uint32_t& nkb, uint32_t& nblocks, uint32_t
     nblocks = nkb * (uint32_t)g.yg1 * (uint32_t)g.xg1;
 }
 
-// the LDS-staged IJKL step: tile RI x KT cells, about kIjklBlocks workgroups.
-// Measured at 512^3 (FP32): 4 x 64 and 16384 workgroups 5.48 ms, 8 x 32 5.51 ms
-// (6144 workgroups 5.66 ms), 16 x 16 7.03 ms, 8 x 16 6.24 ms.
-constexpr int kIjklTileI = 4, kIjklTileK = 64, kIjklBlocks = 16384;
-// the Simple pull through LDS: tile RI x KT cells (halo on both sides)
-constexpr int kIjklPullI = 8, kIjklPullK = 32;
-// TDLB_IJKL_LDS=0 selects the one-row kernel for IJKL (for comparison)
-inline bool ijkl_lds() {
-    static const bool on = [] {
-        const char* v = std::getenv("TDLB_IJKL_LDS");
-        return !(v && v[0] == '0');
-    }();
-    return on;
-}
-
-template <typename PR, int L>
+template <typename PR>
 hipError_t esotwist_t(int mode, int even, void* Q, void* mout, const void* F, void* Nu, const uint64_t* fm,
                       const Grid& g, const CollideArgs& c, float rho0, hipStream_t s) {
     using S = typename PR::S;
@@ -2431,34 +2046,13 @@ hipError_t esotwist_t(int mode, int even, void* Q, void* mout, const void* F, vo
     auto* nu = static_cast<typename PR::N*>(Nu);
     const auto P = to_params<T, typename PR::D>(c);
 #define TDLB_ESO(M, E, H) \
-    hipLaunchKernelGGL((k_esotwist<PR, L, M, E, H>), dim3(nb), dim3(bk), 0, s, q, mo, f, nu, fm, g, P, nkb, rho0)
+    hipLaunchKernelGGL((k_esotwist<PR, M, E, H>), dim3(nb), dim3(bk), 0, s, q, mo, f, nu, fm, g, P, nkb, rho0)
     if (mode == MODE_COLL) { if (even) TDLB_ESO(MODE_COLL, 1, false); else TDLB_ESO(MODE_COLL, 0, false); }
     else if (mode == MODE_MOM) { if (even) TDLB_ESO(MODE_MOM, 1, false); else TDLB_ESO(MODE_MOM, 0, false); }
     else if (mode == MODE_FUSED) {
-        if constexpr (L == LayoutLIJK) {
-            if (line_rows<S>(g)) {
-                if (even) TDLB_ESO(MODE_FUSED, 1, true); else TDLB_ESO(MODE_FUSED, 0, true);
-                return hipGetLastError();
-            }
-        }
-        if constexpr (L == LayoutIJKL && !PR::kShift && std::is_same<typename PR::T, float>::value) {
-            if (ijkl_lds()) {
-                constexpr int RI = kIjklTileI, KT = kIjklTileK;
-                const int nti = (g.xg1 + RI - 1) / RI, ntk = (g.zg1 + KT - 1) / KT;
-                // j chunks: enough workgroups to fill the GPU several times over
-                const int cols = nti * ntk;
-                const int want = (kIjklBlocks + cols - 1) / cols;
-                const int jchunk = std::max(4, (g.yg1 + want - 1) / want);
-                const int nch = (g.yg1 + jchunk - 1) / jchunk;
-                const dim3 grid((uint32_t)(cols * nch)), block((uint32_t)(RI * KT));
-                if (even)
-                    hipLaunchKernelGGL((k_esotwist_ijkl_lds<PR, 1, RI, KT>), grid, block, 0, s, q, f, nu, fm, g, P, nti,
-                                       ntk, jchunk, rho0);
-                else
-                    hipLaunchKernelGGL((k_esotwist_ijkl_lds<PR, 0, RI, KT>), grid, block, 0, s, q, f, nu, fm, g, P, nti,
-                                       ntk, jchunk, rho0);
-                return hipGetLastError();
-            }
+        if (line_rows<S>(g)) {
+            if (even) TDLB_ESO(MODE_FUSED, 1, true); else TDLB_ESO(MODE_FUSED, 0, true);
+            return hipGetLastError();
         }
         if (even) TDLB_ESO(MODE_FUSED, 1, false); else TDLB_ESO(MODE_FUSED, 0, false);
     }
@@ -2467,7 +2061,7 @@ hipError_t esotwist_t(int mode, int even, void* Q, void* mout, const void* F, vo
     return hipGetLastError();
 }
 
-template <typename PR, int L>
+template <typename PR>
 hipError_t simple_t(int mode, const void* src, void* dst, void* mout, const void* F, void* Nu, const uint64_t* fm,
                     const Grid& g, const CollideArgs& c, float rho0, hipStream_t s) {
     using S = typename PR::S;
@@ -2480,21 +2074,8 @@ hipError_t simple_t(int mode, const void* src, void* dst, void* mout, const void
     const T* f = static_cast<const T*>(F);
     auto* nu = static_cast<typename PR::N*>(Nu);
     const auto P = to_params<T, typename PR::D>(c);
-    if constexpr (L == LayoutIJKL && !PR::kShift && std::is_same<typename PR::T, float>::value) {
-        if (mode == MODE_FUSED && ijkl_lds()) {
-            constexpr int RI = kIjklPullI, KT = kIjklPullK;
-            const int nti = (g.xg1 + RI - 1) / RI, ntk = (g.zg1 + KT - 1) / KT;
-            const int cols = nti * ntk;
-            const int want = (kIjklBlocks + cols - 1) / cols;
-            const int jchunk = std::max(4, (g.yg1 + want - 1) / want);
-            const int nch = (g.yg1 + jchunk - 1) / jchunk;
-            hipLaunchKernelGGL((k_simple_ijkl_lds<PR, RI, KT>), dim3((uint32_t)(cols * nch)), dim3((uint32_t)(RI * KT)),
-                               0, s, a, b, f, nu, fm, g, P, nti, ntk, jchunk, rho0);
-            return hipGetLastError();
-        }
-    }
 #define TDLB_SIM(M) \
-    hipLaunchKernelGGL((k_simple<PR, L, M>), dim3(nb), dim3(bk), 0, s, a, b, mo, f, nu, fm, g, P, nkb, rho0)
+    hipLaunchKernelGGL((k_simple<PR, M>), dim3(nb), dim3(bk), 0, s, a, b, mo, f, nu, fm, g, P, nkb, rho0)
     switch (mode) {
         case MODE_COLL: TDLB_SIM(MODE_COLL); break;
         case MODE_MOM: TDLB_SIM(MODE_MOM); break;
@@ -2506,7 +2087,7 @@ hipError_t simple_t(int mode, const void* src, void* dst, void* mout, const void
     return hipGetLastError();
 }
 
-template <typename PR, int L, int STREAM>
+template <typename PR, int STREAM>
 hipError_t force_level_t(int momsrc, int even, const PointsDev& p, int64_t begin, int64_t count, void* F,
                          const void* Q, const Grid& g, double alfa, double beta, float rho0, hipStream_t s) {
     using S = typename PR::S;
@@ -2516,7 +2097,7 @@ hipError_t force_level_t(int momsrc, int even, const PointsDev& p, int64_t begin
     const S* q = static_cast<const S*>(Q);
     const T a = (T)alfa, b = (T)beta;
 #define TDLB_FL(M, E) \
-    hipLaunchKernelGGL((k_force_level<PR, L, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, p, begin, count, f, q, g, a, b, rho0)
+    hipLaunchKernelGGL((k_force_level<PR, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, p, begin, count, f, q, g, a, b, rho0)
     if (momsrc == MOMSRC_STORED) {
         if constexpr (PR::kShift) return hipErrorInvalidValue;
         else { if (even) TDLB_FL(MOMSRC_STORED, 1); else TDLB_FL(MOMSRC_STORED, 0); }
@@ -2543,43 +2124,36 @@ hipError_t force_level_t(int momsrc, int even, const PointsDev& p, int64_t begin
     } while (0)
 
 // ====================================================================== launchers
-hipError_t launch_fill_q(int prec, int layout, void* Q, const Grid& g, double rho, hipStream_t s) {
-    const uint32_t nb = grid_blocks((layout == LayoutIJKL ? g.size : g.qsize) * kQ);
-    if (prec == 0) {
-        if (layout == LayoutIJKL) hipLaunchKernelGGL((k_fill_q<float, LayoutIJKL>), dim3(nb), dim3(kBlock), 0, s, (float*)Q, g, (float)rho);
-        else hipLaunchKernelGGL((k_fill_q<float, LayoutLIJK>), dim3(nb), dim3(kBlock), 0, s, (float*)Q, g, (float)rho);
-    } else {
-        if (layout == LayoutIJKL) hipLaunchKernelGGL((k_fill_q<double, LayoutIJKL>), dim3(nb), dim3(kBlock), 0, s, (double*)Q, g, rho);
-        else hipLaunchKernelGGL((k_fill_q<double, LayoutLIJK>), dim3(nb), dim3(kBlock), 0, s, (double*)Q, g, rho);
-    }
+hipError_t launch_fill_q(int prec, void* Q, const Grid& g, double rho, hipStream_t s) {
+    const uint32_t nb = grid_blocks(g.qsize * kQ);
+    if (prec == 0) hipLaunchKernelGGL(k_fill_q<float>, dim3(nb), dim3(kBlock), 0, s, (float*)Q, g, (float)rho);
+    else hipLaunchKernelGGL(k_fill_q<double>, dim3(nb), dim3(kBlock), 0, s, (double*)Q, g, rho);
     return hipGetLastError();
 }
 
 namespace {
 template <typename W>
-hipError_t q_boundary_t(int dlayout, int blayout, bool to_boundary, const void* src, void* dst, const Grid& g,
-                        hipStream_t s) {
-    const uint32_t nb = grid_blocks(g.size * kQ);
-    const W* a = static_cast<const W*>(src);
-    W* b = static_cast<W*>(dst);
-#define TDLB_QB(DL, BL)                                                                                   \
-    do {                                                                                                  \
-        if (to_boundary) hipLaunchKernelGGL((k_q_boundary<W, DL, BL, true>), dim3(nb), dim3(kBlock), 0, s, a, b, g); \
-        else hipLaunchKernelGGL((k_q_boundary<W, DL, BL, false>), dim3(nb), dim3(kBlock), 0, s, a, b, g); \
-    } while (0)
-    if (dlayout == LayoutIJKL && blayout == LayoutIJKL) TDLB_QB(LayoutIJKL, LayoutIJKL);
-    else if (dlayout == LayoutIJKL) TDLB_QB(LayoutIJKL, LayoutLIJK);
-    else if (blayout == LayoutIJKL) TDLB_QB(LayoutLIJK, LayoutIJKL);
-    else TDLB_QB(LayoutLIJK, LayoutLIJK);
-#undef TDLB_QB
+hipError_t q_boundary_t(int blayout, bool to_boundary, void* Q, void* dense, uint64_t begin, uint64_t end,
+                        const Grid& g, hipStream_t s) {
+    const dim3 nb(grid_blocks(end - begin)), bs(kBlock);
+    W* q = static_cast<W*>(Q);
+    W* d = static_cast<W*>(dense);
+    if (blayout == LayoutIJKL) {
+        if (to_boundary) hipLaunchKernelGGL((k_q_boundary<W, LayoutIJKL, true>), nb, bs, 0, s, q, d, begin, end, g);
+        else hipLaunchKernelGGL((k_q_boundary<W, LayoutIJKL, false>), nb, bs, 0, s, q, d, begin, end, g);
+    } else {
+        if (to_boundary) hipLaunchKernelGGL((k_q_boundary<W, LayoutLIJK, true>), nb, bs, 0, s, q, d, begin, end, g);
+        else hipLaunchKernelGGL((k_q_boundary<W, LayoutLIJK, false>), nb, bs, 0, s, q, d, begin, end, g);
+    }
     return hipGetLastError();
 }
 }  // namespace
 
-hipError_t launch_q_boundary(int esize, int dlayout, int blayout, int to_boundary, const void* src, void* dst,
-                             const Grid& g, hipStream_t s) {
-    if (esize == 4) return q_boundary_t<uint32_t>(dlayout, blayout, to_boundary != 0, src, dst, g, s);
-    if (esize == 8) return q_boundary_t<uint64_t>(dlayout, blayout, to_boundary != 0, src, dst, g, s);
+hipError_t launch_q_boundary(int esize, int blayout, int to_boundary, void* Q, void* dense, uint64_t begin,
+                             uint64_t end, const Grid& g, hipStream_t s) {
+    if (begin >= end) return hipSuccess;
+    if (esize == 4) return q_boundary_t<uint32_t>(blayout, to_boundary != 0, Q, dense, begin, end, g, s);
+    if (esize == 8) return q_boundary_t<uint64_t>(blayout, to_boundary != 0, Q, dense, begin, end, g, s);
     return hipErrorInvalidValue;
 }
 
@@ -2642,48 +2216,38 @@ hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s) 
     return hipGetLastError();
 }
 
-hipError_t launch_esotwist(int prec, int layout, int mode, int even, void* Q, void* mout, const void* F, void* Nu,
+hipError_t launch_esotwist(int prec, int mode, int even, void* Q, void* mout, const void* F, void* Nu,
                            const uint64_t* fmask, const Grid& g, const CollideArgs& c, float rho0, hipStream_t s) {
     hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, e = layout == LayoutIJKL
-                                 ? esotwist_t<PR, LayoutIJKL>(mode, even, Q, mout, F, Nu, fmask, g, c, rho0, s)
-                                 : esotwist_t<PR, LayoutLIJK>(mode, even, Q, mout, F, Nu, fmask, g, c, rho0, s));
+    TDLB_WITH_PREC(prec, e = esotwist_t<PR>(mode, even, Q, mout, F, Nu, fmask, g, c, rho0, s));
     return e;
 }
 
-hipError_t launch_simple(int prec, int layout, int mode, const void* src, void* dst, void* mout, const void* F,
+hipError_t launch_simple(int prec, int mode, const void* src, void* dst, void* mout, const void* F,
                          void* Nu, const uint64_t* fmask, const Grid& g, const CollideArgs& c, float rho0,
                          hipStream_t s) {
     hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, e = layout == LayoutIJKL
-                                 ? simple_t<PR, LayoutIJKL>(mode, src, dst, mout, F, Nu, fmask, g, c, rho0, s)
-                                 : simple_t<PR, LayoutLIJK>(mode, src, dst, mout, F, Nu, fmask, g, c, rho0, s));
+    TDLB_WITH_PREC(prec, e = simple_t<PR>(mode, src, dst, mout, F, Nu, fmask, g, c, rho0, s));
     return e;
 }
 
-// launch KERNEL<W, layout> over NTHREADS grid-stride threads
-#define TDLB_MOVE(KERNEL, W, NTHREADS, ...)                                                                     \
-    do {                                                                                                        \
-        const uint32_t nb_ = grid_blocks(NTHREADS);                                                             \
-        if (layout == LayoutIJKL)                                                                               \
-            hipLaunchKernelGGL((KERNEL<W, LayoutIJKL>), dim3(nb_), dim3(kBlock), 0, s, __VA_ARGS__);            \
-        else                                                                                                    \
-            hipLaunchKernelGGL((KERNEL<W, LayoutLIJK>), dim3(nb_), dim3(kBlock), 0, s, __VA_ARGS__);            \
-    } while (0)
+// launch KERNEL<W> over NTHREADS grid-stride threads
+#define TDLB_MOVE(KERNEL, W, NTHREADS, ...) \
+    hipLaunchKernelGGL(KERNEL<W>, dim3(grid_blocks(NTHREADS)), dim3(kBlock), 0, s, __VA_ARGS__)
 
-hipError_t launch_push_all(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s) {
+hipError_t launch_push_all(int esize, const void* src, void* dst, const Grid& g, hipStream_t s) {
     if (esize == 4) TDLB_MOVE(k_push_all, uint32_t, g.size, (const uint32_t*)src, (uint32_t*)dst, g);
     else TDLB_MOVE(k_push_all, uint64_t, g.size, (const uint64_t*)src, (uint64_t*)dst, g);
     return hipGetLastError();
 }
 
-hipError_t launch_pull_all(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s) {
+hipError_t launch_pull_all(int esize, const void* src, void* dst, const Grid& g, hipStream_t s) {
     if (esize == 4) TDLB_MOVE(k_pull_all, uint32_t, g.size, (const uint32_t*)src, (uint32_t*)dst, g);
     else TDLB_MOVE(k_pull_all, uint64_t, g.size, (const uint64_t*)src, (uint64_t*)dst, g);
     return hipGetLastError();
 }
 
-hipError_t launch_bounce_back(int esize, int layout, void* Q, const Grid& g, hipStream_t s) {
+hipError_t launch_bounce_back(int esize, void* Q, const Grid& g, hipStream_t s) {
     for (int face = 0; face < 6; face++) {
         const int axis = face >> 1;
         const uint64_t n = (uint64_t)(axis == 0 ? g.yg1 : g.xg1) * (axis == 2 ? g.yg1 : g.zg1);
@@ -2698,7 +2262,7 @@ hipError_t launch_bounce_back(int esize, int layout, void* Q, const Grid& g, hip
     return hipGetLastError();
 }
 
-hipError_t launch_ghost_fill(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s) {
+hipError_t launch_ghost_fill(int esize, const void* src, void* dst, const Grid& g, hipStream_t s) {
     if (esize == 4)
         TDLB_MOVE(k_ghost_fill, RawBits<uint32_t>, ghost_count(g), (const uint32_t*)src, (uint32_t*)dst, g, 0.0f);
     else
@@ -2706,7 +2270,7 @@ hipError_t launch_ghost_fill(int esize, int layout, const void* src, void* dst, 
     return hipGetLastError();
 }
 
-hipError_t launch_ghost_fill_decode(int prec, int layout, const void* src, void* dst, const Grid& g, float rho0,
+hipError_t launch_ghost_fill_decode(int prec, const void* src, void* dst, const Grid& g, float rho0,
                                     hipStream_t s) {
     if (prec == 2)
         TDLB_MOVE(k_ghost_fill, PrecF16, ghost_count(g), (const PrecF16::S*)src, (float*)dst, g, rho0);
@@ -2719,7 +2283,7 @@ hipError_t launch_ghost_fill_decode(int prec, int layout, const void* src, void*
     return hipGetLastError();
 }
 
-hipError_t launch_ghost_copy(int esize, int layout, const void* src, void* dst, const Grid& g, hipStream_t s) {
+hipError_t launch_ghost_copy(int esize, const void* src, void* dst, const Grid& g, hipStream_t s) {
     if (esize == 4) TDLB_MOVE(k_ghost_copy, uint32_t, ghost_count(g), (const uint32_t*)src, (uint32_t*)dst, g);
     else TDLB_MOVE(k_ghost_copy, uint64_t, ghost_count(g), (const uint64_t*)src, (uint64_t*)dst, g);
     return hipGetLastError();
@@ -2754,26 +2318,19 @@ hipError_t launch_force_prepare(int prec, const PointsDev& p, int64_t begin, int
     return hipGetLastError();
 }
 
-hipError_t launch_force_level(int prec, int layout, int streaming, int momsrc, int even, const PointsDev& p,
+hipError_t launch_force_level(int prec, int streaming, int momsrc, int even, const PointsDev& p,
                               int64_t begin, int64_t count, void* F, const void* Q, const Grid& g, double alfa,
                               double beta, float rho0, hipStream_t s) {
     if (count <= 0) return hipSuccess;
     hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, {
-        if (layout == LayoutIJKL)
-            e = streaming == StreamEsotwist
-                    ? force_level_t<PR, LayoutIJKL, StreamEsotwist>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s)
-                    : force_level_t<PR, LayoutIJKL, StreamSimple>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s);
-        else
-            e = streaming == StreamEsotwist
-                    ? force_level_t<PR, LayoutLIJK, StreamEsotwist>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s)
-                    : force_level_t<PR, LayoutLIJK, StreamSimple>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s);
-    });
+    TDLB_WITH_PREC(prec, e = streaming == StreamEsotwist
+                                 ? force_level_t<PR, StreamEsotwist>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s)
+                                 : force_level_t<PR, StreamSimple>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s));
     return e;
 }
 
 namespace {
-template <typename PR, int L, int STREAM>
+template <typename PR, int STREAM>
 hipError_t ib_moments_t(int momsrc, int even, const uint32_t* cells, const PointsDev* p, int64_t begin, int64_t n,
                         void* cache, const void* Q, const Grid& g, float rho0, hipStream_t s) {
     using T = typename PR::T;
@@ -2784,8 +2341,8 @@ hipError_t ib_moments_t(int momsrc, int even, const uint32_t* cells, const Point
     const uint32_t nb = (uint32_t)((threads + kBlock - 1) / kBlock);
 #define TDLB_IBM(M, E)                                                                                          \
     do {                                                                                                        \
-        if (cells) hipLaunchKernelGGL((k_ib_moments_cells<PR, L, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, cells, n, c, q, g, rho0); \
-        else hipLaunchKernelGGL((k_ib_moments_points<PR, L, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, *p, begin, n, c, q, g, rho0); \
+        if (cells) hipLaunchKernelGGL((k_ib_moments_cells<PR, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, cells, n, c, q, g, rho0); \
+        else hipLaunchKernelGGL((k_ib_moments_points<PR, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, *p, begin, n, c, q, g, rho0); \
     } while (0)
     if (momsrc == MOMSRC_STORED) {
         if constexpr (PR::kShift) return hipErrorInvalidValue;
@@ -2798,34 +2355,30 @@ hipError_t ib_moments_t(int momsrc, int even, const uint32_t* cells, const Point
 }
 
 template <typename PR>
-hipError_t ib_moments_prec(int layout, int streaming, int momsrc, int even, const uint32_t* cells, const PointsDev* p,
+hipError_t ib_moments_prec(int streaming, int momsrc, int even, const uint32_t* cells, const PointsDev* p,
                            int64_t begin, int64_t n, void* cache, const void* Q, const Grid& g, float rho0,
                            hipStream_t s) {
-    if (layout == LayoutIJKL)
-        return streaming == StreamEsotwist
-                   ? ib_moments_t<PR, LayoutIJKL, StreamEsotwist>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s)
-                   : ib_moments_t<PR, LayoutIJKL, StreamSimple>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s);
     return streaming == StreamEsotwist
-               ? ib_moments_t<PR, LayoutLIJK, StreamEsotwist>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s)
-               : ib_moments_t<PR, LayoutLIJK, StreamSimple>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s);
+               ? ib_moments_t<PR, StreamEsotwist>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s)
+               : ib_moments_t<PR, StreamSimple>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s);
 }
 }  // namespace
 
-hipError_t launch_ib_moments_cells(int prec, int layout, int streaming, int momsrc, int even, const uint32_t* cells,
+hipError_t launch_ib_moments_cells(int prec, int streaming, int momsrc, int even, const uint32_t* cells,
                                    int64_t n, void* cache, const void* Q, const Grid& g, float rho0, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, e = ib_moments_prec<PR>(layout, streaming, momsrc, even, cells, nullptr, 0, n, cache, Q, g,
+    TDLB_WITH_PREC(prec, e = ib_moments_prec<PR>(streaming, momsrc, even, cells, nullptr, 0, n, cache, Q, g,
                                                  rho0, s));
     return e;
 }
 
-hipError_t launch_ib_moments_points(int prec, int layout, int streaming, int momsrc, int even, const PointsDev& p,
+hipError_t launch_ib_moments_points(int prec, int streaming, int momsrc, int even, const PointsDev& p,
                                     int64_t begin, int64_t count, void* cache, const void* Q, const Grid& g,
                                     float rho0, hipStream_t s) {
     if (count <= 0) return hipSuccess;
     hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, e = ib_moments_prec<PR>(layout, streaming, momsrc, even, nullptr, &p, begin, count, cache, Q,
+    TDLB_WITH_PREC(prec, e = ib_moments_prec<PR>(streaming, momsrc, even, nullptr, &p, begin, count, cache, Q,
                                                  g, rho0, s));
     return e;
 }
@@ -2851,37 +2404,34 @@ hipError_t launch_force_level_cached(int prec, const PointsDev& p, int64_t begin
 }
 
 namespace {
-// fn(L, STREAM, MOMSRC, EVEN) with compile-time values (std::integral_constant)
+// fn(STREAM, MOMSRC, EVEN) with compile-time values (std::integral_constant)
 template <int V>
 using IC = std::integral_constant<int, V>;
 
-template <typename PR, int L, int STREAM, typename Fn>
+template <typename PR, int STREAM, typename Fn>
 hipError_t with_source(int momsrc, int even, Fn&& fn) {
     if (momsrc == MOMSRC_STORED) {
         if constexpr (PR::kShift) return hipErrorInvalidValue;
-        else return even ? fn(IC<L>{}, IC<STREAM>{}, IC<MOMSRC_STORED>{}, IC<1>{})
-                         : fn(IC<L>{}, IC<STREAM>{}, IC<MOMSRC_STORED>{}, IC<0>{});
+        else return even ? fn(IC<STREAM>{}, IC<MOMSRC_STORED>{}, IC<1>{})
+                         : fn(IC<STREAM>{}, IC<MOMSRC_STORED>{}, IC<0>{});
     }
     if (momsrc == MOMSRC_ESO_POPS) {
         if constexpr (STREAM != StreamEsotwist) return hipErrorInvalidValue;
-        else return even ? fn(IC<L>{}, IC<STREAM>{}, IC<MOMSRC_ESO_POPS>{}, IC<1>{})
-                         : fn(IC<L>{}, IC<STREAM>{}, IC<MOMSRC_ESO_POPS>{}, IC<0>{});
+        else return even ? fn(IC<STREAM>{}, IC<MOMSRC_ESO_POPS>{}, IC<1>{})
+                         : fn(IC<STREAM>{}, IC<MOMSRC_ESO_POPS>{}, IC<0>{});
     }
     if constexpr (STREAM != StreamSimple) return hipErrorInvalidValue;
-    else return fn(IC<L>{}, IC<STREAM>{}, IC<MOMSRC_PULL_POPS>{}, IC<1>{});
+    else return fn(IC<STREAM>{}, IC<MOMSRC_PULL_POPS>{}, IC<1>{});
 }
 
 template <typename PR, typename Fn>
-hipError_t with_cell_source(int layout, int streaming, int momsrc, int even, Fn&& fn) {
-    if (layout == LayoutIJKL)
-        return streaming == StreamEsotwist ? with_source<PR, LayoutIJKL, StreamEsotwist>(momsrc, even, fn)
-                                           : with_source<PR, LayoutIJKL, StreamSimple>(momsrc, even, fn);
-    return streaming == StreamEsotwist ? with_source<PR, LayoutLIJK, StreamEsotwist>(momsrc, even, fn)
-                                       : with_source<PR, LayoutLIJK, StreamSimple>(momsrc, even, fn);
+hipError_t with_cell_source(int streaming, int momsrc, int even, Fn&& fn) {
+    return streaming == StreamEsotwist ? with_source<PR, StreamEsotwist>(momsrc, even, fn)
+                                       : with_source<PR, StreamSimple>(momsrc, even, fn);
 }
 }  // namespace
 
-hipError_t launch_force_gather(int prec, int layout, int streaming, int momsrc, int even, const ForceGeom& fg,
+hipError_t launch_force_gather(int prec, int streaming, int momsrc, int even, const ForceGeom& fg,
                                const BladeStep& st, const GatherBlocks& gb, const void* Q, void* F,
                                const uint64_t* prev, uint64_t* next, const uint64_t* static_base, const Grid& g,
                                float rho0, hipStream_t s) {
@@ -2891,8 +2441,8 @@ hipError_t launch_force_gather(int prec, int layout, int streaming, int momsrc, 
     TDLB_WITH_PREC(prec, {
         using S = typename PR::S;
         using T = typename PR::T;
-        e = with_cell_source<PR>(layout, streaming, momsrc, even, [&](auto Lc, auto Sc, auto Mc, auto Ec) {
-            hipLaunchKernelGGL((k_force_gather<PR, decltype(Lc)::value, decltype(Sc)::value, decltype(Mc)::value,
+        e = with_cell_source<PR>(streaming, momsrc, even, [&](auto Sc, auto Mc, auto Ec) {
+            hipLaunchKernelGGL((k_force_gather<PR, decltype(Sc)::value, decltype(Mc)::value,
                                                decltype(Ec)::value>),
                                dim3(nb), dim3(kGatherBlock), 0, s, fg, st, gb, (const S*)Q, (T*)F, prev, next,
                                static_base, g, rho0);
@@ -2992,15 +2542,15 @@ int pipe_xcc_check(hipStream_t s) {
     return 1;
 }
 
-hipError_t launch_reduce(int prec, int layout, int streaming, int momsrc, int even, const void* Q, const void* F,
+hipError_t launch_reduce(int prec, int streaming, int momsrc, int even, const void* Q, const void* F,
                          const uint64_t* fmask, const Grid& g, const ReduceArgs& ra, float rho0, double* partial,
                          double* out, hipStream_t s) {
     hipError_t e = hipErrorInvalidValue;
     TDLB_WITH_PREC(prec, {
         using S = typename PR::S;
         using T = typename PR::T;
-        e = with_cell_source<PR>(layout, streaming, momsrc, even, [&](auto Lc, auto Sc, auto Mc, auto Ec) {
-            hipLaunchKernelGGL((k_reduce_cells<PR, decltype(Lc)::value, decltype(Sc)::value, decltype(Mc)::value,
+        e = with_cell_source<PR>(streaming, momsrc, even, [&](auto Sc, auto Mc, auto Ec) {
+            hipLaunchKernelGGL((k_reduce_cells<PR, decltype(Sc)::value, decltype(Mc)::value,
                                                decltype(Ec)::value>),
                                dim3(kReduceBlocks), dim3(kBlock), 0, s, (const S*)Q, (const T*)F, fmask, g, ra, rho0,
                                partial);
@@ -3012,7 +2562,7 @@ hipError_t launch_reduce(int prec, int layout, int streaming, int momsrc, int ev
     return hipGetLastError();
 }
 
-hipError_t launch_macroscopic(int prec, int layout, int streaming, int momsrc, int even, const void* Q,
+hipError_t launch_macroscopic(int prec, int streaming, int momsrc, int even, const void* Q,
                               const void* F, const uint64_t* fmask, const Grid& g, float rho0, void* out,
                               hipStream_t s) {
     const uint32_t nb = grid_blocks((uint64_t)g.xg1 * g.yg1 * g.zg1);
@@ -3020,8 +2570,8 @@ hipError_t launch_macroscopic(int prec, int layout, int streaming, int momsrc, i
     TDLB_WITH_PREC(prec, {
         using S = typename PR::S;
         using T = typename PR::T;
-        e = with_cell_source<PR>(layout, streaming, momsrc, even, [&](auto Lc, auto Sc, auto Mc, auto Ec) {
-            hipLaunchKernelGGL((k_macroscopic<PR, decltype(Lc)::value, decltype(Sc)::value, decltype(Mc)::value,
+        e = with_cell_source<PR>(streaming, momsrc, even, [&](auto Sc, auto Mc, auto Ec) {
+            hipLaunchKernelGGL((k_macroscopic<PR, decltype(Sc)::value, decltype(Mc)::value,
                                               decltype(Ec)::value>),
                                dim3(nb), dim3(kBlock), 0, s, (const S*)Q, (const T*)F, fmask, g, rho0, (T*)out);
             return hipGetLastError();
@@ -3030,19 +2580,13 @@ hipError_t launch_macroscopic(int prec, int layout, int streaming, int momsrc, i
     return e;
 }
 
-hipError_t launch_regrid(int esize, int layout, const void* oldQ, void* newQ, int nu_esize, const void* oldNu,
+hipError_t launch_regrid(int esize, const void* oldQ, void* newQ, int nu_esize, const void* oldNu,
                          void* newNu, const Grid& og, const Grid& ng, hipStream_t s) {
     const uint32_t nb = grid_blocks(ng.size);
     if (esize == 4) {
-        if (layout == LayoutIJKL)
-            hipLaunchKernelGGL((k_regrid_q<uint32_t, LayoutIJKL>), dim3(nb), dim3(kBlock), 0, s, (const uint32_t*)oldQ, (uint32_t*)newQ, og, ng);
-        else
-            hipLaunchKernelGGL((k_regrid_q<uint32_t, LayoutLIJK>), dim3(nb), dim3(kBlock), 0, s, (const uint32_t*)oldQ, (uint32_t*)newQ, og, ng);
+        hipLaunchKernelGGL((k_regrid_q<uint32_t>), dim3(nb), dim3(kBlock), 0, s, (const uint32_t*)oldQ, (uint32_t*)newQ, og, ng);
     } else if (esize == 8) {
-        if (layout == LayoutIJKL)
-            hipLaunchKernelGGL((k_regrid_q<uint64_t, LayoutIJKL>), dim3(nb), dim3(kBlock), 0, s, (const uint64_t*)oldQ, (uint64_t*)newQ, og, ng);
-        else
-            hipLaunchKernelGGL((k_regrid_q<uint64_t, LayoutLIJK>), dim3(nb), dim3(kBlock), 0, s, (const uint64_t*)oldQ, (uint64_t*)newQ, og, ng);
+        hipLaunchKernelGGL((k_regrid_q<uint64_t>), dim3(nb), dim3(kBlock), 0, s, (const uint64_t*)oldQ, (uint64_t*)newQ, og, ng);
     } else {
         return hipErrorInvalidValue;
     }
@@ -3085,25 +2629,23 @@ hipError_t launch_nu_convert(int prec, int to_float, const void* src, void* dst,
     return hipGetLastError();
 }
 
-hipError_t launch_plane_xz(int prec, int layout, const void* Q, const void* F, const uint64_t* fmask,
+hipError_t launch_plane_xz(int prec, const void* Q, const void* F, const uint64_t* fmask,
                            const uint8_t* exclude, const Grid& g, int cut, int64_t i0, int64_t k0, PlaneRec4* q,
                            PlaneRec3* f, uint8_t* flags, hipStream_t s) {
     const uint32_t nb = (uint32_t)(((int64_t)g.xg1 * g.zg1 + kBlock - 1) / kBlock);
-#define TDLB_PLANE(T, L)                                                                                       \
-    hipLaunchKernelGGL((k_plane_xz<T, L>), dim3(nb), dim3(kBlock), 0, s, (const T*)Q, (const T*)F, fmask, exclude, \
+#define TDLB_PLANE(T)                                                                                          \
+    hipLaunchKernelGGL((k_plane_xz<T>), dim3(nb), dim3(kBlock), 0, s, (const T*)Q, (const T*)F, fmask, exclude, \
                        g, cut, i0, k0, q, f, flags)
     if (prec == 1) {
-        if (layout == LayoutIJKL) TDLB_PLANE(double, LayoutIJKL);
-        else TDLB_PLANE(double, LayoutLIJK);
+        TDLB_PLANE(double);
     } else {
-        if (layout == LayoutIJKL) TDLB_PLANE(float, LayoutIJKL);
-        else TDLB_PLANE(float, LayoutLIJK);
+        TDLB_PLANE(float);
     }
 #undef TDLB_PLANE
     return hipGetLastError();
 }
 
-hipError_t launch_vorticity(int prec, int layout, int streaming, int momsrc, int even, const void* Q, const Grid& g,
+hipError_t launch_vorticity(int prec, int streaming, int momsrc, int even, const void* Q, const Grid& g,
                             int axis, int cut, const uint8_t* exclude, void* out, float rho0, hipStream_t s) {
     const int64_t cells = (int64_t)g.xg1 * (axis == 0 ? g.zg1 : g.yg1);
     const uint32_t nb = (uint32_t)((cells + kBlock - 1) / kBlock);
@@ -3111,8 +2653,8 @@ hipError_t launch_vorticity(int prec, int layout, int streaming, int momsrc, int
     TDLB_WITH_PREC(prec, {
         using S = typename PR::S;
         using T = typename PR::T;
-        e = with_cell_source<PR>(layout, streaming, momsrc, even, [&](auto Lc, auto Sc, auto Mc, auto Ec) {
-            hipLaunchKernelGGL((k_vorticity<PR, decltype(Lc)::value, decltype(Sc)::value, decltype(Mc)::value,
+        e = with_cell_source<PR>(streaming, momsrc, even, [&](auto Sc, auto Mc, auto Ec) {
+            hipLaunchKernelGGL((k_vorticity<PR, decltype(Sc)::value, decltype(Mc)::value,
                                             decltype(Ec)::value>),
                                dim3(nb), dim3(kBlock), 0, s, (const S*)Q, g, axis, cut, exclude, (T*)out, rho0);
             return hipGetLastError();
@@ -3186,13 +2728,13 @@ __device__ __forceinline__ bool batch_cell(const Grid& g, int tile, uint32_t b, 
     return j >= 1 && j <= g.yg1 && k >= 1 && k <= g.zg1;
 }
 
-template <typename PR, int L, int STREAM>
+template <typename PR, int STREAM>
 __global__ __launch_bounds__(kRowBlock) void k_batch_fused(const MemberDev* __restrict__ mem,
                                                         const int64_t* __restrict__ off, int n,
                                                         const int32_t* __restrict__ bm) {
     static_assert(std::is_same<typename PR::T, float>::value, "batches compute in float");
     using S = typename PR::S;
-    const uint32_t blk = layout_block<L>();
+    const uint32_t blk = blockIdx.x;
     // one load from the block table instead of a binary search of dependent loads
     const int m = bm ? bm[blk] : find_slot(off, n, blk);
     const MemberDev& md = mem[m];
@@ -3203,17 +2745,17 @@ __global__ __launch_bounds__(kRowBlock) void k_batch_fused(const MemberDev* __re
     if constexpr (STREAM == StreamEsotwist) {
         S* Q = static_cast<S*>(md.Q[0]);
         auto* nu = static_cast<typename PR::N*>(md.Nu);
-        if (md.even) esotwist_cell<PR, L, MODE_FUSED, 1>(Q, nullptr, md.F, nu, fm, md.g, md.P, md.rho0, i, j, k);
-        else esotwist_cell<PR, L, MODE_FUSED, 0>(Q, nullptr, md.F, nu, fm, md.g, md.P, md.rho0, i, j, k);
+        if (md.even) esotwist_cell<PR, MODE_FUSED, 1>(Q, nullptr, md.F, nu, fm, md.g, md.P, md.rho0, i, j, k);
+        else esotwist_cell<PR, MODE_FUSED, 0>(Q, nullptr, md.F, nu, fm, md.g, md.P, md.rho0, i, j, k);
     } else {
-        simple_cell<PR, L, MODE_FUSED>(static_cast<const S*>(md.Q[md.cur]), static_cast<S*>(md.Q[1 - md.cur]),
+        simple_cell<PR, MODE_FUSED>(static_cast<const S*>(md.Q[md.cur]), static_cast<S*>(md.Q[1 - md.cur]),
                                        nullptr, md.F, static_cast<typename PR::N*>(md.Nu), fm, md.g, md.P,
                                        md.rho0, i, j, k);
     }
 }
 
 // the gather of every member (force_gather) from the populations the fused kernel just wrote
-template <typename PR, int L, int STREAM>
+template <typename PR, int STREAM>
 __global__ __launch_bounds__(kGatherBlock) void k_batch_gather(const MemberDev* __restrict__ mem,
                                                                const int64_t* __restrict__ off,
                                                                const int32_t* __restrict__ bm) {
@@ -3228,14 +2770,14 @@ __global__ __launch_bounds__(kGatherBlock) void k_batch_gather(const MemberDev* 
     if constexpr (STREAM == StreamEsotwist) {
         const S* Q = static_cast<const S*>(md.Q[0]);
         if (md.even)
-            force_gather<PR, L, STREAM, MOMSRC_ESO_POPS, 0>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base,
+            force_gather<PR, STREAM, MOMSRC_ESO_POPS, 0>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base,
                                                             md.g, md.rho0);
         else
-            force_gather<PR, L, STREAM, MOMSRC_ESO_POPS, 1>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base,
+            force_gather<PR, STREAM, MOMSRC_ESO_POPS, 1>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base,
                                                             md.g, md.rho0);
     } else {
         const S* Q = static_cast<const S*>(md.Q[1 - md.cur]);
-        force_gather<PR, L, STREAM, MOMSRC_PULL_POPS, 1>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base, md.g,
+        force_gather<PR, STREAM, MOMSRC_PULL_POPS, 1>(md.fg, st, b, md.gb, Q, md.F, prev, next, md.static_base, md.g,
                                                          md.rho0);
     }
 }
@@ -3268,22 +2810,22 @@ __global__ void k_batch_advance(MemberDev* __restrict__ mem, int n) {
 
 inline uint32_t nblk(int64_t n, int bs) { return (uint32_t)((n + bs - 1) / bs); }
 
-template <typename PR, int L, int STREAM>
+template <typename PR, int STREAM>
 hipError_t batch_fused_t(const BatchPlan& p, hipStream_t s) {
     if (p.tot_coll <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_batch_fused<PR, L, STREAM>), dim3((uint32_t)p.tot_coll), dim3(p.bs), 0, s, p.mem,
+    hipLaunchKernelGGL((k_batch_fused<PR, STREAM>), dim3((uint32_t)p.tot_coll), dim3(p.bs), 0, s, p.mem,
                        p.off_coll, p.n_members, p.coll_member);
     return hipGetLastError();
 }
 
-template <typename PR, int L, int STREAM>
+template <typename PR, int STREAM>
 hipError_t batch_step_t(const BatchPlan& p, hipStream_t s) {
     const int n = p.n_members;
     if (p.bs != 256 && p.bs != 512) return hipErrorInvalidValue;
-    hipError_t e = batch_fused_t<PR, L, STREAM>(p, s);
+    hipError_t e = batch_fused_t<PR, STREAM>(p, s);
     if (e != hipSuccess) return e;
     if (p.tot_gather > 0)
-        hipLaunchKernelGGL((k_batch_gather<PR, L, STREAM>), dim3((uint32_t)p.tot_gather), dim3(kGatherBlock), 0, s, p.mem,
+        hipLaunchKernelGGL((k_batch_gather<PR, STREAM>), dim3((uint32_t)p.tot_gather), dim3(kGatherBlock), 0, s, p.mem,
                            p.off_gather, p.gather_member);
     if (p.n_tasks > 0)
         hipLaunchKernelGGL(k_batch_levels, dim3((uint32_t)p.n_tasks), dim3(p.force_bs), (uint32_t)p.force_lds_bytes, s,
@@ -3293,20 +2835,16 @@ hipError_t batch_step_t(const BatchPlan& p, hipStream_t s) {
 }
 
 template <typename Fn>
-hipError_t with_batch_prec(int prec, int layout, int streaming, Fn&& fn) {
-    auto by_layout = [&](auto pr) -> hipError_t {
+hipError_t with_batch_prec(int prec, int streaming, Fn&& fn) {
+    auto by_stream = [&](auto pr) -> hipError_t {
         using PR = decltype(pr);
-        if (layout == LayoutIJKL)
-            return streaming == StreamEsotwist ? fn(PR{}, IC<LayoutIJKL>{}, IC<StreamEsotwist>{})
-                                               : fn(PR{}, IC<LayoutIJKL>{}, IC<StreamSimple>{});
-        return streaming == StreamEsotwist ? fn(PR{}, IC<LayoutLIJK>{}, IC<StreamEsotwist>{})
-                                           : fn(PR{}, IC<LayoutLIJK>{}, IC<StreamSimple>{});
+        return streaming == StreamEsotwist ? fn(PR{}, IC<StreamEsotwist>{}) : fn(PR{}, IC<StreamSimple>{});
     };
     switch (prec) {
-        case 0: return by_layout(PrecF32{});
-        case 2: return by_layout(PrecF16{});
-        case 3: return by_layout(PrecBF16{});
-        case 4: return by_layout(PrecE3M12{});
+        case 0: return by_stream(PrecF32{});
+        case 2: return by_stream(PrecF16{});
+        case 3: return by_stream(PrecBF16{});
+        case 4: return by_stream(PrecE3M12{});
         default: return hipErrorInvalidValue;
     }
 }
@@ -3323,18 +2861,18 @@ int64_t batch_coll_blocks(const Grid& g, int tile, int bs) {
     return (int64_t)g.xg1 * ((plane + bs - 1) / bs);
 }
 
-hipError_t launch_batch_step(int prec, int layout, int streaming, const BatchPlan& plan, int steps, hipStream_t s) {
-    return with_batch_prec(prec, layout, streaming, [&](auto pr, auto lc, auto sc) {
+hipError_t launch_batch_step(int prec, int streaming, const BatchPlan& plan, int steps, hipStream_t s) {
+    return with_batch_prec(prec, streaming, [&](auto pr, auto sc) {
         hipError_t e = hipSuccess;
         for (int k = 0; k < steps && e == hipSuccess; k++)
-            e = batch_step_t<decltype(pr), decltype(lc)::value, decltype(sc)::value>(plan, s);
+            e = batch_step_t<decltype(pr), decltype(sc)::value>(plan, s);
         return e;
     });
 }
 
-hipError_t launch_batch_fused(int prec, int layout, int streaming, const BatchPlan& plan, hipStream_t s) {
-    return with_batch_prec(prec, layout, streaming, [&](auto pr, auto lc, auto sc) {
-        return batch_fused_t<decltype(pr), decltype(lc)::value, decltype(sc)::value>(plan, s);
+hipError_t launch_batch_fused(int prec, int streaming, const BatchPlan& plan, hipStream_t s) {
+    return with_batch_prec(prec, streaming, [&](auto pr, auto sc) {
+        return batch_fused_t<decltype(pr), decltype(sc)::value>(plan, s);
     });
 }
 
