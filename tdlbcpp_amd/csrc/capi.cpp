@@ -39,6 +39,7 @@
 #include "../../include/tdlb.h"
 #include "handle.h"
 #include "kernels.h"
+#include "readback.h"
 #include "rushton.h"
 
 namespace tdlb {
@@ -830,6 +831,7 @@ int tdlb_cu_create(const tdlb_cu_params* p, const tdlb_flow* f, tdlb_cu_t* out) 
         return fail(TDLB_ERR_UNSUPPORTED, "grid too large: at most 2^31 cells including ghosts");
 
     tdlb_cu* cu = new tdlb_cu();
+    readback_handle(1);
     cu->prm = *p;
     cu->flow = *f;
     cu->xg = xg; cu->yg = yg; cu->zg = zg;
@@ -842,6 +844,7 @@ int tdlb_cu_create(const tdlb_cu_params* p, const tdlb_flow* f, tdlb_cu_t* out) 
     cu->ssize = p->precision == TDLB_PREC_F64 ? 8 : p->precision == TDLB_PREC_F32 ? 4 : 2;
     set_q_geometry(cu->g, cu->ssize);
     if (cu->q_cells() >= (1ull << 32)) {
+        readback_handle(-1);
         delete cu;
         return fail(TDLB_ERR_UNSUPPORTED, "grid too large for 32-bit cell indexing");
     }
@@ -853,6 +856,7 @@ int tdlb_cu_create(const tdlb_cu_params* p, const tdlb_flow* f, tdlb_cu_t* out) 
 
     auto bad = [&](int code, const std::string& m) {
         release(cu);
+        readback_handle(-1);
         delete cu;
         return fail(code, m);
     };
@@ -894,6 +898,7 @@ int tdlb_cu_destroy(tdlb_cu_t cu) {
     (void)hipSetDevice(cu->device);
     if (cu->stream) (void)hipStreamSynchronize(cu->stream);
     release(cu);
+    readback_handle(-1);
     delete cu;
     return TDLB_OK;
 }
@@ -1052,26 +1057,30 @@ int tdlb_cu_field_bytes(tdlb_cu_t cu, int field, size_t* bytes) {
     return TDLB_OK;
 }
 
-// The explicit Q to `out` or from `in` (one of them null), converted between the
-// kernels' array and the boundary's in pieces, so that a lattice of more than half
-// the memory still moves.
-static int move_q(tdlb_cu* cu, void* out, const void* in, size_t bytes) {
-    constexpr size_t kPiece = (size_t)1 << 29;
-    const size_t piece = std::min(bytes, kPiece);
+// A result to host memory, formed piece by piece (readback.h).
+static int read_result(tdlb_cu* cu, void* host, size_t bytes, size_t align, const char* what, const PieceFn& piece) {
+    const hipError_t e = read_back(cu->device, cu->stream, host, bytes, align, piece);
+    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
+    return TDLB_OK;
+}
+
+// The explicit Q from host memory, converted to the kernels' array in pieces, so
+// that a lattice of more than half the memory still moves.
+static int upload_q(tdlb_cu* cu, const void* host, size_t bytes) {
+    const size_t piece = std::min(bytes, (size_t)1 << 29);
     void* tmp = nullptr;
-    if (hipMalloc(&tmp, piece) != hipSuccess) return fail(TDLB_ERR_NOMEM, "Q staging");
+    if (hipMalloc(&tmp, piece) != hipSuccess) return fail(TDLB_ERR_NOMEM, "upload Q staging");
     hipError_t e = hipSuccess;
     for (size_t at = 0; at < bytes && e == hipSuccess; at += piece) {
         const size_t n = std::min(piece, bytes - at);
-        if (in) e = hipMemcpyAsync(tmp, (const char*)in + at, n, hipMemcpyHostToDevice, cu->stream);
+        e = hipMemcpyAsync(tmp, (const char*)host + at, n, hipMemcpyHostToDevice, cu->stream);
         if (e == hipSuccess)
-            e = launch_q_boundary((int)cu->tsize, cu->blay(), out ? 1 : 0, cu->eq(), tmp, at / cu->tsize,
-                                  (at + n) / cu->tsize, cu->g, cu->stream);
-        if (e == hipSuccess && out) e = hipMemcpyAsync((char*)out + at, tmp, n, hipMemcpyDeviceToHost, cu->stream);
+            e = launch_q_boundary((int)cu->tsize, cu->blay(), 0, cu->eq(), tmp, at / cu->tsize, (at + n) / cu->tsize,
+                                  cu->g, cu->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
     }
     (void)hipFree(tmp);
-    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string(out ? "download" : "upload") + " Q: " + hipGetErrorString(e));
+    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("upload Q: ") + hipGetErrorString(e));
     return TDLB_OK;
 }
 
@@ -1081,31 +1090,23 @@ int tdlb_cu_download(tdlb_cu_t cu, int field, void* host, size_t bytes) {
     if (!host || bytes != need) return fail(TDLB_ERR_INVALID, "download: buffer size must be " + std::to_string(need));
     CHK(set_device(cu));
     CHK(materialise(cu));
-    if (field == TDLB_FIELD_F) {
-        void* tmp = nullptr;
-        if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "download F staging");
-        hipError_t e = launch_masked_f(cu->prec(), cu->F, cu->fmask[cu->fm], tmp, cu->g, cu->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(host, tmp, need, hipMemcpyDeviceToHost, cu->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
-        (void)hipFree(tmp);
-        if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("download F: ") + hipGetErrorString(e));
-        return TDLB_OK;
-    }
-    if (field == TDLB_FIELD_Q) return move_q(cu, host, nullptr, need);
-    if (field == TDLB_FIELD_NU && cu->shifted()) {
-        void* tmp = nullptr;
-        if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "download Nu staging");
-        hipError_t e = launch_nu_convert(cu->prec(), 1, cu->Nu, tmp, cu->g.size, cu->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(host, tmp, need, hipMemcpyDeviceToHost, cu->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
-        (void)hipFree(tmp);
-        if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("download Nu: ") + hipGetErrorString(e));
-        return TDLB_OK;
-    }
-    const void* src = field == TDLB_FIELD_NU ? cu->Nu : (const void*)cu->O;
-    HIPCHK(hipMemcpyAsync(host, src, need, hipMemcpyDeviceToHost, cu->stream));
-    HIPCHK(hipStreamSynchronize(cu->stream));
-    return TDLB_OK;
+    const size_t ts = cu->tsize;
+    if (field == TDLB_FIELD_F)
+        return read_result(cu, host, need, 3 * ts, "download F", [&](void* dst, size_t a, size_t b, hipStream_t s) {
+            return launch_masked_f(cu->prec(), cu->F, cu->fmask[cu->fm], a / (3 * ts), b / (3 * ts), dst, cu->g, s);
+        });
+    if (field == TDLB_FIELD_Q)
+        return read_result(cu, host, need, ts, "download Q", [&](void* dst, size_t a, size_t b, hipStream_t s) {
+            return launch_q_boundary((int)ts, cu->blay(), 1, cu->eq(), dst, a / ts, b / ts, cu->g, s);
+        });
+    if (field == TDLB_FIELD_NU && cu->shifted())
+        return read_result(cu, host, need, ts, "download Nu", [&](void* dst, size_t a, size_t b, hipStream_t s) {
+            return launch_nu_convert(cu->prec(), 1, (const char*)cu->Nu + a / ts * cu->ssize, dst, (b - a) / ts, s);
+        });
+    const char* src = static_cast<const char*>(field == TDLB_FIELD_NU ? cu->Nu : (const void*)cu->O);
+    return read_result(cu, host, need, 16, "download", [&](void* dst, size_t a, size_t b, hipStream_t s) {
+        return hipMemcpyAsync(dst, src + a, b - a, hipMemcpyDeviceToHost, s);
+    });
 }
 
 int tdlb_cu_upload(tdlb_cu_t cu, int field, const void* host, size_t bytes) {
@@ -1115,7 +1116,7 @@ int tdlb_cu_upload(tdlb_cu_t cu, int field, const void* host, size_t bytes) {
     CHK(set_device(cu));
     CHK(materialise(cu));
     void* dst = field == TDLB_FIELD_F ? cu->F : field == TDLB_FIELD_NU ? cu->Nu : (void*)cu->O;
-    if (field == TDLB_FIELD_Q) return move_q(cu, nullptr, host, need);
+    if (field == TDLB_FIELD_Q) return upload_q(cu, host, need);
     if (field == TDLB_FIELD_NU && cu->shifted()) {
         void* tmp = nullptr;
         if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "upload Nu staging");
@@ -1562,16 +1563,12 @@ int tdlb_cu_macroscopic(tdlb_cu_t cu, void* out, size_t bytes) {
     const size_t need = (size_t)cu->g.xg1 * cu->g.yg1 * cu->g.zg1 * 4 * cu->tsize;
     if (bytes != need) return fail(TDLB_ERR_INVALID, "macroscopic: buffer size must be " + std::to_string(need));
     CHK(set_device(cu));
-    void* tmp = nullptr;
-    if (hipMalloc(&tmp, need) != hipSuccess) return fail(TDLB_ERR_NOMEM, "macroscopic staging");
     const CellSource cs = cell_source(cu);
-    hipError_t e = launch_macroscopic(cs.prec, cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F,
-                                      cu->fmask[cu->fm], cu->g, cu->rho0, tmp, cu->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, need, hipMemcpyDeviceToHost, cu->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
-    (void)hipFree(tmp);
-    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("macroscopic: ") + hipGetErrorString(e));
-    return TDLB_OK;
+    const size_t cell = 4 * cu->tsize;
+    return read_result(cu, out, need, cell, "macroscopic", [&](void* dst, size_t a, size_t b, hipStream_t s) {
+        return launch_macroscopic(cs.prec, cu->prm.streaming, cs.momsrc, cs.even, cs.Q, cu->F, cu->fmask[cu->fm], cu->g,
+                                  cu->rho0, a / cell, b / cell, dst, s);
+    });
 }
 
 int tdlb_cu_double_resolution(tdlb_cu_t cu) {

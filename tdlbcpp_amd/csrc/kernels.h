@@ -96,7 +96,9 @@ hipError_t launch_ghost_copy(int esize, const void* src, void* dst, const Grid& 
 
 hipError_t launch_mask_from_f(int prec, const void* F, uint64_t* mask, uint64_t* gmask, const Grid& g,
                               hipStream_t s);
-hipError_t launch_masked_f(int prec, const void* F, const uint64_t* mask, void* out, const Grid& g, hipStream_t s);
+// F of cells [begin, end), zero where the mask is clear; out points at cell begin
+hipError_t launch_masked_f(int prec, const void* F, const uint64_t* mask, uint64_t begin, uint64_t end, void* out,
+                           const Grid& g, hipStream_t s);
 hipError_t launch_zero_interior_o(uint8_t* O, const Grid& g, hipStream_t s);
 
 hipError_t launch_force_prepare(int prec, const PointsDev& p, int64_t begin, int64_t count, void* F,
@@ -253,9 +255,9 @@ struct ReduceArgs {
 hipError_t launch_reduce(int prec, int streaming, int momsrc, int even, const void* Q, const void* F,
                          const uint64_t* fmask, const Grid& g, const ReduceArgs& ra, float rho0, double* partial,
                          double* out, hipStream_t s);
-// {rho, ux, uy, uz} per interior cell in T, interior cells in (i, j, k) order
-hipError_t launch_macroscopic(int prec, int streaming, int momsrc, int even, const void* Q,
-                              const void* F, const uint64_t* fmask, const Grid& g, float rho0, void* out,
+// {rho, ux, uy, uz} in T of interior cells [begin, end) in (i, j, k) order; out points at cell begin
+hipError_t launch_macroscopic(int prec, int streaming, int momsrc, int even, const void* Q, const void* F,
+                              const uint64_t* fmask, const Grid& g, float rho0, uint64_t begin, uint64_t end, void* out,
                               hipStream_t s);
 
 // doubleResolutionFullCU: Q (esize 4/8) and a per-cell array (nu_esize 2/4/8)

@@ -645,17 +645,19 @@ __global__ void k_mask_from_f(const T* __restrict__ F, uint64_t* __restrict__ ma
     }
 }
 
-// F as the reference holds it: the stored value where the bit is set, else 0.
+// F of cells [begin, end) as the reference holds it: the stored value where the bit is set, else 0.
 template <typename T>
-__global__ void k_masked_f(const T* __restrict__ F, const uint64_t* __restrict__ mask, T* __restrict__ out, Grid g) {
-    for (uint64_t n = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; n < g.size;
+__global__ void k_masked_f(const T* __restrict__ F, const uint64_t* __restrict__ mask, uint64_t begin, uint64_t end,
+                           T* __restrict__ out, Grid g) {
+    for (uint64_t n = begin + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; n < end;
          n += (uint64_t)gridDim.x * blockDim.x) {
         int i, j, k;
         decode_cell(g, n, i, j, k);
         const bool on = mask_test(mask, g, i, j, k);
-        out[3 * n + 0] = on ? F[3 * n + 0] : T(0);
-        out[3 * n + 1] = on ? F[3 * n + 1] : T(0);
-        out[3 * n + 2] = on ? F[3 * n + 2] : T(0);
+        const uint64_t o = 3 * (n - begin);
+        out[o + 0] = on ? F[3 * n + 0] : T(0);
+        out[o + 1] = on ? F[3 * n + 1] : T(0);
+        out[o + 2] = on ? F[3 * n + 2] : T(0);
     }
 }
 
@@ -1854,27 +1856,25 @@ __global__ __launch_bounds__(kReduceFinalBlock) void k_reduce_final(const double
     out[threadIdx.x] = a;
 }
 
-// {rho, ux, uy, uz} per interior cell, u as QVec::velocity(F) forms it
+// {rho, ux, uy, uz} of interior cells [begin, end), u as QVec::velocity(F) forms it
 // (QVec.hpp:125-131: (1.0 / rho) * (j + 0.5 * F), double literals).
 template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __global__ __launch_bounds__(kBlock) void k_macroscopic(const typename PR::S* __restrict__ Q,
                                                         const typename PR::T* __restrict__ F,
                                                         const uint64_t* __restrict__ fmask, Grid g, float rho0,
-                                                        typename PR::T* __restrict__ out) {
+                                                        uint64_t begin, uint64_t end, Mom4<typename PR::T>* __restrict__ out) {
     using T = typename PR::T;
     using D = typename PR::D;
-    const uint64_t n = (uint64_t)g.xg1 * g.yg1 * g.zg1;
-    for (uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t < n; t += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t t = begin + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t < end;
+         t += (uint64_t)gridDim.x * blockDim.x) {
         int i, j, k;
         interior_cell(g, t, i, j, k);
         T rho, jx, jy, jz, fx, fy, fz;
         cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, rho, jx, jy, jz, rho0);
         cell_force(F, fmask, g, i, j, k, fx, fy, fz);
         const D inv = D(1.0) / (D)rho;
-        out[4 * t + 0] = rho;
-        out[4 * t + 1] = (T)(inv * ((D)jx + D(0.5) * (D)fx));
-        out[4 * t + 2] = (T)(inv * ((D)jy + D(0.5) * (D)fy));
-        out[4 * t + 3] = (T)(inv * ((D)jz + D(0.5) * (D)fz));
+        out[t - begin] = Mom4<T>{rho, (T)(inv * ((D)jx + D(0.5) * (D)fx)), (T)(inv * ((D)jy + D(0.5) * (D)fy)),
+                                 (T)(inv * ((D)jz + D(0.5) * (D)fz))};
     }
 }
 
@@ -2298,9 +2298,12 @@ hipError_t launch_mask_from_f(int prec, const void* F, uint64_t* mask, uint64_t*
     return hipGetLastError();
 }
 
-hipError_t launch_masked_f(int prec, const void* F, const uint64_t* mask, void* out, const Grid& g, hipStream_t s) {
-    if (prec != 1) hipLaunchKernelGGL(k_masked_f<float>, dim3(grid_blocks(g.size)), dim3(kBlock), 0, s, (const float*)F, mask, (float*)out, g);
-    else hipLaunchKernelGGL(k_masked_f<double>, dim3(grid_blocks(g.size)), dim3(kBlock), 0, s, (const double*)F, mask, (double*)out, g);
+hipError_t launch_masked_f(int prec, const void* F, const uint64_t* mask, uint64_t begin, uint64_t end, void* out,
+                           const Grid& g, hipStream_t s) {
+    if (begin >= end) return hipSuccess;
+    const dim3 nb(grid_blocks(end - begin)), bs(kBlock);
+    if (prec != 1) hipLaunchKernelGGL(k_masked_f<float>, nb, bs, 0, s, (const float*)F, mask, begin, end, (float*)out, g);
+    else hipLaunchKernelGGL(k_masked_f<double>, nb, bs, 0, s, (const double*)F, mask, begin, end, (double*)out, g);
     return hipGetLastError();
 }
 
@@ -2562,18 +2565,19 @@ hipError_t launch_reduce(int prec, int streaming, int momsrc, int even, const vo
     return hipGetLastError();
 }
 
-hipError_t launch_macroscopic(int prec, int streaming, int momsrc, int even, const void* Q,
-                              const void* F, const uint64_t* fmask, const Grid& g, float rho0, void* out,
+hipError_t launch_macroscopic(int prec, int streaming, int momsrc, int even, const void* Q, const void* F,
+                              const uint64_t* fmask, const Grid& g, float rho0, uint64_t begin, uint64_t end, void* out,
                               hipStream_t s) {
-    const uint32_t nb = grid_blocks((uint64_t)g.xg1 * g.yg1 * g.zg1);
+    if (begin >= end) return hipSuccess;
+    const uint32_t nb = grid_blocks(end - begin);
     hipError_t e = hipErrorInvalidValue;
     TDLB_WITH_PREC(prec, {
         using S = typename PR::S;
         using T = typename PR::T;
         e = with_cell_source<PR>(streaming, momsrc, even, [&](auto Sc, auto Mc, auto Ec) {
-            hipLaunchKernelGGL((k_macroscopic<PR, decltype(Sc)::value, decltype(Mc)::value,
-                                              decltype(Ec)::value>),
-                               dim3(nb), dim3(kBlock), 0, s, (const S*)Q, (const T*)F, fmask, g, rho0, (T*)out);
+            hipLaunchKernelGGL((k_macroscopic<PR, decltype(Sc)::value, decltype(Mc)::value, decltype(Ec)::value>),
+                               dim3(nb), dim3(kBlock), 0, s, (const S*)Q, (const T*)F, fmask, g, rho0, begin, end,
+                               (Mom4<T>*)out);
             return hipGetLastError();
         });
     });

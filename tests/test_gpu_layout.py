@@ -24,3 +24,37 @@ def test_q_round_trip(dims, precision):
         assert np.array_equal(cu.q_ijkl().view(word) if layout != td.LAYOUT_LIJK
                               else np.ascontiguousarray(cu.q_ijkl()).view(word), values), layout
         cu.close()
+
+
+def test_results_read_by_several_threads_at_once():
+    """Six threads, each with a handle and stream of its own, share the pinned buffers of the read-back
+    (four of each size): every field equals the one read alone."""
+    import threading
+    edges = (24, 37, 64, 65, 90, 101)
+    cus = []
+    for n, e in enumerate(edges):
+        cu = td.ComputeUnit(e, precision=td.PREC_F16 if n % 2 else td.PREC_F32, **td.flow_for_tank(e))
+        cu.initialise(1.0)
+        cu.bind_rushton(td.rushton_defaults(e, startup_steps=2))
+        cu.run(3)
+        cus.append(cu)
+    for cu in cus:
+        cu.get(td.FIELD_F)  # leaves the handle with its moments stored, as every later read finds it
+    alone = [(cu.macroscopic(), cu.get(td.FIELD_F), cu.get(td.FIELD_NU)) for cu in cus]
+    got = [None] * len(cus)
+    print("[gpu case] read-back from six threads", flush=True)
+
+    def read(n):
+        got[n] = [(cus[n].macroscopic(), cus[n].get(td.FIELD_F), cus[n].get(td.FIELD_NU)) for _ in range(3)]
+
+    threads = [threading.Thread(target=read, args=(n,)) for n in range(len(cus))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(alone, got):
+        assert b is not None
+        for r in b:
+            assert all(np.array_equal(x, y) for x, y in zip(a, r))
+    for cu in cus:
+        cu.close()
