@@ -109,7 +109,7 @@ void release(tdlb_cu* cu) {
     cu->pts.release();
     cu->api_pts.release();
     cu->static_set.release();
-    cu->api_set.release();
+    cu->api_lists.release();
     if (cu->rot_cache) (void)hipFree(cu->rot_cache);
     for (hipEvent_t e : cu->events) (void)hipEventDestroy(e);
     cu->events.clear();
@@ -219,7 +219,7 @@ int check_points(const tdlb_cu* cu, const tdlb_ib_point* p, int64_t n) {
 // levels of a list; returns the permutation ordering points by level (stable)
 // and CSR offsets (offsets[0] = 0 .. offsets[L] = n)
 void compute_levels(const tdlb_cu* cu, const tdlb_ib_point* p, int64_t n, std::vector<int64_t>& order,
-                    std::vector<int64_t>& offsets, int base_level = 0) {
+                    std::vector<int64_t>& offsets) {
     std::unordered_map<uint64_t, int32_t> last;
     last.reserve((size_t)n * 4 + 16);
     std::vector<int32_t> lev(n);
@@ -228,7 +228,7 @@ void compute_levels(const tdlb_cu* cu, const tdlb_ib_point* p, int64_t n, std::v
     const int64_t gh = cu->prm.ghost;
     for (int64_t q = 0; q < n; q++) {
         stencil_cells(cu, p[q].i + gh, p[q].j + gh, p[q].k + gh, cells);
-        int32_t l = base_level;
+        int32_t l = 0;
         for (uint64_t c : cells) {
             auto it = last.find(c);
             if (it != last.end()) l = std::max(l, it->second + 1);
@@ -237,13 +237,13 @@ void compute_levels(const tdlb_cu* cu, const tdlb_ib_point* p, int64_t n, std::v
         lev[q] = l;
         maxl = std::max(maxl, l);
     }
-    const int nl = maxl + 1 - base_level;
+    const int nl = maxl + 1;
     offsets.assign(std::max(nl, 0) + 1, 0);
-    for (int64_t q = 0; q < n; q++) offsets[lev[q] - base_level + 1]++;
+    for (int64_t q = 0; q < n; q++) offsets[lev[q] + 1]++;
     for (int l = 0; l < nl; l++) offsets[l + 1] += offsets[l];
     order.resize(n);
     std::vector<int64_t> fill(offsets.begin(), offsets.end() - 1);
-    for (int64_t q = 0; q < n; q++) order[fill[lev[q] - base_level]++] = q;
+    for (int64_t q = 0; q < n; q++) order[fill[lev[q]]++] = q;
 }
 
 void to_host_points(const tdlb_cu* cu, const tdlb_ib_point* p, const std::vector<int64_t>& order, HostPoints& h) {
@@ -278,95 +278,6 @@ int upload_points(tdlb_cu* cu, DevPoints& dp, int64_t offset, const HostPoints& 
     HIPCHK(hipMemcpyAsync((char*)dp.d.v + offset * ts, h.v.data(), n * ts, hipMemcpyHostToDevice, cu->stream));
     HIPCHK(hipMemcpyAsync((char*)dp.d.w + offset * ts, h.w.data(), n * ts, hipMemcpyHostToDevice, cu->stream));
     HIPCHK(hipStreamSynchronize(cu->stream));  // host staging buffers end with the caller
-    return TDLB_OK;
-}
-
-// Build the unique-cell moment cache description of points (in device order)
-// and upload it; sidx entries are indexed by the point's position + offset.
-int build_indexed_set(tdlb_cu* cu, const tdlb_ib_point* p, const std::vector<int64_t>& order, IndexedSet& set) {
-    set.release();
-    const int64_t n = (int64_t)order.size();
-    if (n == 0) return TDLB_OK;
-    std::vector<uint32_t> all(9 * n);
-    uint64_t cells[9];
-    const int64_t gh = cu->prm.ghost;
-    for (int64_t a = 0; a < n; a++) {
-        const tdlb_ib_point& q = p[order[a]];
-        stencil_cells(cu, q.i + gh, q.j + gh, q.k + gh, cells);
-        for (int s = 0; s < 9; s++) all[9 * a + s] = (uint32_t)cells[s];
-    }
-    std::vector<uint32_t> uniq(all);
-    std::sort(uniq.begin(), uniq.end());
-    uniq.erase(std::unique(uniq.begin(), uniq.end()), uniq.end());
-    std::vector<int32_t> sidx(9 * n);
-    for (int64_t e = 0; e < 9 * n; e++)
-        sidx[e] = (int32_t)(std::lower_bound(uniq.begin(), uniq.end(), all[e]) - uniq.begin());
-    set.n_cells = (int64_t)uniq.size();
-    set.n_points = n;
-    if (hipMalloc((void**)&set.cells, uniq.size() * 4) != hipSuccess ||
-        hipMalloc((void**)&set.sidx, sidx.size() * 4) != hipSuccess ||
-        hipMalloc(&set.cache, uniq.size() * 4 * cu->tsize) != hipSuccess)
-        return fail(TDLB_ERR_NOMEM, "IB moment cache");
-    HIPCHK(hipMemcpyAsync(set.cells, uniq.data(), uniq.size() * 4, hipMemcpyHostToDevice, cu->stream));
-    HIPCHK(hipMemcpyAsync(set.sidx, sidx.data(), sidx.size() * 4, hipMemcpyHostToDevice, cu->stream));
-    HIPCHK(hipStreamSynchronize(cu->stream));
-    return TDLB_OK;
-}
-
-// Point ranges of one forcing pass sharing a source of stencil moments.
-struct ForceSegment {
-    const IndexedSet* set = nullptr;  // unique-cell cache (sidx by point index)
-    void* direct_cache = nullptr;     // or 9 entries per point from cache_base
-    int64_t cache_base = 0, n_points = 0;
-    std::vector<std::pair<int64_t, int64_t>> levels;
-};
-
-// One forcing pass: levels of every segment in order.  prepare: point ranges
-// whose stencil cells may be missing from the previous occupancy mask.  base:
-// bits the new mask starts from.
-int forcing_pass(tdlb_cu* cu, const DevPoints& dp, const std::vector<ForceSegment>& segs,
-                 const std::vector<std::pair<int64_t, int64_t>>& prepare, const uint64_t* base, int momsrc) {
-    uint64_t* prev = cu->fmask[cu->fm];
-    uint64_t* next = cu->fmask[1 - cu->fm];
-    const int even = cu->even ? 1 : 0;
-    // stored moments live in the explicit Q, populations in the lattice
-    const bool stored = momsrc == MOMSRC_STORED;
-    const void* Qsrc = stored ? cu->eq() : cu->Q[cu->cur];
-    const int qp = stored ? cu->eprec() : cu->prec();
-    HIPCHK(launch_copy(next, base, cu->mask_bytes(), cu->stream));
-    for (auto& r : prepare)
-        HIPCHK(launch_force_prepare(cu->eprec(), dp.d, r.first, r.second - r.first, cu->F, prev, next, cu->g,
-                                    cu->stream));
-    // stencils wrap onto themselves below 3 interior cells: keep the plain kernel there
-    const bool tiny = cu->g.xg1 < 3 || cu->g.zg1 < 3;
-    if (!tiny) {
-        for (auto& sg : segs) {
-            if (sg.set)
-                HIPCHK(launch_ib_moments_cells(qp, cu->prm.streaming, momsrc, even, sg.set->cells,
-                                               sg.set->n_cells, sg.set->cache, Qsrc, cu->g, cu->rho0, cu->stream));
-            else
-                HIPCHK(launch_ib_moments_points(qp, cu->prm.streaming, momsrc, even, dp.d,
-                                                sg.cache_base, sg.n_points, sg.direct_cache, Qsrc, cu->g, cu->rho0,
-                                                cu->stream));
-        }
-    }
-    for (auto& sg : segs)
-        for (auto& r : sg.levels) {
-            if (tiny)
-                HIPCHK(launch_force_level(qp, cu->prm.streaming, momsrc, even, dp.d, r.first,
-                                          r.second - r.first, cu->F, Qsrc, cu->g, cu->alfa, cu->beta, cu->rho0,
-                                          cu->stream));
-            else
-                HIPCHK(launch_force_level_cached(cu->eprec(), dp.d, r.first, r.second - r.first,
-                                                 sg.set ? sg.set->sidx : nullptr, sg.cache_base,
-                                                 sg.set ? sg.set->cache : sg.direct_cache, cu->F, cu->g, cu->alfa,
-                                                 cu->beta, cu->stream));
-        }
-    if (cu->o_dirty) {
-        HIPCHK(launch_zero_interior_o(cu->O, cu->g, cu->stream));
-        cu->o_dirty = false;
-    }
-    cu->fm = 1 - cu->fm;
     return TDLB_OK;
 }
 
@@ -1022,27 +933,28 @@ int tdlb_cu_forcing(tdlb_cu_t cu, const tdlb_ib_point* points, int64_t n, double
     CHK(set_device(cu));
     CHK(check_points(cu, points, n));
     CHK(materialise(cu));
-    std::vector<int64_t> order, offsets;
-    compute_levels(cu, points, n, order, offsets);
-    HostPoints h;
-    to_host_points(cu, points, order, h);
+    // the caller's points as they are, spread and ordered on the device
     CHK(cu->api_pts.reserve(n, cu->tsize));
-    CHK(upload_points(cu, cu->api_pts, 0, h));
-    CHK(build_indexed_set(cu, points, order, cu->api_set));
-    std::vector<ForceSegment> segs(1);
-    segs[0].set = &cu->api_set;
-    segs[0].n_points = n;
-    for (size_t l = 0; l + 1 < offsets.size(); l++) segs[0].levels.push_back({offsets[l], offsets[l + 1]});
-    std::vector<std::pair<int64_t, int64_t>> prep;
-    if (n > 0) prep.push_back({0, n});
-    const double a0 = cu->alfa, b0 = cu->beta;
-    cu->alfa = alfa;
-    cu->beta = beta;
-    int r = forcing_pass(cu, cu->api_pts, segs, prep, cu->gmask, MOMSRC_STORED);
-    cu->alfa = a0;
-    cu->beta = b0;
+    CHK(cu->api_lists.reserve(n, list_marks_bytes(cu->g, nullptr)));
+    uint64_t* prev = cu->fmask[cu->fm];
+    uint64_t* next = cu->fmask[1 - cu->fm];
+    if (n > 0) {
+        HIPCHK(hipMemcpyAsync(cu->api_lists.raw, points, sizeof(tdlb_ib_point) * (size_t)n, hipMemcpyHostToDevice,
+                              cu->stream));
+        HIPCHK(hipStreamSynchronize(cu->stream));  // the caller's buffer is free again when this returns
+    }
+    HIPCHK(launch_list_unpack(cu->prec(), cu->api_lists.raw, n, (int)cu->prm.ghost, cu->api_pts.d, cu->gmask, next,
+                              cu->mask_words, cu->stream));
+    HIPCHK(launch_list_planes(cu->prec(), cu->prm.streaming, cu->even ? 1 : 0, cu->api_pts.d, n, cu->api_lists.list,
+                              cu->api_lists.marks, cu->eq(), cu->F, prev, next, cu->g, alfa, beta, cu->rho0,
+                              cu->stream));
+    if (cu->o_dirty) {
+        HIPCHK(launch_zero_interior_o(cu->O, cu->g, cu->stream));
+        cu->o_dirty = false;
+    }
+    cu->fm = 1 - cu->fm;
     cu->static_in_prev = false;
-    return r;
+    return TDLB_OK;
 }
 
 int tdlb_cu_field_bytes(tdlb_cu_t cu, int field, size_t* bytes) {

@@ -79,10 +79,43 @@ inline void set_q_geometry(Grid& g, size_t ssize) {
     g.qsize = (cells + align - 1) / align * align;
 }
 
-// Stencil cells of a point list with a moments cache: the sorted unique cells,
-// and for every point the 9 positions of its stencil cells in that list.
-// A bound tank's static set also carries its plane tasks (PlaneDesc): cells
-// grouped by plane, points ordered plane by plane and level by level.
+// Buffers of the per-call forcing, as large as its longest list so far.
+struct ListBuffers {
+    tdlb_ib_point* raw = nullptr;  // the caller's points
+    int64_t* list = nullptr;       // positions, plane by plane
+    uint32_t* marks = nullptr;     // planes of marks, for grids whose plane the LDS does not hold
+    int64_t cap = 0;
+    void release() {
+        for (void* p : {(void*)raw, (void*)list, (void*)marks})
+            if (p) (void)hipFree(p);
+        raw = nullptr;
+        list = nullptr;
+        marks = nullptr;
+        cap = 0;
+    }
+    int reserve(int64_t n, size_t marks_bytes) {
+        if (n > cap) {
+            const int64_t c = std::max<int64_t>(n, 256);
+            for (void** p : {(void**)&raw, (void**)&list}) {
+                if (*p) (void)hipFree(*p);
+                *p = nullptr;
+            }
+            cap = 0;
+            if (hipMalloc((void**)&raw, sizeof(tdlb_ib_point) * (size_t)c) != hipSuccess ||
+                hipMalloc((void**)&list, sizeof(int64_t) * (size_t)c) != hipSuccess)
+                return fail(TDLB_ERR_NOMEM, "IB list buffers");
+            cap = c;
+        }
+        if (n > 0 && marks_bytes > 0 && !marks && hipMalloc((void**)&marks, marks_bytes) != hipSuccess) {
+            marks = nullptr;
+            return fail(TDLB_ERR_NOMEM, "IB list marks");
+        }
+        return TDLB_OK;
+    }
+};
+
+// A bound tank's static points and their plane tasks (PlaneDesc): the unique
+// stencil cells grouped by plane, points ordered plane by plane and level by level.
 struct IndexedSet {
     uint32_t* cells = nullptr;
     int32_t* sidx = nullptr;
@@ -196,7 +229,7 @@ struct tdlb_cu {
     uint32_t* pctr = nullptr;
 
     DevPoints api_pts;  // points of the generic forcing call
-    IndexedSet api_set;
+    ListBuffers api_lists;
 
     // event timing of tdlb_cu_run (tdlb_cu_profile)
     bool prof = false;

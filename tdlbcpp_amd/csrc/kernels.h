@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include "../../include/tdlb.h"
 #include "device.h"
 #include "es_collide.h"
 
@@ -103,23 +104,19 @@ hipError_t launch_zero_interior_o(uint8_t* O, const Grid& g, hipStream_t s);
 
 hipError_t launch_force_prepare(int prec, const PointsDev& p, int64_t begin, int64_t count, void* F,
                                 const uint64_t* prev, uint64_t* next, const Grid& g, hipStream_t s);
-hipError_t launch_force_level(int prec, int streaming, int momsrc, int even, const PointsDev& p,
-                              int64_t begin, int64_t count, void* F, const void* Q, const Grid& g, double alfa,
-                              double beta, float rho0, hipStream_t s);
+// ---- IB forcing of a caller's list (fp32, fp64; moments stored in Q)
+// n points into arrays p (cell indices with the ghost offset), and next = base (words)
+hipError_t launch_list_unpack(int prec, const tdlb_ib_point* in, int64_t n, int ghost, const PointsDev& p,
+                              const uint64_t* base, uint64_t* next, uint64_t words, hipStream_t s);
+// Bytes of the marks array launch_list_planes needs in HBM (0: a plane's marks fit
+// the LDS), and its workgroups.
+constexpr size_t kListLdsBytes = 152 * 1024;  // of a CU's 160 KB
+size_t list_marks_bytes(const Grid& g, int* blocks);
+// The forcing of the list in its order; list: room for n positions.
+hipError_t launch_list_planes(int prec, int streaming, int even, const PointsDev& p, int64_t n, int64_t* list,
+                              uint32_t* marks, const void* Q, void* F, const uint64_t* prev, uint64_t* next,
+                              const Grid& g, double alfa, double beta, float rho0, hipStream_t s);
 
-// Density and momentum of IB stencil cells, 4 values of T per entry {rho, jx, jy, jz}.
-// cells: sorted cell indices (one entry per cell).
-hipError_t launch_ib_moments_cells(int prec, int streaming, int momsrc, int even, const uint32_t* cells,
-                                   int64_t n, void* cache, const void* Q, const Grid& g, float rho0, hipStream_t s);
-// one entry per (point, stencil cell): entry 9*t + s for point begin + t
-hipError_t launch_ib_moments_points(int prec, int streaming, int momsrc, int even, const PointsDev& p,
-                                    int64_t begin, int64_t count, void* cache, const void* Q, const Grid& g,
-                                    float rho0, hipStream_t s);
-// One forcing level reading stencil moments from a cache.  sidx: per point 9 cache
-// indices (static lists); null: the entries of point begin+t are 9*(t + cache_base) ...
-hipError_t launch_force_level_cached(int prec, const PointsDev& p, int64_t begin, int64_t count,
-                                     const int32_t* sidx, int64_t cache_base, const void* cache, void* F,
-                                     const Grid& g, double alfa, double beta, hipStream_t s);
 // ---- IB forcing of a bound tank by j planes.  Stencils span i and k at the
 // point's j, so points of different planes never share a cell and each plane
 // is an independent task.  A pass is two launches: the gather (blade points,

@@ -758,22 +758,62 @@ __device__ __forceinline__ void cell_rho_j(const typename PR::S* __restrict__ Q,
     }
 }
 
-// One level of the forcing: points of a level have pairwise disjoint stencils,
-// so each thread runs the reference's gather / correct / spread for one point
-// (Forcing.hpp:73-135) with the F values left by all earlier levels.
-template <typename PR, int STREAM, int MOMSRC, int EVEN>
-__global__ __launch_bounds__(kBlock) void k_force_level(PointsDev p, int64_t begin, int64_t count,
-                                                        typename PR::T* __restrict__ F,
-                                                        const typename PR::S* __restrict__ Q, Grid g,
-                                                        typename PR::T alfa, typename PR::T beta, float rho0) {
+// Density and momentum of a cell, or the three force components (the fourth unused).
+template <typename T>
+struct alignas(4 * sizeof(T)) Mom4 {
+    T r, x, y, z;
+};
+
+// ------------------------------------------------------------------ IB forcing of a list
+// The per-call forcing (any list, in its order) in two launches.  k_list_unpack
+// spreads the caller's points into arrays and starts the next occupancy mask.
+// k_list_planes takes a j plane per workgroup: points of different planes never
+// share a cell.  It collects the plane's points in list order, prepares their cells
+// and then runs rounds over the first unfinished ones, one a lane: each marks its
+// nine cells with the lowest position that wants them (atomicMin), and those that
+// hold all their cells run the reference's gather / correct / spread
+// (Forcing.hpp:73-135) and make room for the next.  They share no cell, and no
+// earlier point is unfinished on theirs, so every cell sees its points in list
+// order.  The rounds are bound by the latency of a point's loads.  A call over the
+// 13,431 points of a 60^3 tank: 0.29 ms, the kernel 110 us of them; with levels from
+// a hash map on the host and a launch per level 8.5 ms.
+template <typename T>
+__global__ void k_list_unpack(const tdlb_ib_point* __restrict__ in, int64_t n, int ghost, PointsDev p,
+                              const uint64_t* __restrict__ base, uint64_t* __restrict__ next, uint64_t words) {
+    for (uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t < max((uint64_t)n, words);
+         t += (uint64_t)gridDim.x * blockDim.x) {
+        if (t < words) next[t] = base[t];
+        if (t >= (uint64_t)n) continue;
+        const tdlb_ib_point q = in[t];
+        p.i[t] = (int32_t)(q.i + ghost);
+        p.j[t] = (int32_t)(q.j + ghost);
+        p.k[t] = (int32_t)(q.k + ghost);
+        static_cast<T*>(p.ifrac)[t] = (T)q.i_frac;
+        static_cast<T*>(p.kfrac)[t] = (T)q.k_frac;
+        static_cast<T*>(p.u)[t] = (T)q.u_delta;
+        static_cast<T*>(p.v)[t] = (T)q.v_delta;
+        static_cast<T*>(p.w)[t] = (T)q.w_delta;
+    }
+}
+
+// gather, correct and spread of point q, all nine cells by one lane, from stored moments
+template <typename PR, int STREAM, int EVEN>
+__device__ __forceinline__ void list_point(const PointsDev& p, int64_t q, typename PR::T* __restrict__ F,
+                                           const typename PR::S* __restrict__ Q, const Grid& g,
+                                           typename PR::T alfa, typename PR::T beta, float rho0) {
     using T = typename PR::T;
     using D = typename PR::D;
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    const int64_t q = begin + t;
     const int pi = p.i[q], pj = p.j[q], pk = p.k[q];
     const T ifr = static_cast<const T*>(p.ifrac)[q], kfr = static_cast<const T*>(p.kfrac)[q];
     T wx[3], wz[3];
+    uint64_t at[9];
+    T f[9][3];
+#pragma unroll
+    for (int s = 0; s < 9; s++) {
+        at[s] = 3ull * cell_index(g, wrap_ik(pi + s % 3 - 1, g.xg1), pj, wrap_ik(pk + s / 3 - 1, g.zg1));
+#pragma unroll
+        for (int d = 0; d < 3; d++) f[s][d] = F[at[s] + d];
+    }
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         wx[a] = ib_weight<T>(-ifr + T(a - 1));
@@ -781,183 +821,142 @@ __global__ __launch_bounds__(kBlock) void k_force_level(PointsDev p, int64_t beg
     }
     T rhoSum = T(0.0), xSum = T(0.0), ySum = T(0.0), zSum = T(0.0);
 #pragma unroll
-    for (int k1 = -1; k1 <= 1; k1++)
-#pragma unroll
-        for (int i1 = -1; i1 <= 1; i1++) {
-            const int i2 = wrap_ik(pi + i1, g.xg1), k2 = wrap_ik(pk + k1, g.zg1);
-            T rho, jx, jy, jz;
-            cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i2, pj, k2, rho, jx, jy, jz, rho0);
-            const uint64_t c = cell_index(g, i2, pj, k2);
-            const T ppp = wx[i1 + 1] * wz[k1 + 1];
-            const T xx = (T)((D)jx + D(0.5) * (D)F[3 * c + 0]);
-            const T yy = (T)((D)jy + D(0.5) * (D)F[3 * c + 1]);
-            const T zz = (T)((D)jz + D(0.5) * (D)F[3 * c + 2]);
-            rhoSum += ppp * rho;
-            xSum += ppp * xx;
-            ySum += ppp * yy;
-            zSum += ppp * zz;
-        }
+    for (int s = 0; s < 9; s++) {
+        T rho, jx, jy, jz;
+        cell_rho_j<PR, STREAM, MOMSRC_STORED, EVEN>(Q, g, wrap_ik(pi + s % 3 - 1, g.xg1), pj,
+                                                    wrap_ik(pk + s / 3 - 1, g.zg1), rho, jx, jy, jz, rho0);
+        const T ppp = wx[s % 3] * wz[s / 3];
+        const T xx = (T)((D)jx + D(0.5) * (D)f[s][0]);
+        const T yy = (T)((D)jy + D(0.5) * (D)f[s][1]);
+        const T zz = (T)((D)jz + D(0.5) * (D)f[s][2]);
+        rhoSum += ppp * rho;
+        xSum += ppp * xx;
+        ySum += ppp * yy;
+        zSum += ppp * zz;
+    }
     xSum -= rhoSum * static_cast<const T*>(p.u)[q];
     ySum -= rhoSum * static_cast<const T*>(p.v)[q];
     zSum -= rhoSum * static_cast<const T*>(p.w)[q];
+    // below 3 interior cells a stencil meets itself: one cell after the other
+    const bool meets = g.xg1 < 3 || g.zg1 < 3;
 #pragma unroll
-    for (int k1 = -1; k1 <= 1; k1++)
+    for (int s = 0; s < 9; s++) {
+        const T bp = beta * (wx[s % 3] * wz[s / 3]);
+        if (meets)
 #pragma unroll
-        for (int i1 = -1; i1 <= 1; i1++) {
-            const int i2 = wrap_ik(pi + i1, g.xg1), k2 = wrap_ik(pk + k1, g.zg1);
-            const uint64_t c = cell_index(g, i2, pj, k2);
-            const T bp = beta * (wx[i1 + 1] * wz[k1 + 1]);
-            F[3 * c + 0] = alfa * F[3 * c + 0] - bp * xSum;
-            F[3 * c + 1] = alfa * F[3 * c + 1] - bp * ySum;
-            F[3 * c + 2] = alfa * F[3 * c + 2] - bp * zSum;
-        }
-}
-
-// ------------------------------------------------------------------ IB forcing with a moments cache
-// Density and momentum of the stencil cells are computed once per forcing pass
-// (they do not change while F is updated), so the level kernels issue only
-// independent cache / F loads instead of 18 scattered population loads per
-// stencil cell.
-template <typename T>
-struct alignas(4 * sizeof(T)) Mom4 {
-    T r, x, y, z;
-};
-
-template <typename PR, int STREAM, int MOMSRC, int EVEN>
-__global__ __launch_bounds__(kBlock) void k_ib_moments_cells(const uint32_t* __restrict__ cells, int64_t n,
-                                                             Mom4<typename PR::T>* __restrict__ cache,
-                                                             const typename PR::S* __restrict__ Q, Grid g,
-                                                             float rho0) {
-    using T = typename PR::T;
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const uint32_t c = cells[t];
-    const int i = (int)(c / g.yz);
-    const uint32_t r = c - (uint32_t)i * g.yz;
-    const int j = (int)(r / (uint32_t)g.zg);
-    const int k = (int)(r - (uint32_t)j * (uint32_t)g.zg);
-    Mom4<T> m;
-    cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i, j, k, m.r, m.x, m.y, m.z, rho0);
-    cache[t] = m;
-}
-
-template <typename PR, int STREAM, int MOMSRC, int EVEN>
-__global__ __launch_bounds__(kBlock) void k_ib_moments_points(PointsDev p, int64_t begin, int64_t count,
-                                                              Mom4<typename PR::T>* __restrict__ cache,
-                                                              const typename PR::S* __restrict__ Q, Grid g,
-                                                              float rho0) {
-    using T = typename PR::T;
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= count * 9) return;
-    const int64_t q = begin + t / 9;
-    const int s = (int)(t % 9);
-    const int i2 = wrap_ik(p.i[q] + (s % 3) - 1, g.xg1), k2 = wrap_ik(p.k[q] + (s / 3) - 1, g.zg1);
-    Mom4<T> m;
-    cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i2, p.j[q], k2, m.r, m.x, m.y, m.z, rho0);
-    cache[t] = m;
-}
-
-// Same arithmetic as k_force_level, one point per 3 lanes of a wavefront: lane
-// c of the group holds the stencil row k1 = c - 1, its cells s = 3c + m for
-// i1 = m - 1 (s = (k1+1)*3 + (i1+1)), so the 9 gathers of a point run in
-// parallel, three per lane.  Stencil cell s reads cache[sidx[9q+s]] (INDEXED)
-// or cache[9(q-cache_base)+s].  Every lane of the group adds the 9 terms in
-// the reference's order (s = 0..8, each product rounded before the add), so
-// the sums are those of the sequential loop bit for bit.  The 9 cells of a
-// point are distinct (the cached path needs 3 interior cells in x and z) and
-// the points of a level have disjoint stencils, so each F entry has one writer.
-// Three lanes per point put 21 points in a wavefront (7 with a lane per cell):
-// a level's passes, each a chain of dependent loads, are a third as many.
-constexpr int kGroup = 3;                    // lanes per point
-constexpr int kGroupsPerWave = 64 / kGroup;  // 21 points per wavefront, lane 63 idle
-
-template <typename T, typename D, bool INDEXED>
-__device__ __forceinline__ void force_point9(const PointsDev& p, int64_t q, bool valid, int c, int base,
-                                             const int32_t* __restrict__ sidx, int64_t cache_base,
-                                             const Mom4<T>* __restrict__ cache, T* __restrict__ F, const Grid& g,
-                                             T alfa, T beta) {
-    T w[3], tr[3], tx[3], ty[3], tz[3], fo[3][3];
-    uint64_t cell[3];
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-        w[m] = tr[m] = tx[m] = ty[m] = tz[m] = fo[m][0] = fo[m][1] = fo[m][2] = T(0);
-        cell[m] = 0;
-    }
-    if (valid) {
-        const T ifr = static_cast<const T*>(p.ifrac)[q], kfr = static_cast<const T*>(p.kfrac)[q];
-        const T wk = ib_weight<T>(-kfr + T(c - 1));
-        const int pi = p.i[q], pj = p.j[q], k2 = wrap_ik(p.k[q] + c - 1, g.zg1);
-        Mom4<T> mo[3];
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            const int i2 = wrap_ik(pi + m - 1, g.xg1);
-            cell[m] = cell_index(g, i2, pj, k2);
-            mo[m] = cache[INDEXED ? (int64_t)sidx[9 * q + 3 * c + m] : 9 * (q - cache_base) + 3 * c + m];
-            fo[m][0] = F[3 * cell[m] + 0];
-            fo[m][1] = F[3 * cell[m] + 1];
-            fo[m][2] = F[3 * cell[m] + 2];
-        }
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            w[m] = ib_weight<T>(-ifr + T(m - 1)) * wk;
-            const T xx = (T)((D)mo[m].x + D(0.5) * (D)fo[m][0]);
-            const T yy = (T)((D)mo[m].y + D(0.5) * (D)fo[m][1]);
-            const T zz = (T)((D)mo[m].z + D(0.5) * (D)fo[m][2]);
-            tr[m] = w[m] * mo[m].r;
-            tx[m] = w[m] * xx;
-            ty[m] = w[m] * yy;
-            tz[m] = w[m] * zz;
-        }
-    }
-    // terms s = 3 c2 + m in the order s = 0..8: row c2 from lane base + c2
-    T rhoSum = T(0.0), xSum = T(0.0), ySum = T(0.0), zSum = T(0.0);
-#pragma unroll
-    for (int c2 = 0; c2 < kGroup; c2++)
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            rhoSum += __shfl(tr[m], base + c2, 64);
-            xSum += __shfl(tx[m], base + c2, 64);
-            ySum += __shfl(ty[m], base + c2, 64);
-            zSum += __shfl(tz[m], base + c2, 64);
-        }
-    if (!valid) return;
-    xSum -= rhoSum * static_cast<const T*>(p.u)[q];
-    ySum -= rhoSum * static_cast<const T*>(p.v)[q];
-    zSum -= rhoSum * static_cast<const T*>(p.w)[q];
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-        const T bp = beta * w[m];
-        F[3 * cell[m] + 0] = alfa * fo[m][0] - bp * xSum;
-        F[3 * cell[m] + 1] = alfa * fo[m][1] - bp * ySum;
-        F[3 * cell[m] + 2] = alfa * fo[m][2] - bp * zSum;
+            for (int d = 0; d < 3; d++) f[s][d] = F[at[s] + d];
+        F[at[s] + 0] = alfa * f[s][0] - bp * xSum;
+        F[at[s] + 1] = alfa * f[s][1] - bp * ySum;
+        F[at[s] + 2] = alfa * f[s][2] - bp * zSum;
     }
 }
 
-// lane -> (point index within the launch, stencil row, group base lane)
-__device__ __forceinline__ int64_t group_point(int& c, int& base) {
-    const int lane = (int)(threadIdx.x & 63), grp = lane / kGroup;
-    c = lane - grp * kGroup;
-    base = grp * kGroup;
-    const int64_t wave = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6);
-    return grp < kGroupsPerWave ? wave * kGroupsPerWave + grp : -1;
-}
-
-inline uint32_t group_blocks(int64_t points, int bs) {
-    const int64_t waves = (points + kGroupsPerWave - 1) / kGroupsPerWave;
-    const int64_t per_block = bs / 64;
-    return (uint32_t)((waves + per_block - 1) / per_block);
-}
-
-template <typename T, typename D, bool INDEXED>
-__global__ __launch_bounds__(kBlock) void k_force_level_cached(PointsDev p, int64_t begin, int64_t count,
-                                                               const int32_t* __restrict__ sidx, int64_t cache_base,
-                                                               const Mom4<T>* __restrict__ cache, T* __restrict__ F,
-                                                               Grid g, T alfa, T beta) {
-    int s, base;
-    const int64_t t = group_point(s, base);
-    const bool valid = t >= 0 && t < count;
-    force_point9<T, D, INDEXED>(p, begin + (valid ? t : 0), valid, s, base, sidx, cache_base, cache, F, g, alfa,
-                                beta);
+constexpr int kListBlock = 512;
+constexpr uint32_t kNoPoint = 0xffffffffu;
+// list: n positions, the planes' points one plane after the other.  marks_hbm: a
+// plane of marks per workgroup where the LDS does not hold one; a mark there may sit
+// in this CU's L1 from the round before and is read where the atomics put it.
+template <typename PR, int STREAM, int EVEN, bool MARKS_LDS>
+__global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t n, int64_t* __restrict__ list,
+                                                            uint32_t* __restrict__ marks_hbm,
+                                                            typename PR::T* __restrict__ F,
+                                                            const typename PR::S* __restrict__ Q,
+                                                            const uint64_t* __restrict__ prev,
+                                                            uint64_t* __restrict__ next, Grid g,
+                                                            typename PR::T alfa, typename PR::T beta, float rho0) {
+    extern __shared__ uint32_t list_lds[];
+    constexpr int kWaves = kListBlock / 64;
+    __shared__ int64_t s_less[kWaves];
+    __shared__ int s_wave[2][kWaves];
+    __shared__ uint32_t s_next, s_done;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int plane = g.xg1 * g.zg1;
+    uint32_t* const hbm = MARKS_LDS ? nullptr : marks_hbm + (uint64_t)blockIdx.x * plane;
+    auto set_mark = [&](int c) {
+        if (MARKS_LDS) list_lds[c] = kNoPoint;
+        else hbm[c] = kNoPoint;
+    };
+    auto min_mark = [&](int c, uint32_t t) {
+        if (MARKS_LDS) atomicMin(&list_lds[c], t);
+        else atomicMin(hbm + c, t);
+    };
+    auto mark = [&](int c) -> uint32_t {
+        return MARKS_LDS ? list_lds[c] : __hip_atomic_load(hbm + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    for (int c = tid; c < plane; c += kListBlock) set_mark(c);
+    for (int j = 1 + (int)blockIdx.x; j <= g.yg1; j += (int)gridDim.x) {
+        // the plane's part of the list begins after the points of lower planes
+        int64_t less = 0;
+        for (int64_t q = tid; q < n; q += kListBlock) less += p.j[q] < j ? 1 : 0;
+        for (int o = 32; o > 0; o >>= 1) less += __shfl_down(less, o, 64);
+        if (lane == 0) s_less[wave] = less;
+        __syncthreads();
+        int64_t first = 0;
+        for (int w = 0; w < kWaves; w++) first += s_less[w];
+        int64_t* const mine = list + first;
+        // its points in list order
+        uint32_t count = 0;
+        int turn = 0;
+        for (int64_t q0 = 0; q0 < n; q0 += kListBlock, turn ^= 1) {
+            const int64_t q = q0 + tid;
+            const bool in = q < n && p.j[q] == j;
+            const uint64_t vote = __ballot(in);
+            if (lane == 0) s_wave[turn][wave] = __popcll(vote);
+            __syncthreads();  // the last reader of s_wave[turn] has passed the turn between
+            uint32_t at = count;
+            for (int w = 0; w < kWaves; w++) {
+                at += w < wave ? s_wave[turn][w] : 0;
+                count += s_wave[turn][w];
+            }
+            if (in) mine[at + __popcll(vote & ((1ull << lane) - 1ull))] = q;
+        }
+        if (tid == 0) {
+            s_next = kListBlock;
+            s_done = 0;
+        }
+        __syncthreads();
+        for (uint32_t t = tid; t < count; t += kListBlock) prepare_point(p, mine[t], F, prev, next, g);
+        // the lanes hold a prefix of the plane's list: a lane that finishes its point takes the next
+        uint32_t t = tid;
+        bool have = t < count;
+        int64_t q = 0;
+        int cells[9];
+        auto take = [&] {
+            q = mine[t];
+            const int pi = p.i[q], pk = p.k[q];
+#pragma unroll
+            for (int s = 0; s < 9; s++)
+                cells[s] = (wrap_ik(pi + s % 3 - 1, g.xg1) - 1) * g.zg1 + wrap_ik(pk + s / 3 - 1, g.zg1) - 1;
+        };
+        if (have) take();
+        __syncthreads();
+        // One barrier ends a turn for every lane, so the loop has one way back: with a
+        // lane's take() as a second one the compiler made a loop of its own of it, and
+        // the barriers of a wavefront's lanes parted.
+        for (uint32_t done = 0; done < count;) {
+            if (have)
+#pragma unroll
+                for (int s = 0; s < 9; s++) min_mark(cells[s], t);
+            __syncthreads();
+            bool ready = have;
+            if (have)
+#pragma unroll
+                for (int s = 0; s < 9; s++) ready = (mark(cells[s]) == t) && ready;
+            __syncthreads();
+            if (have)
+#pragma unroll
+                for (int s = 0; s < 9; s++) set_mark(cells[s]);
+            if (ready) {
+                list_point<PR, STREAM, EVEN>(p, q, F, Q, g, alfa, beta, rho0);
+                atomicAdd(&s_done, 1u);
+                t = atomicAdd(&s_next, 1u);
+                have = t < count;
+                if (have) take();
+            }
+            __syncthreads();
+            done = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_done);  // changes two barriers from here
+        }
+    }
 }
 
 // ------------------------------------------------------------------ IB forcing by planes
@@ -2087,27 +2086,6 @@ hipError_t simple_t(int mode, const void* src, void* dst, void* mout, const void
     return hipGetLastError();
 }
 
-template <typename PR, int STREAM>
-hipError_t force_level_t(int momsrc, int even, const PointsDev& p, int64_t begin, int64_t count, void* F,
-                         const void* Q, const Grid& g, double alfa, double beta, float rho0, hipStream_t s) {
-    using S = typename PR::S;
-    using T = typename PR::T;
-    const uint32_t nb = (uint32_t)((count + kBlock - 1) / kBlock);
-    T* f = static_cast<T*>(F);
-    const S* q = static_cast<const S*>(Q);
-    const T a = (T)alfa, b = (T)beta;
-#define TDLB_FL(M, E) \
-    hipLaunchKernelGGL((k_force_level<PR, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, p, begin, count, f, q, g, a, b, rho0)
-    if (momsrc == MOMSRC_STORED) {
-        if constexpr (PR::kShift) return hipErrorInvalidValue;
-        else { if (even) TDLB_FL(MOMSRC_STORED, 1); else TDLB_FL(MOMSRC_STORED, 0); }
-    }
-    else if (momsrc == MOMSRC_ESO_POPS) { if (even) TDLB_FL(MOMSRC_ESO_POPS, 1); else TDLB_FL(MOMSRC_ESO_POPS, 0); }
-    else { TDLB_FL(MOMSRC_PULL_POPS, 1); }
-#undef TDLB_FL
-    return hipGetLastError();
-}
-
 }  // namespace
 
 // precision index -> traits: 0 fp32, 1 fp64, 2 fp16 storage, 3 bf16 storage,
@@ -2321,95 +2299,59 @@ hipError_t launch_force_prepare(int prec, const PointsDev& p, int64_t begin, int
     return hipGetLastError();
 }
 
-hipError_t launch_force_level(int prec, int streaming, int momsrc, int even, const PointsDev& p,
-                              int64_t begin, int64_t count, void* F, const void* Q, const Grid& g, double alfa,
-                              double beta, float rho0, hipStream_t s) {
-    if (count <= 0) return hipSuccess;
-    hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, e = streaming == StreamEsotwist
-                                 ? force_level_t<PR, StreamEsotwist>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s)
-                                 : force_level_t<PR, StreamSimple>(momsrc, even, p, begin, count, F, Q, g, alfa, beta, rho0, s));
-    return e;
-}
+template <int V>
+using IC = std::integral_constant<int, V>;
 
-namespace {
-template <typename PR, int STREAM>
-hipError_t ib_moments_t(int momsrc, int even, const uint32_t* cells, const PointsDev* p, int64_t begin, int64_t n,
-                        void* cache, const void* Q, const Grid& g, float rho0, hipStream_t s) {
-    using T = typename PR::T;
-    using S = typename PR::S;
-    Mom4<T>* c = static_cast<Mom4<T>*>(cache);
-    const S* q = static_cast<const S*>(Q);
-    const int64_t threads = cells ? n : 9 * n;
-    const uint32_t nb = (uint32_t)((threads + kBlock - 1) / kBlock);
-#define TDLB_IBM(M, E)                                                                                          \
-    do {                                                                                                        \
-        if (cells) hipLaunchKernelGGL((k_ib_moments_cells<PR, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, cells, n, c, q, g, rho0); \
-        else hipLaunchKernelGGL((k_ib_moments_points<PR, STREAM, M, E>), dim3(nb), dim3(kBlock), 0, s, *p, begin, n, c, q, g, rho0); \
-    } while (0)
-    if (momsrc == MOMSRC_STORED) {
-        if constexpr (PR::kShift) return hipErrorInvalidValue;
-        else { if (even) TDLB_IBM(MOMSRC_STORED, 1); else TDLB_IBM(MOMSRC_STORED, 0); }
-    }
-    else if (momsrc == MOMSRC_ESO_POPS) { if (even) TDLB_IBM(MOMSRC_ESO_POPS, 1); else TDLB_IBM(MOMSRC_ESO_POPS, 0); }
-    else TDLB_IBM(MOMSRC_PULL_POPS, 1);
-#undef TDLB_IBM
+hipError_t launch_list_unpack(int prec, const tdlb_ib_point* in, int64_t n, int ghost, const PointsDev& p,
+                              const uint64_t* base, uint64_t* next, uint64_t words, hipStream_t s) {
+    const dim3 nb(grid_blocks(std::max<uint64_t>((uint64_t)n, words))), bs(kBlock);
+    if (prec != 1) hipLaunchKernelGGL(k_list_unpack<float>, nb, bs, 0, s, in, n, ghost, p, base, next, words);
+    else hipLaunchKernelGGL(k_list_unpack<double>, nb, bs, 0, s, in, n, ghost, p, base, next, words);
     return hipGetLastError();
 }
 
-template <typename PR>
-hipError_t ib_moments_prec(int streaming, int momsrc, int even, const uint32_t* cells, const PointsDev* p,
-                           int64_t begin, int64_t n, void* cache, const void* Q, const Grid& g, float rho0,
-                           hipStream_t s) {
-    return streaming == StreamEsotwist
-               ? ib_moments_t<PR, StreamEsotwist>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s)
-               : ib_moments_t<PR, StreamSimple>(momsrc, even, cells, p, begin, n, cache, Q, g, rho0, s);
+size_t list_marks_bytes(const Grid& g, int* blocks) {
+    const size_t plane = (size_t)g.xg1 * g.zg1 * sizeof(uint32_t);
+    const bool lds = plane <= kListLdsBytes;
+    // a workgroup per plane; with marks in HBM at most one per CU
+    const int n = lds ? g.yg1 : std::min(g.yg1, 256);
+    if (blocks) *blocks = n;
+    return lds ? 0 : plane * (size_t)n;
 }
-}  // namespace
 
-hipError_t launch_ib_moments_cells(int prec, int streaming, int momsrc, int even, const uint32_t* cells,
-                                   int64_t n, void* cache, const void* Q, const Grid& g, float rho0, hipStream_t s) {
+hipError_t launch_list_planes(int prec, int streaming, int even, const PointsDev& p, int64_t n, int64_t* list,
+                              uint32_t* marks, const void* Q, void* F, const uint64_t* prev, uint64_t* next,
+                              const Grid& g, double alfa, double beta, float rho0, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, e = ib_moments_prec<PR>(streaming, momsrc, even, cells, nullptr, 0, n, cache, Q, g,
-                                                 rho0, s));
-    return e;
-}
-
-hipError_t launch_ib_moments_points(int prec, int streaming, int momsrc, int even, const PointsDev& p,
-                                    int64_t begin, int64_t count, void* cache, const void* Q, const Grid& g,
-                                    float rho0, hipStream_t s) {
-    if (count <= 0) return hipSuccess;
-    hipError_t e = hipErrorInvalidValue;
-    TDLB_WITH_PREC(prec, e = ib_moments_prec<PR>(streaming, momsrc, even, nullptr, &p, begin, count, cache, Q,
-                                                 g, rho0, s));
-    return e;
-}
-
-hipError_t launch_force_level_cached(int prec, const PointsDev& p, int64_t begin, int64_t count,
-                                     const int32_t* sidx, int64_t cache_base, const void* cache, void* F,
-                                     const Grid& g, double alfa, double beta, hipStream_t s) {
-    if (count <= 0) return hipSuccess;
-    constexpr int bs = 64;  // one wavefront per block: levels are small, spread them over the CUs
-    const uint32_t nb = group_blocks(count, bs);
-    TDLB_WITH_PREC(prec, {
+    int blocks = 0;
+    const size_t hbm = list_marks_bytes(g, &blocks);
+    if ((hbm != 0) != (marks != nullptr)) return hipErrorInvalidValue;
+    const uint32_t lds = hbm ? 0u : (uint32_t)((size_t)g.xg1 * g.zg1 * sizeof(uint32_t));
+    auto go = [&](auto pr, auto Sc, auto Ec) -> hipError_t {
+        using PR = decltype(pr);
         using T = typename PR::T;
-        using D = typename PR::D;
-        const auto* c = static_cast<const Mom4<T>*>(cache);
-        if (sidx)
-            hipLaunchKernelGGL((k_force_level_cached<T, D, true>), dim3(nb), dim3(bs), 0, s, p, begin, count, sidx,
-                               cache_base, c, (T*)F, g, (T)alfa, (T)beta);
-        else
-            hipLaunchKernelGGL((k_force_level_cached<T, D, false>), dim3(nb), dim3(bs), 0, s, p, begin, count, sidx,
-                               cache_base, c, (T*)F, g, (T)alfa, (T)beta);
-    });
-    return hipGetLastError();
+        constexpr int S = decltype(Sc)::value, E = decltype(Ec)::value;
+        auto* k = hbm ? &k_list_planes<PR, S, E, false> : &k_list_planes<PR, S, E, true>;
+        if (lds > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(k, dim3((uint32_t)blocks), dim3(kListBlock), lds, s, p, n, list, marks, (T*)F, (const T*)Q, prev,
+                           next, g, (T)alfa, (T)beta, rho0);
+        return hipGetLastError();
+    };
+    auto by_stream = [&](auto pr) {
+        if (streaming != StreamEsotwist) return go(pr, IC<StreamSimple>{}, IC<1>{});  // plain addressing
+        return even ? go(pr, IC<StreamEsotwist>{}, IC<1>{}) : go(pr, IC<StreamEsotwist>{}, IC<0>{});
+    };
+    if (prec == 0) return by_stream(PrecF32{});
+    if (prec == 1) return by_stream(PrecF64{});
+    return hipErrorInvalidValue;
 }
 
 namespace {
 // fn(STREAM, MOMSRC, EVEN) with compile-time values (std::integral_constant)
-template <int V>
-using IC = std::integral_constant<int, V>;
 
 template <typename PR, int STREAM, typename Fn>
 hipError_t with_source(int momsrc, int even, Fn&& fn) {

@@ -10,6 +10,7 @@ import pytest
 import tdlbcpp_amd as td
 from oracle import oracle as O
 from tests.helpers import ReferenceLoop, flow_for_tank
+from tests.test_gpu_parity import LAYOUTS, STREAMS, random_points, seeded_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -100,3 +101,24 @@ def test_batch_levels_match_solo_runs(block, monkeypatch):
     batch.close()
     for cu in members:
         cu.close()
+
+
+# A caller's list: more points in a plane than a workgroup has lanes, one cell many times, stencils that meet
+# themselves, planes whose cells the LDS has no room for.
+@pytest.mark.parametrize("shape,n,same", [((8, 5, 7), 3000, 0), ((6, 3, 70), 600, 700), ((2, 3, 2), 60, 0),
+                                          ((200, 2, 200), 3000, 100)])
+@pytest.mark.parametrize("precision", [td.PREC_F32, td.PREC_F64], ids=["fp32", "fp64"])
+@pytest.mark.parametrize("stream", STREAMS, ids=["Simple", "Esotwist"])
+def test_forcing_of_a_list_matches_oracle(shape, n, same, precision, stream):
+    print(f"[gpu case] list of {n} + {same} points in {shape}, precision {precision}", flush=True)
+    for even in (True, False):
+        o, g = seeded_pair(LAYOUTS[0], stream, precision, False, shape=shape, seed=5, even=even)
+        rng = np.random.default_rng(6)
+        pts = random_points(rng, shape, n + same)
+        for axis in "ijk":
+            pts[axis][n // 2:n // 2 + same] = pts[axis][0]
+        for part in (pts, pts[::3].copy()):
+            o.forcing(part, 0.97, 1.9)
+            g.forcing(part, 0.97, 1.9)
+            np.testing.assert_array_equal(g.get(td.FIELD_F), o.get(O.FIELD_F))
+        g.close()
