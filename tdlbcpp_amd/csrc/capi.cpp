@@ -300,8 +300,7 @@ void level_shape(const Grid& g, const std::vector<PlaneDesc>& planes, const std:
     // static cells: moments and force values; blades: rows and moments of a plane's points and, if it fits, the
     // plane's force values
     const int64_t per = 7 * (int64_t)tsize, rows = blade_points * blade_row_bytes(tsize);
-    int64_t want = std::max(most * per, rows + plane_force_bytes(g, tsize));
-    if (want > (int64_t)kCuLdsBytes) want = std::min<int64_t>(std::max(most * per, rows), kCuLdsBytes);
+    const int64_t want = std::min<int64_t>(rows + std::max(most * per, plane_force_bytes(g, tsize)), kCuLdsBytes);
     set.level_lds = (int32_t)((want + 15) / 16 * 16);
     const int most_lanes = tsize > 4 ? level_block<double>() : level_block<float>();
     set.level_lanes = (int32_t)std::min<int64_t>(most_lanes, std::max<int64_t>(4 * wide[at], cells[at]) / 64 * 64 + 64);

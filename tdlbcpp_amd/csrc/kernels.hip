@@ -975,7 +975,8 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
 // many points then needed several workgroups meeting at barriers in HBM (24^3: 205
 // us).  Whole pass, gather and levels in one -> two launches: 24^3 205 -> 33 us,
 // 60^3 41 -> 29, 96^3 47 -> 37, 192^3 FP64 219 -> 132, 256^3 226 -> 166, 512^3
-// 597 -> 549 (gather 390, 5.1 TB/s of lines; levels 140).
+// 597 -> 549 (gather 390, 5.1 TB/s of lines; levels 140).  With rows asked for three
+// passes ahead (run_levels): 24^3 33 -> 31 us, 96^3 35 -> 32, 131^3 45 -> 42, 256^3 166 -> 158.
 
 // ---- A point of a plane task on a quad of lanes: lane c = 0..2 of the quad
 // takes stencil row k1 = c - 1 (cells s = 3c + m for i1 = m - 1), lane 3 repeats
@@ -1023,13 +1024,14 @@ template <typename T>
 __device__ __forceinline__ void force_row(const ForceRow<T>& r, const Mom4<T> (&mo)[3], T (&f)[3][3], T alfa, T beta) {
     T tr[3], tx[3], ty[3], tz[3];
 #pragma unroll
+    for (int m = 0; m < 3; m++) tr[m] = r.w[m] * mo[m].r;
+    const T rho = quad_sum(tr);
+#pragma unroll
     for (int m = 0; m < 3; m++) {
-        tr[m] = r.w[m] * mo[m].r;
         tx[m] = r.w[m] * add_half(mo[m].x, f[m][0]);
         ty[m] = r.w[m] * add_half(mo[m].y, f[m][1]);
         tz[m] = r.w[m] * add_half(mo[m].z, f[m][2]);
     }
-    const T rho = quad_sum(tr);
     T x = quad_sum(tx), y = quad_sum(ty), z = quad_sum(tz);
     x -= rho * quad_lane<0>(r.vel);
     y -= rho * quad_lane<1>(r.vel);
@@ -1075,12 +1077,6 @@ __global__ void k_static_rows(PointsDev p, int64_t n, const int32_t* __restrict_
 // share a stencil cell.  Blades at least 3 sqrt(2) cells apart at the inner
 // radius never share one either, so one level then takes all blades' points of a
 // radial class (5 levels, merged); in smaller tanks a level is one class.
-struct BladeLevel {
-    BladeEnum e;
-    int rmod, nr;        // radial class and its points per blade
-    int first, stride;   // blades first, first + stride, ...
-    int count;           // points of the level on one plane
-};
 __device__ __forceinline__ BladeEnum blade_enum_of(const BladeLayout& bl) {
     BladeEnum e;
     e.n_blades = bl.n_blades;
@@ -1089,16 +1085,11 @@ __device__ __forceinline__ BladeEnum blade_enum_of(const BladeLayout& bl) {
     e.n_bcol = bl.n_bcol;
     return e;
 }
-__device__ __forceinline__ BladeLevel blade_level(const BladeLayout& bl, int l) {
-    BladeLevel v;
-    v.e = blade_enum_of(bl);
-    v.rmod = l % 5;
-    v.nr = v.e.n_radial > v.rmod ? (v.e.n_radial - v.rmod + 4) / 5 : 0;
-    v.first = bl.merged ? 0 : l / 5;
-    v.stride = bl.merged ? 1 : v.e.n_bcol;
-    const int nb = v.e.n_blades > v.first ? (v.e.n_blades - v.first + v.stride - 1) / v.stride : 0;
-    v.count = nb * v.nr;
-    return v;
+// points of level l on one plane
+__device__ __forceinline__ int blade_level_count(const BladeLayout& bl, int l) {
+    const int rmod = l % 5, nr = bl.n_radial > rmod ? (bl.n_radial - rmod + 4) / 5 : 0;
+    const int first = bl.merged ? 0 : l / 5, stride = bl.merged ? 1 : bl.n_bcol;
+    return (bl.n_blades > first ? (bl.n_blades - first + stride - 1) / stride : 0) * nr;
 }
 // list index of radial point r of blade b on blade plane bp
 __device__ __forceinline__ int blade_index(const BladeEnum& e, int b, int r, int bp) {
@@ -1109,11 +1100,6 @@ __device__ __forceinline__ int blade_index(const BladeEnum& e, int b, int r, int
     before *= e.n_radial;
     for (int a = 0; a < rmod; a++) before += nb * (e.n_radial > a ? (e.n_radial - a + 4) / 5 : 0);
     return before * e.n_planes + (bi * e.n_planes + bp) * ((e.n_radial - rmod + 4) / 5) + r / 5;
-}
-// list index of point t of the level on blade plane bp
-__device__ __forceinline__ int level_index(const BladeLevel& v, int t, int bp) {
-    const int s = t / v.nr, ri = t - s * v.nr;
-    return blade_index(v.e, v.first + s * v.stride, v.rmod + 5 * ri, bp);
 }
 // position of radial point r of blade b among the plane's points in level order
 __device__ __forceinline__ int level_slot(const BladeLayout& bl, int b, int r) {
@@ -1182,13 +1168,15 @@ __device__ __forceinline__ void gather_blade_cell(const ForceGeom& fg, const Bla
         static_cast<T*>(fg.pts.v)[q] = (T)p.v_delta;
         static_cast<T*>(fg.pts.w)[q] = (T)p.w_delta;
     }
+    // the plane's points in the order of its levels, for contiguous reads there
+    const int64_t at = (int64_t)pl * be.n_blades * be.n_radial + level_slot(bl, b, r);
     if (s == 3 * c) {
         ForceRow<T> row = make_row<T>((T)p.i_frac, (T)p.k_frac, c,
                                       (T)(c == 0 ? p.u_delta : c == 1 ? p.v_delta : p.w_delta));
 #pragma unroll
         for (int m = 0; m < 3; m++)
             row.e[m] = (int32_t)cell_index(g, wrap_ik(i + m - 1, g.xg1), j, wrap_ik(k + c - 1, g.zg1));
-        static_cast<ForceRow<T>*>(fg.rows)[3 * q + c] = row;
+        static_cast<ForceRow<T>*>(fg.rows)[3 * (fg.n_static + at) + c] = row;
     }
     const int i2 = wrap_ik(i + (s - 3 * c) - 1, g.xg1), k2 = wrap_ik(k + c - 1, g.zg1);
     if (!mask_test(prev, g, i2, j, k2)) {
@@ -1199,7 +1187,7 @@ __device__ __forceinline__ void gather_blade_cell(const ForceGeom& fg, const Bla
     }
     Mom4<T> m;
     cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, i2, j, k2, m.r, m.x, m.y, m.z, rho0);
-    static_cast<Mom4<T>*>(fg.rcache)[9 * (int64_t)e + s] = m;
+    static_cast<Mom4<T>*>(fg.rcache)[9 * at + s] = m;
 }
 
 // Block b of a tank's gather: the blades' blocks first (their points cost the
@@ -1250,19 +1238,88 @@ __device__ __forceinline__ X uniform_copy(const X& x) {
     return __builtin_bit_cast(X, a);
 }
 
-// The plane's static levels, passes of a point per quad of lanes, with a barrier
-// after every level.  Rows are loaded two passes ahead and moments in HBM one
-// pass ahead: neither changes during the pass.  lm: the moments by entry of the
-// plane, in LDS (MOM_LDS) or the cache in HBM; the force values by entry: lf in
-// LDS (F_LDS), else four T an entry in the plane's scratch fs.  Loads return in
-// order, so in HBM a pass asks for its force values before the rows and moments
-// of later passes, and within a level for the next pass's before it stores its own.
+// The levels of a plane: passes of a point per quad of lanes, a barrier after every
+// level.  level_end(l): end of level l's points, called for l = 0, 1, ...; row_at(q):
+// the lane's stencil row of point q; mom_at(q, row, m): its moments; get and
+// put(row, f): its force values.  A turn of the loop is one pass.  Rows are asked
+// for three passes ahead and moments one, since neither changes meanwhile.  The
+// turn is written out for each place of the ring of rows: with rows moved from one
+// variable to the next, every move waited for the row in flight (24^3: 0.72 us a
+// level, now 0.55, which is the instruction stream of one wavefront per SIMD).
+// Rows in HBM are asked for by every lane, without a branch (a lane without a point
+// takes the level's last): past a branch that may have skipped loads the compiler
+// waits for all of them.  Loads return in order, so in HBM a pass asks for its force
+// values before the moments and rows of later passes, and within a level for the
+// next pass's before it stores its own.
+template <typename T, bool ROWS_LDS, bool F_LDS, typename End, typename RowAt, typename MomAt, typename Get, typename Put>
+__device__ __forceinline__ void run_levels(int nlev, T alfa, T beta, End&& level_end, RowAt&& row_at, MomAt&& mom_at,
+                                           Get&& get, Put&& put) {
+    const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), per = (int)(blockDim.x >> 2);
+    struct Pass {
+        int l;       // level, nlev after the last
+        int q, end;  // first point, end of the level
+    };
+    auto next = [&](Pass a) {
+        if (a.q + per < a.end) return Pass{a.l, a.q + per, a.end};
+        int l = a.l + 1;
+        for (; l < nlev; l++) {
+            const int end = level_end(l);
+            if (end > a.end) return Pass{l, a.end, end};
+        }
+        return Pass{l, a.end, a.end};
+    };
+    auto on = [&](const Pass& a) { return a.q + slot < a.end; };
+    ForceRow<T> r0, r1, r2, r3;
+    Mom4<T> m0[3], m1[3];
+    T f0[3][3], f1[3][3];
+    Pass a0 = next(Pass{-1, 0, 0}), a1 = next(a0), a2 = next(a1);
+    if (a0.l >= nlev) return;
+    auto load = [&](ForceRow<T>& r, const Pass& a) {
+        if (!ROWS_LDS) r = row_at(min(a.q + slot, a.end - 1));
+        else if (on(a)) r = row_at(a.q + slot);
+    };
+    load(r0, a0);
+    load(r1, a1);
+    load(r2, a2);
+    if (on(a0)) mom_at(a0.q + slot, r0, m0);
+    bool have = false;  // the pass's force values were asked for in the pass before
+    // this pass, the next and the one three ahead
+    auto turn = [&](ForceRow<T>& cr, ForceRow<T>& nr, ForceRow<T>& ar, Mom4<T> (&cm)[3], Mom4<T> (&nm)[3],
+                    T (&cf)[3][3], T (&nf)[3][3]) {
+        const bool on0 = on(a0), on1 = on(a1), same = a1.l == a0.l;
+        if ((F_LDS || !have) && on0) get(cr, cf);
+        if (!F_LDS && same && on1) get(nr, nf);
+        if (on1) mom_at(a1.q + slot, nr, nm);
+        const Pass a3 = next(a2);
+        __builtin_amdgcn_sched_barrier(0);  // the row behind them: no wait for moments or forces includes it
+        load(ar, a3);
+        if (on0) {
+            force_row(cr, cm, cf, alfa, beta);
+            if (lane < 3) put(cr, cf);
+        }
+        if (!same) __syncthreads();
+        a0 = a1;
+        a1 = a2;
+        a2 = a3;
+        have = same;
+        return a0.l < nlev;
+    };
+    for (;;) {
+        if (!turn(r0, r1, r3, m0, m1, f0, f1)) break;
+        if (!turn(r1, r2, r0, m1, m0, f1, f0)) break;
+        if (!turn(r2, r3, r1, m0, m1, f0, f1)) break;
+        if (!turn(r3, r0, r2, m1, m0, f1, f0)) break;
+    }
+}
+
+// Static levels.  lm: the moments by entry of the plane, in LDS (MOM_LDS) or the
+// cache in HBM; the force values by entry: lf in LDS (F_LDS), else four T an entry
+// in the plane's scratch fs.
 template <typename T, bool MOM_LDS, bool F_LDS>
 __device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDesc& pd, const Mom4<T>* lm, T* lf,
                                               Mom4<T>* fs, T alfa, T beta) {
-    const ForceRow<T>* rows = static_cast<const ForceRow<T>*>(fg.rows);
-    const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), c = min(lane, 2);
-    const int per = (int)(blockDim.x >> 2), nlev = pd.n_levels;
+    const int c = min((int)(threadIdx.x & 3), 2), nlev = pd.n_levels;
+    if (nlev == 0) return;
     // Level ends without a load in the loop, whose wait would include every load
     // before it: lane i of the wave holds the end of level base + i.
     const int64_t* off = fg.lev_off + pd.lev;
@@ -1272,102 +1329,44 @@ __device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDe
         base = l;
         ends = (int)(off[min(l + (int)(threadIdx.x & 63), nlev - 1) + 1] - q0);
     };
-    auto level_end = [&](int l) {
-        if (l - base >= 64) hold(l);
-        return __builtin_amdgcn_readlane(ends, l - base);
-    };
-    if (nlev > 0) hold(0);
-    rows += 3 * q0;
-    struct Pass {
-        int l;       // level, nlev after the last
-        int q, end;  // first point, end of the level
-    };
-    auto next = [&](Pass a) {
-        if (a.l >= nlev) return a;
-        if (a.q + per < a.end) return Pass{a.l, a.q + per, a.end};
-        return Pass{a.l + 1, a.end, a.l + 1 < nlev ? level_end(a.l + 1) : a.end};
-    };
-    struct Row {
-        ForceRow<T> r;
-        Mom4<T> mo[MOM_LDS ? 1 : 3];
-        bool ok;
-    };
-    auto load = [&](Pass a) {
-        Row x{};
-        x.ok = a.l < nlev && a.q + slot < a.end;
-        if (x.ok) x.r = rows[3 * (int64_t)(a.q + slot) + c];
-        return x;
-    };
-    auto complete = [&](Row& x) {
-        if constexpr (!MOM_LDS)
-            if (x.ok)
+    hold(0);
+    const ForceRow<T>* rows = static_cast<const ForceRow<T>*>(fg.rows) + 3 * q0 + c;
+    run_levels<T, false, F_LDS>(
+        nlev, alfa, beta,
+        [&](int l) {
+            if (l - base >= 64) hold(l);
+            return __builtin_amdgcn_readlane(ends, l - base);
+        },
+        [&](int q) { return rows[3 * (int64_t)q]; },
+        [&](int, const ForceRow<T>& r, Mom4<T> (&m)[3]) {
 #pragma unroll
-                for (int m = 0; m < 3; m++) x.mo[m] = lm[x.r.e[m]];
-    };
-    struct Force {
-        T f[3][3];
-    };
-    auto fetch = [&](const Row& x, Force& v) {
-        if (!x.ok) return;
+            for (int b = 0; b < 3; b++) m[b] = lm[r.e[b]];
+        },
+        [&](const ForceRow<T>& r, T (&f)[3][3]) {
 #pragma unroll
-        for (int m = 0; m < 3; m++) {
-            const int e = x.r.e[m];
-            if constexpr (F_LDS) {
+            for (int b = 0; b < 3; b++) {
+                if constexpr (F_LDS) {
 #pragma unroll
-                for (int a = 0; a < 3; a++) v.f[m][a] = lf[3 * e + a];
-            } else {
-                const Mom4<T> w = fs[e];
-                v.f[m][0] = w.r;
-                v.f[m][1] = w.x;
-                v.f[m][2] = w.y;
-            }
-        }
-    };
-    Pass a0{0, 0, nlev > 0 ? level_end(0) : 0}, a1 = next(a0);
-    Row r0 = load(a0), r1 = load(a1);
-    complete(r0);
-    Force v0{}, v1{};
-    bool have = false;  // v0 was asked for in the pass before
-    while (a0.l < nlev) {
-        if (F_LDS || !have) fetch(r0, v0);
-        const Pass a2 = next(a1);
-        const bool same = a1.l == a0.l;
-        if constexpr (!F_LDS) {
-            if (same) fetch(r1, v1);
-        }
-        complete(r1);
-        __builtin_amdgcn_sched_barrier(0);  // the rows behind them: no wait for moments or forces includes theirs
-        Row r2 = load(a2);
-        if (r0.ok) {
-            Mom4<T> mo[3];
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                if constexpr (MOM_LDS) mo[m] = lm[r0.r.e[m]];
-                else mo[m] = r0.mo[m];
-            }
-            force_row(r0.r, mo, v0.f, alfa, beta);
-            if (lane < 3)
-#pragma unroll
-                for (int m = 0; m < 3; m++) {
-                    const int e = r0.r.e[m];
-                    if constexpr (F_LDS) {
-#pragma unroll
-                        for (int a = 0; a < 3; a++) lf[3 * e + a] = v0.f[m][a];
-                    } else {
-                        fs[e] = Mom4<T>{v0.f[m][0], v0.f[m][1], v0.f[m][2], T(0)};
-                    }
+                    for (int a = 0; a < 3; a++) f[b][a] = lf[3 * r.e[b] + a];
+                } else {
+                    const Mom4<T> w = fs[r.e[b]];
+                    f[b][0] = w.r;
+                    f[b][1] = w.x;
+                    f[b][2] = w.y;
                 }
-        }
-        if (!same) __syncthreads();
-        a0 = a1;
-        a1 = a2;
-        r0 = r1;
-        r1 = r2;
-        if constexpr (!F_LDS) {
-            v0 = v1;
-            have = same;
-        }
-    }
+            }
+        },
+        [&](const ForceRow<T>& r, const T (&f)[3][3]) {
+#pragma unroll
+            for (int b = 0; b < 3; b++) {
+                if constexpr (F_LDS) {
+#pragma unroll
+                    for (int a = 0; a < 3; a++) lf[3 * r.e[b] + a] = f[b][a];
+                } else {
+                    fs[r.e[b]] = Mom4<T>{f[b][0], f[b][1], f[b][2], T(0)};
+                }
+            }
+        });
 }
 
 // cell n of plane j in the plane's own (i, k) order
@@ -1377,106 +1376,103 @@ __device__ __forceinline__ int plane_index(const Grid& g, uint32_t n, int j) {
 }
 
 // The blade levels of a plane.  With room in LDS the rows and moments of all its
-// points come there first, in level order, and if a copy of the whole plane's
-// force values fits beside them the stencil cells' too: a level then waits on
-// LDS alone (1.7 us a level from the caches, most of it the latency of the next
-// rows).  Otherwise the force values stay in F, and without any room the rows and
-// moments in the caches.
+// points come there first (blade_rows), and if a copy of the whole plane's force
+// values fits beside them the stencil cells' too: a level then waits on LDS alone.
+// Otherwise the force values stay in F, and without any room the rows and moments
+// in the caches.
 template <typename T>
 struct BladeRow {
     ForceRow<T> r;
     Mom4<T> mo[3];
 };
 static_assert(3 * sizeof(BladeRow<float>) == blade_row_bytes(4) && 3 * sizeof(BladeRow<double>) == blade_row_bytes(8), "LDS");
+
+// rows and moments of blade plane bp to LDS
+template <typename T>
+__device__ __forceinline__ void blade_rows(const ForceGeom& fg, int bp, BladeRow<T>* lr) {
+    const int n3 = 3 * fg.blade.n_blades * fg.blade.n_radial;
+    const ForceRow<T>* __restrict__ rows = static_cast<const ForceRow<T>*>(fg.rows) + 3 * fg.n_static + (int64_t)bp * n3;
+    const Mom4<T>* __restrict__ cache = static_cast<const Mom4<T>*>(fg.rcache) + (int64_t)bp * n3 * 3;
+    for (int t = (int)threadIdx.x; t < n3; t += (int)blockDim.x) {
+        const ForceRow<T> r = rows[t];
+        const Mom4<T> a = cache[3 * t], b = cache[3 * t + 1], c = cache[3 * t + 2];
+        lr[t].r = r;
+        lr[t].mo[0] = a;
+        lr[t].mo[1] = b;
+        lr[t].mo[2] = c;
+    }
+}
+
+// lr: the plane's rows, in LDS already (ROWS_LDS); ld: room for its force values (F_LDS)
 template <typename T, bool ROWS_LDS, bool F_LDS>
 __device__ __forceinline__ void blade_levels(const ForceGeom& fg, const Grid& g, int j, int bp, int nlev,
                                              T* __restrict__ F, uint64_t* __restrict__ next, BladeRow<T>* lr, T* ld,
                                              T alfa, T beta) {
-    const ForceRow<T>* __restrict__ rows = static_cast<const ForceRow<T>*>(fg.rows) + 3 * fg.n_static;
-    const Mom4<T>* __restrict__ cache = static_cast<const Mom4<T>*>(fg.rcache);
-    const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), c = min(lane, 2);
-    const int per = (int)(blockDim.x >> 2);
-    // the occupancy bits of the rows' cells, and what the levels need in LDS, rows in level order
-    const BladeEnum be = blade_enum_of(fg.blade);
-    const int n3 = 3 * be.n_blades * be.n_radial;
+    const int c = min((int)(threadIdx.x & 3), 2), n3 = 3 * fg.blade.n_blades * fg.blade.n_radial;
+    const ForceRow<T>* __restrict__ rows = static_cast<const ForceRow<T>*>(fg.rows) + 3 * fg.n_static + (int64_t)bp * n3;
+    const Mom4<T>* __restrict__ cache = static_cast<const Mom4<T>*>(fg.rcache) + (int64_t)bp * n3 * 3;
+    // the occupancy bits of the rows' cells, and the cells' force values
     for (int t = (int)threadIdx.x; t < n3; t += (int)blockDim.x) {
-        const int pt = t / 3, row = t - 3 * pt, b = pt / be.n_radial, r = pt - b * be.n_radial;
-        const int64_t e = blade_index(be, b, r, bp);
-        BladeRow<T> x;
-        x.r = rows[3 * e + row];
-        if constexpr (ROWS_LDS)
-#pragma unroll
-            for (int m = 0; m < 3; m++) x.mo[m] = cache[9 * e + 3 * row + m];
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            const uint32_t n = (uint32_t)x.r.e[m];
+            const uint32_t n = (uint32_t)(ROWS_LDS ? lr[t].r.e[m] : rows[t].e[m]);
             const int i = (int)(n / g.yz), k = (int)(n - (uint32_t)i * g.yz - (uint32_t)j * (uint32_t)g.zg);
-            atomicOr((unsigned long long*)&next[mask_word_index(g, i, j, k)], 1ull << (k & 63));
             if constexpr (F_LDS) {
-                x.r.e[m] = (i - 1) * g.zg1 + k - 1;
+                const int e = (i - 1) * g.zg1 + k - 1;
+                lr[t].r.e[m] = e;
 #pragma unroll
-                for (int a = 0; a < 3; a++) ld[3 * x.r.e[m] + a] = F[3 * (uint64_t)n + a];
+                for (int a = 0; a < 3; a++) ld[3 * e + a] = F[3 * (uint64_t)n + a];
             }
+            atomicOr((unsigned long long*)&next[mask_word_index(g, i, j, k)], 1ull << (k & 63));
         }
-        if constexpr (ROWS_LDS) lr[3 * level_slot(fg.blade, b, r) + row] = x;
     }
-    if constexpr (ROWS_LDS) __syncthreads();
-    struct Pass {
-        ForceRow<T> r;
-        Mom4<T> mo[3];
-        bool ok;
-    };
-    auto load = [&](int l, int at, int t) {
-        Pass a{};
-        if (l >= nlev) return a;
-        const BladeLevel v = blade_level(fg.blade, l);
-        a.ok = t < v.count;
-        if (a.ok) {
-            if constexpr (ROWS_LDS) {
-                const BladeRow<T>& x = lr[3 * (at + t) + c];
-                a.r = x.r;
-#pragma unroll
-                for (int m = 0; m < 3; m++) a.mo[m] = x.mo[m];
-            } else {
-                const int64_t e = level_index(v, t, bp);
-                a.r = rows[3 * e + c];
-#pragma unroll
-                for (int m = 0; m < 3; m++) a.mo[m] = cache[9 * e + 3 * c + m];
-            }
-        }
-        return a;
-    };
-    for (int l = 0, at = 0; l < nlev; l++) {
-        const int count = blade_level(fg.blade, l).count;  // 0 with fewer than 5 radial points
-        for (int u = 0; u < count; u += per) {
-            const Pass cur = load(l, at, u + slot);
-            if (cur.ok) {
-                T f[3][3];
-                uint64_t p[3];
-#pragma unroll
-                for (int m = 0; m < 3; m++) {
-                    p[m] = 3 * (uint64_t)(uint32_t)cur.r.e[m];
-#pragma unroll
-                    for (int a = 0; a < 3; a++) f[m][a] = F_LDS ? ld[(int)p[m] + a] : F[p[m] + a];
+    if constexpr (F_LDS) __syncthreads();
+    // lane i of the wave holds the end of level base + i (of the first 64, then the next)
+    int base = -64, ends = 0;
+    run_levels<T, ROWS_LDS, F_LDS>(
+        nlev, alfa, beta,
+        [&](int l) {
+            if (l - base >= 64) {
+                const int before = base < 0 ? 0 : __builtin_amdgcn_readlane(ends, 63), at = (int)(threadIdx.x & 63);
+                base += 64;
+                ends = base + at < nlev ? blade_level_count(fg.blade, base + at) : 0;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int up = __shfl_up(ends, o, 64);
+                    if (at >= o) ends += up;
                 }
-                force_row(cur.r, cur.mo, f, alfa, beta);
-                if (lane < 3)
-#pragma unroll
-                    for (int m = 0; m < 3; m++)
-#pragma unroll
-                        for (int a = 0; a < 3; a++) {
-                            if constexpr (F_LDS) ld[(int)p[m] + a] = f[m][a];
-                            else F[p[m] + a] = f[m][a];
-                        }
+                ends += before;
             }
-        }
-        if (count > 0) __syncthreads();
-        at += count;
-    }
+            return __builtin_amdgcn_readlane(ends, l - base);
+        },
+        [&](int q) {
+            if constexpr (ROWS_LDS) return lr[3 * q + c].r;
+            else return rows[3 * q + c];
+        },
+        [&](int q, const ForceRow<T>&, Mom4<T> (&m)[3]) {
+#pragma unroll
+            for (int b = 0; b < 3; b++) {
+                if constexpr (ROWS_LDS) m[b] = lr[3 * q + c].mo[b];
+                else m[b] = cache[3 * (3 * q + c) + b];
+            }
+        },
+        [&](const ForceRow<T>& r, T (&f)[3][3]) {
+#pragma unroll
+            for (int b = 0; b < 3; b++)
+#pragma unroll
+                for (int a = 0; a < 3; a++) f[b][a] = F_LDS ? ld[3 * r.e[b] + a] : F[3 * (uint64_t)(uint32_t)r.e[b] + a];
+        },
+        [&](const ForceRow<T>& r, const T (&f)[3][3]) {
+#pragma unroll
+            for (int b = 0; b < 3; b++)
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    if constexpr (F_LDS) ld[3 * r.e[b] + a] = f[b][a];
+                    else F[3 * (uint64_t)(uint32_t)r.e[b] + a] = f[b][a];
+                }
+        });
     if constexpr (F_LDS) {
         // back to F, once per point and cell: points that share a cell write the same value
-        const int n9 = 9 * fg.blade.n_blades * fg.blade.n_radial;
-        for (int t = (int)threadIdx.x; t < n9; t += (int)blockDim.x) {
+        for (int t = (int)threadIdx.x; t < 3 * n3; t += (int)blockDim.x) {
             const int pr = t / 3, p = lr[pr].r.e[t - 3 * pr];
             const int i = p / g.zg1, k = p - i * g.zg1;
             const uint64_t n = cell_index(g, i + 1, j, k + 1);
@@ -1498,6 +1494,19 @@ __device__ __forceinline__ void plane_levels(const ForceGeom& fg, const PlaneDes
     const int tid = (int)threadIdx.x, nt = (int)blockDim.x, nc = (int)(pd.cell_end - pd.cell_begin);
     const int64_t mom_bytes = (int64_t)nc * sizeof(Mom4<T>), f_bytes = (int64_t)nc * 3 * sizeof(T);
     const bool f_lds = f_bytes <= lds_bytes, mom_lds = mom_bytes + f_bytes <= lds_bytes;
+    // The blades' rows come at the start if they fit beside what the static levels
+    // keep: after them the wait for the rows was 1 to 2 us of a plane's 20.
+    int nlev;
+    const int bp = blade_plane(fg, pd.j, nlev);
+    const bool blades = nlev > 0 && pd.blades;
+    const int64_t row_bytes = 3 * (int64_t)fg.blade.n_blades * fg.blade.n_radial * sizeof(BladeRow<T>);
+    const bool early = blades && row_bytes + (mom_lds ? mom_bytes + f_bytes : f_lds ? f_bytes : 0) <= lds_bytes;
+    auto* const lr = static_cast<BladeRow<T>*>(lds);
+    auto* const ld = reinterpret_cast<T*>(static_cast<char*>(lds) + row_bytes);
+    if (early) {
+        blade_rows(fg, bp, lr);
+        lds = ld;
+    }
     const auto* gm = static_cast<const Mom4<T>*>(fg.scache) + pd.cell_begin;
     auto* fs = static_cast<Mom4<T>*>(fg.fscr) + pd.cell_begin;
     auto* lm = static_cast<Mom4<T>*>(lds);
@@ -1531,17 +1540,17 @@ __device__ __forceinline__ void plane_levels(const ForceGeom& fg, const PlaneDes
             F[3 * n + 2] = v.y;
         }
     }
-    int nlev;
-    const int bp = blade_plane(fg, pd.j, nlev);
-    if (nlev == 0 || !pd.blades) return;
+    if (!blades) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const int64_t row_bytes = 3 * (int64_t)fg.blade.n_blades * fg.blade.n_radial * sizeof(BladeRow<T>);
-    auto* lr = static_cast<BladeRow<T>*>(lds);
-    T* ld = reinterpret_cast<T*>(static_cast<char*>(lds) + row_bytes);
+    const bool rows_lds = row_bytes <= lds_bytes;
+    if (rows_lds && !early) {
+        blade_rows(fg, bp, lr);
+        __syncthreads();
+    }
     if (row_bytes + plane_force_bytes(g, sizeof(T)) <= lds_bytes)
         blade_levels<T, true, true>(fg, g, pd.j, bp, nlev, F, next, lr, ld, alfa, beta);
-    else if (row_bytes <= lds_bytes)
+    else if (rows_lds)
         blade_levels<T, true, false>(fg, g, pd.j, bp, nlev, F, next, lr, nullptr, alfa, beta);
     else blade_levels<T, false, false>(fg, g, pd.j, bp, nlev, F, next, nullptr, nullptr, alfa, beta);
 }
