@@ -236,6 +236,23 @@ __global__ void k_copy_bytes(uint8_t* __restrict__ d, const uint8_t* __restrict_
         d[a] = s[a];
 }
 
+// A block takes consecutive cells of one interior i plane, rows back to back, so
+// only the plane's last block has lanes without a cell.
+constexpr int kFlatBlock = 256;
+struct FlatTile {
+    uint32_t blocks;  // of an i plane
+    uint32_t recip;   // ceil(2^32 / zg1): the high word of r * recip is r / zg1 while yg1 * zg1 * zg1 < 2^32
+};
+__device__ __forceinline__ bool flat_cell(const Grid& g, const FlatTile& tile, int& i, int& j, int& k) {
+    const uint32_t ip = blockIdx.x / tile.blocks, r = (blockIdx.x - ip * tile.blocks) * blockDim.x + threadIdx.x;
+    if (r >= (uint32_t)g.yg1 * (uint32_t)g.zg1) return false;
+    const uint32_t jp = __umulhi(r, tile.recip);
+    i = (int)ip + 1;
+    j = (int)jp + 1;
+    k = (int)(r - jp * (uint32_t)g.zg1) + 1;
+    return true;
+}
+
 // ------------------------------------------------------------------ Esotwist
 // Direction d of cell c is stored at home(c,d) = c + (1 where e_d < 0, periodic
 // on the interior), in slot d at even parity and opp(d) at odd parity.  read
@@ -342,6 +359,18 @@ __global__ __launch_bounds__(kRowBlock) void k_esotwist(typename PR::S* __restri
     esotwist_cell<PR, MODE, EVEN, HINT>(Q, mout, F, Nu, fmask, g, P, rho0, rb.i, rb.j, k);
 }
 
+// Fused step over the cells of an i plane back to back (flat_tile)
+template <typename PR, int EVEN>
+__global__ __launch_bounds__(kFlatBlock) void k_esotwist_flat(typename PR::S* __restrict__ Q,
+                                                              const typename PR::T* __restrict__ F,
+                                                              typename PR::N* __restrict__ Nu,
+                                                              const uint64_t* __restrict__ fmask, Grid g,
+                                                              CollideParams<typename PR::T> P, FlatTile tile, float rho0) {
+    int i, j, k;
+    if (!flat_cell(g, tile, i, j, k)) return;
+    esotwist_cell<PR, MODE_FUSED, EVEN>(Q, nullptr, F, Nu, fmask, g, P, rho0, i, j, k);
+}
+
 // ------------------------------------------------------------------ Simple
 // In-place collide / moments, or pull from src (the two-lattice form of the
 // reference's in-place push: slot d of an interior cell c takes src[c-e_d][d]
@@ -425,6 +454,17 @@ __global__ __launch_bounds__(kRowBlock) void k_simple(const typename PR::S* src,
     const int k = rb.k0 + (int)threadIdx.x;
     if (k > g.zg1) return;
     simple_cell<PR, MODE>(src, dst, mout, F, Nu, fmask, g, P, rho0, rb.i, rb.j, k);
+}
+
+template <typename PR>
+__global__ __launch_bounds__(kFlatBlock) void k_simple_flat(const typename PR::S* src, typename PR::S* dst,
+                                                            const typename PR::T* __restrict__ F,
+                                                            typename PR::N* __restrict__ Nu,
+                                                            const uint64_t* __restrict__ fmask, Grid g,
+                                                            CollideParams<typename PR::T> P, FlatTile tile, float rho0) {
+    int i, j, k;
+    if (!flat_cell(g, tile, i, j, k)) return;
+    simple_cell<PR, MODE_FUSED>(src, dst, nullptr, F, Nu, fmask, g, P, rho0, i, j, k);
 }
 
 // ------------------------------------------------------------------ data movement on every cell
@@ -2041,6 +2081,35 @@ inline void row_launch(const Grid& g, uint32_t& nkb, uint32_t& nblocks, uint32_t
     nblocks = nkb * (uint32_t)g.yg1 * (uint32_t)g.xg1;
 }
 
+// Rows of k that are not whole wavefronts leave lanes idle (131: 192 lanes a row);
+// over the cells of a plane back to back nearly none are, at the price of a
+// division and its own j per lane.  The line, from both mappings at 56 edges from
+// 24 to 448 (stream-collide, us, rows -> flat):
+//   rows that waste a tenth of their lanes or more gain while the memory does not
+//   bound the step: FP32 70^3 22 -> 17, 131^3 79 -> 71, 270^3 636 -> 617, 330^3 1150
+//   -> 1113 but Simple 1231 -> 1235; FP16 70^3 18 -> 14, 131^3 49 -> 40, 270^3 343 ->
+//   334, 330^3 Simple 686 -> 697: below 2^25 cells.  FP64 131^3 137 -> 128, but 170^3
+//   285 -> 290, and rows within a wavefront 36^3 12.0 -> 12.4: 65 to 2^22 cells;
+//   16-bit storage is bound by its arithmetic and gains with any idle lane (60^3 15.1
+//   -> 13.7, 120^3 35 -> 33) up to 2^22 cells (184^3 122 -> 122);
+//   rows of whole lines keep their streaming hints (hints: 224^3 FP32 292 against 337
+//   flat, 144^3 FP64 154 against 172), but for small lattices (96^3 FP32 34.6 -> 30.7).
+bool flat_tile(const Grid& g, size_t ssize, bool hints, FlatTile& tile, uint32_t& nblocks, uint32_t& bk) {
+    const uint64_t row = (uint64_t)g.zg1, lanes = (row + 63) / 64 * 64, plane = row * (uint64_t)g.yg1;
+    const uint64_t cells = plane * (uint64_t)g.xg1;
+    if (row < 2 || row == lanes || plane * row >= (1ull << 32) || (hints && cells >= (1ull << 20))) return false;
+    const bool waste = 10 * row <= 9 * lanes;
+    const bool gains = ssize > 4   ? waste && row > 64 && cells < (1ull << 22)
+                       : ssize < 4 ? cells < (1ull << 22) || (waste && cells < (1ull << 25))
+                                   : waste && cells < (1ull << 25);
+    if (!gains) return false;
+    bk = kFlatBlock;
+    tile.blocks = (uint32_t)((plane + bk - 1) / bk);
+    tile.recip = (uint32_t)(((1ull << 32) + row - 1) / row);
+    nblocks = tile.blocks * (uint32_t)g.xg1;
+    return true;
+}
+
 template <typename PR>
 hipError_t esotwist_t(int mode, int even, void* Q, void* mout, const void* F, void* Nu, const uint64_t* fm,
                       const Grid& g, const CollideArgs& c, float rho0, hipStream_t s) {
@@ -2058,6 +2127,12 @@ hipError_t esotwist_t(int mode, int even, void* Q, void* mout, const void* F, vo
     if (mode == MODE_COLL) { if (even) TDLB_ESO(MODE_COLL, 1, false); else TDLB_ESO(MODE_COLL, 0, false); }
     else if (mode == MODE_MOM) { if (even) TDLB_ESO(MODE_MOM, 1, false); else TDLB_ESO(MODE_MOM, 0, false); }
     else if (mode == MODE_FUSED) {
+        FlatTile tile;
+        if (flat_tile(g, sizeof(S), line_rows<S>(g), tile, nb, bk)) {
+            auto* k = even ? &k_esotwist_flat<PR, 1> : &k_esotwist_flat<PR, 0>;
+            hipLaunchKernelGGL(k, dim3(nb), dim3(bk), 0, s, q, f, nu, fm, g, P, tile, rho0);
+            return hipGetLastError();
+        }
         if (line_rows<S>(g)) {
             if (even) TDLB_ESO(MODE_FUSED, 1, true); else TDLB_ESO(MODE_FUSED, 0, true);
             return hipGetLastError();
@@ -2087,7 +2162,13 @@ hipError_t simple_t(int mode, const void* src, void* dst, void* mout, const void
     switch (mode) {
         case MODE_COLL: TDLB_SIM(MODE_COLL); break;
         case MODE_MOM: TDLB_SIM(MODE_MOM); break;
-        case MODE_FUSED: TDLB_SIM(MODE_FUSED); break;
+        case MODE_FUSED: {
+            FlatTile tile;
+            if (flat_tile(g, sizeof(S), false, tile, nb, bk))
+                hipLaunchKernelGGL(k_simple_flat<PR>, dim3(nb), dim3(bk), 0, s, a, b, f, nu, fm, g, P, tile, rho0);
+            else TDLB_SIM(MODE_FUSED);
+            break;
+        }
         case MODE_MOM_PULL: TDLB_SIM(MODE_MOM_PULL); break;
         default: return hipErrorInvalidValue;
     }

@@ -5,6 +5,8 @@ import numpy as np
 import pytest
 
 import tdlbcpp_amd as td
+from oracle import oracle as O
+from tests.test_gpu_forcing import compare
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +60,14 @@ def test_results_read_by_several_threads_at_once():
             assert all(np.array_equal(x, y) for x, y in zip(a, r))
     for cu in cus:
         cu.close()
+
+
+# Rows that end inside a wavefront: the fused step takes the cells of a plane back to back (a row of one
+# cell more than a wavefront, of an odd size, and FP64 rows within one wavefront, which stay rows).
+@pytest.mark.parametrize("T", [30, 65, 71, 116])
+@pytest.mark.parametrize("precision", [td.PREC_F32, td.PREC_F64], ids=["fp32", "fp64"])
+@pytest.mark.parametrize("streaming", [(td.STREAM_ESOTWIST, O.ESOTWIST), (td.STREAM_SIMPLE, O.SIMPLE)],
+                         ids=["Esotwist", "Simple"])
+def test_rows_ending_inside_a_wavefront_match_oracle(T, precision, streaming):
+    print(f"[gpu case] rows of {T}, precision {precision}", flush=True)
+    compare(T, 3, precision, streaming=streaming)
