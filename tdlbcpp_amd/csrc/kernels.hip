@@ -815,8 +815,9 @@ struct alignas(4 * sizeof(T)) Mom4 {
 // (Forcing.hpp:73-135) and make room for the next.  They share no cell, and no
 // earlier point is unfinished on theirs, so every cell sees its points in list
 // order.  The rounds are bound by the latency of a point's loads.  A call over the
-// 13,431 points of a 60^3 tank: 0.29 ms, the kernel 110 us of them; with levels from
-// a hash map on the host and a launch per level 8.5 ms.
+// 13,431 points of a 60^3 tank: 0.12 to 0.28 ms, the kernel 77 us of them (115 with
+// the points' moments read when they run); with levels from a hash map on the host
+// and a launch per level 8.5 ms.
 template <typename T>
 __global__ void k_list_unpack(const tdlb_ib_point* __restrict__ in, int64_t n, int ghost, PointsDev p,
                               const uint64_t* __restrict__ base, uint64_t* __restrict__ next, uint64_t words) {
@@ -836,62 +837,77 @@ __global__ void k_list_unpack(const tdlb_ib_point* __restrict__ in, int64_t n, i
     }
 }
 
-// gather, correct and spread of point q, all nine cells by one lane, from stored moments
+// A point in a lane's registers with everything the forcing does not change: the
+// moments of its nine cells are asked for when the lane takes it, rounds before use.
+template <typename T>
+struct ListPoint {
+    T wx[3], wz[3], vel[3];
+    T rho[9], jx[9], jy[9], jz[9];
+    uint32_t at[9];  // cell indices
+};
+
 template <typename PR, int STREAM, int EVEN>
-__device__ __forceinline__ void list_point(const PointsDev& p, int64_t q, typename PR::T* __restrict__ F,
-                                           const typename PR::S* __restrict__ Q, const Grid& g,
-                                           typename PR::T alfa, typename PR::T beta, float rho0) {
+__device__ __forceinline__ void list_take(ListPoint<typename PR::T>& a, const PointsDev& p, int64_t q, int pi, int pk,
+                                          int pj, const typename PR::S* __restrict__ Q, const Grid& g, float rho0) {
     using T = typename PR::T;
-    using D = typename PR::D;
-    const int pi = p.i[q], pj = p.j[q], pk = p.k[q];
     const T ifr = static_cast<const T*>(p.ifrac)[q], kfr = static_cast<const T*>(p.kfrac)[q];
-    T wx[3], wz[3];
-    uint64_t at[9];
-    T f[9][3];
+    a.vel[0] = static_cast<const T*>(p.u)[q];
+    a.vel[1] = static_cast<const T*>(p.v)[q];
+    a.vel[2] = static_cast<const T*>(p.w)[q];
 #pragma unroll
     for (int s = 0; s < 9; s++) {
-        at[s] = 3ull * cell_index(g, wrap_ik(pi + s % 3 - 1, g.xg1), pj, wrap_ik(pk + s / 3 - 1, g.zg1));
-#pragma unroll
-        for (int d = 0; d < 3; d++) f[s][d] = F[at[s] + d];
+        const int i2 = wrap_ik(pi + s % 3 - 1, g.xg1), k2 = wrap_ik(pk + s / 3 - 1, g.zg1);
+        a.at[s] = cell_index(g, i2, pj, k2);
+        cell_rho_j<PR, STREAM, MOMSRC_STORED, EVEN>(Q, g, i2, pj, k2, a.rho[s], a.jx[s], a.jy[s], a.jz[s], rho0);
     }
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        wx[a] = ib_weight<T>(-ifr + T(a - 1));
-        wz[a] = ib_weight<T>(-kfr + T(a - 1));
+    for (int b = 0; b < 3; b++) {
+        a.wx[b] = ib_weight<T>(-ifr + T(b - 1));
+        a.wz[b] = ib_weight<T>(-kfr + T(b - 1));
     }
+}
+
+// gather, correct and spread of a point, all nine cells by one lane
+template <typename PR>
+__device__ __forceinline__ void list_point(const ListPoint<typename PR::T>& a, typename PR::T* __restrict__ F,
+                                           typename PR::T alfa, typename PR::T beta, bool meets) {
+    using T = typename PR::T;
+    using D = typename PR::D;
+    T f[9][3];
+#pragma unroll
+    for (int s = 0; s < 9; s++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) f[s][d] = F[3 * (uint64_t)a.at[s] + d];
     T rhoSum = T(0.0), xSum = T(0.0), ySum = T(0.0), zSum = T(0.0);
 #pragma unroll
     for (int s = 0; s < 9; s++) {
-        T rho, jx, jy, jz;
-        cell_rho_j<PR, STREAM, MOMSRC_STORED, EVEN>(Q, g, wrap_ik(pi + s % 3 - 1, g.xg1), pj,
-                                                    wrap_ik(pk + s / 3 - 1, g.zg1), rho, jx, jy, jz, rho0);
-        const T ppp = wx[s % 3] * wz[s / 3];
-        const T xx = (T)((D)jx + D(0.5) * (D)f[s][0]);
-        const T yy = (T)((D)jy + D(0.5) * (D)f[s][1]);
-        const T zz = (T)((D)jz + D(0.5) * (D)f[s][2]);
-        rhoSum += ppp * rho;
+        const T ppp = a.wx[s % 3] * a.wz[s / 3];
+        const T xx = (T)((D)a.jx[s] + D(0.5) * (D)f[s][0]);
+        const T yy = (T)((D)a.jy[s] + D(0.5) * (D)f[s][1]);
+        const T zz = (T)((D)a.jz[s] + D(0.5) * (D)f[s][2]);
+        rhoSum += ppp * a.rho[s];
         xSum += ppp * xx;
         ySum += ppp * yy;
         zSum += ppp * zz;
     }
-    xSum -= rhoSum * static_cast<const T*>(p.u)[q];
-    ySum -= rhoSum * static_cast<const T*>(p.v)[q];
-    zSum -= rhoSum * static_cast<const T*>(p.w)[q];
-    // below 3 interior cells a stencil meets itself: one cell after the other
-    const bool meets = g.xg1 < 3 || g.zg1 < 3;
+    xSum -= rhoSum * a.vel[0];
+    ySum -= rhoSum * a.vel[1];
+    zSum -= rhoSum * a.vel[2];
+    // meets: below 3 interior cells a stencil meets itself, one cell after the other
 #pragma unroll
     for (int s = 0; s < 9; s++) {
-        const T bp = beta * (wx[s % 3] * wz[s / 3]);
+        T* const c = F + 3 * (uint64_t)a.at[s];
+        const T bp = beta * (a.wx[s % 3] * a.wz[s / 3]);
         if (meets)
 #pragma unroll
-            for (int d = 0; d < 3; d++) f[s][d] = F[at[s] + d];
-        F[at[s] + 0] = alfa * f[s][0] - bp * xSum;
-        F[at[s] + 1] = alfa * f[s][1] - bp * ySum;
-        F[at[s] + 2] = alfa * f[s][2] - bp * zSum;
+            for (int d = 0; d < 3; d++) f[s][d] = c[d];
+        c[0] = alfa * f[s][0] - bp * xSum;
+        c[1] = alfa * f[s][1] - bp * ySum;
+        c[2] = alfa * f[s][2] - bp * zSum;
     }
 }
 
-constexpr int kListBlock = 512;
+constexpr int kListBlock = 512, kListRun = 8;  // lanes, and points a lane looks at between two barriers
 constexpr uint32_t kNoPoint = 0xffffffffu;
 // list: n positions, the planes' points one plane after the other.  marks_hbm: a
 // plane of marks per workgroup where the LDS does not hold one; a mark there may sit
@@ -907,7 +923,7 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
     extern __shared__ uint32_t list_lds[];
     constexpr int kWaves = kListBlock / 64;
     __shared__ int64_t s_less[kWaves];
-    __shared__ int s_wave[2][kWaves];
+    __shared__ int s_wave[2][kListRun][kWaves];
     __shared__ uint32_t s_next, s_done;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int plane = g.xg1 * g.zg1;
@@ -927,6 +943,7 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
     for (int j = 1 + (int)blockIdx.x; j <= g.yg1; j += (int)gridDim.x) {
         // the plane's part of the list begins after the points of lower planes
         int64_t less = 0;
+#pragma unroll 8
         for (int64_t q = tid; q < n; q += kListBlock) less += p.j[q] < j ? 1 : 0;
         for (int o = 32; o > 0; o >>= 1) less += __shfl_down(less, o, 64);
         if (lane == 0) s_less[wave] = less;
@@ -937,18 +954,30 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
         // its points in list order
         uint32_t count = 0;
         int turn = 0;
-        for (int64_t q0 = 0; q0 < n; q0 += kListBlock, turn ^= 1) {
-            const int64_t q = q0 + tid;
-            const bool in = q < n && p.j[q] == j;
-            const uint64_t vote = __ballot(in);
-            if (lane == 0) s_wave[turn][wave] = __popcll(vote);
-            __syncthreads();  // the last reader of s_wave[turn] has passed the turn between
-            uint32_t at = count;
-            for (int w = 0; w < kWaves; w++) {
-                at += w < wave ? s_wave[turn][w] : 0;
-                count += s_wave[turn][w];
+        for (int64_t q0 = 0; q0 < n; q0 += kListBlock * kListRun, turn ^= 1) {
+            int pj[kListRun];
+            uint64_t vote[kListRun];
+#pragma unroll
+            for (int u = 0; u < kListRun; u++) {
+                const int64_t q = q0 + u * kListBlock + tid;
+                pj[u] = q < n ? p.j[q] : 0;
             }
-            if (in) mine[at + __popcll(vote & ((1ull << lane) - 1ull))] = q;
+#pragma unroll
+            for (int u = 0; u < kListRun; u++) {
+                vote[u] = __ballot(pj[u] == j);
+                if (lane == 0) s_wave[turn][u][wave] = __popcll(vote[u]);
+            }
+            __syncthreads();  // the last reader of s_wave[turn] has passed the turn between
+#pragma unroll
+            for (int u = 0; u < kListRun; u++) {
+                uint32_t at = count;
+#pragma unroll
+                for (int w = 0; w < kWaves; w++) {
+                    at += w < wave ? s_wave[turn][u][w] : 0;
+                    count += s_wave[turn][u][w];
+                }
+                if (pj[u] == j) mine[at + __popcll(vote[u] & ((1ull << lane) - 1ull))] = q0 + u * kListBlock + tid;
+            }
         }
         if (tid == 0) {
             s_next = kListBlock;
@@ -959,11 +988,12 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
         // the lanes hold a prefix of the plane's list: a lane that finishes its point takes the next
         uint32_t t = tid;
         bool have = t < count;
-        int64_t q = 0;
+        ListPoint<typename PR::T> a;
         int cells[9];
         auto take = [&] {
-            q = mine[t];
+            const int64_t q = mine[t];
             const int pi = p.i[q], pk = p.k[q];
+            list_take<PR, STREAM, EVEN>(a, p, q, pi, pk, j, Q, g, rho0);
 #pragma unroll
             for (int s = 0; s < 9; s++)
                 cells[s] = (wrap_ik(pi + s % 3 - 1, g.xg1) - 1) * g.zg1 + wrap_ik(pk + s / 3 - 1, g.zg1) - 1;
@@ -987,7 +1017,7 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
 #pragma unroll
                 for (int s = 0; s < 9; s++) set_mark(cells[s]);
             if (ready) {
-                list_point<PR, STREAM, EVEN>(p, q, F, Q, g, alfa, beta, rho0);
+                list_point<PR>(a, F, alfa, beta, g.xg1 < 3 || g.zg1 < 3);
                 atomicAdd(&s_done, 1u);
                 t = atomicAdd(&s_next, 1u);
                 have = t < count;
