@@ -409,7 +409,7 @@ int build_plan(tdlb_batch* b, int64_t K, bool* structure_changed) {
     p.tot_gather = tot_gather;
     p.n_tasks = (int64_t)tasks.size();
     p.bs = b->bs;
-    // launches: fused, forcing gather, forcing levels, advance
+    // launches of a step alone: fused, forcing gather, forcing levels, advance
     b->launches_per_step = 4;
     // A captured step bakes in every launch size and kernel argument: recapture
     // whenever any of them differs (member identity alone is not enough, a freed

@@ -295,8 +295,8 @@ hipError_t launch_solid_mask(double cx, double cz, double radius, uint8_t* out, 
 // layout) advance together: every kernel of a main-loop step is one launch over
 // all members, blocks mapped to members through prefix tables.  Per-member
 // state that changes from step to step (parity, lattice, occupancy mask, step
-// index) lives in MemberDev on the device and is advanced by a kernel, so one
-// step is a fixed launch sequence that can be captured in a HIP graph.
+// index) lives in MemberDev on the device and is advanced by a kernel, so a run of
+// steps is a fixed launch sequence that can be captured in a HIP graph.
 enum Tile : int32_t {
     TILE_ROW64 = 0,  // a wavefront takes 64 consecutive k of one (i, j) row
     TILE_PLANE = 1,  // a block takes consecutive cells of one i plane (ghost cells idle)
@@ -319,7 +319,7 @@ struct MemberDev {
     GatherBlocks gb;         // its blocks in the gather launch
     const BladeStep* steps;  // blade orientation of step done + 1, done + 2, ...
     int64_t n_steps;         // steps this member may still take in the batch
-    // advanced on the device after every step
+    // advanced on the device after every launch_batch_step
     int32_t even, cur, fm, active;
     int64_t done;
 };
@@ -348,7 +348,8 @@ struct BatchPlan {
 };
 
 // Enqueue `steps` main-loop steps of every active member: per step the fused
-// stream-collide, the forcing gather, the forcing levels, advance.
+// stream-collide, the forcing gather and the forcing levels; then the advance of
+// the members' state.
 hipError_t launch_batch_step(int prec, int streaming, const BatchPlan& plan, int steps, hipStream_t s);
 // blocks of the fused kernel for one member with the given tile and block size
 int64_t batch_coll_blocks(const Grid& g, int tile, int bs);
