@@ -178,11 +178,11 @@ TDLB_HD inline int64_t plane_force_bytes(const Grid& g, size_t tsize) {
 constexpr size_t kCuLdsBytes = 160 * 1024;  // LDS of a gfx950 CU
 // Workgroup of a batch's forcing planes for a mean of `cells` static stencil
 // cells per task: a lane per ~4 cells, a power of two from 128 to
-// kForcePlaneBlock lanes (batches of 48^3 tanks: 128 lanes 1.7x faster than
-// 1024; the mixed 48..160 batch: 256 lanes 9 % faster; 160^3 tanks: 256
-// lanes 2 % faster, 512 lanes 4 %).  A batch has thousands of tasks; a single
-// tank's few hundred planes leave CUs idle anyway and run faster with 1024
-// lanes (512^3: 0.653 against 0.734 ms per pass with 512 lanes).
+// kForcePlaneBlock lanes, which is the fastest of 128, 256, 512 and 1024 lanes for
+// steps of 100 tanks of 48^3 (0.42 ms with 128; 0.43, 0.48, 0.55), of 64 mixed from 48
+// to 160 (2.48 ms with 256; 2.65, 2.56, 2.60) and of 8 of 160^3 (0.87 ms with 256;
+// 1.01, 0.89, 0.88).  A batch of few tanks leaves CUs idle and runs faster with 1024
+// lanes (3 of 90^3: 85 us; 103, 91, 86).
 inline int forcing_block_for(double cells) {
     int t = 128;
     while (t < kForcePlaneBlock && 2.0 * t <= cells / 4.0) t *= 2;
