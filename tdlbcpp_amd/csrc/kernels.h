@@ -112,6 +112,10 @@ hipError_t launch_list_unpack(int prec, const tdlb_ib_point* in, int64_t n, int 
 // the LDS), and its workgroups.
 constexpr size_t kListLdsBytes = 152 * 1024;  // of a CU's 160 KB
 size_t list_marks_bytes(const Grid& g, int* blocks);
+// Level of every point of a list within its j plane (i, j, k of p): one more than the
+// highest level of an earlier point of the list that shares a stencil cell.
+hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint32_t* marks, int32_t* lev,
+                              const Grid& g, hipStream_t s);
 // The forcing of the list in its order; list: room for n positions.
 hipError_t launch_list_planes(int prec, int streaming, int even, const PointsDev& p, int64_t n, int64_t* list,
                               uint32_t* marks, const void* Q, void* F, const uint64_t* prev, uint64_t* next,

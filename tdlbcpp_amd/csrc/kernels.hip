@@ -909,9 +909,135 @@ __device__ __forceinline__ void list_point(const ListPoint<typename PR::T>& a, t
 
 constexpr int kListBlock = 512, kListRun = 8;  // lanes, and points a lane looks at between two barriers
 constexpr uint32_t kNoPoint = 0xffffffffu;
+struct ListShared {
+    int64_t less[kListBlock / 64];
+    int wave[2][kListRun][kListBlock / 64];
+};
+// The points of plane j (pj: the planes of all n) to their part of list, in list order, by the whole workgroup;
+// returns their number, mine their part.  A barrier is needed before they are read.
+__device__ __forceinline__ uint32_t plane_points(const int32_t* __restrict__ pj, int64_t n, int j,
+                                                 int64_t* __restrict__ list, int64_t*& mine, ListShared& sh) {
+    constexpr int kWaves = kListBlock / 64;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // the plane's part of the list begins after the points of lower planes
+    int64_t less = 0;
+#pragma unroll 8
+    for (int64_t q = tid; q < n; q += kListBlock) less += pj[q] < j ? 1 : 0;
+    for (int o = 32; o > 0; o >>= 1) less += __shfl_down(less, o, 64);
+    if (lane == 0) sh.less[wave] = less;
+    __syncthreads();
+    int64_t first = 0;
+    for (int w = 0; w < kWaves; w++) first += sh.less[w];
+    mine = list + first;
+    // its points in list order
+    uint32_t count = 0;
+    int turn = 0;
+    for (int64_t q0 = 0; q0 < n; q0 += kListBlock * kListRun, turn ^= 1) {
+        int at_j[kListRun];
+        uint64_t vote[kListRun];
+#pragma unroll
+        for (int u = 0; u < kListRun; u++) {
+            const int64_t q = q0 + u * kListBlock + tid;
+            at_j[u] = q < n ? pj[q] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < kListRun; u++) {
+            vote[u] = __ballot(at_j[u] == j);
+            if (lane == 0) sh.wave[turn][u][wave] = __popcll(vote[u]);
+        }
+        __syncthreads();  // the last reader of sh.wave[turn] has passed the turn between
+#pragma unroll
+        for (int u = 0; u < kListRun; u++) {
+            uint32_t at = count;
+#pragma unroll
+            for (int w = 0; w < kWaves; w++) {
+                at += w < wave ? sh.wave[turn][u][w] : 0;
+                count += sh.wave[turn][u][w];
+            }
+            if (at_j[u] == j) mine[at + __popcll(vote[u] & ((1ull << lane) - 1ull))] = q0 + u * kListBlock + tid;
+        }
+    }
+    return count;
+}
+
+// The marks of a plane's cells, in LDS or, where it does not hold them, in HBM: there a
+// mark may sit in this CU's L1 from the round before and is read where the atomics put it.
+template <bool LDS>
+struct Marks {
+    uint32_t* p;
+    __device__ __forceinline__ void clear(int c) const { p[c] = kNoPoint; }
+    __device__ __forceinline__ void lower(int c, uint32_t t) const { atomicMin(p + c, t); }
+    __device__ __forceinline__ uint32_t get(int c) const {
+        return LDS ? p[c] : __hip_atomic_load(p + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+// a stencil's nine cells in a plane's own (i, k) order
+__device__ __forceinline__ void plane_cells(int (&cells)[9], int pi, int pk, const Grid& g) {
+#pragma unroll
+    for (int s = 0; s < 9; s++)
+        cells[s] = (wrap_ik(pi + s % 3 - 1, g.xg1) - 1) * g.zg1 + wrap_ik(pk + s / 3 - 1, g.zg1) - 1;
+}
+
+// Levels of a list within its planes, one more than the highest level of an earlier
+// point that shares a stencil cell: the round in which a point holds all its cells when
+// every unfinished point of the plane marks.  list, marks_hbm as in k_list_planes.
+template <bool MARKS_LDS>
+__global__ __launch_bounds__(kListBlock) void k_list_levels(PointsDev p, int64_t n, int64_t* __restrict__ list,
+                                                            uint32_t* __restrict__ marks_hbm, int32_t* __restrict__ lev,
+                                                            Grid g) {
+    extern __shared__ uint32_t list_lds[];
+    __shared__ ListShared s_list;
+    __shared__ uint32_t s_done;
+    const int tid = (int)threadIdx.x;
+    const int plane = g.xg1 * g.zg1;
+    const Marks<MARKS_LDS> marks{MARKS_LDS ? list_lds : marks_hbm + (uint64_t)blockIdx.x * plane};
+    for (int c = tid; c < plane; c += kListBlock) marks.clear(c);
+    for (int j = 1 + (int)blockIdx.x; j <= g.yg1; j += (int)gridDim.x) {
+        int64_t* mine;
+        const uint32_t count = plane_points(p.j, n, j, list, mine, s_list);
+        if (tid == 0) s_done = 0;
+        __syncthreads();
+        int32_t round = 0;
+        for (uint32_t done = 0; done < count; round++) {
+            int cells[9];
+            for (uint32_t t = tid; t < count; t += kListBlock) {
+                const int64_t q = mine[t];
+                if (q < 0) continue;
+                plane_cells(cells, p.i[q], p.k[q], g);
+#pragma unroll
+                for (int s = 0; s < 9; s++) marks.lower(cells[s], t);
+            }
+            __syncthreads();
+            uint32_t ended = 0;
+            for (uint32_t t = tid; t < count; t += kListBlock) {
+                const int64_t q = mine[t];
+                if (q < 0) continue;
+                plane_cells(cells, p.i[q], p.k[q], g);
+                bool ready = true;
+#pragma unroll
+                for (int s = 0; s < 9; s++) ready = marks.get(cells[s]) == t && ready;
+                if (!ready) continue;
+                lev[q] = round;
+                mine[t] = -1 - q;
+                ended++;
+            }
+            if (ended) atomicAdd(&s_done, ended);
+            __syncthreads();
+            for (uint32_t t = tid; t < count; t += kListBlock) {
+                const int64_t q = mine[t];
+                const int64_t a = q < 0 ? -1 - q : q;
+                plane_cells(cells, p.i[a], p.k[a], g);
+#pragma unroll
+                for (int s = 0; s < 9; s++) marks.clear(cells[s]);
+            }
+            done = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_done);
+            __syncthreads();
+        }
+    }
+}
+
 // list: n positions, the planes' points one plane after the other.  marks_hbm: a
-// plane of marks per workgroup where the LDS does not hold one; a mark there may sit
-// in this CU's L1 from the round before and is read where the atomics put it.
+// plane of marks per workgroup where the LDS does not hold one.
 template <typename PR, int STREAM, int EVEN, bool MARKS_LDS>
 __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t n, int64_t* __restrict__ list,
                                                             uint32_t* __restrict__ marks_hbm,
@@ -921,64 +1047,15 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
                                                             uint64_t* __restrict__ next, Grid g,
                                                             typename PR::T alfa, typename PR::T beta, float rho0) {
     extern __shared__ uint32_t list_lds[];
-    constexpr int kWaves = kListBlock / 64;
-    __shared__ int64_t s_less[kWaves];
-    __shared__ int s_wave[2][kListRun][kWaves];
+    __shared__ ListShared s_list;
     __shared__ uint32_t s_next, s_done;
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = (int)threadIdx.x;
     const int plane = g.xg1 * g.zg1;
-    uint32_t* const hbm = MARKS_LDS ? nullptr : marks_hbm + (uint64_t)blockIdx.x * plane;
-    auto set_mark = [&](int c) {
-        if (MARKS_LDS) list_lds[c] = kNoPoint;
-        else hbm[c] = kNoPoint;
-    };
-    auto min_mark = [&](int c, uint32_t t) {
-        if (MARKS_LDS) atomicMin(&list_lds[c], t);
-        else atomicMin(hbm + c, t);
-    };
-    auto mark = [&](int c) -> uint32_t {
-        return MARKS_LDS ? list_lds[c] : __hip_atomic_load(hbm + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    for (int c = tid; c < plane; c += kListBlock) set_mark(c);
+    const Marks<MARKS_LDS> marks{MARKS_LDS ? list_lds : marks_hbm + (uint64_t)blockIdx.x * plane};
+    for (int c = tid; c < plane; c += kListBlock) marks.clear(c);
     for (int j = 1 + (int)blockIdx.x; j <= g.yg1; j += (int)gridDim.x) {
-        // the plane's part of the list begins after the points of lower planes
-        int64_t less = 0;
-#pragma unroll 8
-        for (int64_t q = tid; q < n; q += kListBlock) less += p.j[q] < j ? 1 : 0;
-        for (int o = 32; o > 0; o >>= 1) less += __shfl_down(less, o, 64);
-        if (lane == 0) s_less[wave] = less;
-        __syncthreads();
-        int64_t first = 0;
-        for (int w = 0; w < kWaves; w++) first += s_less[w];
-        int64_t* const mine = list + first;
-        // its points in list order
-        uint32_t count = 0;
-        int turn = 0;
-        for (int64_t q0 = 0; q0 < n; q0 += kListBlock * kListRun, turn ^= 1) {
-            int pj[kListRun];
-            uint64_t vote[kListRun];
-#pragma unroll
-            for (int u = 0; u < kListRun; u++) {
-                const int64_t q = q0 + u * kListBlock + tid;
-                pj[u] = q < n ? p.j[q] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < kListRun; u++) {
-                vote[u] = __ballot(pj[u] == j);
-                if (lane == 0) s_wave[turn][u][wave] = __popcll(vote[u]);
-            }
-            __syncthreads();  // the last reader of s_wave[turn] has passed the turn between
-#pragma unroll
-            for (int u = 0; u < kListRun; u++) {
-                uint32_t at = count;
-#pragma unroll
-                for (int w = 0; w < kWaves; w++) {
-                    at += w < wave ? s_wave[turn][u][w] : 0;
-                    count += s_wave[turn][u][w];
-                }
-                if (pj[u] == j) mine[at + __popcll(vote[u] & ((1ull << lane) - 1ull))] = q0 + u * kListBlock + tid;
-            }
-        }
+        int64_t* mine;
+        const uint32_t count = plane_points(p.j, n, j, list, mine, s_list);
         if (tid == 0) {
             s_next = kListBlock;
             s_done = 0;
@@ -994,9 +1071,7 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
             const int64_t q = mine[t];
             const int pi = p.i[q], pk = p.k[q];
             list_take<PR, STREAM, EVEN>(a, p, q, pi, pk, j, Q, g, rho0);
-#pragma unroll
-            for (int s = 0; s < 9; s++)
-                cells[s] = (wrap_ik(pi + s % 3 - 1, g.xg1) - 1) * g.zg1 + wrap_ik(pk + s / 3 - 1, g.zg1) - 1;
+            plane_cells(cells, pi, pk, g);
         };
         if (have) take();
         __syncthreads();
@@ -1006,16 +1081,16 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
         for (uint32_t done = 0; done < count;) {
             if (have)
 #pragma unroll
-                for (int s = 0; s < 9; s++) min_mark(cells[s], t);
+                for (int s = 0; s < 9; s++) marks.lower(cells[s], t);
             __syncthreads();
             bool ready = have;
             if (have)
 #pragma unroll
-                for (int s = 0; s < 9; s++) ready = (mark(cells[s]) == t) && ready;
+                for (int s = 0; s < 9; s++) ready = marks.get(cells[s]) == t && ready;
             __syncthreads();
             if (have)
 #pragma unroll
-                for (int s = 0; s < 9; s++) set_mark(cells[s]);
+                for (int s = 0; s < 9; s++) marks.clear(cells[s]);
             if (ready) {
                 list_point<PR>(a, F, alfa, beta, g.xg1 < 3 || g.zg1 < 3);
                 atomicAdd(&s_done, 1u);
@@ -2437,6 +2512,23 @@ size_t list_marks_bytes(const Grid& g, int* blocks) {
     const int n = lds ? g.yg1 : std::min(g.yg1, 256);
     if (blocks) *blocks = n;
     return lds ? 0 : plane * (size_t)n;
+}
+
+hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint32_t* marks, int32_t* lev,
+                              const Grid& g, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    int blocks = 0;
+    const size_t hbm = list_marks_bytes(g, &blocks);
+    if ((hbm != 0) != (marks != nullptr)) return hipErrorInvalidValue;
+    const uint32_t lds = hbm ? 0u : (uint32_t)((size_t)g.xg1 * g.zg1 * sizeof(uint32_t));
+    auto* k = hbm ? &k_list_levels<false> : &k_list_levels<true>;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(k, dim3((uint32_t)blocks), dim3(kListBlock), lds, s, p, n, list, marks, lev, g);
+    return hipGetLastError();
 }
 
 hipError_t launch_list_planes(int prec, int streaming, int even, const PointsDev& p, int64_t n, int64_t* list,
