@@ -503,47 +503,50 @@ __global__ void k_pull_all(const W* __restrict__ src, W* __restrict__ dst, Grid 
     }
 }
 
-// One face of the bounce-back, in place: ghost slot d (5 inward directions) of a
-// face cell takes slot opp(d) of the neighbour g+e_d.  Faces run in the
-// reference's order as separate launches because face rims read ghosts of
-// faces handled later.
+// The bounce-back, in place, in one launch: ghost slot d (5 inward directions) of a
+// face cell takes slot opp(d) of the neighbour g+e_d, and the 12 edge lines theirs
+// (Boundary.hpp:41-132: on an edge the one direction pointing inward on both
+// boundary axes).  The reference's faces follow one another (i, j, k), and at a rim a
+// face reads a ghost cell of another: of a later face its old value, while the later
+// face would read back the very value that the earlier one took from it, so it keeps
+// its own and nothing that is read is written.  Six faces and the edges as launches
+// of their own took 23 us a call at 60^3, this one 5.
 template <typename W>
-__global__ void k_bb_face(W* __restrict__ Q, Grid g, int face) {
-    const int axis = face >> 1;        // 0 i, 1 j, 2 k
-    const int inward = (face & 1) ? -1 : 1;
-    const int pos = (face & 1) ? (axis == 0 ? g.xg1 + 1 : axis == 1 ? g.yg1 + 1 : g.zg1 + 1) : 0;
-    const int na = axis == 0 ? g.yg1 : g.xg1;                 // first free axis extent
-    const int nb = axis == 2 ? g.yg1 : g.zg1;                 // second free axis extent
-    const uint64_t total = (uint64_t)na * nb;
-    for (uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t < total;
-         t += (uint64_t)gridDim.x * blockDim.x) {
-        const int a = (int)(t / nb) + 1, b = (int)(t % nb) + 1;
-        int i, j, k;
-        if (axis == 0) { i = pos; j = a; k = b; }
-        else if (axis == 1) { i = a; j = pos; k = b; }
-        else { i = a; j = b; k = pos; }
-        const uint32_t c = qcell(g, i, j, k);
-#pragma unroll
-        for (int d = 0; d < kQ; d++) {
-            const int comp = axis == 0 ? dir_x(d) : axis == 1 ? dir_y(d) : dir_z(d);
-            if (comp != inward) continue;
-            const uint32_t s = qcell(g, i + dir_x(d), j + dir_y(d), k + dir_z(d));
-            Q[qaddr(g, c, d)] = Q[qaddr(g, s, opposite(d))];
-        }
-    }
-}
-
-// The 12 edge lines of the bounce-back (Boundary.hpp:41-132): on an edge the
-// one direction pointing inward on both boundary axes takes opp(d) of g+e_d.
-template <typename W>
-__global__ void k_bb_edges(W* __restrict__ Q, Grid g) {
+__global__ void k_bounce_back(W* __restrict__ Q, Grid g) {
+    const uint64_t fi = (uint64_t)g.yg1 * g.zg1, fj = (uint64_t)g.xg1 * g.zg1, fk = (uint64_t)g.xg1 * g.yg1;
+    const uint64_t faces = 2 * (fi + fj + fk);
     const int nmax = max(g.xg1, max(g.yg1, g.zg1));
-    const uint64_t total = 12ull * nmax;
-    for (uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t < total;
-         t += (uint64_t)gridDim.x * blockDim.x) {
+    const int X0 = g.xg1 + 1, Y0 = g.yg1 + 1, Z0 = g.zg1 + 1;
+    for (uint64_t u = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; u < faces + 12ull * nmax;
+         u += (uint64_t)gridDim.x * blockDim.x) {
+        int i, j, k;
+        if (u < faces) {
+            const int axis = u < 2 * fi ? 0 : u < 2 * (fi + fj) ? 1 : 2;  // 0 i, 1 j, 2 k
+            const uint64_t per = axis == 0 ? fi : axis == 1 ? fj : fk;
+            uint64_t t = u - (axis == 0 ? 0 : axis == 1 ? 2 * fi : 2 * (fi + fj));
+            const bool far = t >= per;
+            if (far) t -= per;
+            const int inward = far ? -1 : 1;
+            const int nb = axis == 2 ? g.yg1 : g.zg1;  // second free axis extent
+            const int a = (int)(t / nb) + 1, b = (int)(t % nb) + 1;
+            if (axis == 0) { i = far ? X0 : 0; j = a; k = b; }
+            else if (axis == 1) { i = a; j = far ? Y0 : 0; k = b; }
+            else { i = a; j = b; k = far ? Z0 : 0; }
+            const uint32_t c = qcell(g, i, j, k);
+#pragma unroll
+            for (int d = 0; d < kQ; d++) {
+                const int comp = axis == 0 ? dir_x(d) : axis == 1 ? dir_y(d) : dir_z(d);
+                if (comp != inward) continue;
+                const int i2 = i + dir_x(d), j2 = j + dir_y(d), k2 = k + dir_z(d);
+                if (axis > 0 && (i2 == 0 || i2 == X0)) continue;
+                if (axis > 1 && (j2 == 0 || j2 == Y0)) continue;
+                Q[qaddr(g, c, d)] = Q[qaddr(g, qcell(g, i2, j2, k2), opposite(d))];
+            }
+            continue;
+        }
+        const uint64_t t = u - faces;
         const int line = (int)(t / nmax), s = (int)(t % nmax) + 1;
-        const int X0 = g.xg1 + 1, Y0 = g.yg1 + 1, Z0 = g.zg1 + 1;
-        int i, j, k, d;
+        int d;
         switch (line) {
             case 0: i = 0; j = 0; k = s; d = Q07; break;
             case 1: i = X0; j = 0; k = s; d = Q14; break;
@@ -2421,17 +2424,10 @@ hipError_t launch_pull_all(int esize, const void* src, void* dst, const Grid& g,
 }
 
 hipError_t launch_bounce_back(int esize, void* Q, const Grid& g, hipStream_t s) {
-    for (int face = 0; face < 6; face++) {
-        const int axis = face >> 1;
-        const uint64_t n = (uint64_t)(axis == 0 ? g.yg1 : g.xg1) * (axis == 2 ? g.yg1 : g.zg1);
-        if (esize == 4) TDLB_MOVE(k_bb_face, uint32_t, n, (uint32_t*)Q, g, face);
-        else TDLB_MOVE(k_bb_face, uint64_t, n, (uint64_t*)Q, g, face);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    const uint64_t n = 12ull * (uint64_t)std::max(g.xg1, std::max(g.yg1, g.zg1));
-    if (esize == 4) TDLB_MOVE(k_bb_edges, uint32_t, n, (uint32_t*)Q, g);
-    else TDLB_MOVE(k_bb_edges, uint64_t, n, (uint64_t*)Q, g);
+    const uint64_t x = (uint64_t)g.xg1, y = (uint64_t)g.yg1, z = (uint64_t)g.zg1;
+    const uint64_t n = 2 * (y * z + x * z + x * y) + 12 * std::max(x, std::max(y, z));
+    if (esize == 4) TDLB_MOVE(k_bounce_back, uint32_t, n, (uint32_t*)Q, g);
+    else TDLB_MOVE(k_bounce_back, uint64_t, n, (uint64_t*)Q, g);
     return hipGetLastError();
 }
 

@@ -71,3 +71,23 @@ def test_results_read_by_several_threads_at_once():
 def test_rows_ending_inside_a_wavefront_match_oracle(T, precision, streaming):
     print(f"[gpu case] rows of {T}, precision {precision}", flush=True)
     compare(T, 3, precision, streaming=streaming)
+
+
+# one launch writes every face and edge: rims where faces meet, extents of one cell
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 4, 2), (3, 1, 5), (66, 3, 2), (5, 6, 130)])
+@pytest.mark.parametrize("precision", [td.PREC_F32, td.PREC_F64], ids=["fp32", "fp64"])
+def test_bounce_back_of_all_faces_matches_oracle(shape, precision):
+    print(f"[gpu case] bounce-back {shape}, precision {precision}", flush=True)
+    o = O.OracleCU(*shape, dtype=O.F32 if precision == td.PREC_F32 else O.F64, layout=O.LIJK, streaming=O.SIMPLE,
+                   use_les=False, nu=0.003)
+    g = td.ComputeUnit(*shape, layout=td.LAYOUT_LIJK, streaming=td.STREAM_SIMPLE, precision=precision, nu=0.003)
+    q = np.random.default_rng(3).standard_normal(o.get(O.FIELD_Q).shape)
+    o.set(O.FIELD_Q, q)
+    g.set(td.FIELD_Q, o.get(O.FIELD_Q))
+    for _ in range(2):
+        o.bounce_back()
+        g.bounce_back()
+        assert np.array_equal(g.get(td.FIELD_Q), o.get(O.FIELD_Q))
+        o.streaming_push()
+        g.streaming_push()
+    g.close()
