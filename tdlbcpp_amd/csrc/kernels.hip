@@ -1124,7 +1124,9 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
 // us).  Whole pass, gather and levels in one -> two launches: 24^3 205 -> 33 us,
 // 60^3 41 -> 29, 96^3 47 -> 37, 192^3 FP64 219 -> 132, 256^3 226 -> 166, 512^3
 // 597 -> 549 (gather 390, 5.1 TB/s of lines; levels 140).  With rows asked for three
-// passes ahead (run_levels): 24^3 33 -> 31 us, 96^3 35 -> 32, 131^3 45 -> 42, 256^3 166 -> 158.
+// passes ahead (run_levels): 24^3 33 -> 31 us, 96^3 35 -> 32, 131^3 45 -> 42, 256^3 166
+// -> 158; with the blades' indexes in closed form (blade_group; loops of integer divisions
+// before) and branch-free passes: 24^3 31 -> 27, 60^3 27 -> 25, 96^3 32 -> 30, 131^3 42 -> 40.
 
 // ---- A point of a plane task on a quad of lanes: lane c = 0..2 of the quad
 // takes stencil row k1 = c - 1 (cells s = 3c + m for i1 = m - 1), lane 3 repeats
@@ -1233,38 +1235,45 @@ __device__ __forceinline__ BladeEnum blade_enum_of(const BladeLayout& bl) {
     e.n_bcol = bl.n_bcol;
     return e;
 }
-// points of level l on one plane
-__device__ __forceinline__ int blade_level_count(const BladeLayout& bl, int l) {
-    const int rmod = l % 5, nr = bl.n_radial > rmod ? (bl.n_radial - rmod + 4) / 5 : 0;
-    const int first = bl.merged ? 0 : l / 5, stride = bl.merged ? 1 : bl.n_bcol;
-    return (bl.n_blades > first ? (bl.n_blades - first + stride - 1) / stride : 0) * nr;
+// radial classes with points: no level of a plane is empty
+__device__ __forceinline__ int radial_classes(const BladeLayout& bl) { return min(bl.n_radial, 5); }
+// Blades dealt to `groups` in turn (blade b to group b mod groups): how many a group has and how many the
+// groups before it have together.
+struct BladeGroup {
+    int n, before;
+};
+__device__ __forceinline__ BladeGroup blade_group(int n_blades, int groups, int g) {
+    const int q = n_blades / groups, rem = n_blades - q * groups;
+    return BladeGroup{q + (g < rem ? 1 : 0), g * q + min(g, rem)};
+}
+// radial points of the first m classes of a blade (index mod 5 below m)
+__device__ __forceinline__ int radial_before(int n_radial, int m) { return n_radial / 5 * m + min(m, n_radial % 5); }
+// points of levels 0..l on one plane
+__device__ __forceinline__ int blade_level_end(const BladeLayout& bl, int l) {
+    const int per = radial_classes(bl), g = l / per;
+    const BladeGroup bg = blade_group(bl.n_blades, bl.merged ? 1 : bl.n_bcol, g);
+    return bg.before * bl.n_radial + bg.n * radial_before(bl.n_radial, l - g * per + 1);
 }
 // list index of radial point r of blade b on blade plane bp
 __device__ __forceinline__ int blade_index(const BladeEnum& e, int b, int r, int bp) {
-    const int bcol = b % e.n_bcol, bi = b / e.n_bcol, rmod = r % 5;
-    const int nb = (e.n_blades - bcol + e.n_bcol - 1) / e.n_bcol;
-    int before = 0;  // points per plane of the colours before bcol, then of this colour's radial classes before rmod
-    for (int a = 0; a < bcol; a++) before += (e.n_blades - a + e.n_bcol - 1) / e.n_bcol;
-    before *= e.n_radial;
-    for (int a = 0; a < rmod; a++) before += nb * (e.n_radial > a ? (e.n_radial - a + 4) / 5 : 0);
+    const int bi = b / e.n_bcol, rmod = r % 5;
+    const BladeGroup bg = blade_group(e.n_blades, e.n_bcol, b - bi * e.n_bcol);
+    // points per plane of the colours before the blade's, then of its colour's radial classes before rmod
+    const int before = bg.before * e.n_radial + bg.n * radial_before(e.n_radial, rmod);
     return before * e.n_planes + (bi * e.n_planes + bp) * ((e.n_radial - rmod + 4) / 5) + r / 5;
 }
 // position of radial point r of blade b among the plane's points in level order
 __device__ __forceinline__ int level_slot(const BladeLayout& bl, int b, int r) {
-    const BladeEnum e = blade_enum_of(bl);
-    const int groups = bl.merged ? 1 : e.n_bcol, grp = b % groups, bi = b / groups, rmod = r % 5;
-    const int nb = (e.n_blades - grp + groups - 1) / groups;
-    int before = 0;
-    for (int a = 0; a < grp; a++) before += (e.n_blades - a + groups - 1) / groups;
-    before *= e.n_radial;
-    for (int a = 0; a < rmod; a++) before += nb * (e.n_radial > a ? (e.n_radial - a + 4) / 5 : 0);
-    return before + bi * ((e.n_radial - rmod + 4) / 5) + r / 5;
+    const int groups = bl.merged ? 1 : bl.n_bcol, bi = b / groups, rmod = r % 5;
+    const BladeGroup bg = blade_group(bl.n_blades, groups, b - bi * groups);
+    return bg.before * bl.n_radial + bg.n * radial_before(bl.n_radial, rmod) +
+           bi * ((bl.n_radial - rmod + 4) / 5) + r / 5;
 }
 // blade plane index of plane j and its blade levels (0: no blades)
 __device__ __forceinline__ int blade_plane(const ForceGeom& fg, int j, int& nlev) {
     const BladeLayout& bl = fg.blade;
     const int bp = j - bl.ghost - bl.j_lo;
-    nlev = (bl.n_blades > 0 && fg.n_rot > 0 && bp >= 0 && bp < bl.n_planes) ? (bl.merged ? 5 : 5 * bl.n_bcol) : 0;
+    nlev = (bl.n_blades > 0 && fg.n_rot > 0 && bp >= 0 && bp < bl.n_planes) ? radial_classes(bl) * (bl.merged ? 1 : bl.n_bcol) : 0;
     return bp;
 }
 
@@ -1387,76 +1396,80 @@ __device__ __forceinline__ X uniform_copy(const X& x) {
 }
 
 // The levels of a plane: passes of a point per quad of lanes, a barrier after every
-// level.  level_end(l): end of level l's points, called for l = 0, 1, ...; row_at(q):
+// level; none is empty.  end_of(l): the end of level l's points, on any lane; row_at(q):
 // the lane's stencil row of point q; mom_at(q, row, m): its moments; get and
 // put(row, f): its force values.  A turn of the loop is one pass.  Rows are asked
 // for three passes ahead and moments one, since neither changes meanwhile.  The
 // turn is written out for each place of the ring of rows: with rows moved from one
 // variable to the next, every move waited for the row in flight (24^3: 0.72 us a
-// level, now 0.55, which is the instruction stream of one wavefront per SIMD).
+// level, 0.55 without).  Level ends come from lanes of a register (64 levels at a
+// time), the next pass from selects, and what a lane with a point does is the straight
+// path: a level is then bound by the latency of its reads, sums, writes and barrier.
 // Rows in HBM are asked for by every lane, without a branch (a lane without a point
 // takes the level's last): past a branch that may have skipped loads the compiler
 // waits for all of them.  Loads return in order, so in HBM a pass asks for its force
 // values before the moments and rows of later passes, and within a level for the
 // next pass's before it stores its own.
 template <typename T, bool ROWS_LDS, bool F_LDS, typename End, typename RowAt, typename MomAt, typename Get, typename Put>
-__device__ __forceinline__ void run_levels(int nlev, T alfa, T beta, End&& level_end, RowAt&& row_at, MomAt&& mom_at,
+__device__ __forceinline__ void run_levels(int nlev, T alfa, T beta, End&& end_of, RowAt&& row_at, MomAt&& mom_at,
                                            Get&& get, Put&& put) {
     const int slot = (int)(threadIdx.x >> 2), lane = (int)(threadIdx.x & 3), per = (int)(blockDim.x >> 2);
-    struct Pass {
-        int l;       // level, nlev after the last
-        int q, end;  // first point, end of the level
-    };
-    auto next = [&](Pass a) {
-        if (a.q + per < a.end) return Pass{a.l, a.q + per, a.end};
-        int l = a.l + 1;
-        for (; l < nlev; l++) {
-            const int end = level_end(l);
-            if (end > a.end) return Pass{l, a.end, end};
+    int begin = 0;
+    for (int base = 0; base < nlev; base += 64) {
+        const int levels = min(nlev - base, 64);
+        // lane i of the wave: the end of level base + i, of the last beyond it
+        const int ends = end_of(base + min((int)(threadIdx.x & 63), levels - 1));
+        struct Pass {
+            int l;       // level from base, `levels` after the last
+            int q, end;  // first point, end of the level
+        };
+        auto next = [&](Pass a) {
+            const bool same = a.q + per < a.end;
+            const int l = same ? a.l : a.l + 1;
+            return Pass{min(l, levels), same ? a.q + per : a.end, __builtin_amdgcn_readlane(ends, min(l, 63))};
+        };
+        auto on = [&](const Pass& a) { return a.q + slot < a.end; };
+        ForceRow<T> r0, r1, r2, r3;
+        Mom4<T> m0[3], m1[3];
+        T f0[3][3], f1[3][3];
+        Pass a0{0, begin, __builtin_amdgcn_readlane(ends, 0)}, a1 = next(a0), a2 = next(a1);
+        begin = __builtin_amdgcn_readlane(ends, 63);
+        auto load = [&](ForceRow<T>& r, const Pass& a) {
+            if (!ROWS_LDS) r = row_at(min(a.q + slot, a.end - 1));
+            else if (on(a)) r = row_at(a.q + slot);
+        };
+        load(r0, a0);
+        load(r1, a1);
+        load(r2, a2);
+        if (on(a0)) mom_at(a0.q + slot, r0, m0);
+        bool have = false;  // the pass's force values were asked for in the pass before
+        // this pass, the next and the one three ahead
+        auto turn = [&](ForceRow<T>& cr, ForceRow<T>& nr, ForceRow<T>& ar, Mom4<T> (&cm)[3], Mom4<T> (&nm)[3],
+                        T (&cf)[3][3], T (&nf)[3][3]) {
+            const bool on0 = on(a0), on1 = on(a1), same = a1.l == a0.l;
+            if ((F_LDS || !have) && __builtin_expect(on0, true)) get(cr, cf);
+            if (!F_LDS && same && on1) get(nr, nf);
+            if (__builtin_expect(on1, true)) mom_at(a1.q + slot, nr, nm);
+            const Pass a3 = next(a2);
+            __builtin_amdgcn_sched_barrier(0);  // the row behind them: no wait for moments or forces includes it
+            load(ar, a3);
+            if (__builtin_expect(on0, true)) {
+                force_row(cr, cm, cf, alfa, beta);
+                if (lane < 3) put(cr, cf);
+            }
+            if (!same) __syncthreads();
+            a0 = a1;
+            a1 = a2;
+            a2 = a3;
+            have = same;
+            return a0.l < levels;
+        };
+        for (;;) {
+            if (!turn(r0, r1, r3, m0, m1, f0, f1)) break;
+            if (!turn(r1, r2, r0, m1, m0, f1, f0)) break;
+            if (!turn(r2, r3, r1, m0, m1, f0, f1)) break;
+            if (!turn(r3, r0, r2, m1, m0, f1, f0)) break;
         }
-        return Pass{l, a.end, a.end};
-    };
-    auto on = [&](const Pass& a) { return a.q + slot < a.end; };
-    ForceRow<T> r0, r1, r2, r3;
-    Mom4<T> m0[3], m1[3];
-    T f0[3][3], f1[3][3];
-    Pass a0 = next(Pass{-1, 0, 0}), a1 = next(a0), a2 = next(a1);
-    if (a0.l >= nlev) return;
-    auto load = [&](ForceRow<T>& r, const Pass& a) {
-        if (!ROWS_LDS) r = row_at(min(a.q + slot, a.end - 1));
-        else if (on(a)) r = row_at(a.q + slot);
-    };
-    load(r0, a0);
-    load(r1, a1);
-    load(r2, a2);
-    if (on(a0)) mom_at(a0.q + slot, r0, m0);
-    bool have = false;  // the pass's force values were asked for in the pass before
-    // this pass, the next and the one three ahead
-    auto turn = [&](ForceRow<T>& cr, ForceRow<T>& nr, ForceRow<T>& ar, Mom4<T> (&cm)[3], Mom4<T> (&nm)[3],
-                    T (&cf)[3][3], T (&nf)[3][3]) {
-        const bool on0 = on(a0), on1 = on(a1), same = a1.l == a0.l;
-        if ((F_LDS || !have) && on0) get(cr, cf);
-        if (!F_LDS && same && on1) get(nr, nf);
-        if (on1) mom_at(a1.q + slot, nr, nm);
-        const Pass a3 = next(a2);
-        __builtin_amdgcn_sched_barrier(0);  // the row behind them: no wait for moments or forces includes it
-        load(ar, a3);
-        if (on0) {
-            force_row(cr, cm, cf, alfa, beta);
-            if (lane < 3) put(cr, cf);
-        }
-        if (!same) __syncthreads();
-        a0 = a1;
-        a1 = a2;
-        a2 = a3;
-        have = same;
-        return a0.l < nlev;
-    };
-    for (;;) {
-        if (!turn(r0, r1, r3, m0, m1, f0, f1)) break;
-        if (!turn(r1, r2, r0, m1, m0, f1, f0)) break;
-        if (!turn(r2, r3, r1, m0, m1, f0, f1)) break;
-        if (!turn(r3, r0, r2, m1, m0, f1, f0)) break;
     }
 }
 
@@ -1468,23 +1481,11 @@ __device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDe
                                               Mom4<T>* fs, T alfa, T beta) {
     const int c = min((int)(threadIdx.x & 3), 2), nlev = pd.n_levels;
     if (nlev == 0) return;
-    // Level ends without a load in the loop, whose wait would include every load
-    // before it: lane i of the wave holds the end of level base + i.
     const int64_t* off = fg.lev_off + pd.lev;
     const int64_t q0 = off[0];
-    int base = 0, ends = 0;
-    auto hold = [&](int l) {
-        base = l;
-        ends = (int)(off[min(l + (int)(threadIdx.x & 63), nlev - 1) + 1] - q0);
-    };
-    hold(0);
     const ForceRow<T>* rows = static_cast<const ForceRow<T>*>(fg.rows) + 3 * q0 + c;
     run_levels<T, false, F_LDS>(
-        nlev, alfa, beta,
-        [&](int l) {
-            if (l - base >= 64) hold(l);
-            return __builtin_amdgcn_readlane(ends, l - base);
-        },
+        nlev, alfa, beta, [&](int l) { return (int)(off[l + 1] - q0); },
         [&](int q) { return rows[3 * (int64_t)q]; },
         [&](int, const ForceRow<T>& r, Mom4<T> (&m)[3]) {
 #pragma unroll
@@ -1495,7 +1496,7 @@ __device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDe
             for (int b = 0; b < 3; b++) {
                 if constexpr (F_LDS) {
 #pragma unroll
-                    for (int a = 0; a < 3; a++) f[b][a] = lf[3 * r.e[b] + a];
+                    for (int a = 0; a < 3; a++) f[b][a] = lf[__umul24(r.e[b], 3) + a];
                 } else {
                     const Mom4<T> w = fs[r.e[b]];
                     f[b][0] = w.r;
@@ -1509,7 +1510,7 @@ __device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDe
             for (int b = 0; b < 3; b++) {
                 if constexpr (F_LDS) {
 #pragma unroll
-                    for (int a = 0; a < 3; a++) lf[3 * r.e[b] + a] = f[b][a];
+                    for (int a = 0; a < 3; a++) lf[__umul24(r.e[b], 3) + a] = f[b][a];
                 } else {
                     fs[r.e[b]] = Mom4<T>{f[b][0], f[b][1], f[b][2], T(0)};
                 }
@@ -1575,23 +1576,9 @@ __device__ __forceinline__ void blade_levels(const ForceGeom& fg, const Grid& g,
         }
     }
     if constexpr (F_LDS) __syncthreads();
-    // lane i of the wave holds the end of level base + i (of the first 64, then the next)
-    int base = -64, ends = 0;
     run_levels<T, ROWS_LDS, F_LDS>(
         nlev, alfa, beta,
-        [&](int l) {
-            if (l - base >= 64) {
-                const int before = base < 0 ? 0 : __builtin_amdgcn_readlane(ends, 63), at = (int)(threadIdx.x & 63);
-                base += 64;
-                ends = base + at < nlev ? blade_level_count(fg.blade, base + at) : 0;
-                for (int o = 1; o < 64; o <<= 1) {
-                    const int up = __shfl_up(ends, o, 64);
-                    if (at >= o) ends += up;
-                }
-                ends += before;
-            }
-            return __builtin_amdgcn_readlane(ends, l - base);
-        },
+        [&](int l) { return blade_level_end(fg.blade, l); },
         [&](int q) {
             if constexpr (ROWS_LDS) return lr[3 * q + c].r;
             else return rows[3 * q + c];
@@ -1607,14 +1594,14 @@ __device__ __forceinline__ void blade_levels(const ForceGeom& fg, const Grid& g,
 #pragma unroll
             for (int b = 0; b < 3; b++)
 #pragma unroll
-                for (int a = 0; a < 3; a++) f[b][a] = F_LDS ? ld[3 * r.e[b] + a] : F[3 * (uint64_t)(uint32_t)r.e[b] + a];
+                for (int a = 0; a < 3; a++) f[b][a] = F_LDS ? ld[__umul24(r.e[b], 3) + a] : F[3 * (uint64_t)(uint32_t)r.e[b] + a];
         },
         [&](const ForceRow<T>& r, const T (&f)[3][3]) {
 #pragma unroll
             for (int b = 0; b < 3; b++)
 #pragma unroll
                 for (int a = 0; a < 3; a++) {
-                    if constexpr (F_LDS) ld[3 * r.e[b] + a] = f[b][a];
+                    if constexpr (F_LDS) ld[__umul24(r.e[b], 3) + a] = f[b][a];
                     else F[3 * (uint64_t)(uint32_t)r.e[b] + a] = f[b][a];
                 }
         });
