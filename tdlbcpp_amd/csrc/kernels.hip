@@ -37,11 +37,6 @@ constexpr int kRowBlock = 512;
 template <typename S>
 constexpr int row_block_max() { return kRowBlock; }
 
-inline uint32_t blocks_for(uint64_t n, int bs = kBlock) {
-    uint64_t b = (n + bs - 1) / bs;
-    return (uint32_t)(b > 0x7fffffffull ? 0x7fffffffull : (b ? b : 1));
-}
-
 // Blocks take rows in dispatch order (round-robin over the 8 XCDs): every line is
 // read by one row only, and all XCDs streaming through one region of HBM together
 // are 5 % faster than each XCD on a contiguous range of its own.
@@ -1518,12 +1513,6 @@ __device__ __forceinline__ void static_levels(const ForceGeom& fg, const PlaneDe
         });
 }
 
-// cell n of plane j in the plane's own (i, k) order
-__device__ __forceinline__ int plane_index(const Grid& g, uint32_t n, int j) {
-    const int i = (int)(n / g.yz), k = (int)(n - (uint32_t)i * g.yz - (uint32_t)j * (uint32_t)g.zg);
-    return (i - 1) * g.zg1 + k - 1;
-}
-
 // The blade levels of a plane.  With room in LDS the rows and moments of all its
 // points come there first (blade_rows), and if a copy of the whole plane's force
 // values fits beside them the stencil cells' too: a level then waits on LDS alone.
@@ -1744,13 +1733,6 @@ __device__ __forceinline__ void pipe_wait(const uint32_t* a, uint32_t ta, const 
     }
     __syncthreads();
 }
-// every store of the workgroup is complete in L2, then thread 0 counts it
-__device__ __forceinline__ void pipe_done(uint32_t* ctr) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // rows of one item of the pipe (consecutive j of one i step)
 constexpr uint32_t kPipeRows = 8;
 
