@@ -190,7 +190,9 @@ int tdlb_rushton_solid_mask(const tdlb_rushton_params* p, int64_t xg, int64_t yg
  * The impeller must lie inside the interior (TDLB_ERR_INVALID otherwise); the
  * blades are forced in colour classes of non-overlapping stencils, a class per
  * blade in tanks too small for shared classes (the generator's rotating list
- * follows the same classes), so every tank size binds. */
+ * follows the same classes), so every tank size binds.  Arguments that are
+ * refused leave an earlier geometry bound; a bind that fails later (memory)
+ * leaves the handle without one (TDLB_ERR_STATE from tdlb_cu_run). */
 int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t step, double angle, double alfa,
                          double beta);
 /* Run nsteps iterations of the main loop: step += 1; angle += increment(step);

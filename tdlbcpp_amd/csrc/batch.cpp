@@ -575,6 +575,9 @@ int tdlb_batch_run(tdlb_batch_t b, int64_t nsteps, int64_t* steps_run) {
     // every member takes min(nsteps, remaining) steps; one whose state is not
     // the steady fused state takes the first of them alone
     int64_t most = 0, K = 0;
+    for (auto& m : b->members)
+        if (m.remaining > 0 && !m.cu->bound)
+            return fail(TDLB_ERR_STATE, "a member has no bound geometry (its last tdlb_cu_bind_rushton failed)");
     for (auto& m : b->members) {
         HIPCHK(hipStreamSynchronize(m.cu->stream));
         m.call = std::min<int64_t>(m.remaining, nsteps);

@@ -1229,6 +1229,9 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     CHK(check_points(cu, stat.data(), (int64_t)stat.size()));
     CHK(check_points(cu, rot.data(), (int64_t)rot.size()));
 
+    // the tables of an earlier bind go from here on: a bind that fails leaves the handle unbound
+    cu->bound = false;
+    cu->pipe = false;
     cu->n_static = (int64_t)stat.size();
     cu->n_rot = (int64_t)rot.size();
     cu->n_blade_classes = cu->n_rot > 0 ? 5 * be.n_bcol : 0;
@@ -1283,7 +1286,6 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
         HIPCHK(hipMemcpyAsync(cu->static_base, a.data(), cu->mask_bytes(), hipMemcpyHostToDevice, cu->stream));
         HIPCHK(hipStreamSynchronize(cu->stream));
     }
-    cu->bound = true;
     cu->alfa = alfa;
     cu->beta = beta;
     HIPCHK(allow_level_lds(cu->eprec()));
@@ -1291,6 +1293,7 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
 
     // initial forcing of main.cpp:305 on the current density and momentum
     CHK(bound_forcing(cu, cell_source(cu).momsrc, true, blade_step(cu, angle, delta)));
+    cu->bound = true;
     return TDLB_OK;
 }
 

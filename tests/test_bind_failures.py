@@ -1,0 +1,58 @@
+"""A bind that fails leaves no half-made geometry to run on (CPU)."""
+from tests.host_library import host_library  # noqa: F401
+
+
+def test_failed_rebind_leaves_the_handle_unbound(host_library):  # noqa: F811
+    """Whichever allocation of a second bind fails: run and batches refuse the handle (TDLB_ERR_STATE), no
+    forcing is launched on it, and a bind that succeeds makes it runnable again."""
+    host_library("""
+    rp = td.rushton_defaults(36)
+    one, ang = ctypes.c_uint64(1), ctypes.c_double(0.0)
+    n = 0
+    while True:
+        cu = td.ComputeUnit(48)
+        cu.initialise(1.0)
+        cu.bind_rushton(td.rushton_defaults(24))  # fewer points than the second geometry: its buffers grow
+        batch, other = td.Batch(td.PREC_F32), td.Batch(td.PREC_F32)
+        batch.add(cu, 1000)
+        batch.run(2)
+        L.fake_fail_malloc(n)
+        rc = L.tdlb_cu_bind_rushton(cu._h, ctypes.byref(rp), 1, 0.0, 0.97, 1.9)
+        L.fake_fail_malloc(-1)
+        L.hipGetLastError()
+        if rc != 0:
+            assert rc == NOMEM, rc
+            before = L.fake_gathers()
+            assert L.tdlb_cu_run(cu._h, 1, ctypes.byref(one), ctypes.byref(ang)) == STATE, n
+            assert L.tdlb_batch_run(batch._b, 1, None) == STATE, n
+            assert L.tdlb_batch_add(other._b, cu._h, 1, 0.0, 5) == STATE, n
+            assert L.fake_gathers() == before
+            cu.bind_rushton(rp)
+        cu.run(1)
+        batch.run(1)
+        batch.close()
+        other.close()
+        cu.close()
+        if rc == 0:
+            break
+        n += 1
+    assert n > 8
+    """)
+
+
+def test_refused_rebind_keeps_the_earlier_geometry(host_library):  # noqa: F811
+    """Arguments that are refused are refused before anything of the bound geometry changes."""
+    host_library("""
+    cu = tank(36)
+    info = cu.forcing_info()
+    rp = td.rushton_defaults(36)
+    rp.n_blades = 17
+    try:
+        cu.bind_rushton(rp)
+        raise SystemExit("17 blades accepted")
+    except td.TdlbError:
+        pass
+    cu.run(2)
+    assert cu.forcing_info() == info
+    cu.close()
+    """)
