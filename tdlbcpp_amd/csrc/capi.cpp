@@ -971,9 +971,12 @@ int tdlb_cu_field_bytes(tdlb_cu_t cu, int field, size_t* bytes) {
 }
 
 // A result to host memory, formed piece by piece (readback.h).
-static int read_result(tdlb_cu* cu, void* host, size_t bytes, size_t align, const char* what, const PieceFn& piece) {
-    const hipError_t e = read_back(cu->device, cu->stream, host, bytes, align, piece);
-    if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
+static int read_result(tdlb_cu* cu, void* host, size_t bytes, size_t align, const char* what, const PieceFn& piece,
+                       const void* array = nullptr) {
+    const hipError_t e = read_back(cu->device, cu->stream, host, bytes, align, piece, array);
+    if (e != hipSuccess)
+        return fail(e == hipErrorOutOfMemory ? TDLB_ERR_NOMEM : TDLB_ERR_HIP,
+                    std::string(what) + ": " + hipGetErrorString(e));
     return TDLB_OK;
 }
 
@@ -1017,9 +1020,12 @@ int tdlb_cu_download(tdlb_cu_t cu, int field, void* host, size_t bytes) {
             return launch_nu_convert(cu->prec(), 1, (const char*)cu->Nu + a / ts * cu->ssize, dst, (b - a) / ts, s);
         });
     const char* src = static_cast<const char*>(field == TDLB_FIELD_NU ? cu->Nu : (const void*)cu->O);
-    return read_result(cu, host, need, 16, "download", [&](void* dst, size_t a, size_t b, hipStream_t s) {
-        return hipMemcpyAsync(dst, src + a, b - a, hipMemcpyDeviceToHost, s);
-    });
+    return read_result(
+        cu, host, need, 16, "download",
+        [&](void* dst, size_t a, size_t b, hipStream_t s) {
+            return hipMemcpyAsync(dst, src + a, b - a, hipMemcpyDeviceToHost, s);
+        },
+        src);
 }
 
 int tdlb_cu_upload(tdlb_cu_t cu, int field, const void* host, size_t bytes) {

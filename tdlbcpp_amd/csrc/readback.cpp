@@ -12,17 +12,18 @@
 // The pinned buffers are kept between calls (fresh ones fault page by page on the
 // host's first reads, at 2 GB/s): at most kMaxRings of each of two sizes, shared by
 // all handles and threads, given back with the last handle.  A caller that finds
-// all of its size in use waits for one.
+// all of its size in use waits for one; where pinned memory is not to be had, pieces
+// are formed in device memory and copied from there.  No C++ exception leaves here:
+// fewer threads do the work where more are not to be had.
 #include "readback.h"
 
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 namespace tdlb {
 namespace {
@@ -35,26 +36,52 @@ constexpr size_t kRingBytes[2] = {kMinPiece, (size_t)kMaxThreads << 22};
 
 std::mutex g_mu;
 std::condition_variable g_cv;
-std::vector<void*> g_idle[2];
-int g_rings[2] = {0, 0}, g_handles = 0;
+void* g_idle[2][kMaxRings];
+int g_n_idle[2] = {0, 0}, g_rings[2] = {0, 0}, g_handles = 0;
 
-hipError_t take_ring(int kind, void** ring) {
+// null: no buffer of this size is there and none can be made
+void* take_ring(int kind) {
     std::unique_lock<std::mutex> lk(g_mu);
-    g_cv.wait(lk, [&] { return !g_idle[kind].empty() || g_rings[kind] < kMaxRings; });
-    if (!g_idle[kind].empty()) {
-        *ring = g_idle[kind].back();
-        g_idle[kind].pop_back();
-        return hipSuccess;
+    for (;;) {
+        if (g_n_idle[kind] > 0) return g_idle[kind][--g_n_idle[kind]];
+        if (g_rings[kind] < kMaxRings) {
+            void* ring = nullptr;
+            if (hipHostMalloc(&ring, kRingBytes[kind], hipHostMallocPortable) == hipSuccess) {
+                g_rings[kind]++;
+                return ring;
+            }
+            (void)hipGetLastError();  // not the next launch's
+            if (g_rings[kind] == 0) return nullptr;
+        }
+        g_cv.wait(lk, [&] { return g_n_idle[kind] > 0; });
     }
-    const hipError_t e = hipHostMalloc(ring, kRingBytes[kind], hipHostMallocPortable);
-    if (e == hipSuccess) g_rings[kind]++;
-    return e;
 }
 
 void give_ring(int kind, void* ring) {
     std::lock_guard<std::mutex> lk(g_mu);
-    g_idle[kind].push_back(ring);
+    g_idle[kind][g_n_idle[kind]++] = ring;
     g_cv.notify_all();
+}
+
+// Without pinned memory: pieces in device memory, copied from there one after the other.
+hipError_t by_device_pieces(hipStream_t s, char* host, size_t bytes, size_t align, const PieceFn& piece) {
+    size_t part = std::min(bytes, (size_t)1 << 29);
+    void* buf = nullptr;
+    for (;; part /= 2) {
+        if (hipMalloc(&buf, part) == hipSuccess) break;
+        (void)hipGetLastError();
+        if (part / 2 < kMinPiece) return hipErrorOutOfMemory;
+    }
+    part = part / align * align;
+    hipError_t e = hipSuccess;
+    for (size_t begin = 0; begin < bytes && e == hipSuccess; begin += part) {
+        const size_t end = std::min(bytes, begin + part);
+        e = piece(buf, begin, end, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(host + begin, buf, end - begin, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+    }
+    (void)hipFree(buf);
+    return e;
 }
 
 }  // namespace
@@ -64,18 +91,22 @@ void readback_handle(int change) {
     g_handles += change;
     if (g_handles > 0) return;
     for (int kind = 0; kind < 2; kind++) {
-        for (void* p : g_idle[kind]) (void)hipHostFree(p);
-        g_rings[kind] -= (int)g_idle[kind].size();
-        g_idle[kind].clear();
+        for (int a = 0; a < g_n_idle[kind]; a++) (void)hipHostFree(g_idle[kind][a]);
+        g_rings[kind] -= g_n_idle[kind];
+        g_n_idle[kind] = 0;
     }
 }
 
-hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece) {
+hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece,
+                     const void* array) {
     if (bytes == 0) return hipStreamSynchronize(s);
     const int kind = bytes <= kMinPiece ? 0 : 1;
-    void* ring = nullptr;
-    hipError_t e = take_ring(kind, &ring);
-    if (e != hipSuccess) return e;
+    void* const ring = take_ring(kind);
+    if (!ring && array) {
+        const hipError_t e = hipMemcpyAsync(host, array, bytes, hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    }
+    if (!ring) return by_device_pieces(s, static_cast<char*>(host), bytes, align, piece);
     // a thread per piece in flight; small results take the calling thread only
     const int cpus = std::max(1, (int)std::thread::hardware_concurrency());
     const int most = (int)std::min<size_t>(std::max(1, std::min(kMaxThreads, cpus / 2)), (bytes + kMinPiece - 1) / kMinPiece);
@@ -100,15 +131,16 @@ hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t
         if (done) (void)hipEventDestroy(done);
         if (r != hipSuccess) failed.store(r);
     };
-    std::vector<std::thread> threads;
+    std::thread threads[kMaxThreads];
+    int started = 1;
     try {
-        for (int t = 1; t < most; t++) threads.emplace_back(work, t);
-    } catch (const std::system_error&) {
-        // no more threads to be had: the ones there are do the work
+        for (; started < most; started++) threads[started] = std::thread(work, started);
+    } catch (const std::exception&) {
+        // no more threads (std::system_error) or memory for one: the ones there are do the work
     }
     work(0);
-    for (std::thread& t : threads) t.join();
-    e = (hipError_t)failed.load();
+    for (int t = 1; t < started; t++) threads[t].join();
+    const hipError_t e = (hipError_t)failed.load();
     if (e != hipSuccess) (void)hipStreamSynchronize(s);  // nothing may write to the ring any more
     give_ring(kind, ring);
     return e;

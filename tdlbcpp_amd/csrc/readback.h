@@ -3,17 +3,34 @@
 
 #include <hip/hip_runtime.h>
 #include <cstddef>
-#include <functional>
 
 namespace tdlb {
 
-// Enqueues on `s` whatever writes bytes [begin, end) of the result to dst, which
-// is pinned host memory that the GPU can write.
-using PieceFn = std::function<hipError_t(void* dst, size_t begin, size_t end, hipStream_t s)>;
+// A reference to a callable (dst, begin, end, stream) that enqueues whatever writes
+// bytes [begin, end) of the result to dst: pinned host memory that the GPU can
+// write, or device memory.
+class PieceFn {
+public:
+    template <typename Fn>
+    PieceFn(const Fn& fn)
+        : fn_(&fn), call_([](const void* f, void* dst, size_t begin, size_t end, hipStream_t s) {
+              return (*static_cast<const Fn*>(f))(dst, begin, end, s);
+          }) {}
+    hipError_t operator()(void* dst, size_t begin, size_t end, hipStream_t s) const {
+        return call_(fn_, dst, begin, end, s);
+    }
+
+private:
+    const void* fn_;
+    hipError_t (*call_)(const void*, void*, size_t, size_t, hipStream_t);
+};
 
 // `bytes` of a result to host memory, after the work already on `s`; returns when
-// they are there.  Pieces are multiples of `align` bytes.
-hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece);
+// they are there.  Pieces are multiples of `align` bytes.  array: the result where it
+// lies in device memory as it is, else null.  hipErrorOutOfMemory: neither pinned nor
+// device memory for a piece.
+hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece,
+                     const void* array = nullptr);
 
 // A handle came or went: the pinned buffers are given back with the last one.
 void readback_handle(int change);

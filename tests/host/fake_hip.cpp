@@ -28,6 +28,11 @@ int64_t fail_malloc = -1, fail_pinned = -1;  // allocations until one fails, -1:
 int64_t mallocs = 0, pinned_mallocs = 0, gathers = 0;
 std::atomic<int64_t> fail_new{-1};
 thread_local hipError_t last = hipSuccess;
+thread_local int within = 0;  // allocations of this file's own do not fail
+struct Within {
+    Within() { within++; }
+    ~Within() { within--; }
+};
 
 hipError_t error(hipError_t e) { return last = e; }
 hipError_t launched() {  // what a launcher ends with
@@ -75,7 +80,7 @@ int64_t fake_gathers() { return gathers; }
 }
 
 void* operator new(size_t n) {
-    if (fail_new.load() >= 0 && fail_new.fetch_sub(1) == 0) throw std::bad_alloc();
+    if (!within && fail_new.load() >= 0 && fail_new.fetch_sub(1) == 0) throw std::bad_alloc();
     if (void* p = std::malloc(n ? n : 1)) return p;
     throw std::bad_alloc();
 }
@@ -85,6 +90,7 @@ void operator delete(void* p, size_t) noexcept { std::free(p); }
 // ---------------------------------------------------------------- the runtime
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
+    Within own;
     std::lock_guard<std::mutex> lk(mu);
     *p = nullptr;
     mallocs++;
@@ -106,6 +112,7 @@ hipError_t hipFree(void* p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    Within own;
     std::lock_guard<std::mutex> lk(mu);
     *p = nullptr;
     if (fails(fail_pinned)) return error(hipErrorOutOfMemory);

@@ -39,7 +39,7 @@ def tank(T, prec=td.PREC_F32, bind=True, **kw):
 
 @pytest.fixture(scope="session")
 def host_library(tmp_path_factory):
-    """run(body): the Python code of a test over the host library, in a child process"""
+    """run(*bodies): the Python code of a test over the host library, in a child process"""
     out = tmp_path_factory.mktemp("host")
     flags = ["-D__HIP_PLATFORM_AMD__", "-D__align__(n)=__attribute__((aligned(n)))", "-DHIP_SYMBOL(x)=(x)",
              "-I/opt/rocm/include", "-O1", "-std=c++17", "-fPIC", "-ffp-contract=off", "-w"]
@@ -53,8 +53,8 @@ def host_library(tmp_path_factory):
     subprocess.run(["g++", "-shared", "-pthread", "-Wl,-Bsymbolic,-z,defs", "-o", lib] + [o for o, _ in jobs],
                    check=True)
 
-    def run(body, timeout=120):
-        code = PRELUDE.format(root=ROOT, lib=lib) + textwrap.dedent(body)
+    def run(*bodies, timeout=120):
+        code = PRELUDE.format(root=ROOT, lib=lib) + "".join(textwrap.dedent(b) for b in bodies)
         r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=timeout)
         assert r.returncode == 0, f"exit {r.returncode}\n{r.stdout}\n{r.stderr[-4000:]}"
 
