@@ -34,17 +34,38 @@ constexpr size_t kMinPiece = (size_t)1 << 20;
 // results of one piece, and larger ones: a slot of 4 MiB per thread
 constexpr size_t kRingBytes[2] = {kMinPiece, (size_t)kMaxThreads << 22};
 
+// Making a buffer and giving it back costs 1 to 4 ms where the buffer is large (the
+// next allocations pay for it), so programs that read little between their first
+// handle and their last take the plain copy.  A tank created, read and destroyed, by
+// plain copies and through buffers made at once: 60^3 with three results (10 MB) 0.92
+// and 1.8 ms, 80^3 (23 MB) 1.7 and 2.9, 96^3 one result (14 MB) 2.7 and 2.6, 128^3
+// (34 MB) 5.9 and 3.3; of small results 36^3 one (0.7 MB) 0.24 and 0.35.
+constexpr int kSmallReads = 4;                      // the small buffer from the fourth small result on
+constexpr size_t kLargeRead = (size_t)12 << 20;     // the large one for a result of this size
+constexpr size_t kLargeBytes = (size_t)64 << 20;    // or from this many bytes of larger ones on
+// Arrays that lie in device memory as they are come by a plain copy up to here: O of
+// 30^3 11 us (through a buffer 19), of 100^3 (1.1 MB) 68 (80), Nu of 100^3 (4.2 MB) 240 (205).
+constexpr size_t kPlainArray = (size_t)2 << 20;
+
 std::mutex g_mu;
 std::condition_variable g_cv;
 void* g_idle[2][kMaxRings];
 int g_n_idle[2] = {0, 0}, g_rings[2] = {0, 0}, g_handles = 0;
+int g_reads[2] = {0, 0};  // reads while there was no buffer, and their bytes
+size_t g_bytes[2] = {0, 0};
 
-// null: no buffer of this size is there and none can be made
-void* take_ring(int kind) {
+// null: no buffer of this size is there, and none can be made or is worth it yet
+void* take_ring(int kind, size_t bytes) {
     std::unique_lock<std::mutex> lk(g_mu);
     for (;;) {
         if (g_n_idle[kind] > 0) return g_idle[kind][--g_n_idle[kind]];
         if (g_rings[kind] < kMaxRings) {
+            if (g_rings[kind] == 0) {
+                g_reads[kind]++;
+                g_bytes[kind] += bytes;
+                if (kind == 0 ? g_reads[kind] < kSmallReads : bytes < kLargeRead && g_bytes[kind] < kLargeBytes)
+                    return nullptr;
+            }
             void* ring = nullptr;
             if (hipHostMalloc(&ring, kRingBytes[kind], hipHostMallocPortable) == hipSuccess) {
                 g_rings[kind]++;
@@ -94,6 +115,8 @@ void readback_handle(int change) {
         for (int a = 0; a < g_n_idle[kind]; a++) (void)hipHostFree(g_idle[kind][a]);
         g_rings[kind] -= g_n_idle[kind];
         g_n_idle[kind] = 0;
+        g_reads[kind] = 0;
+        g_bytes[kind] = 0;
     }
 }
 
@@ -101,7 +124,7 @@ hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t
                      const void* array) {
     if (bytes == 0) return hipStreamSynchronize(s);
     const int kind = bytes <= kMinPiece ? 0 : 1;
-    void* const ring = take_ring(kind);
+    void* const ring = array && bytes <= kPlainArray ? nullptr : take_ring(kind, bytes);
     if (!ring && array) {
         const hipError_t e = hipMemcpyAsync(host, array, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;

@@ -68,3 +68,35 @@ def test_host_memory_short_while_threads_start(host_library, n):  # noqa: F811
         assert np.array_equal(out.reshape(-1, 4)[:, 0], np.arange(101 ** 3))
     cu.close()
     """)
+
+
+def test_pinned_memory_is_made_where_it_pays(host_library):  # noqa: F811
+    """Programs that read little between their first handle and their last make no pinned memory; it is given
+    back with the last handle, and arrays that lie in device memory as they are do without while small."""
+    host_library("""
+    def reads(T, n, read, want):
+        L.fake_limit(1 << 40)
+        before, cu = L.fake_pinned_mallocs(), tank(T, bind=False)
+        for _ in range(n):
+            read(cu)
+        assert L.fake_pinned_mallocs() - before == want, (T, n, L.fake_pinned_mallocs() - before)
+        cu.close()
+        assert L.fake_pinned() == 0
+    field = lambda cu: cu.macroscopic()
+    for _ in range(2):
+        reads(36, 3, field, 0)
+        reads(36, 9, field, 1)
+        reads(80, 3, field, 0)     # 8.2 MB each: from 64 MiB on
+        reads(80, 9, field, 1)
+        reads(96, 1, field, 1)     # 14 MB
+        reads(30, 20, lambda cu: cu.get(td.FIELD_O), 0)
+        reads(60, 20, lambda cu: cu.get(td.FIELD_NU), 0)
+    a, b = tank(36, bind=False), tank(36, bind=False)
+    for _ in range(4):
+        a.macroscopic()
+    a.close()
+    assert L.fake_pinned() == 1    # the other handle's reads find it
+    b.macroscopic()
+    b.close()
+    assert L.fake_pinned() == 0 and L.fake_live() == 0
+    """)
