@@ -980,22 +980,23 @@ static int read_result(tdlb_cu* cu, void* host, size_t bytes, size_t align, cons
     return TDLB_OK;
 }
 
-// The explicit Q from host memory, converted to the kernels' array in pieces, so
-// that a lattice of more than half the memory still moves.
+// The explicit Q from host memory, converted to the kernels' array piece by piece: the
+// stream orders a piece's copy after the conversion of the one before.
 static int upload_q(tdlb_cu* cu, const void* host, size_t bytes) {
-    const size_t piece = std::min(bytes, (size_t)1 << 29);
-    void* tmp = nullptr;
-    if (hipMalloc(&tmp, piece) != hipSuccess) return fail(TDLB_ERR_NOMEM, "upload Q staging");
+    size_t piece = 0;
+    void* const stage = take_stage(cu->device, &piece);
+    if (!stage) return fail(TDLB_ERR_NOMEM, "upload Q staging");
     hipError_t e = hipSuccess;
     for (size_t at = 0; at < bytes && e == hipSuccess; at += piece) {
         const size_t n = std::min(piece, bytes - at);
-        e = hipMemcpyAsync(tmp, (const char*)host + at, n, hipMemcpyHostToDevice, cu->stream);
+        e = hipMemcpyAsync(stage, (const char*)host + at, n, hipMemcpyHostToDevice, cu->stream);
         if (e == hipSuccess)
-            e = launch_q_boundary((int)cu->tsize, cu->blay(), 0, cu->eq(), tmp, at / cu->tsize, (at + n) / cu->tsize,
-                                  cu->g, cu->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
+            e = launch_q_boundary((int)cu->tsize, cu->blay(), 0, cu->eq(), stage, at / cu->tsize,
+                                  (at + n) / cu->tsize, cu->g, cu->stream);
     }
-    (void)hipFree(tmp);
+    const hipError_t end = hipStreamSynchronize(cu->stream);
+    give_stage(cu->device, stage, piece);
+    if (e == hipSuccess) e = end;
     if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("upload Q: ") + hipGetErrorString(e));
     return TDLB_OK;
 }

@@ -54,6 +54,9 @@ int g_n_idle[2] = {0, 0}, g_rings[2] = {0, 0}, g_handles = 0;
 int g_reads[2] = {0, 0};  // reads while there was no buffer, and their bytes
 size_t g_bytes[2] = {0, 0};
 
+constexpr int kStageDevices = 64;  // tdlb_cu_create refuses device ids beyond
+void* g_stage[kStageDevices] = {};
+
 // null: no buffer of this size is there, and none can be made or is worth it yet
 void* take_ring(int kind, size_t bytes) {
     std::unique_lock<std::mutex> lk(g_mu);
@@ -111,6 +114,10 @@ void readback_handle(int change) {
     std::lock_guard<std::mutex> lk(g_mu);
     g_handles += change;
     if (g_handles > 0) return;
+    for (void*& p : g_stage) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    }
     for (int kind = 0; kind < 2; kind++) {
         for (int a = 0; a < g_n_idle[kind]; a++) (void)hipHostFree(g_idle[kind][a]);
         g_rings[kind] -= g_n_idle[kind];
@@ -118,6 +125,34 @@ void readback_handle(int change) {
         g_reads[kind] = 0;
         g_bytes[kind] = 0;
     }
+}
+
+void* take_stage(int device, size_t* bytes) {
+    *bytes = kStageBytes;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if (void* p = g_stage[device]) {
+            g_stage[device] = nullptr;
+            return p;
+        }
+    }
+    for (; *bytes >= kMinPiece; *bytes /= 2) {
+        void* p = nullptr;
+        if (hipMalloc(&p, *bytes) == hipSuccess) return p;
+        (void)hipGetLastError();  // not the next launch's
+    }
+    return nullptr;
+}
+
+void give_stage(int device, void* stage, size_t bytes) {
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if (bytes == kStageBytes && !g_stage[device]) {
+            g_stage[device] = stage;
+            return;
+        }
+    }
+    (void)hipFree(stage);
 }
 
 hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece,

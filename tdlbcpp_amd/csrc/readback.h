@@ -1,4 +1,5 @@
-// Device results into pageable host memory (private to the library).
+// Device results into pageable host memory, and the staging of uploads (private to
+// the library).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -32,7 +33,15 @@ private:
 hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece,
                      const void* array = nullptr);
 
-// A handle came or went: the pinned buffers are given back with the last one.
+// A piece of device memory for an upload that is converted on the device, kStageBytes or,
+// where memory is short, less (bytes says how much; null: there is none).  One a device
+// is kept between uploads: allocating and freeing it costs 50 us, a tenth of a 60^3
+// tank's Q.  The caller's work on it has ended when it is given back.
+constexpr size_t kStageBytes = (size_t)16 << 20;
+void* take_stage(int device, size_t* bytes);
+void give_stage(int device, void* stage, size_t bytes);
+
+// A handle came or went: what is kept between calls is given back with the last one.
 void readback_handle(int change);
 
 }  // namespace tdlb

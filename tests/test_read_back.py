@@ -100,3 +100,31 @@ def test_pinned_memory_is_made_where_it_pays(host_library):  # noqa: F811
     b.close()
     assert L.fake_pinned() == 0 and L.fake_live() == 0
     """)
+
+
+def test_uploads_share_a_stage(host_library):  # noqa: F811
+    """Uploads of Q allocate device memory once, whatever the number of handles and sizes; short memory makes the
+    pieces smaller, none is TDLB_ERR_NOMEM, and the stage goes with the last handle."""
+    host_library("""
+    a, b = tank(30, td.PREC_F64, bind=False), tank(70, bind=False)
+    def upload(cu):
+        q = np.random.default_rng(1).random(cu.field_bytes(td.FIELD_Q) // np.dtype(cu.np_dtype).itemsize).astype(cu.np_dtype)
+        cu.set(td.FIELD_Q, q)
+        assert np.array_equal(cu.get(td.FIELD_Q), q)
+    upload(a)
+    n = L.fake_mallocs()
+    a.set(td.FIELD_Q, a.get(td.FIELD_Q))
+    b.set(td.FIELD_Q, np.zeros(b.field_bytes(td.FIELD_Q) // 4, dtype=np.float32))
+    assert L.fake_mallocs() == n + 1        # the download's piece
+    a.close()
+    b.close()
+    assert L.fake_live() == 0
+    b = tank(70, bind=False)
+    L.fake_limit(L.fake_live() + (3 << 20))
+    upload(b)
+    L.fake_limit(L.fake_live() + 1000)
+    q = np.zeros(b.field_bytes(td.FIELD_Q) // 4, dtype=np.float32)
+    assert L.tdlb_cu_upload(b._h, td.FIELD_Q, q.ctypes.data, q.nbytes) == NOMEM
+    b.close()
+    assert L.fake_live() == 0
+    """)
