@@ -229,10 +229,15 @@ int list_levels(tdlb_cu* cu, const std::vector<tdlb_ib_point>& pts, std::vector<
         ijk[n + q] = (int32_t)pts[q].j + gh;
         ijk[2 * n + q] = (int32_t)pts[q].k + gh;
     }
-    const size_t marks = list_marks_bytes(cu->g, nullptr);
-    char* buf = nullptr;  // positions, i, j, k, levels, marks
-    if (hipMalloc((void**)&buf, n * (sizeof(int64_t) + 4 * sizeof(int32_t)) + marks) != hipSuccess)
+    char* buf = nullptr;  // positions, i, j, k, levels
+    if (hipMalloc((void**)&buf, n * (sizeof(int64_t) + 4 * sizeof(int32_t))) != hipSuccess)
         return fail(TDLB_ERR_NOMEM, "IB level buffers");
+    uint32_t* marks = nullptr;
+    int blocks = 0;
+    if (const int rc = reserve_marks(cu->g, &marks, &blocks)) {
+        (void)hipFree(buf);
+        return rc;
+    }
     auto* list = reinterpret_cast<int64_t*>(buf);
     auto* i32 = reinterpret_cast<int32_t*>(list + n);
     PointsDev p{};
@@ -241,12 +246,12 @@ int list_levels(tdlb_cu* cu, const std::vector<tdlb_ib_point>& pts, std::vector<
     p.k = i32 + 2 * n;
     hipError_t e = hipMemcpyAsync(i32, ijk.data(), 3 * n * sizeof(int32_t), hipMemcpyHostToDevice, cu->stream);
     if (e == hipSuccess)
-        e = launch_list_levels(p, (int64_t)n, list, marks ? reinterpret_cast<uint32_t*>(i32 + 4 * n) : nullptr,
-                               i32 + 3 * n, cu->g, cu->stream);
+        e = launch_list_levels(p, (int64_t)n, list, marks, blocks, i32 + 3 * n, cu->g, cu->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(lev.data(), i32 + 3 * n, n * sizeof(int32_t), hipMemcpyDeviceToHost, cu->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(cu->stream);
     (void)hipFree(buf);
+    if (marks) (void)hipFree(marks);
     if (e != hipSuccess) return fail(TDLB_ERR_HIP, std::string("IB levels: ") + hipGetErrorString(e));
     return TDLB_OK;
 }
@@ -936,7 +941,7 @@ int tdlb_cu_forcing(tdlb_cu_t cu, const tdlb_ib_point* points, int64_t n, double
     CHK(materialise(cu));
     // the caller's points as they are, spread and ordered on the device
     CHK(cu->api_pts.reserve(n, cu->tsize));
-    CHK(cu->api_lists.reserve(n, list_marks_bytes(cu->g, nullptr)));
+    CHK(cu->api_lists.reserve(n, cu->g));
     uint64_t* prev = cu->fmask[cu->fm];
     uint64_t* next = cu->fmask[1 - cu->fm];
     if (n > 0) {
@@ -947,7 +952,7 @@ int tdlb_cu_forcing(tdlb_cu_t cu, const tdlb_ib_point* points, int64_t n, double
     HIPCHK(launch_list_unpack(cu->prec(), cu->api_lists.raw, n, (int)cu->prm.ghost, cu->api_pts.d, cu->gmask, next,
                               cu->mask_words, cu->stream));
     HIPCHK(launch_list_planes(cu->prec(), cu->prm.streaming, cu->even ? 1 : 0, cu->api_pts.d, n, cu->api_lists.list,
-                              cu->api_lists.marks, cu->eq(), cu->F, prev, next, cu->g, alfa, beta, cu->rho0,
+                              cu->api_lists.marks, cu->api_lists.blocks, cu->eq(), cu->F, prev, next, cu->g, alfa, beta, cu->rho0,
                               cu->stream));
     if (cu->o_dirty) {
         HIPCHK(launch_zero_interior_o(cu->O, cu->g, cu->stream));

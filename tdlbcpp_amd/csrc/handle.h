@@ -79,11 +79,25 @@ inline void set_q_geometry(Grid& g, size_t ssize) {
     g.qsize = (cells + align - 1) / align * align;
 }
 
+// Workgroups of the list kernels and, where the LDS does not hold a plane's, their marks in
+// HBM: for fewer workgroups (more planes for each) where memory is short.
+inline int reserve_marks(const Grid& g, uint32_t** marks, int* blocks) {
+    const size_t each = list_marks_bytes(g, blocks);
+    if (each == 0) return TDLB_OK;
+    for (;; *blocks /= 2) {
+        if (*blocks < 1) return fail(TDLB_ERR_NOMEM, "IB list marks");
+        if (hipMalloc((void**)marks, each * (size_t)*blocks) == hipSuccess) return TDLB_OK;
+        *marks = nullptr;
+        (void)hipGetLastError();  // not the next launch's
+    }
+}
+
 // Buffers of the per-call forcing, as large as its longest list so far.
 struct ListBuffers {
     tdlb_ib_point* raw = nullptr;  // the caller's points
     int64_t* list = nullptr;       // positions, plane by plane
-    uint32_t* marks = nullptr;     // planes of marks, for grids whose plane the LDS does not hold
+    uint32_t* marks = nullptr;     // reserve_marks
+    int blocks = 0;                // workgroups
     int64_t cap = 0;
     void release() {
         for (void* p : {(void*)raw, (void*)list, (void*)marks})
@@ -91,9 +105,10 @@ struct ListBuffers {
         raw = nullptr;
         list = nullptr;
         marks = nullptr;
+        blocks = 0;
         cap = 0;
     }
-    int reserve(int64_t n, size_t marks_bytes) {
+    int reserve(int64_t n, const Grid& g) {
         if (n > cap) {
             const int64_t c = std::max<int64_t>(n, 256);
             for (void** p : {(void**)&raw, (void**)&list}) {
@@ -106,11 +121,7 @@ struct ListBuffers {
                 return fail(TDLB_ERR_NOMEM, "IB list buffers");
             cap = c;
         }
-        if (n > 0 && marks_bytes > 0 && !marks && hipMalloc((void**)&marks, marks_bytes) != hipSuccess) {
-            marks = nullptr;
-            return fail(TDLB_ERR_NOMEM, "IB list marks");
-        }
-        return TDLB_OK;
+        return n > 0 && blocks == 0 ? reserve_marks(g, &marks, &blocks) : TDLB_OK;
     }
 };
 

@@ -108,18 +108,18 @@ hipError_t launch_force_prepare(int prec, const PointsDev& p, int64_t begin, int
 // n points into arrays p (cell indices with the ghost offset), and next = base (words)
 hipError_t launch_list_unpack(int prec, const tdlb_ib_point* in, int64_t n, int ghost, const PointsDev& p,
                               const uint64_t* base, uint64_t* next, uint64_t words, hipStream_t s);
-// Bytes of the marks array launch_list_planes needs in HBM (0: a plane's marks fit
-// the LDS), and its workgroups.
+// Workgroups of the list kernels, a plane each at a time, and the bytes of a plane's marks
+// that each needs in HBM (0: the LDS holds them).  Fewer workgroups do as well.
 constexpr size_t kListLdsBytes = 152 * 1024;  // of a CU's 160 KB
 size_t list_marks_bytes(const Grid& g, int* blocks);
 // Level of every point of a list within its j plane (i, j, k of p): one more than the
 // highest level of an earlier point of the list that shares a stencil cell.
-hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint32_t* marks, int32_t* lev,
+hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint32_t* marks, int blocks, int32_t* lev,
                               const Grid& g, hipStream_t s);
 // The forcing of the list in its order; list: room for n positions.
 hipError_t launch_list_planes(int prec, int streaming, int even, const PointsDev& p, int64_t n, int64_t* list,
-                              uint32_t* marks, const void* Q, void* F, const uint64_t* prev, uint64_t* next,
-                              const Grid& g, double alfa, double beta, float rho0, hipStream_t s);
+                              uint32_t* marks, int blocks, const void* Q, void* F, const uint64_t* prev,
+                              uint64_t* next, const Grid& g, double alfa, double beta, float rho0, hipStream_t s);
 
 // ---- IB forcing of a bound tank by j planes.  Stencils span i and k at the
 // point's j, so points of different planes never share a cell and each plane

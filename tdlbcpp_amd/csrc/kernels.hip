@@ -2474,17 +2474,16 @@ size_t list_marks_bytes(const Grid& g, int* blocks) {
     const size_t plane = (size_t)g.xg1 * g.zg1 * sizeof(uint32_t);
     const bool lds = plane <= kListLdsBytes;
     // a workgroup per plane; with marks in HBM at most one per CU
-    const int n = lds ? g.yg1 : std::min(g.yg1, 256);
-    if (blocks) *blocks = n;
-    return lds ? 0 : plane * (size_t)n;
+    *blocks = lds ? g.yg1 : std::min(g.yg1, 256);
+    return lds ? 0 : plane;
 }
 
-hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint32_t* marks, int32_t* lev,
+hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint32_t* marks, int blocks, int32_t* lev,
                               const Grid& g, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    int blocks = 0;
-    const size_t hbm = list_marks_bytes(g, &blocks);
-    if ((hbm != 0) != (marks != nullptr)) return hipErrorInvalidValue;
+    int most = 0;
+    const size_t hbm = list_marks_bytes(g, &most);
+    if ((hbm != 0) != (marks != nullptr) || blocks < 1 || blocks > most) return hipErrorInvalidValue;
     const uint32_t lds = hbm ? 0u : (uint32_t)((size_t)g.xg1 * g.zg1 * sizeof(uint32_t));
     auto* k = hbm ? &k_list_levels<false> : &k_list_levels<true>;
     if (lds > 64 * 1024) {
@@ -2497,12 +2496,12 @@ hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint
 }
 
 hipError_t launch_list_planes(int prec, int streaming, int even, const PointsDev& p, int64_t n, int64_t* list,
-                              uint32_t* marks, const void* Q, void* F, const uint64_t* prev, uint64_t* next,
-                              const Grid& g, double alfa, double beta, float rho0, hipStream_t s) {
+                              uint32_t* marks, int blocks, const void* Q, void* F, const uint64_t* prev,
+                              uint64_t* next, const Grid& g, double alfa, double beta, float rho0, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    int blocks = 0;
-    const size_t hbm = list_marks_bytes(g, &blocks);
-    if ((hbm != 0) != (marks != nullptr)) return hipErrorInvalidValue;
+    int most = 0;
+    const size_t hbm = list_marks_bytes(g, &most);
+    if ((hbm != 0) != (marks != nullptr) || blocks < 1 || blocks > most) return hipErrorInvalidValue;
     const uint32_t lds = hbm ? 0u : (uint32_t)((size_t)g.xg1 * g.zg1 * sizeof(uint32_t));
     auto go = [&](auto pr, auto Sc, auto Ec) -> hipError_t {
         using PR = decltype(pr);

@@ -250,16 +250,16 @@ hipError_t launch_list_unpack(int, const tdlb_ib_point*, int64_t, int, const Poi
 size_t list_marks_bytes(const Grid& g, int* blocks) {
     const size_t plane = (size_t)g.xg1 * g.zg1 * sizeof(uint32_t);
     const bool lds = plane <= kListLdsBytes;
-    const int n = lds ? g.yg1 : std::min(g.yg1, 256);
-    if (blocks) *blocks = n;
-    return lds ? 0 : plane * (size_t)n;
+    *blocks = lds ? g.yg1 : std::min(g.yg1, 256);
+    return lds ? 0 : plane;
 }
-hipError_t launch_list_levels(const PointsDev&, int64_t, int64_t*, uint32_t*, int32_t*, const Grid&, hipStream_t) {
-    return launched();
+hipError_t launch_list_levels(const PointsDev&, int64_t, int64_t*, uint32_t*, int blocks, int32_t*, const Grid&,
+                              hipStream_t) {
+    return blocks < 1 ? hipErrorInvalidValue : launched();
 }
-hipError_t launch_list_planes(int, int, int, const PointsDev&, int64_t, int64_t*, uint32_t*, const void*, void*,
-                              const uint64_t*, uint64_t*, const Grid&, double, double, float, hipStream_t) {
-    return launched();
+hipError_t launch_list_planes(int, int, int, const PointsDev&, int64_t, int64_t*, uint32_t*, int blocks, const void*,
+                              void*, const uint64_t*, uint64_t*, const Grid&, double, double, float, hipStream_t) {
+    return blocks < 1 ? hipErrorInvalidValue : launched();
 }
 hipError_t launch_force_gather(int, int, int, int, const ForceGeom&, const BladeStep&, const GatherBlocks&,
                                const void*, void*, const uint64_t*, uint64_t*, const uint64_t*, const Grid&, float,

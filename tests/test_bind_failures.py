@@ -56,3 +56,47 @@ def test_refused_rebind_keeps_the_earlier_geometry(host_library):  # noqa: F811
     assert cu.forcing_info() == info
     cu.close()
     """)
+
+
+def test_marks_of_large_planes_take_what_memory_there_is(host_library):  # noqa: F811
+    """A plane beyond the LDS has its marks in HBM, a plane a workgroup: with little memory left a bind and a
+    forcing call run with fewer workgroups, and with no room for one plane they are TDLB_ERR_NOMEM."""
+    host_library("""
+    def grid():
+        cu = td.ComputeUnit(220, 60, 220)
+        cu.initialise(1.0)
+        return cu
+    plane = 220 * 220 * 4
+    rp = td.rushton_defaults(60)
+    cu = grid()
+    L.fake_reset_peak()
+    start = L.fake_live()
+    cu.bind_rushton(rp)
+    tank_bytes = L.fake_live() - start        # what stays
+    assert L.fake_peak() - start > 60 * plane
+    n_static = cu.forcing_info()[0]
+    pts = td.rushton_generate(rp, td.GEOM_FIXED)
+    cu.forcing(pts, 0.97, 1.9)
+    assert L.fake_live() - start > tank_bytes + 60 * plane
+    cu.close()
+    assert tank_bytes < 45 * plane
+    for room, ok in ((20 * plane, True), (plane + 100, True), (plane - 1000, False)):
+        cu = grid()
+        # what stays and the transients of its tables; or the list's positions, indices and levels
+        few = n_static * 24 + room
+        L.fake_limit(L.fake_live() + (max(few, tank_bytes + n_static * 36 + cu.xg * cu.yg * 32) if ok else few))
+        rc = L.tdlb_cu_bind_rushton(cu._h, ctypes.byref(rp), 1, 0.0, 0.97, 1.9)
+        L.fake_limit(1 << 40)
+        assert rc == (0 if ok else NOMEM), (room, rc)
+        cu.close()
+        cu = grid()
+        L.fake_limit(L.fake_live() + len(pts) * (64 + 8 + 12 + 20) + room)
+        p = np.ascontiguousarray(pts)
+        for _ in range(2):
+            rc = L.tdlb_cu_forcing(cu._h, p.ctypes.data, len(p), 0.97, 1.9)
+            assert rc == (0 if ok else NOMEM), (room, rc)
+        L.fake_limit(1 << 40)
+        cu.forcing(pts, 0.97, 1.9)
+        cu.close()
+        assert L.fake_live() == 0
+    """)
