@@ -75,9 +75,15 @@ struct tdlb_server {
 
 namespace {
 
-// bytes a tank holds on the device: lattices, F, Nu, O and the masks, plus 10 %
-// for the IB lists, level tables and caches
-size_t footprint(const tdlb_server* s, int64_t edge) {
+// Bytes of a tank of this edge: `lattice`, its lattices, F, Nu, O and the masks plus
+// 10 %, which is what a request may ask for at most, and `all`, what admission reserves
+// for it, with everything that its forcing holds.  The generator's default tank has at
+// most 3.75 edge^2 static points and 12.6 edge^2 of their stencil cells, and 0.17 edge^2
+// blade points (12^3 to 320^3; the first two grow, the last falls with the edge).
+struct Footprint {
+    size_t lattice, all;
+};
+Footprint footprint(const tdlb_server* s, int64_t edge) {
     const size_t n = (size_t)(edge + 2) * (edge + 2) * (edge + 2);
     const size_t pop = s->prec == TDLB_PREC_F64 ? 8 : s->prec == TDLB_PREC_F32 ? 4 : 2;
     const size_t t = s->prec == TDLB_PREC_F64 ? 8 : 4;
@@ -92,7 +98,18 @@ size_t footprint(const tdlb_server* s, int64_t edge) {
     set_q_geometry(g, pop);
     const size_t qcells = (size_t)g.qsize;
     const size_t masks = 5 * (size_t)zg * zg * ((zg + 63) / 64) * 8;
-    return (size_t)((double)(nq * 18 * pop * qcells + n * (3 * t + (pop == 2 ? 2 : t) + 1) + masks) * 1.10);
+    const size_t arrays = nq * 18 * pop * qcells + n * (3 * t + (pop == 2 ? 2 : t) + 1) + masks;
+    const double e2 = (double)edge * (double)edge;
+    const size_t row = t == 4 ? sizeof(ForceRow<float>) : sizeof(ForceRow<double>);
+    const double points = 3 * 4 + 5 * t + 3 * row;  // of either kind
+    const double forcing = 3.75 * e2 * (points + 9 * 4) +       // and a static point's positions, while it is bound
+                           12.6 * e2 * (4 + 4 * t + 4 * t) +    // cells, moments, force values beyond the LDS
+                           0.17 * e2 * (points + 9 * 4 * t) +   // blades and their moments
+                           (double)edge * 512;                  // levels and tasks of the planes
+    // the sums' partials, the batch's tables, small lists' least sizes
+    const size_t fixed = (size_t)384 << 10;
+    const size_t lattice = (size_t)((double)arrays * 1.10);
+    return {lattice, std::max(lattice, arrays + (size_t)forcing + fixed)};
 }
 
 // The tank of a request: FlowParams as main.cpp leaves them (nu from
@@ -242,8 +259,9 @@ int tdlb_server_submit(tdlb_server_t s, const tdlb_tank_request* req, int64_t* t
     j->ticket = s->next_ticket++;
     j->req = *req;
     j->submit_s = s->now();
-    j->footprint = footprint(s, req->edge);
-    if ((double)j->footprint > s->budget) return fail(TDLB_ERR_NOMEM, "request larger than the HBM budget");
+    const Footprint f = footprint(s, req->edge);
+    j->footprint = f.all;
+    if ((double)f.lattice > s->budget) return fail(TDLB_ERR_NOMEM, "request larger than the HBM budget");
     if (ticket) *ticket = j->ticket;
     s->queue.push_back(std::move(j));
     return TDLB_OK;
@@ -258,7 +276,9 @@ int tdlb_server_tick(tdlb_server_t s, int64_t* resident, int64_t* queued, int64_
         auto admitted = [&]() {
             return (int64_t)(s->running.size() + s->prepared.size()) + s->preparing;
         };
-        while (!s->queue.empty() && (double)(s->reserved + s->queue.front()->footprint) <= s->budget &&
+        // a tank alone is always admitted (its lattice fitted the budget when it was submitted)
+        while (!s->queue.empty() &&
+               (s->reserved == 0 || (double)(s->reserved + s->queue.front()->footprint) <= s->budget) &&
                (s->max_resident == 0 || admitted() < s->max_resident)) {
             std::unique_ptr<Job> j = std::move(s->queue.front());
             s->queue.pop_front();
