@@ -203,7 +203,8 @@ int tdlb_cu_run(tdlb_cu_t cu, int64_t nsteps, uint64_t* step, double* angle);
 int tdlb_cu_rotating_points(tdlb_cu_t cu, tdlb_ib_point* out, int64_t cap, int64_t* n);
 /* getExternalPoints mask computed on the device (xg*yg*zg bytes) */
 int tdlb_cu_solid_mask(tdlb_cu_t cu, uint8_t* out, size_t bytes);
-/* number of IB points and forcing levels of the bound geometry */
+/* number of IB points of the bound geometry, and the levels that its forcing runs one
+ * after the other: the most static levels of a plane, and the blade levels */
 int tdlb_cu_forcing_info(tdlb_cu_t cu, int64_t* n_static, int64_t* n_rotating, int64_t* n_levels);
 /* 1 when tdlb_cu_run advances this bound tank with the one-launch step (no
  * counterpart in the reference; opt-in: the environment variable TDLB_PIPE=1
@@ -309,7 +310,8 @@ int tdlb_batch_remove(tdlb_batch_t b, tdlb_cu_t cu);
 int tdlb_batch_run(tdlb_batch_t b, int64_t nsteps, int64_t* steps_run);
 /* a member's RunningParams and remaining budget */
 int tdlb_batch_member(tdlb_batch_t b, tdlb_cu_t cu, uint64_t* step, double* angle, int64_t* remaining);
-/* members, kernel launches per step of the last run, and each member's tile (0 row, 1 plane, 2 flat) */
+/* members, kernel launches of a step (recorded alone: a graph of several advances the
+ * members' state once), and each member's tile (0 row, 1 plane, 2 flat) */
 int tdlb_batch_info(tdlb_batch_t b, int64_t* n_members, int64_t* launches_per_step, int32_t* tiles, int64_t cap);
 /* the fused kernel's block size of the last run, the steps one graph replay
  * advances and the workgroup size of the forcing levels (chosen from the members'

@@ -384,7 +384,7 @@ std::vector<uint8_t> plane_parts(const tdlb_cu* cu, const std::vector<tdlb_ib_po
 // tasks are ordered by an estimate of their duration, longest first, so the
 // disk plane starts at once.
 int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const BladeEnum& be, int64_t blade_j0,
-                    std::vector<int64_t>& order, IndexedSet& set) {
+                    int32_t blade_levels, std::vector<int64_t>& order, IndexedSet& set) {
     set.release();
     const int64_t n = (int64_t)stat.size();
     const int64_t gh = cu->prm.ghost;
@@ -396,7 +396,6 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
     std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) {
         return stat[a].j != stat[b].j ? stat[a].j < stat[b].j : part[a] != part[b] ? part[a] < part[b] : lev[a] < lev[b];
     });
-    const int n_classes = be.n_blades > 0 ? 5 * be.n_bcol : 0;
     std::vector<int32_t> widest;  // points of the largest level of each plane
     std::vector<PlaneDesc> planes;
     std::vector<double> cost;
@@ -413,7 +412,7 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
         const uint8_t pt = (uint8_t)(jp & 1);
         int64_t a1 = a0;
         while (a1 < n && stat[order[a1]].j + gh == j && part[order[a1]] == pt) a1++;
-        const bool blades = pt == 0 && n_classes > 0 && j >= blade_j0 && j < blade_j0 + be.n_planes;
+        const bool blades = pt == 0 && blade_levels > 0 && j >= blade_j0 && j < blade_j0 + be.n_planes;
         if (a1 == a0 && !blades) {
             a0 = a1;
             continue;
@@ -450,7 +449,7 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
         planes.push_back(pd);
         widest.push_back((int32_t)wide);
         // about 1 us a level, 2 us a blade level, and the copies of cells and passes
-        cost.push_back(nl + 2.0 * (blades ? n_classes : 0) + (double)(a1 - a0) / 256.0 +
+        cost.push_back(nl + 2.0 * (blades ? blade_levels : 0) + (double)(a1 - a0) / 256.0 +
                        (double)(pd.cell_end - pd.cell_begin) / 1024.0);
         a0 = a1;
     }
@@ -1246,21 +1245,8 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     cu->pipe = false;
     cu->n_static = (int64_t)stat.size();
     cu->n_rot = (int64_t)rot.size();
-    cu->n_blade_classes = cu->n_rot > 0 ? 5 * be.n_bcol : 0;
     cu->rp = *p;
     cu->blade_wraps = wraps;
-    std::vector<int64_t> order;
-    CHK(build_plane_set(cu, stat, be, p->blade_plane_lo + cu->prm.ghost, order, cu->static_set));
-    HostPoints hs;
-    to_host_points(cu, stat.data(), order, hs);
-    CHK(cu->pts.reserve(cu->n_static + cu->n_rot, cu->tsize));
-    CHK(upload_points(cu, cu->pts, 0, hs));
-    CHK(build_rows(cu));
-    if (cu->rot_cache) (void)hipFree(cu->rot_cache);
-    cu->rot_cache = nullptr;
-    if (cu->n_rot > 0 && hipMalloc(&cu->rot_cache, (size_t)cu->n_rot * 9 * 4 * cu->tsize) != hipSuccess)
-        return fail(TDLB_ERR_NOMEM, "blade moment cache");
-
     cu->blade.n_blades = p->n_blades;
     cu->blade.n_bcol = be.n_bcol;
     cu->blade.j_lo = (int32_t)p->blade_plane_lo;
@@ -1271,6 +1257,18 @@ int tdlb_cu_bind_rushton(tdlb_cu_t cu, const tdlb_rushton_params* p, uint64_t st
     cu->blade.cz = p->center_z;
     cu->blade.ghost = (int32_t)cu->prm.ghost;
     cu->blade.merged = !wraps && blades_apart(p->n_blades, p->blade_inner_radius) ? 1 : 0;
+    cu->n_blade_levels = cu->n_rot > 0 ? blade_level_count(be, cu->blade.merged != 0) : 0;
+    std::vector<int64_t> order;
+    CHK(build_plane_set(cu, stat, be, p->blade_plane_lo + cu->prm.ghost, cu->n_blade_levels, order, cu->static_set));
+    HostPoints hs;
+    to_host_points(cu, stat.data(), order, hs);
+    CHK(cu->pts.reserve(cu->n_static + cu->n_rot, cu->tsize));
+    CHK(upload_points(cu, cu->pts, 0, hs));
+    CHK(build_rows(cu));
+    if (cu->rot_cache) (void)hipFree(cu->rot_cache);
+    cu->rot_cache = nullptr;
+    if (cu->n_rot > 0 && hipMalloc(&cu->rot_cache, (size_t)cu->n_rot * 9 * 4 * cu->tsize) != hipSuccess)
+        return fail(TDLB_ERR_NOMEM, "blade moment cache");
 
     // static occupancy bits: run the prepare kernel on an empty mask
     if (!cu->static_bits && hipMalloc((void**)&cu->static_bits, cu->mask_bytes()) != hipSuccess)
@@ -1663,7 +1661,7 @@ int tdlb_cu_forcing_info(tdlb_cu_t cu, int64_t* n_static, int64_t* n_rotating, i
     if (!cu) return fail(TDLB_ERR_INVALID, "null handle");
     if (n_static) *n_static = cu->n_static;
     if (n_rotating) *n_rotating = cu->n_rot;
-    if (n_levels) *n_levels = (int64_t)cu->static_set.max_levels + cu->n_blade_classes;
+    if (n_levels) *n_levels = (int64_t)cu->static_set.max_levels + cu->n_blade_levels;
     return TDLB_OK;
 }
 

@@ -230,7 +230,7 @@ struct tdlb_cu {
     IndexedSet static_set;               // stencil cells of the static points
     void* rot_cache = nullptr;           // 9 moment entries per blade point
     int64_t n_static = 0, n_rot = 0;
-    int32_t n_blade_classes = 0;         // blade colour classes of the generated list
+    int32_t n_blade_levels = 0;          // blade levels of a plane
     BladeLayout blade{};
     double alfa = 0.97, beta = 1.9;
 

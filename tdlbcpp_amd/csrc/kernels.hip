@@ -1268,7 +1268,7 @@ __device__ __forceinline__ int level_slot(const BladeLayout& bl, int b, int r) {
 __device__ __forceinline__ int blade_plane(const ForceGeom& fg, int j, int& nlev) {
     const BladeLayout& bl = fg.blade;
     const int bp = j - bl.ghost - bl.j_lo;
-    nlev = (bl.n_blades > 0 && fg.n_rot > 0 && bp >= 0 && bp < bl.n_planes) ? radial_classes(bl) * (bl.merged ? 1 : bl.n_bcol) : 0;
+    nlev = (bl.n_blades > 0 && fg.n_rot > 0 && bp >= 0 && bp < bl.n_planes) ? blade_level_count(blade_enum_of(bl), bl.merged != 0) : 0;
     return bp;
 }
 

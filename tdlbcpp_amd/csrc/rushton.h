@@ -67,6 +67,12 @@ TDLB_HD inline bool blades_apart(int32_t n_blades, double r_inner) {
     return 2.0 * r_inner * sin(3.14159265358979323846 / n_blades) >= 3.0 * 1.4142135623730951 + 1e-9;
 }
 
+// Levels that the blade points of a plane take: one per radial class with points, or per
+// blade colour and radial class where blades are not merged.
+TDLB_HD inline int32_t blade_level_count(const BladeEnum& e, bool merged) {
+    return (e.n_radial < 5 ? e.n_radial : 5) * (merged ? 1 : e.n_bcol);
+}
+
 // Number of blade points of colour class c (c = bcol*5 + rmod).
 TDLB_HD inline int64_t blade_class_size(const BladeEnum& e, int c) {
     int bcol = c / 5, rmod = c % 5;
