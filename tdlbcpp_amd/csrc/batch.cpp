@@ -29,6 +29,7 @@
 #include "../../include/tdlb.h"
 #include "handle.h"
 #include "kernels.h"
+#include "readback.h"
 #include "rushton.h"
 
 namespace {
@@ -480,6 +481,7 @@ int tdlb_batch_create(int32_t precision, int32_t layout, int32_t streaming, int3
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, b->device) == hipSuccess && ncu > 0)
         b->n_cu = ncu;
+    readback_handle(1);
     *out = b;
     return TDLB_OK;
 }
@@ -495,6 +497,7 @@ int tdlb_batch_destroy(tdlb_batch_t b) {
     b->d_steps.release();
     b->d_bm.release();
     (void)hipStreamDestroy(b->stream);
+    readback_handle(-1);
     delete b;
     return TDLB_OK;
 }

@@ -11,7 +11,7 @@
 //
 // The pinned buffers are kept between calls (fresh ones fault page by page on the
 // host's first reads, at 2 GB/s): at most kMaxRings of each of two sizes, shared by
-// all handles and threads, given back with the last handle.  A caller that finds
+// all handles and threads, given back with the last handle or batch.  A caller that finds
 // all of its size in use waits for one; where pinned memory is not to be had, pieces
 // are formed in device memory and copied from there.  No C++ exception leaves here:
 // fewer threads do the work where more are not to be had.
@@ -44,8 +44,8 @@ constexpr int kSmallReads = 4;                      // the small buffer from the
 constexpr size_t kLargeRead = (size_t)12 << 20;     // the large one for a result of this size
 constexpr size_t kLargeBytes = (size_t)64 << 20;    // or from this many bytes of larger ones on
 // Arrays that lie in device memory as they are come by a plain copy up to here: O of
-// 30^3 11 us (through a buffer 19), of 100^3 (1.1 MB) 68 (80), Nu of 100^3 (4.2 MB) 240 (205).
-constexpr size_t kPlainArray = (size_t)2 << 20;
+// 30^3 11 us (through a buffer 19), of 60^3 (0.24 MB) 21 (29), of 80^3 (0.55 MB) 35 either way.
+constexpr size_t kPlainArray = (size_t)1 << 19;
 
 std::mutex g_mu;
 std::condition_variable g_cv;
@@ -174,16 +174,16 @@ hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t
     std::atomic<int> failed{hipSuccess};
     auto work = [&](int t) {
         hipError_t r = hipSetDevice(device);
-        hipEvent_t done = nullptr;
-        if (r == hipSuccess) r = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+        hipEvent_t done = nullptr;  // of this thread's pieces among those of several
+        if (r == hipSuccess && most > 1) r = hipEventCreateWithFlags(&done, hipEventDisableTiming);
         char* buf = static_cast<char*>(ring) + (size_t)t * slot;
         while (r == hipSuccess && failed.load() == hipSuccess) {
             const size_t begin = next.fetch_add(part);
             if (begin >= bytes) break;
             const size_t end = std::min(bytes, begin + part);
             r = piece(buf, begin, end, s);
-            if (r == hipSuccess) r = hipEventRecord(done, s);
-            if (r == hipSuccess) r = hipEventSynchronize(done);
+            if (r == hipSuccess && done) r = hipEventRecord(done, s);
+            if (r == hipSuccess) r = done ? hipEventSynchronize(done) : hipStreamSynchronize(s);
             if (r == hipSuccess) std::memcpy(static_cast<char*>(host) + begin, buf, end - begin);
         }
         if (done) (void)hipEventDestroy(done);

@@ -41,7 +41,8 @@ constexpr size_t kStageBytes = (size_t)16 << 20;
 void* take_stage(int device, size_t* bytes);
 void give_stage(int device, void* stage, size_t bytes);
 
-// A handle came or went: what is kept between calls is given back with the last one.
+// A handle or a batch (a server's too) came or went: what is kept between calls is given
+// back with the last one.
 void readback_handle(int change);
 
 }  // namespace tdlb

@@ -90,7 +90,8 @@ def test_pinned_memory_is_made_where_it_pays(host_library):  # noqa: F811
         reads(80, 9, field, 1)
         reads(96, 1, field, 1)     # 14 MB
         reads(30, 20, lambda cu: cu.get(td.FIELD_O), 0)
-        reads(60, 20, lambda cu: cu.get(td.FIELD_NU), 0)
+        reads(60, 20, lambda cu: cu.get(td.FIELD_O), 0)
+        reads(60, 20, lambda cu: cu.get(td.FIELD_NU), 1)
     a, b = tank(36, bind=False), tank(36, bind=False)
     for _ in range(4):
         a.macroscopic()
@@ -98,6 +99,23 @@ def test_pinned_memory_is_made_where_it_pays(host_library):  # noqa: F811
     assert L.fake_pinned() == 1    # the other handle's reads find it
     b.macroscopic()
     b.close()
+    assert L.fake_pinned() == 0 and L.fake_live() == 0
+    """)
+
+
+def test_a_server_keeps_the_buffers_between_its_tanks(host_library):  # noqa: F811
+    """Tanks of a server come and go; its reads make the pinned buffers once, and they go with the server."""
+    host_library("""
+    s = td.Server(td.PREC_F16, tick_steps=50, keep_handles=True)
+    for n in range(3):
+        t = s.submit(100, 0.1, 5000.0, 20)
+        while not s.poll():
+            s.tick()
+        cu = s.take(t, 100)
+        cu.macroscopic()
+        cu.close()
+        assert L.fake_pinned() == 1 and L.fake_pinned_mallocs() == 1
+    s.close()
     assert L.fake_pinned() == 0 and L.fake_live() == 0
     """)
 
