@@ -2478,6 +2478,12 @@ size_t list_marks_bytes(const Grid& g, int* blocks) {
     return lds ? 0 : plane;
 }
 
+// A launch of a list kernel may ask for more than 64 KB of LDS: the same most for every
+// grid, so that threads with planes of different sizes never lower another's.
+static hipError_t allow_list_lds(const void* kernel) {
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kListLdsBytes);
+}
+
 hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint32_t* marks, int blocks, int32_t* lev,
                               const Grid& g, hipStream_t s) {
     if (n <= 0) return hipSuccess;
@@ -2487,8 +2493,7 @@ hipError_t launch_list_levels(const PointsDev& p, int64_t n, int64_t* list, uint
     const uint32_t lds = hbm ? 0u : (uint32_t)((size_t)g.xg1 * g.zg1 * sizeof(uint32_t));
     auto* k = hbm ? &k_list_levels<false> : &k_list_levels<true>;
     if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = allow_list_lds(reinterpret_cast<const void*>(k));
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k, dim3((uint32_t)blocks), dim3(kListBlock), lds, s, p, n, list, marks, lev, g);
@@ -2509,8 +2514,7 @@ hipError_t launch_list_planes(int prec, int streaming, int even, const PointsDev
         constexpr int S = decltype(Sc)::value, E = decltype(Ec)::value;
         auto* k = hbm ? &k_list_planes<PR, S, E, false> : &k_list_planes<PR, S, E, true>;
         if (lds > 64 * 1024) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            const hipError_t e = allow_list_lds(reinterpret_cast<const void*>(k));
             if (e != hipSuccess) return e;
         }
         hipLaunchKernelGGL(k, dim3((uint32_t)blocks), dim3(kListBlock), lds, s, p, n, list, marks, (T*)F, (const T*)Q, prev,
