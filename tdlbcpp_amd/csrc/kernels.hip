@@ -909,6 +909,7 @@ constexpr int kListBlock = 512, kListRun = 8;  // lanes, and points a lane looks
 constexpr uint32_t kNoPoint = 0xffffffffu;
 struct ListShared {
     int64_t less[kListBlock / 64];
+    int same[kListBlock / 64];
     int wave[2][kListRun][kListBlock / 64];
 };
 // The points of plane j (pj: the planes of all n) to their part of list, in list order, by the whole workgroup;
@@ -919,14 +920,27 @@ __device__ __forceinline__ uint32_t plane_points(const int32_t* __restrict__ pj,
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the plane's part of the list begins after the points of lower planes
     int64_t less = 0;
+    int same = 0;  // of a lane: whether the plane has points
 #pragma unroll 8
-    for (int64_t q = tid; q < n; q += kListBlock) less += pj[q] < j ? 1 : 0;
+    for (int64_t q = tid; q < n; q += kListBlock) {
+        less += pj[q] < j ? 1 : 0;
+        same |= pj[q] == j ? 1 : 0;
+    }
     for (int o = 32; o > 0; o >>= 1) less += __shfl_down(less, o, 64);
-    if (lane == 0) sh.less[wave] = less;
+    const bool any = __ballot(same) != 0;
+    if (lane == 0) {
+        sh.less[wave] = less;
+        sh.same[wave] = any ? 1 : 0;
+    }
     __syncthreads();
     int64_t first = 0;
-    for (int w = 0; w < kWaves; w++) first += sh.less[w];
+    int points = 0;
+    for (int w = 0; w < kWaves; w++) {
+        first += sh.less[w];
+        points |= sh.same[w];
+    }
     mine = list + first;
+    if (__builtin_amdgcn_readfirstlane(points) == 0) return 0;  // the same for every lane of every wave
     // its points in list order
     uint32_t count = 0;
     int turn = 0;
@@ -2470,11 +2484,15 @@ hipError_t launch_list_unpack(int prec, const tdlb_ib_point* in, int64_t n, int 
     return hipGetLastError();
 }
 
+// At most this many workgroups where the LDS holds the marks: four times what the chip
+// holds at once.  With a workgroup for each of 100,000 planes of 16 x 16 cells and 300
+// points a call took 1.0 ms, most of it for planes without any.
+constexpr int kListBlocks = 4096;
 size_t list_marks_bytes(const Grid& g, int* blocks) {
     const size_t plane = (size_t)g.xg1 * g.zg1 * sizeof(uint32_t);
     const bool lds = plane <= kListLdsBytes;
-    // a workgroup per plane; with marks in HBM at most one per CU
-    *blocks = lds ? g.yg1 : std::min(g.yg1, 256);
+    // a workgroup per plane at a time; with marks in HBM at most one per CU
+    *blocks = std::min(g.yg1, lds ? kListBlocks : 256);
     return lds ? 0 : plane;
 }
 

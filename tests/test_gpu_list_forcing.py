@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 import tdlbcpp_amd as td
-from tests.test_gpu_parity import random_points
+from oracle import oracle as O
+from tests.test_gpu_parity import LAYOUTS, STREAMS, random_points, seeded_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +43,21 @@ def test_threads_with_planes_of_different_sizes():
         t.join()
     for w, g in zip(want, got):
         np.testing.assert_array_equal(g, w)
+
+
+# more planes than workgroups, most of them without points: a few in every so many planes, in the last ones only,
+# in all
+@pytest.mark.parametrize("n,planes", [(300, None), (40, (8990, 9000)), (1, (0, 1)), (30000, None)])
+def test_many_planes_match_oracle(n, planes):
+    shape = (5, 9000, 6)
+    print(f"[gpu case] list of {n} points in {shape}, planes {planes}", flush=True)
+    o, g = seeded_pair(LAYOUTS[0], STREAMS[1], td.PREC_F32, False, shape=shape, seed=3, even=True)
+    rng = np.random.default_rng(n)
+    for _ in range(2):
+        pts = random_points(rng, shape, n)
+        if planes:
+            pts["j"] = rng.integers(planes[0], planes[1], n)
+        o.forcing(pts, 0.97, 1.9)
+        g.forcing(pts, 0.97, 1.9)
+        np.testing.assert_array_equal(g.get(td.FIELD_F), o.get(O.FIELD_F))
+    g.close()
