@@ -988,11 +988,12 @@ static int read_result(tdlb_cu* cu, void* host, size_t bytes, size_t align, cons
 // stream orders a piece's copy after the conversion of the one before.
 static int upload_q(tdlb_cu* cu, const void* host, size_t bytes) {
     size_t piece = 0;
-    void* const stage = take_stage(cu->device, &piece);
+    void* const stage = take_stage(cu->device, bytes, &piece);
     if (!stage) return fail(TDLB_ERR_NOMEM, "upload Q staging");
     hipError_t e = hipSuccess;
-    for (size_t at = 0; at < bytes && e == hipSuccess; at += piece) {
-        const size_t n = std::min(piece, bytes - at);
+    const size_t part = piece / cu->tsize * cu->tsize;
+    for (size_t at = 0; at < bytes && e == hipSuccess; at += part) {
+        const size_t n = std::min(part, bytes - at);
         e = hipMemcpyAsync(stage, (const char*)host + at, n, hipMemcpyHostToDevice, cu->stream);
         if (e == hipSuccess)
             e = launch_q_boundary((int)cu->tsize, cu->blay(), 0, cu->eq(), stage, at / cu->tsize,

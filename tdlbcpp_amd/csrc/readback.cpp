@@ -56,6 +56,8 @@ size_t g_bytes[2] = {0, 0};
 
 constexpr int kStageDevices = 64;  // tdlb_cu_create refuses device ids beyond
 void* g_stage[kStageDevices] = {};
+constexpr int kStageUses = 4;
+int g_stage_uses[kStageDevices] = {};  // without a piece that was kept
 
 // null: no buffer of this size is there, and none can be made or is worth it yet
 void* take_ring(int kind, size_t bytes) {
@@ -87,36 +89,16 @@ void give_ring(int kind, void* ring) {
     g_cv.notify_all();
 }
 
-// Without pinned memory: pieces in device memory, copied from there one after the other.
-hipError_t by_device_pieces(hipStream_t s, char* host, size_t bytes, size_t align, const PieceFn& piece) {
-    size_t part = std::min(bytes, (size_t)1 << 29);
-    void* buf = nullptr;
-    for (;; part /= 2) {
-        if (hipMalloc(&buf, part) == hipSuccess) break;
-        (void)hipGetLastError();
-        if (part / 2 < kMinPiece) return hipErrorOutOfMemory;
-    }
-    part = part / align * align;
-    hipError_t e = hipSuccess;
-    for (size_t begin = 0; begin < bytes && e == hipSuccess; begin += part) {
-        const size_t end = std::min(bytes, begin + part);
-        e = piece(buf, begin, end, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(host + begin, buf, end - begin, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-    }
-    (void)hipFree(buf);
-    return e;
-}
-
 }  // namespace
 
 void readback_handle(int change) {
     std::lock_guard<std::mutex> lk(g_mu);
     g_handles += change;
     if (g_handles > 0) return;
-    for (void*& p : g_stage) {
-        if (p) (void)hipFree(p);
-        p = nullptr;
+    for (int d = 0; d < kStageDevices; d++) {
+        if (g_stage[d]) (void)hipFree(g_stage[d]);
+        g_stage[d] = nullptr;
+        g_stage_uses[d] = 0;
     }
     for (int kind = 0; kind < 2; kind++) {
         for (int a = 0; a < g_n_idle[kind]; a++) (void)hipHostFree(g_idle[kind][a]);
@@ -127,19 +109,21 @@ void readback_handle(int change) {
     }
 }
 
-void* take_stage(int device, size_t* bytes) {
-    *bytes = kStageBytes;
+void* take_stage(int device, size_t want, size_t* bytes) {
     {
         std::lock_guard<std::mutex> lk(g_mu);
         if (void* p = g_stage[device]) {
             g_stage[device] = nullptr;
+            *bytes = kStageBytes;
             return p;
         }
+        *bytes = ++g_stage_uses[device] < kStageUses ? std::min(want, kStageBytes) : kStageBytes;
     }
-    for (; *bytes >= kMinPiece; *bytes /= 2) {
+    for (;; *bytes /= 2) {
         void* p = nullptr;
         if (hipMalloc(&p, *bytes) == hipSuccess) return p;
         (void)hipGetLastError();  // not the next launch's
+        if (*bytes / 2 < kMinPiece) break;
     }
     return nullptr;
 }
@@ -155,6 +139,24 @@ void give_stage(int device, void* stage, size_t bytes) {
     (void)hipFree(stage);
 }
 
+// Without pinned memory: pieces in device memory, copied from there one after the other.
+static hipError_t by_device_pieces(int device, hipStream_t s, char* host, size_t bytes, size_t align,
+                                   const PieceFn& piece) {
+    size_t room = 0;
+    void* const stage = take_stage(device, bytes, &room);
+    if (!stage) return hipErrorOutOfMemory;
+    const size_t part = room / align * align;
+    hipError_t e = hipSuccess;
+    for (size_t begin = 0; begin < bytes && e == hipSuccess; begin += part) {
+        const size_t end = std::min(bytes, begin + part);
+        e = piece(stage, begin, end, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(host + begin, stage, end - begin, hipMemcpyDeviceToHost, s);
+    }
+    const hipError_t done = hipStreamSynchronize(s);
+    give_stage(device, stage, room);
+    return e == hipSuccess ? done : e;
+}
+
 hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece,
                      const void* array) {
     if (bytes == 0) return hipStreamSynchronize(s);
@@ -164,7 +166,7 @@ hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t
         const hipError_t e = hipMemcpyAsync(host, array, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    if (!ring) return by_device_pieces(s, static_cast<char*>(host), bytes, align, piece);
+    if (!ring) return by_device_pieces(device, s, static_cast<char*>(host), bytes, align, piece);
     // a thread per piece in flight; small results take the calling thread only
     const int cpus = std::max(1, (int)std::thread::hardware_concurrency());
     const int most = (int)std::min<size_t>(std::max(1, std::min(kMaxThreads, cpus / 2)), (bytes + kMinPiece - 1) / kMinPiece);

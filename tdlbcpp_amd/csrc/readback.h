@@ -33,12 +33,14 @@ private:
 hipError_t read_back(int device, hipStream_t s, void* host, size_t bytes, size_t align, const PieceFn& piece,
                      const void* array = nullptr);
 
-// A piece of device memory for an upload that is converted on the device, kStageBytes or,
-// where memory is short, less (bytes says how much; null: there is none).  One a device
-// is kept between uploads: allocating and freeing it costs 50 us, a tenth of a 60^3
-// tank's Q.  The caller's work on it has ended when it is given back.
+// Device memory for `want` bytes of data that are converted on the device on their way,
+// piece by piece: kStageBytes, or less where little is wanted or memory is short (bytes says
+// how much; null: there is none).  From the fourth call on one piece a device is kept
+// between calls: allocating and freeing it costs 50 us, a tenth of the upload of a 60^3
+// tank's Q, but more than a small one where a program has a single use for it.  The
+// caller's work on it has ended when it is given back.
 constexpr size_t kStageBytes = (size_t)16 << 20;
-void* take_stage(int device, size_t* bytes);
+void* take_stage(int device, size_t want, size_t* bytes);
 void give_stage(int device, void* stage, size_t bytes);
 
 // A handle or a batch (a server's too) came or went: what is kept between calls is given
