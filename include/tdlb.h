@@ -216,8 +216,9 @@ int tdlb_cu_forcing_info(tdlb_cu_t cu, int64_t* n_static, int64_t* n_rotating, i
 int tdlb_cu_one_launch(tdlb_cu_t cu, int32_t* on);
 /* Phase times of the last one-launch step, in microseconds from its first work
  * item (no counterpart in the reference): for each of the 8 XCDs, when its
- * last row was written, its last forcing gather done and its last forcing
- * level done: us[3 x + 0 .. 2], n >= 24.  Synchronises the handle's stream. */
+ * last row was written and its last forcing gather done: us[3 x + 0], us[3 x + 1],
+ * and us[3 x + 2] as us[3 x + 1] (the forcing levels run in a launch of their own);
+ * n >= 24.  Synchronises the handle's stream. */
 int tdlb_cu_one_launch_phases(tdlb_cu_t cu, double* us, int32_t n);
 /* Kernel timing of the fused path (no counterpart in the reference, which only
  * has wall-clock phase timers, timer.cpp:127-222): while enabled, tdlb_cu_run

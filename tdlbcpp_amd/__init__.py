@@ -399,7 +399,7 @@ class ComputeUnit:
         return bool(v.value)
 
     def one_launch_phases(self):
-        """Per XCD (rows written, forcing gathers done, forcing levels done), in
+        """Per XCD (rows written, forcing gathers done, the latter again), in
         microseconds from the first work item of the last one-launch step."""
         out = (ctypes.c_double * 24)()
         check(lib().tdlb_cu_one_launch_phases(self._h, out, 24))

@@ -33,6 +33,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/tdlb.h"
@@ -294,9 +295,10 @@ int upload_points(tdlb_cu* cu, DevPoints& dp, int64_t offset, const HostPoints& 
 // Workgroup of a tank's levels launch, from all but the few largest planes (the
 // impeller disk's).  lanes: a lane per static cell for the copies in and out,
 // which is more than a quad per point of a level (96^3: 192 lanes 43 us a pass,
-// 1024 lanes 38).  LDS: what holds everything of every plane, at most a CU's (a
-// workgroup's registers leave room for one a CU anyway); what a plane cannot hold
-// there stays in HBM.
+// 1024 lanes 38).  LDS: what holds everything of every plane, at most a CU's; what a
+// plane cannot hold there stays in HBM.  Workgroups of few lanes could share a CU by
+// their registers but not by this LDS, which counts only with more planes than CUs:
+// 96 x 1024 x 96 runs its 1024 planes four to a CU one after the other (a pass 180 us).
 void level_shape(const Grid& g, const std::vector<PlaneDesc>& planes, const std::vector<int32_t>& widest,
                  int64_t blade_points, size_t tsize, IndexedSet& set) {
     if (planes.empty()) return;
@@ -465,7 +467,6 @@ int build_plane_set(tdlb_cu* cu, const std::vector<tdlb_ib_point>& stat, const B
         set.plane_cost[t] = (float)cost[by[t]];
     }
     set.n_cells = (int64_t)cells.size();
-    set.n_points = n;
     set.n_planes = (int32_t)sorted.size();
     set.max_levels = max_levels;
     set.plane_list = sorted;
@@ -526,6 +527,7 @@ int setup_pipe(tdlb_cu* cu) {
     cu->rowcell = nullptr;
     cu->pctr = nullptr;
     const Grid& g = cu->g;
+    // (LAYOUT_IJKL handles are refused as ever; their lattice would do)
     const bool shape = !cu->simple() && cu->prm.layout != TDLB_LAYOUT_IJKL && cu->prm.precision != TDLB_PREC_F64 &&
                        g.xg1 >= 4 && g.yg1 >= 3 * kXcds && g.zg1 >= 64;
     if (!shape || !pipe_device_ok(cu)) return TDLB_OK;
@@ -581,8 +583,8 @@ int pipe_step(tdlb_cu* cu, const BladeStep& st) {
     a.ctr = cu->pctr;
     HIPCHK(launch_zero(cu->pctr, pipe_counter_words(cu->g) * 4, cu->stream));
     const int hint = line_rows_bytes(cu->g, cu->ssize) ? 1 : 0;
-    HIPCHK(launch_eso_pipe(cu->prec(), cu->even ? 1 : 0, hint, a, cu->g, cu->cargs(), cu->rho0, cu->alfa, cu->beta,
-                           0, row_lanes(cu->g), cu->stream));
+    HIPCHK(launch_eso_pipe(cu->prec(), cu->even ? 1 : 0, hint, a, cu->g, cu->cargs(), cu->rho0, 0,
+                           row_lanes(cu->g), cu->stream));
     // the levels read the populations of the next step's collision
     const GatherBlocks gb = gather_blocks(cu->n_rot, 0, 0);
     HIPCHK(launch_force_gather(cu->prec(), cu->prm.streaming, MOMSRC_ESO_POPS, cu->even ? 0 : 1, a.fg, st,

@@ -135,7 +135,7 @@ struct IndexedSet {
     void* fscr = nullptr;  // bound tank: force scratch of planes beyond the LDS
     PlaneDesc* planes = nullptr;
     int64_t* lev_off = nullptr;
-    int64_t n_cells = 0, n_points = 0;
+    int64_t n_cells = 0;
     int32_t n_planes = 0, max_levels = 0;
     int32_t level_lanes = 64, level_lds = 0;  // workgroup of the levels launch
     std::vector<float> plane_cost;       // host: duration estimate of each plane (planes order)
@@ -151,7 +151,7 @@ struct IndexedSet {
         fscr = nullptr;
         planes = nullptr;
         lev_off = nullptr;
-        n_cells = n_points = 0;
+        n_cells = 0;
         n_planes = max_levels = 0;
         plane_cost.clear();
         plane_list.clear();

@@ -1,8 +1,8 @@
 // Host-side launchers of the gfx950 kernels (implemented in kernels.hip).
 // Pointers are device pointers; every launcher enqueues on `s` and returns the
-// launch status.  prec: 0 float, 1 double, 2 fp16 storage, 3 bf16 storage (the
-// last two compute in float and store Nu in their 16-bit format; F and point
-// arrays are float).  Population arrays are LIJK (device.h) whatever the layout at the boundary.
+// launch status.  prec: 0 float, 1 double, 2 fp16, 3 bf16, 4 e3m12 storage (the
+// last three compute in float and store Nu in 16 bits; F and point arrays are
+// float).  Population arrays are LIJK (device.h) whatever the layout at the boundary.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -235,7 +235,7 @@ TDLB_HD inline void pipe_range(int yg1, int x, int& jlo, int& jhi) {
 // prec 0, 2, 3, 4 (float arithmetic); hint: the streaming cache hint of the
 // fused kernel (line_rows); blocks: the persistent grid
 hipError_t launch_eso_pipe(int prec, int even, int hint, const PipeArgs& a, const Grid& g, const CollideArgs& c,
-                           float rho0, double alfa, double beta, uint32_t blocks, uint32_t lanes, hipStream_t s);
+                           float rho0, uint32_t blocks, uint32_t lanes, hipStream_t s);
 // lanes per row block of the stream-collide kernels for this grid (the pipe's block size)
 uint32_t row_lanes(const Grid& g);
 // every k-row of the population planes (stored values of ssize bytes) is whole 128 B lines

@@ -1127,15 +1127,12 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
 // the sequential list order of Forcing.hpp:73-135 within the plane: static
 // levels, then blade levels, passes of a point per quad of lanes with a barrier
 // after every level, bound by the latency of that chain.  Gathering inside the
-// plane's workgroup instead left the gather to one CU per plane (96 of 256 CUs
-// at 96^3: 12 us) and, beyond 256 planes, to rounds of workgroups; a plane with
-// many points then needed several workgroups meeting at barriers in HBM (24^3: 205
-// us).  Whole pass, gather and levels in one -> two launches: 24^3 205 -> 33 us,
-// 60^3 41 -> 29, 96^3 47 -> 37, 192^3 FP64 219 -> 132, 256^3 226 -> 166, 512^3
-// 597 -> 549 (gather 390, 5.1 TB/s of lines; levels 140).  With rows asked for three
-// passes ahead (run_levels): 24^3 33 -> 31 us, 96^3 35 -> 32, 131^3 45 -> 42, 256^3 166
-// -> 158; with the blades' indexes in closed form (blade_group; loops of integer divisions
-// before) and branch-free passes: 24^3 31 -> 27, 60^3 27 -> 25, 96^3 32 -> 30, 131^3 42 -> 40.
+// plane's workgroup instead leaves the gather to one CU per plane (96 of 256 CUs at
+// 96^3) and, beyond 256 planes, to rounds of workgroups, and a plane with many points
+// then needs several workgroups meeting at barriers in HBM.  Whole pass, that form ->
+// this: 24^3 252 -> 27 us, 36^3 69 -> 23, 60^3 Simple 80 -> 25, 96^3 91 -> 30, 131^3 FP16
+// 94 -> 40, 192^3 FP64 274 -> 126, 256^3 290 -> 158, 512^3 633 -> 547 (gather 379: 1.63 GB
+// read and 0.07 written, 4.5 TB/s; levels 166).
 
 // ---- A point of a plane task on a quad of lanes: lane c = 0..2 of the quad
 // takes stencil row k1 = c - 1 (cells s = 3c + m for i1 = m - 1), lane 3 repeats
@@ -1148,8 +1145,7 @@ __global__ __launch_bounds__(kListBlock) void k_list_planes(PointsDev p, int64_t
 // beyond the add's own.  A level is a chain (gather, sums, spread, barrier) of a
 // few hundred lanes, bound by latency: three lanes per point with LDS shuffles
 // and the weights' FP64 square roots in every pass took about 9 us a level,
-// this form 1 us with the plane in LDS.  Whole forcing pass of a tank, FP32:
-// 36^3 68 -> 37 us, 60^3 80 -> 41, 96^3 91 -> 47, 256^3 290 -> 226, 512^3 633 -> 597.
+// this form 0.5 us with the plane in LDS.
 template <int C>
 __device__ __forceinline__ float quad_lane(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), C * 0x55, 0xf, 0xf, true));
@@ -1758,8 +1754,7 @@ constexpr int pipe_waves() { return std::is_same<typename PR::S, float>::value ?
 
 template <typename PR, int EVEN, bool HINT>
 __global__ __launch_bounds__(kRowBlock) __attribute__((amdgpu_waves_per_eu(pipe_waves<PR>(), 8)))
-void k_eso_pipe(PipeArgs a, Grid g, CollideParams<float> P, uint32_t nkb,
-                                                      float rho0, float alfa, float beta) {
+void k_eso_pipe(PipeArgs a, Grid g, CollideParams<float> P, uint32_t nkb, float rho0) {
     using S = typename PR::S;
     constexpr int STREAM = StreamEsotwist;
     constexpr int MS = MOMSRC_ESO_POPS;
@@ -1827,7 +1822,7 @@ void k_eso_pipe(PipeArgs a, Grid g, CollideParams<float> P, uint32_t nkb,
         __syncthreads();
         if (tid == 0 &&
             __hip_atomic_fetch_add(cx + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gathers)
-            tx[2] = tx[3] = (uint64_t)wall_clock64();
+            tx[2] = tx[3] = (uint64_t)wall_clock64();  // the third phase ends with the second: the levels follow in a launch of their own
     };
 
     // the next item is taken while the current one runs (each waits only for earlier items)
@@ -2629,16 +2624,14 @@ uint32_t row_lanes(const Grid& g) {
 }
 
 hipError_t launch_eso_pipe(int prec, int even, int hint, const PipeArgs& a, const Grid& g, const CollideArgs& c,
-                           float rho0, double alfa, double beta, uint32_t blocks, uint32_t lanes, hipStream_t s) {
+                           float rho0, uint32_t blocks, uint32_t lanes, hipStream_t s) {
     uint32_t nkb, nb, bk;
     row_launch(g, nkb, nb, bk, kPipeLanes);
     if (lanes != bk) return hipErrorInvalidValue;
     auto go = [&](auto pr) -> hipError_t {
         using PR = decltype(pr);
         const auto P = to_params<float, typename PR::D>(c);
-#define TDLB_PIPE(E, H)                                                                                         \
-    hipLaunchKernelGGL((k_eso_pipe<PR, E, H>), dim3(blocks), dim3(bk), 0, s, a, g, P, nkb, rho0, (float)alfa,    \
-                       (float)beta)
+#define TDLB_PIPE(E, H) hipLaunchKernelGGL((k_eso_pipe<PR, E, H>), dim3(blocks), dim3(bk), 0, s, a, g, P, nkb, rho0)
         if (blocks == 0) {
             // persistent grid: every workgroup resident at once
             int per_cu = 0, dev = 0;

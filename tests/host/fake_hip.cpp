@@ -271,8 +271,8 @@ hipError_t launch_force_levels(int, const ForceGeom&, void*, uint64_t*, const Gr
     return launched();
 }
 hipError_t allow_level_lds(int) { return launched(); }
-hipError_t launch_eso_pipe(int, int, int, const PipeArgs&, const Grid&, const CollideArgs&, float, double, double,
-                           uint32_t, uint32_t, hipStream_t) { return launched(); }
+hipError_t launch_eso_pipe(int, int, int, const PipeArgs&, const Grid&, const CollideArgs&, float, uint32_t, uint32_t,
+                           hipStream_t) { return launched(); }
 uint32_t row_lanes(const Grid&) { return 256; }
 bool line_rows_bytes(const Grid&, size_t) { return false; }
 int pipe_xcc_check(hipStream_t) { return 1; }
