@@ -744,7 +744,8 @@ __global__ void k_force_prepare(PointsDev p, int64_t begin, int64_t count, T* __
     prepare_point(p, begin + t, F, prev, next, g);
 }
 
-// density and momentum of cell (i,j,k) as the reference's moments() would leave them
+// density and momentum of cell (i,j,k) as the reference's moments() would leave them; 1 <= k <= zg1 for Esotwist,
+// whose homes are found by the pitches of the interior rows
 template <typename PR, int STREAM, int MOMSRC, int EVEN>
 __device__ __forceinline__ void cell_rho_j(const typename PR::S* __restrict__ Q, const Grid& g, int i, int j, int k,
                                            typename PR::T& rho, typename PR::T& jx, typename PR::T& jy,
@@ -2106,7 +2107,19 @@ __global__ void k_vorticity(const typename PR::S* __restrict__ Q, Grid g, int ax
             return;
         }
         T rho, jx, jy, jz;
-        cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, a, b, e, rho, jx, jy, jz, rho0);
+        if (STREAM == StreamEsotwist && MOMSRC == MOMSRC_STORED && e == 0) {
+            // a ghost cell at k = 0 has its homes in the side region too, whose rows lie closer than the interior's
+            T m[4];
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                static_assert(!twist_dz(0) && !twist_dz(1) && !twist_dz(2) && !twist_dz(3), "density and momentum stay at k");
+                const int a2 = twist_dx(d) ? (a == g.xg1 ? 1 : a + 1) : a, b2 = twist_dy(d) ? (b == g.yg1 ? 1 : b + 1) : b;
+                m[d] = (T)Q[qaddr(g, qcell(g, a2, b2, 0), EVEN ? d : opposite(d))];
+            }
+            rho = m[0]; jx = m[1]; jy = m[2]; jz = m[3];
+        } else {
+            cell_rho_j<PR, STREAM, MOMSRC, EVEN>(Q, g, a, b, e, rho, jx, jy, jz, rho0);
+        }
         ux = jx / rho;
         uy = jy / rho;
         uz = jz / rho;
