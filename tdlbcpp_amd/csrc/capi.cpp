@@ -46,6 +46,7 @@ namespace tdlb {
 namespace detail {
 thread_local std::string g_err;
 int fail(int code, const std::string& msg) {
+    if (code == TDLB_ERR_NOMEM) (void)hipGetLastError();  // the failed allocation's, not the next launch's
     g_err = msg;
     return code;
 }

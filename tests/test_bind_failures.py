@@ -19,7 +19,6 @@ def test_failed_rebind_leaves_the_handle_unbound(host_library):  # noqa: F811
         L.fake_fail_malloc(n)
         rc = L.tdlb_cu_bind_rushton(cu._h, ctypes.byref(rp), 1, 0.0, 0.97, 1.9)
         L.fake_fail_malloc(-1)
-        L.hipGetLastError()
         if rc != 0:
             assert rc == NOMEM, rc
             before = L.fake_gathers()
@@ -99,4 +98,38 @@ def test_marks_of_large_planes_take_what_memory_there_is(host_library):  # noqa:
         cu.forcing(pts, 0.97, 1.9)
         cu.close()
         assert L.fake_live() == 0
+    """)
+
+
+def test_a_call_after_an_allocation_that_failed(host_library):  # noqa: F811
+    """TDLB_ERR_NOMEM is the error of its own call: the next call on the thread, with memory again, succeeds."""
+    host_library("""
+    pts = np.ascontiguousarray(td.rushton_generate(td.rushton_defaults(24), td.GEOM_FIXED))
+    rp = td.rushton_defaults(24)
+    out = (ctypes.c_double * 8)()
+    for n in range(3):
+        cu, half = tank(24, bind=False), tank(24, td.PREC_F16, bind=False)
+        batch = td.Batch(td.PREC_F32)
+        nu = np.zeros(half.size, dtype=np.float32)
+        solid = np.zeros(cu.size, dtype=np.uint8)
+        bound = tank(24)
+        def calls():
+            yield L.tdlb_cu_forcing(cu._h, pts.ctypes.data, len(pts), 0.97, 1.9)
+            yield L.tdlb_cu_reductions(cu._h, out)
+            yield L.tdlb_cu_upload(half._h, td.FIELD_NU, nu.ctypes.data, nu.nbytes)
+            yield L.tdlb_cu_solid_mask(bound._h, solid.ctypes.data, solid.nbytes)
+            yield L.tdlb_batch_add(batch._b, bound._h, 1, 0.0, 5)
+            yield L.tdlb_cu_bind_rushton(cu._h, ctypes.byref(rp), 1, 0.0, 0.97, 1.9)
+        it = calls()
+        while True:
+            L.fake_fail_malloc(n)
+            rc = next(it, None)
+            L.fake_fail_malloc(-1)
+            if rc is None:
+                break
+            assert rc in (0, NOMEM), rc
+            assert L.tdlb_cu_collision(cu._h) == 0, rc
+        batch.close()
+        for c in (cu, half, bound):
+            c.close()
     """)
